@@ -9,6 +9,7 @@
 
 #include "../../include/tplr_hip.h"
 #include "tplr_device.h"
+#include "tplr_launch.h"
 
 namespace tplr {
 
@@ -340,45 +341,6 @@ __global__ __launch_bounds__(64) void k_dct1d(const float* __restrict__ in, int6
         if (r < left)
             reinterpret_cast<float4*>(out + base * 64)[q] =
                 *reinterpret_cast<const float4*>(tile + r * kLd + ((q & 15) << 2));
-    }
-}
-
-// dense contraction for chunk sizes other than 64 (h, w <= 64)
-__global__ __launch_bounds__(256) void k_dct2d_dense(const float* __restrict__ in, int64_t C, int h, int w,
-                                                     const float* __restrict__ bh, const float* __restrict__ bw,
-                                                     int in_chunked, int out_chunked,
-                                                     float* __restrict__ out) {
-    __shared__ float sx[64 * 64];
-    __shared__ float st[64 * 64];
-    __shared__ float sbh[64 * 64];
-    __shared__ float sbw[64 * 64];
-    const int tid = threadIdx.x;
-    const int64_t X = C / w;
-    const int64_t chunk = blockIdx.x;
-    const int64_t y = chunk / X, xc = chunk - y * X;
-    const int hw = h * w;
-    for (int i = tid; i < h * h; i += 256) sbh[i] = bh[i];
-    for (int i = tid; i < w * w; i += 256) sbw[i] = bw[i];
-    for (int i = tid; i < hw; i += 256) {
-        const int r = i / w, c = i - r * w;
-        sx[i] = in_chunked ? in[chunk * hw + i] : in[(y * h + r) * C + xc * w + c];
-    }
-    __syncthreads();
-    for (int i = tid; i < hw; i += 256) {
-        const int b = i / w, l = i - b * w;
-        float acc = 0.f;
-        for (int k = 0; k < h; ++k) acc = __builtin_fmaf(sbh[k * h + b], sx[k * w + l], acc);
-        st[i] = acc;
-    }
-    __syncthreads();
-    for (int i = tid; i < hw; i += 256) {
-        const int b = i / w, d = i - b * w;
-        float acc = 0.f;
-        for (int l = 0; l < w; ++l) acc = __builtin_fmaf(st[b * w + l], sbw[l * w + d], acc);
-        if (out_chunked)
-            out[chunk * hw + i] = acc;
-        else
-            out[(y * h + b) * C + xc * w + d] = acc;
     }
 }
 
@@ -3680,30 +3642,6 @@ __global__ __launch_bounds__(256, 2) void k_fill_lds(uint32_t word, uint32_t* __
 // =========================================================================================
 using namespace tplr;
 
-static inline int launch_status() {
-    const hipError_t e = hipGetLastError();
-    return e == hipSuccess ? 0 : static_cast<int>(e);
-}
-
-static inline unsigned grid8(int64_t n) { return static_cast<unsigned>(((n + 7) / 8) * 8); }
-
-// persistent grids: exactly one resident set of workgroups of `threads` threads (one wave, or a team of
-// waves), as the occupancy calculator reports it for the kernel at hand (registers or LDS bound it); a
-// larger grid would leave a second, mostly empty round
-template <typename Kernel>
-static int persistent_grid(Kernel kernel, int64_t total, int threads = 64) {
-    int n_cu = 256, per_cu = 0, dev = 0, v = 0;
-    if (hipGetDevice(&dev) == hipSuccess &&
-        hipDeviceGetAttribute(&v, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && v > 0)
-        n_cu = v;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernel, threads, 0) != hipSuccess || per_cu < 1)
-        per_cu = threads > 64 ? 2 : 4;
-    int64_t g = static_cast<int64_t>(n_cu) * per_cu;
-    g = g < 8 ? 8 : (g / 8) * 8;
-    const int64_t need = ((total + 7) / 8) * 8;
-    return static_cast<int>(need < g ? need : g);
-}
-
 // kTeam: waves per workgroup of the kernel (encode_team<> of its instantiation)
 template <int kTeam = 1, typename Kernel>
 static int launch_encode_as(Kernel kernel, const tplr_tensor_desc* d_desc, const tplr_tensor_desc& single,
@@ -3819,18 +3757,6 @@ int tplr_dct1d(const float* d_in, int64_t n_vec, int inverse, float* d_out, void
     if (!d_in || !d_out) return TPLR_E_BADARG;
     hipLaunchKernelGGL(k_dct1d, dim3(static_cast<unsigned>((n_vec + 63) / 64)), dim3(64), 0,
                        static_cast<hipStream_t>(stream), d_in, n_vec, inverse, d_out);
-    return launch_status();
-}
-
-int tplr_dct2d_dense(const float* d_in, int64_t R, int64_t C, int h, int w, const float* d_bh,
-                     const float* d_bw, int in_chunked, int out_chunked, float* d_out, void* stream) {
-    if (!d_in || !d_out || !d_bh || !d_bw || R < 0 || C < 0 || h < 1 || w < 1 || h > 64 || w > 64)
-        return TPLR_E_BADARG;
-    if ((R % h) || (C % w)) return TPLR_E_SHAPE;
-    const int64_t n = (R / h) * (C / w);
-    if (n == 0) return 0;
-    hipLaunchKernelGGL(k_dct2d_dense, dim3(static_cast<unsigned>(n)), dim3(256), 0,
-                       static_cast<hipStream_t>(stream), d_in, C, h, w, d_bh, d_bw, in_chunked, out_chunked, d_out);
     return launch_status();
 }
 

@@ -1,0 +1,33 @@
+// Host-side launch helpers shared by the library's translation units.
+#pragma once
+
+#include <hip/hip_runtime.h>
+#include <stdint.h>
+
+namespace tplr {
+
+inline int launch_status() {
+    const hipError_t e = hipGetLastError();
+    return e == hipSuccess ? 0 : static_cast<int>(e);
+}
+
+inline unsigned grid8(int64_t n) { return static_cast<unsigned>(((n + 7) / 8) * 8); }
+
+// persistent grids: exactly one resident set of workgroups of `threads` threads (one wave, or a team of
+// waves), as the occupancy calculator reports it for the kernel at hand (registers or LDS bound it); a
+// larger grid would leave a second, mostly empty round
+template <typename Kernel>
+int persistent_grid(Kernel kernel, int64_t total, int threads = 64) {
+    int n_cu = 256, per_cu = 0, dev = 0, v = 0;
+    if (hipGetDevice(&dev) == hipSuccess &&
+        hipDeviceGetAttribute(&v, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && v > 0)
+        n_cu = v;
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernel, threads, 0) != hipSuccess || per_cu < 1)
+        per_cu = threads > 64 ? 2 : 4;
+    int64_t g = static_cast<int64_t>(n_cu) * per_cu;
+    g = g < 8 ? 8 : (g / 8) * 8;
+    const int64_t need = ((total + 7) / 8) * 8;
+    return static_cast<int>(need < g ? need : g);
+}
+
+}  // namespace tplr
