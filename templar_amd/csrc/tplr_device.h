@@ -851,4 +851,19 @@ __device__ __forceinline__ void emit_selected(const Selected& s, int lane, int k
     }
 }
 
+// Pointers that come out of descriptor tables are not kernel arguments, so the compiler
+// cannot tell that they are global memory; say so, or it emits FLAT accesses (which also
+// count as LDS traffic and serialise against the tile).
+typedef float v4f __attribute__((ext_vector_type(4)));
+using gfloat = __attribute__((address_space(1))) float;
+using gbyte = __attribute__((address_space(1))) uint8_t;
+
+// 12-bit index j of a packed row (byte pointer to the row start)
+template <typename BytePtr>
+__device__ __forceinline__ uint32_t load_idx12(BytePtr row, int j) {
+    BytePtr b = row + 3 * (j >> 1) + (j & 1);
+    const uint32_t w = b[0] | (static_cast<uint32_t>(b[1]) << 8);
+    return (j & 1) ? (w >> 4) : (w & 0xfffu);
+}
+
 }  // namespace tplr

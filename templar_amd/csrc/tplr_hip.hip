@@ -170,13 +170,6 @@ __device__ __forceinline__ void chunk_inverse(float (&v)[64], float* tile, int l
 // Persistent kernels walk a contiguous range of the batch's chunk list.  A cursor keeps the
 // current tensor's descriptor and the chunk's (y, x) position in wave-uniform registers.
 // -----------------------------------------------------------------------------------------
-// Pointers that come out of descriptor tables are not kernel arguments, so the compiler
-// cannot tell that they are global memory; say so, or it emits FLAT accesses (which also
-// count as LDS traffic and serialise against the tile).
-typedef float v4f __attribute__((ext_vector_type(4)));
-using gfloat = __attribute__((address_space(1))) float;
-using gbyte = __attribute__((address_space(1))) uint8_t;
-
 struct Cursor {
     const tplr_tensor_desc* table;
     int n_tensors;
@@ -304,214 +297,6 @@ __global__ __launch_bounds__(64) void k_dct2d_inv(const float* __restrict__ coef
     float v[64];
     chunk_inverse<true, true>(v, tile, lane);
     store_chunk_cols(v, x, ld, y, xc, lane);
-}
-
-__global__ __launch_bounds__(64) void k_dct1d(const float* __restrict__ in, int64_t n_vec, int inverse,
-                                              float* __restrict__ out) {
-    __shared__ __align__(16) float tile[kTileFloats];
-    const int lane = threadIdx.x;
-    const int64_t base = static_cast<int64_t>(blockIdx.x) * 64;  // 64 vectors per wave
-    const int64_t left = n_vec - base;
-    // stage 64 vectors (rows) through the tile so that global accesses stay coalesced
-#pragma unroll
-    for (int c = 0; c < 16; ++c) {
-        const int q = c * 64 + lane;
-        const int r = q >> 4;
-        float4 t = make_float4(0.f, 0.f, 0.f, 0.f);
-        if (r < left) t = reinterpret_cast<const float4*>(in + base * 64)[q];
-        *reinterpret_cast<float4*>(tile + r * kLd + ((q & 15) << 2)) = t;
-    }
-    __syncthreads();
-    float v[64];
-    tile_rows_to_regs(v, tile, lane);
-    if (inverse)
-        dct64_inv(v);
-    else
-        dct64_fwd(v);
-    // one pass is sqrt(32) times the orthonormal transform
-#pragma unroll
-    for (int d = 0; d < 64; ++d) v[d] *= 0.17677669529663687f;
-    __syncthreads();
-    regs_to_tile_rows(v, tile, lane);
-    __syncthreads();
-#pragma unroll
-    for (int c = 0; c < 16; ++c) {
-        const int q = c * 64 + lane;
-        const int r = q >> 4;
-        if (r < left)
-            reinterpret_cast<float4*>(out + base * 64)[q] =
-                *reinterpret_cast<const float4*>(tile + r * kLd + ((q & 15) << 2));
-    }
-}
-
-// =========================================================================================
-// top-k select + pack
-// =========================================================================================
-template <bool kTwo>
-__global__ __launch_bounds__(64) void k_topk_rows(const float* __restrict__ coef, int64_t n_rows, int row_len,
-                                                  int k, uint8_t* __restrict__ idx12, float* __restrict__ val) {
-    __shared__ __align__(16) float tile[kTileFloats];
-    __shared__ uint64_t cand[kCandCap];
-    const int lane = threadIdx.x;
-    const int64_t row = xcd_contiguous(blockIdx.x, gridDim.x);
-    if (row >= n_rows) return;
-    const float* src = coef + row * row_len;
-    if (row_len == 4096) {
-        flat_to_tile(src, tile, lane);
-    } else {
-#pragma unroll 4
-        for (int i = 0; i < 64; ++i) {
-            const int e = i * 64 + lane;
-            tile[i * kLd + lane] = e < row_len ? src[e] : 0.0f;
-        }
-    }
-    __syncthreads();
-    float w[64];
-    tile_rows_to_regs(w, tile, lane);
-    __syncthreads();
-    const Selected s = select_topk<kTwo>(w, tile, cand, lane, k, 1.0f);
-    emit_selected<kTwo>(s, lane, k, row, idx12, val);
-}
-
-// Any k up to the row length: the whole row sorted.  One workgroup of 256 threads per row, the row as
-// 4096 keys (magnitude, 4095 - index, sign: the canonical order of select_topk, elements past the row
-// as zeros at their own indices, which no real element ranks below) in LDS, a bitonic network of 78
-// steps in descending order, then the k leading keys unpacked as select_topk unpacks its candidates.
-// Not a fast path: it serves selections larger than the register-resident select holds (k > 128).
-__global__ __launch_bounds__(256) void k_topk_rows_sorted(const float* __restrict__ coef, int64_t n_rows, int row_len,
-                                                          int k, uint8_t* __restrict__ idx12, float* __restrict__ val) {
-    __shared__ uint64_t keys[4096];
-    const int tid = threadIdx.x;
-    const int64_t row = xcd_contiguous(blockIdx.x, gridDim.x);
-    if (row >= n_rows) return;  // (the whole workgroup)
-    const float* src = coef + row * row_len;
-    for (int e = tid; e < 4096; e += 256) {
-        const uint32_t bits = e < row_len ? __float_as_uint(src[e]) : 0u;
-        keys[e] = (static_cast<uint64_t>(mag_key(bits)) << 32) | ((4095u - static_cast<uint32_t>(e)) << 1) | (bits >> 31);
-    }
-    __syncthreads();
-    for (int size = 2; size <= 4096; size <<= 1) {
-        for (int stride = size >> 1; stride > 0; stride >>= 1) {
-            for (int i = tid; i < 2048; i += 256) {
-                const int pos = 2 * i - (i & (stride - 1));
-                const uint64_t a = keys[pos], b = keys[pos + stride];
-                const bool down = (pos & size) == 0;  // this run is sorted in descending order
-                if ((a < b) == down) {
-                    keys[pos] = b;
-                    keys[pos + stride] = a;
-                }
-            }
-            __syncthreads();
-        }
-    }
-    float* vrow = val + row * k;
-    uint8_t* irow = idx12 + row * (k + (k >> 1));
-    for (int j = tid; j < (k >> 1); j += 256) {
-        uint32_t ix[2];
-#pragma unroll
-        for (int h = 0; h < 2; ++h) {
-            const uint64_t e = keys[2 * j + h];
-            const uint32_t lo = static_cast<uint32_t>(e), key = static_cast<uint32_t>(e >> 32);
-            ix[h] = 4095u - ((lo >> 1) & 4095u);
-            const uint32_t mag = key == 0x7fffffffu ? 0x7fc00000u : key;
-            vrow[2 * j + h] = __uint_as_float(mag | (lo << 31));
-        }
-        const uint32_t w = ix[0] | (ix[1] << 12);
-        irow[3 * j] = static_cast<uint8_t>(w);
-        irow[3 * j + 1] = static_cast<uint8_t>(w >> 8);
-        irow[3 * j + 2] = static_cast<uint8_t>(w >> 16);
-    }
-}
-
-// The 1-D parameters of a set (norm vectors), every tensor a run of rows of 64 elements: transform,
-// top-k and pack of all of them in one launch, each tensor read where it lies.  One wave takes up to 64
-// rows of one tensor: staged through the tile, a row per lane in registers, the 64-point transform and
-// its scale exactly as k_dct1d applies them, then every lane sorts its own 64 coefficients in registers -
-// a bitonic network over 64-bit keys (magnitude, 63 - index), the canonical order of select_topk - and
-// writes its row's payload: the k leading indices, and their values fetched back from the tile.
-template <bool kUseDct>
-__global__ __launch_bounds__(64) void k_encode_rows(const tplr_tensor_desc* __restrict__ table, int n_tensors, int k,
-                                                    uint8_t* __restrict__ idx12, float* __restrict__ val) {
-    __shared__ __align__(16) float tile[kTileFloats];
-    const int lane = threadIdx.x;
-    // this wave's tensor and group of rows: tensor t has ceil(rows / 64) groups
-    int t = 0, grp = blockIdx.x;
-    for (; t < n_tensors; ++t) {
-        const int groups = (table[t].x_chunks + 63) >> 6;
-        if (grp < groups) break;
-        grp -= groups;
-    }
-    if (t >= n_tensors) return;
-    const tplr_tensor_desc d = table[t];
-    const int left = d.x_chunks - grp * 64;  // rows from this group's first to the tensor's end
-    const gfloat* src = (const gfloat*)d.dense + static_cast<int64_t>(grp) * 4096;
-#pragma unroll
-    for (int c = 0; c < 16; ++c) {
-        const int q = c * 64 + lane;
-        const int r = q >> 4;
-        v4f x = {0.f, 0.f, 0.f, 0.f};
-        if (r < left) x = *reinterpret_cast<const __attribute__((address_space(1))) v4f*>(src + q * 4);
-        *reinterpret_cast<v4f*>(tile + r * kLd + ((q & 15) << 2)) = x;
-    }
-    wave_lds_fence();
-    float w[64];
-    tile_rows_to_regs(w, tile, lane);
-    if (kUseDct) {
-        dct64_fwd(w);
-#pragma unroll
-        for (int e = 0; e < 64; ++e) w[e] *= 0.17677669529663687f;  // one pass is sqrt(32) times the orthonormal transform
-    }
-    wave_lds_fence();
-    regs_to_tile_rows(w, tile, lane);
-    // Keys (magnitude bits, 63 - index) ordered as unsigned 64-bit integers - held as doubles: for positive,
-    // normal, finite doubles the two orders are the same, and a compare-exchange is then one v_max_f64 and one
-    // v_min_f64.  One is added to the exponent field so that a zero magnitude is a normal double, and NaNs share
-    // a magnitude key just below where that addition would reach the doubles' own infinities and NaNs.
-    double key[64];
-#pragma unroll
-    for (int e = 0; e < 64; ++e) {
-        const uint32_t a = __builtin_bit_cast(uint32_t, w[e]) & 0x7fffffffu;
-        const uint32_t mag = (a > 0x7f800000u ? 0x7fdfffffu : a) + 0x00100000u;
-        key[e] = __builtin_bit_cast(double, (static_cast<uint64_t>(mag) << 32) | static_cast<uint32_t>(63 - e));
-    }
-    // bitonic sort, descending
-#pragma unroll
-    for (int size = 2; size <= 64; size <<= 1) {
-#pragma unroll
-        for (int stride = size >> 1; stride > 0; stride >>= 1) {
-#pragma unroll
-            for (int i = 0; i < 64; ++i) {
-                const int l = i ^ stride;
-                if (l > i) {
-                    const bool up = (i & size) != 0 && size < 64;  // this run ascends
-                    const double a = key[i], b = key[l];
-                    const double hi = __builtin_fmax(a, b), lo = __builtin_fmin(a, b);
-                    key[i] = up ? lo : hi;
-                    key[l] = up ? hi : lo;
-                }
-            }
-        }
-    }
-    wave_lds_fence();
-    if (lane >= left) return;
-    const int64_t row = d.chunk_begin + static_cast<int64_t>(grp) * 64 + lane;
-    float* vrow = val + row * k;
-    uint8_t* irow = idx12 + row * (k + (k >> 1));
-    const float* mine = tile + lane * kLd;
-#pragma unroll
-    for (int j = 0; j < 64; j += 2) {
-        if (j < k) {  // k is even
-            const uint32_t i0 = 63u - static_cast<uint32_t>(__builtin_bit_cast(uint64_t, key[j]));
-            const uint32_t i1 = 63u - static_cast<uint32_t>(__builtin_bit_cast(uint64_t, key[j + 1]));
-            vrow[j] = mine[i0];
-            vrow[j + 1] = mine[i1];
-            const uint32_t pair = i0 | (i1 << 12);
-            uint8_t* o = irow + 3 * (j >> 1);
-            o[0] = static_cast<uint8_t>(pair);
-            o[1] = static_cast<uint8_t>(pair >> 8);
-            o[2] = static_cast<uint8_t>(pair >> 16);
-        }
-    }
 }
 
 // the wave's issue priority (0 .. 3; the instruction takes an immediate, hence the ladder); `level` is wave-uniform
@@ -667,14 +452,6 @@ struct PeerPtrs {
 };
 
 __device__ __forceinline__ int tile_pos(uint32_t idx) { return (idx >> 6) * kLd + (idx & 63); }
-
-// 12-bit index j of a packed row (byte pointer to the row start)
-template <typename BytePtr>
-__device__ __forceinline__ uint32_t load_idx12(BytePtr row, int j) {
-    BytePtr b = row + 3 * (j >> 1) + (j & 1);
-    const uint32_t w = b[0] | (static_cast<uint32_t>(b[1]) << 8);
-    return (j & 1) ? (w >> 4) : (w & 0xfffu);
-}
 
 typedef uint16_t __attribute__((aligned(1))) unaligned_u16;
 using gu16 = __attribute__((address_space(1))) unaligned_u16;
@@ -2638,63 +2415,6 @@ __global__ __launch_bounds__(256) void k_dequantize_batch(const uint8_t* __restr
     }
 }
 
-// generic rows (1-D tensors, un-chunked 2-D rows): exact source-order accumulation
-__global__ __launch_bounds__(64) void k_scatter_rows(const uint8_t* __restrict__ idx12,
-                                                     const int64_t* __restrict__ idx64,
-                                                     const float* __restrict__ val, int64_t k_per_row,
-                                                     int row_len, int reduce_mode, float* __restrict__ out,
-                                                     int32_t* __restrict__ err) {
-    __shared__ float acc[TPLR_MAX_ROW];
-    __shared__ uint32_t cnt[TPLR_MAX_ROW];
-    const int lane = threadIdx.x;
-    const int64_t row = blockIdx.x;
-    for (int i = lane; i < row_len; i += 64) {
-        acc[i] = 0.f;
-        cnt[i] = 0;
-    }
-    __syncthreads();
-    const uint8_t* irow = idx12 ? idx12 + row * (k_per_row + (k_per_row >> 1)) : nullptr;
-    for (int64_t j0 = 0; j0 < k_per_row; j0 += 64) {
-        const int64_t j = j0 + lane;
-        int64_t ix = -1;
-        float a = 0.f;
-        if (j < k_per_row) {
-            ix = idx12 ? static_cast<int64_t>(load_idx12(irow, static_cast<int>(j))) : idx64[row * k_per_row + j];
-            a = val[row * k_per_row + j];
-            if (ix < 0 || ix >= row_len) {
-                if (err) atomicMax(err, ix < 0 || ix > 0x7fffffff ? 0x7fffffff : static_cast<int32_t>(ix));
-                ix = -1;
-            }
-        }
-        // rank among earlier lanes of this batch that hit the same destination
-        const int me = static_cast<int>(ix);
-        int rank = 0;
-        for (int i = 0; i < 63; ++i) {
-            const int other = __shfl(me, i);
-            rank += (i < lane && other == me && me >= 0) ? 1 : 0;
-        }
-        int maxrank = rank;
-#pragma unroll
-        for (int off = 32; off > 0; off >>= 1) {
-            const int o = __shfl_xor(maxrank, off);
-            maxrank = o > maxrank ? o : maxrank;
-        }
-        for (int r = 0; r <= maxrank; ++r) {
-            if (me >= 0 && rank == r) {
-                acc[me] += a;
-                cnt[me] += 1;
-            }
-            __syncthreads();
-        }
-    }
-    float* orow = out + row * row_len;
-    for (int i = lane; i < row_len; i += 64) {
-        const uint32_t c = cnt[i];
-        const float s = acc[i];
-        orow[i] = (reduce_mode == TPLR_REDUCE_MEAN && c > 1) ? s / static_cast<float>(c) : s;
-    }
-}
-
 // =========================================================================================
 // peer statistics
 // =========================================================================================
@@ -3751,34 +3471,6 @@ int tplr_dct2d_inv(const float* d_coef, int64_t R, int64_t C, float* d_x, int64_
     return launch_status();
 }
 
-int tplr_dct1d(const float* d_in, int64_t n_vec, int inverse, float* d_out, void* stream) {
-    if (n_vec < 0) return TPLR_E_BADARG;
-    if (n_vec == 0) return 0;
-    if (!d_in || !d_out) return TPLR_E_BADARG;
-    hipLaunchKernelGGL(k_dct1d, dim3(static_cast<unsigned>((n_vec + 63) / 64)), dim3(64), 0,
-                       static_cast<hipStream_t>(stream), d_in, n_vec, inverse, d_out);
-    return launch_status();
-}
-
-int tplr_topk_pack(const float* d_coef, int64_t n_rows, int64_t row_len, int k, uint8_t* d_idx12,
-                   float* d_val, void* stream) {
-    if (n_rows < 0 || row_len < 1 || k < 2 || (k & 1) || k > row_len) return TPLR_E_BADARG;
-    if (row_len > TPLR_MAX_ROW) return TPLR_E_TOOMANY;
-    if (n_rows == 0) return 0;
-    if (!d_coef || !d_idx12 || !d_val) return TPLR_E_BADARG;
-    const int rl = static_cast<int>(row_len);
-    if (k > kCandCap)
-        hipLaunchKernelGGL(k_topk_rows_sorted, dim3(grid8(n_rows)), dim3(256), 0, static_cast<hipStream_t>(stream),
-                           d_coef, n_rows, rl, k, d_idx12, d_val);
-    else if (k > 32)
-        hipLaunchKernelGGL(k_topk_rows<true>, dim3(grid8(n_rows)), dim3(64), 0,
-                           static_cast<hipStream_t>(stream), d_coef, n_rows, rl, k, d_idx12, d_val);
-    else
-        hipLaunchKernelGGL(k_topk_rows<false>, dim3(grid8(n_rows)), dim3(64), 0,
-                           static_cast<hipStream_t>(stream), d_coef, n_rows, rl, k, d_idx12, d_val);
-    return launch_status();
-}
-
 static int launch_encode(const tplr_tensor_desc* d_desc, const tplr_tensor_desc& single, int n_tensors,
                          int64_t total, int k, int use_dct, uint8_t* d_idx12, float* d_val, void* stream) {
     if (k > 32) {
@@ -3814,22 +3506,6 @@ int tplr_encode_topk_pack_batch(const tplr_tensor_desc* d_desc, int n_tensors, i
     if (total_chunks == 0) return 0;
     tplr_tensor_desc none = {};
     return launch_encode(d_desc, none, n_tensors, total_chunks, k, use_dct, d_idx12, d_val, stream);
-}
-
-int tplr_encode_rows_batch(const tplr_tensor_desc* d_desc, int n_tensors, int64_t total_groups, int k, int use_dct,
-                           uint8_t* d_idx12, float* d_val, void* stream) {
-    if (!d_desc || n_tensors < 1 || total_groups < 0 || !d_idx12 || !d_val || k < 2 || (k & 1) || k > 64)
-        return TPLR_E_BADARG;
-    if (total_groups == 0) return 0;
-    if (total_groups > 0x7fffffff) return TPLR_E_TOOMANY;
-    const dim3 grid(static_cast<unsigned>(total_groups)), block(64);
-    if (use_dct)
-        hipLaunchKernelGGL(k_encode_rows<true>, grid, block, 0, static_cast<hipStream_t>(stream), d_desc, n_tensors, k,
-                           d_idx12, d_val);
-    else
-        hipLaunchKernelGGL(k_encode_rows<false>, grid, block, 0, static_cast<hipStream_t>(stream), d_desc, n_tensors, k,
-                           d_idx12, d_val);
-    return launch_status();
 }
 
 int tplr_ef_encode_topk_pack_batch(const tplr_tensor_desc* d_ef_desc, const tplr_tensor_desc* d_grad_desc,
@@ -4384,21 +4060,6 @@ int tplr_flat_update(float* d_a, const float* d_b, int64_t n, float decay, int s
     blocks = blocks > 4096 ? 4096 : blocks;
     hipLaunchKernelGGL(k_flat_update, dim3(static_cast<unsigned>(blocks)), dim3(256), 0, static_cast<hipStream_t>(stream),
                        d_a, d_b, n, decay, subtract);
-    return launch_status();
-}
-
-int tplr_scatter_rows(const uint8_t* d_idx12, const int64_t* d_idx64, const float* d_val, int64_t n_rows,
-                      int64_t k_per_row, int64_t row_len, int reduce_mode, float* d_out, int32_t* d_err,
-                      void* stream) {
-    if (n_rows < 0 || k_per_row < 0 || row_len < 1 || (!d_idx12 == !d_idx64) || !d_val || !d_out ||
-        (reduce_mode != TPLR_REDUCE_MEAN && reduce_mode != TPLR_REDUCE_SUM))
-        return TPLR_E_BADARG;
-    if (d_idx12 && (k_per_row & 1)) return TPLR_E_ODD;
-    if (row_len > TPLR_MAX_ROW) return TPLR_E_TOOMANY;
-    if (n_rows == 0) return 0;
-    hipLaunchKernelGGL(k_scatter_rows, dim3(static_cast<unsigned>(n_rows)), dim3(64), 0,
-                       static_cast<hipStream_t>(stream), d_idx12, d_idx64, d_val, k_per_row,
-                       static_cast<int>(row_len), reduce_mode, d_out, d_err);
     return launch_status();
 }
 

@@ -3,9 +3,11 @@ import numpy as np
 import pytest
 import torch
 
-import templar_amd.compress as tc
-
 pytestmark = pytest.mark.gpu
+
+from oracle import codec as orc  # noqa: E402  (the checker)
+import templar_amd.compress as tc  # noqa: E402
+from templar_amd import _lib  # noqa: E402
 
 
 @pytest.fixture(scope="module")
@@ -33,3 +35,66 @@ def test_dense_transform_at_tile_edges(dev, h, w, Y, X):
                                             torch.from_numpy(bw).to(dev), in_chunked, out_chunked).cpu().numpy()
         ref, tol = (want, bound) if out_chunked else (rows(want), rows(bound))
         assert (np.abs(got - ref) <= tol).all(), (in_chunked, out_chunked)
+
+
+def _rows(kind, n_rows, n, rng):
+    if kind == "normal":
+        return rng.standard_normal((n_rows, n)).astype(np.float32)
+    if kind == "levels":  # ties everywhere, zeros and both signs among them
+        return rng.integers(-3, 4, (n_rows, n)).astype(np.float32)
+    x = np.where(rng.random((n_rows, n)) < 0.01, rng.standard_normal((n_rows, n)), 0.0).astype(np.float32)
+    x[0] = 0.0  # fewer non-zero values than are selected: zeros of the row itself have to follow, lowest index first
+    x[-1, -1] = np.nan
+    return x
+
+
+@pytest.mark.parametrize("kind", ["normal", "levels", "sparse"])
+@pytest.mark.parametrize("n,k", [(2, 2), (37, 6), (63, 62), (64, 32), (64, 64), (65, 64), (100, 10), (127, 126), (128, 128),
+                                 (129, 32), (129, 128), (400, 32), (1000, 64), (2500, 32), (3000, 128), (4032, 2), (4033, 32),
+                                 (4095, 64), (4096, 32)])
+def test_rows_select_at_every_length(dev, n, k, kind):
+    rows = _rows(kind, 7, n, np.random.default_rng(n * 131 + k))
+    idx12, val = tc._topk_rows(torch.from_numpy(rows).to(dev), k)
+    want_i, want_v = orc.topk_rows(rows, k)
+    assert np.array_equal(idx12.cpu().numpy(), orc.pack12(want_i))
+    assert np.array_equal(val.cpu().numpy().view(np.uint32), np.asarray(want_v, np.float32).view(np.uint32))
+
+
+@pytest.mark.parametrize("repeats", [False, True])
+@pytest.mark.parametrize("n,k", [(2, 2), (37, 6), (64, 64), (1001, 32), (3000, 32), (4093, 64), (4096, 2)])
+def test_scatter_into_rows(dev, n, k, repeats):
+    rng = np.random.default_rng(n + k)
+    n_rows = 6
+    idx = np.stack([rng.permutation(n)[:k] for _ in range(n_rows)]).astype(np.int64)
+    if repeats:
+        idx[1] = idx[1, 0]  # one element named by every entry
+        idx[4, k // 2:] = idx[4, :k - k // 2]
+    val = rng.standard_normal((n_rows, k)).astype(np.float32)
+    got = tc._scatter_rows(torch.from_numpy(orc.pack12(idx)).to(dev), torch.from_numpy(val).to(dev), n_rows, k, n)
+    # entries of one element added in entry order, divided by their number
+    want = np.zeros((n_rows, n), np.float32)
+    count = np.zeros((n_rows, n), np.float32)
+    for r in range(n_rows):
+        for j in range(k):
+            want[r, idx[r, j]] += val[r, j]
+            count[r, idx[r, j]] += 1
+    want = np.where(count > 1, want / np.maximum(count, 1), want)
+    assert np.array_equal(got.cpu().numpy(), want)
+
+
+@pytest.mark.parametrize("inverse", [0, 1])
+@pytest.mark.parametrize("n_vec", [1, 3, 4, 5, 32, 63, 16384, 16385])
+def test_vectors_transform_alike_in_both_forms(dev, n_vec, inverse):
+    # the launch changes form past 16384 vectors; every vector's bits are the same in either
+    x = torch.from_numpy(np.random.default_rng(n_vec).standard_normal((n_vec, 64)).astype(np.float32)).to(dev)
+    lib = _lib.load()
+
+    def run(a):
+        out = torch.full_like(a, float("nan"))
+        assert lib.tplr_dct1d(a.data_ptr(), a.shape[0], inverse, out.data_ptr(), None) == 0
+        torch.cuda.synchronize()
+        return out
+
+    many = torch.zeros((16384 + 64 + n_vec, 64), device=dev)
+    many[:n_vec] = x
+    assert torch.equal(run(x), run(many)[:n_vec])
