@@ -390,7 +390,7 @@ int tplr_dequantize_peers(const uint8_t* const* h_codes, int n_peers, int64_t n,
  * payload (the reference runs it per parameter inside compress, :419-421): per tensor t,
  * shift = mean of its values, scale = range_in_sigmas * std / n_bins (1 when that is 0, NaN or
  * infinite), d_codes[i] = clamp(round_half_even((v - shift) / scale + n_bins / 2), 0, n_bins - 1),
- * d_lookup[t * n_bins + b] = mean of the centred values coded b (0 for an unused bin).  Four
+ * d_lookup[t * n_bins + b] = mean of the centred values coded b (0 for an unused bin).  Three
  * launches; every tensor is cut into n_slices (1..1024) runs of rows whose partial sums (double)
  * pass through d_work: n_tensors * n_slices * (2 + 2 * n_bins) doubles, contents irrelevant on
  * entry.  d_shift, d_scale: n_tensors floats.  k a multiple of 4, n_bins <= 256, d_val 16-byte

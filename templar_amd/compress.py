@@ -753,7 +753,7 @@ class TopKCompressor:
             q = torch.empty(val.shape, dtype=torch.uint8, device=dev)
             stats = torch.empty(2, dtype=torch.float32, device=dev)
             lookup = torch.empty(self.n_bins, dtype=torch.float32, device=dev)
-            slices = max(1, min(256, n // 16384))
+            slices = max(1, min(256, n // 1024))  # one load per thread, a workgroup per compute unit
             work = torch.empty(slices * (2 + 2 * self.n_bins), dtype=torch.float64, device=dev)
             with _on(dev):
                 st = lib.tplr_quantize_batch(_ptr(v), 4, _ptr(_flat_desc(n // 4, dev)), 1, self.n_bins,

@@ -187,6 +187,22 @@ __device__ __forceinline__ float wave_sum_f32(float x) {
     return x;
 }
 
+__device__ __forceinline__ double wave_sum_f64(double x) {
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) x += __shfl_xor(x, off);
+    return x;
+}
+
+// sum over the 256 threads of a workgroup, in every thread; `part`: four doubles of LDS
+__device__ __forceinline__ double block256_sum_f64(double x, double* part, int tid) {
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) x += __shfl_down(x, off);
+    __syncthreads();  // `part` may still be read from the previous call
+    if ((tid & 63) == 0) part[tid >> 6] = x;
+    __syncthreads();
+    return (part[0] + part[1]) + (part[2] + part[3]);
+}
+
 // registers (lane = row) -> tile rows
 __device__ __forceinline__ void regs_to_tile_rows(const float (&v)[64], float* tile, int lane) {
     float4* row = reinterpret_cast<float4*>(tile + lane * kLd);

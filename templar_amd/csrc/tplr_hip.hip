@@ -5,8 +5,6 @@
 #include <stdint.h>
 #include <string.h>
 
-#include <mutex>
-
 #include "../../include/tplr_hip.h"
 #include "tplr_device.h"
 #include "tplr_launch.h"
@@ -2212,209 +2210,6 @@ __global__ __launch_bounds__(64) void k_index_stats(const IdxPtrs ip, int P, int
     flush_totals(t_cur);
 }
 
-// De-quantise one peer's flat payload of 8-bit codes: value = lookup[t][code] + shift[t], the
-// tensor t found from the row id (TopKCompressor._dequantize_values, src/tplr/compress.py:637-643,
-// for every parameter of the set at once).  Four codes per thread.
-// The statistical quantiser over each tensor's sent values (src/tplr/compress.py:582-621): the
-// reference's three passes - mean, norm of the centred values, codes with per-bin means - as three
-// launches over slices of every tensor plus one that finishes the tables.  Partial sums are carried
-// in double, kept per (tensor, slice) in a caller-provided workspace and added in slice order by
-// whoever needs the total, so every workgroup of a tensor derives the same shift and scale.
-// Workspace layout (doubles): sum[T][S], sumsq[T][S], then bins[T][S][2 * n_bins] (sums, counts).
-struct QuantSlice {
-    const float4* v;
-    uchar4* q;
-    int64_t n4;  // float4 groups in this slice
-    int64_t n;   // values in the whole tensor
-    int t, s;
-};
-
-__device__ __forceinline__ QuantSlice quant_slice(const float* val, uint8_t* codes, const tplr_tensor_desc* table,
-                                                   int k, int S) {
-    QuantSlice qs;
-    qs.t = blockIdx.x / S;
-    qs.s = blockIdx.x - qs.t * S;
-    const tplr_tensor_desc d = table[qs.t];
-    const int64_t rows = static_cast<int64_t>(d.x_chunks) * d.y_chunks;
-    const int64_t r0 = rows * qs.s / S, r1 = rows * (qs.s + 1) / S;
-    qs.v = reinterpret_cast<const float4*>(val + (d.chunk_begin + r0) * k);
-    qs.q = codes ? reinterpret_cast<uchar4*>(codes + (d.chunk_begin + r0) * k) : nullptr;
-    qs.n4 = (r1 - r0) * k >> 2;  // k is a multiple of 4
-    qs.n = rows * k;
-    return qs;
-}
-
-__device__ __forceinline__ double block256_sum_f64(double x, double* part, int tid) {
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) x += __shfl_down(x, off);
-    __syncthreads();  // `part` may still be read from the previous call
-    if ((tid & 63) == 0) part[tid >> 6] = x;
-    __syncthreads();
-    return (part[0] + part[1]) + (part[2] + part[3]);
-}
-
-__device__ __forceinline__ double slices_total(const double* w, int S) {
-    double s = 0.0;
-    for (int i = 0; i < S; ++i) s += w[i];
-    return s;
-}
-
-__device__ __forceinline__ float quant_shift(const double* work, int t, int S, int64_t n) {
-    return static_cast<float>(slices_total(work + static_cast<int64_t>(t) * S, S) / static_cast<double>(n));  // :594
-}
-
-__device__ __forceinline__ float quant_scale(const double* work, int T, int t, int S, int64_t n, int n_bins,
-                                             float range_in_sigmas) {
-    const double ss = slices_total(work + (static_cast<int64_t>(T) + t) * S, S);
-    const float sd = static_cast<float>(sqrt(ss) / sqrt(static_cast<double>(n - 1)));  // :597
-    const float scale = range_in_sigmas * sd / static_cast<float>(n_bins);              // :598
-    return (scale == 0.f || scale != scale || __builtin_isinf(scale)) ? 1.0f : scale;   // :599-600
-}
-
-__global__ __launch_bounds__(256) void k_quant_sum(const float* __restrict__ val, int k,
-                                                   const tplr_tensor_desc* __restrict__ table, int S,
-                                                   double* __restrict__ work) {
-    __shared__ double part[4];
-    const int tid = threadIdx.x;
-    const QuantSlice qs = quant_slice(val, nullptr, table, k, S);
-    double acc = 0.0;
-    for (int64_t i = tid; i < qs.n4; i += 256) {
-        const float4 x = qs.v[i];
-        acc += (static_cast<double>(x.x) + x.y) + (static_cast<double>(x.z) + x.w);
-    }
-    acc = block256_sum_f64(acc, part, tid);
-    if (tid == 0) work[blockIdx.x] = acc;
-}
-
-__global__ __launch_bounds__(256) void k_quant_sumsq(const float* __restrict__ val, int k,
-                                                     const tplr_tensor_desc* __restrict__ table, int T, int S,
-                                                     double* __restrict__ work) {
-    __shared__ double part[4];
-    const int tid = threadIdx.x;
-    const QuantSlice qs = quant_slice(val, nullptr, table, k, S);
-    const float shift = quant_shift(work, qs.t, S, qs.n);
-    double acc = 0.0;
-    for (int64_t i = tid; i < qs.n4; i += 256) {
-        const float4 x = qs.v[i];
-        const float a = x.x - shift, b = x.y - shift, c = x.z - shift, e = x.w - shift;  // :595
-        acc += (static_cast<double>(a) * a + static_cast<double>(b) * b) +
-               (static_cast<double>(c) * c + static_cast<double>(e) * e);
-    }
-    acc = block256_sum_f64(acc, part, tid);
-    if (tid == 0) work[static_cast<int64_t>(T) * S + blockIdx.x] = acc;
-}
-
-__global__ __launch_bounds__(256) void k_quant_codes(const float* __restrict__ val, int k,
-                                                     const tplr_tensor_desc* __restrict__ table, int T, int S, int n_bins,
-                                                     float range_in_sigmas, uint8_t* __restrict__ codes,
-                                                     double* __restrict__ work) {
-    __shared__ double part[4];
-    __shared__ double bin_sum[256];
-    __shared__ unsigned int bin_cnt[256];
-    const int tid = threadIdx.x;
-    const QuantSlice qs = quant_slice(val, codes, table, k, S);
-    const float shift = quant_shift(work, qs.t, S, qs.n);
-    const float scale = quant_scale(work, T, qs.t, S, qs.n, n_bins, range_in_sigmas);
-    double* out = work + 2 * static_cast<int64_t>(T) * S + static_cast<int64_t>(blockIdx.x) * 2 * n_bins;
-    const float offset = static_cast<float>(n_bins / 2), top = static_cast<float>(n_bins - 1);
-    auto code = [&](float x, float& c) {
-        c = x - shift;
-        float r = __builtin_rintf(c / scale + offset);  // :604-605, ties to even as torch.round
-        r = r < 0.f ? 0.f : r;
-        r = r > top ? top : r;                          // :606
-        return static_cast<uint32_t>(r);
-    };
-    if (n_bins <= 8) {
-        // a handful of bins (templar runs four): per-thread sums, no contended atomics
-        double s8[8], c8[8];
-#pragma unroll
-        for (int b = 0; b < 8; ++b) s8[b] = c8[b] = 0.0;
-        auto tally = [&](uint32_t qq, float c) {
-#pragma unroll
-            for (int b = 0; b < 8; ++b) {
-                s8[b] += qq == static_cast<uint32_t>(b) ? static_cast<double>(c) : 0.0;  // :614-617
-                c8[b] += qq == static_cast<uint32_t>(b) ? 1.0 : 0.0;
-            }
-        };
-        for (int64_t i = tid; i < qs.n4; i += 256) {
-            const float4 x = qs.v[i];
-            float c0, c1, c2, c3;
-            const uint32_t q0 = code(x.x, c0), q1 = code(x.y, c1), q2 = code(x.z, c2), q3 = code(x.w, c3);
-            qs.q[i] = make_uchar4(static_cast<unsigned char>(q0), static_cast<unsigned char>(q1),
-                                  static_cast<unsigned char>(q2), static_cast<unsigned char>(q3));
-            tally(q0, c0), tally(q1, c1), tally(q2, c2), tally(q3, c3);
-        }
-#pragma unroll
-        for (int b = 0; b < 8; ++b) {
-            const double sum = block256_sum_f64(s8[b], part, tid), cnt = block256_sum_f64(c8[b], part, tid);
-            if (tid == 0 && b < n_bins) out[b] = sum, out[n_bins + b] = cnt;
-        }
-    } else {
-        bin_sum[tid] = 0.0, bin_cnt[tid] = 0u;
-        __syncthreads();
-        for (int64_t i = tid; i < qs.n4; i += 256) {
-            const float4 x = qs.v[i];
-            float c0, c1, c2, c3;
-            const uint32_t q0 = code(x.x, c0), q1 = code(x.y, c1), q2 = code(x.z, c2), q3 = code(x.w, c3);
-            qs.q[i] = make_uchar4(static_cast<unsigned char>(q0), static_cast<unsigned char>(q1),
-                                  static_cast<unsigned char>(q2), static_cast<unsigned char>(q3));
-            atomicAdd(&bin_sum[q0], static_cast<double>(c0)), atomicAdd(&bin_cnt[q0], 1u);  // :614-617
-            atomicAdd(&bin_sum[q1], static_cast<double>(c1)), atomicAdd(&bin_cnt[q1], 1u);
-            atomicAdd(&bin_sum[q2], static_cast<double>(c2)), atomicAdd(&bin_cnt[q2], 1u);
-            atomicAdd(&bin_sum[q3], static_cast<double>(c3)), atomicAdd(&bin_cnt[q3], 1u);
-        }
-        __syncthreads();
-        if (tid < n_bins) out[tid] = bin_sum[tid], out[n_bins + tid] = static_cast<double>(bin_cnt[tid]);
-    }
-}
-
-__global__ __launch_bounds__(256) void k_quant_tables(const tplr_tensor_desc* __restrict__ table, int k, int T, int S,
-                                                      int n_bins, float range_in_sigmas,
-                                                      const double* __restrict__ work, float* __restrict__ shift_out,
-                                                      float* __restrict__ scale_out, float* __restrict__ lookup) {
-    const int t = blockIdx.x, tid = threadIdx.x;
-    const tplr_tensor_desc d = table[t];
-    const int64_t n = static_cast<int64_t>(d.x_chunks) * d.y_chunks * k;
-    if (tid < n_bins) {
-        const double* bins = work + 2 * static_cast<int64_t>(T) * S + static_cast<int64_t>(t) * S * 2 * n_bins;
-        double sum = 0.0, cnt = 0.0;
-        for (int s = 0; s < S; ++s) sum += bins[s * 2 * n_bins + tid], cnt += bins[s * 2 * n_bins + n_bins + tid];
-        lookup[static_cast<int64_t>(t) * n_bins + tid] = cnt > 0.0 ? static_cast<float>(sum / cnt) : 0.f;  // :619
-    }
-    if (tid == 0) {
-        shift_out[t] = quant_shift(work, t, S, n);
-        scale_out[t] = quant_scale(work, T, t, S, n, n_bins, range_in_sigmas);
-    }
-}
-
-__global__ __launch_bounds__(256) void k_dequantize_batch(const uint8_t* __restrict__ q,
-                                                          const float* __restrict__ lookup,
-                                                          const float* __restrict__ shift, int n_bins, int k,
-                                                          const tplr_tensor_desc* __restrict__ table, int n_tensors,
-                                                          int64_t n4, float* __restrict__ val) {
-    const int64_t stride = static_cast<int64_t>(gridDim.x) * 256;
-    for (int64_t i = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x; i < n4; i += stride) {
-        const int64_t row = (i * 4) / k;  // k is a multiple of 4 here: the four codes share a row
-        int lo = 0, hi = n_tensors;
-        while (hi - lo > 1) {
-            const int mid = (lo + hi) >> 1;
-            if (table[mid].chunk_begin <= row)
-                lo = mid;
-            else
-                hi = mid;
-        }
-        const uchar4 c = reinterpret_cast<const uchar4*>(q)[i];
-        const float* lk = lookup + static_cast<int64_t>(lo) * n_bins;
-        const float sh = shift[lo];
-        float4 o;
-        o.x = lk[c.x < n_bins ? c.x : n_bins - 1] + sh;
-        o.y = lk[c.y < n_bins ? c.y : n_bins - 1] + sh;
-        o.z = lk[c.z < n_bins ? c.z : n_bins - 1] + sh;
-        o.w = lk[c.w < n_bins ? c.w : n_bins - 1] + sh;
-        reinterpret_cast<float4*>(val)[i] = o;
-    }
-}
-
 // =========================================================================================
 // peer statistics
 // =========================================================================================
@@ -4208,105 +4003,6 @@ int tplr_index_stats_batch(const uint8_t* const* h_idx12, int n_peers, int k, co
     return launch_status();
 }
 
-struct DeqPtrs {
-    const uint8_t* codes[TPLR_MAX_PEERS];
-    float* out[TPLR_MAX_PEERS];
-};
-
-// One parameter's codes of P peers, each with its own lookup and shift: block row p serves peer p.
-__global__ __launch_bounds__(256) void k_dequantize_peers(const DeqPtrs pp, int64_t n4,
-                                                          const float* __restrict__ lookup,
-                                                          const float* __restrict__ shift, int n_bins) {
-    const int p = blockIdx.y;
-    const uchar4* q = reinterpret_cast<const uchar4*>(pp.codes[p]);
-    float4* o = reinterpret_cast<float4*>(pp.out[p]);
-    const float* lk = lookup + static_cast<int64_t>(p) * n_bins;
-    const float sh = shift[p];
-    const int64_t stride = static_cast<int64_t>(gridDim.x) * 256;
-    for (int64_t i = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x; i < n4; i += stride) {
-        const uchar4 c = q[i];
-        float4 r;
-        r.x = lk[c.x < n_bins ? c.x : n_bins - 1] + sh;
-        r.y = lk[c.y < n_bins ? c.y : n_bins - 1] + sh;
-        r.z = lk[c.z < n_bins ? c.z : n_bins - 1] + sh;
-        r.w = lk[c.w < n_bins ? c.w : n_bins - 1] + sh;
-        o[i] = r;
-    }
-}
-
-int tplr_dequantize_peers(const uint8_t* const* h_codes, int n_peers, int64_t n, const float* d_lookup,
-                          const float* d_shift, int n_bins, float* const* h_out, void* stream) {
-    if (!h_codes || !h_out || !d_lookup || !d_shift || n_peers < 1 || n < 0 || (n & 3) || n_bins < 1 || n_bins > 256)
-        return TPLR_E_BADARG;
-    if (n_peers > TPLR_MAX_PEERS) return TPLR_E_TOOMANY;
-    if (n == 0) return 0;
-    DeqPtrs pp;
-    for (int p = 0; p < TPLR_MAX_PEERS; ++p) {
-        pp.codes[p] = p < n_peers ? h_codes[p] : nullptr;
-        pp.out[p] = p < n_peers ? h_out[p] : nullptr;
-        if (p < n_peers && (!pp.codes[p] || !pp.out[p] || (reinterpret_cast<uintptr_t>(pp.codes[p]) & 3) ||
-                            (reinterpret_cast<uintptr_t>(pp.out[p]) & 15)))
-            return TPLR_E_BADARG;
-    }
-    const int64_t n4 = n >> 2;
-    int64_t bx = (n4 + 255) / 256;
-    bx = bx > 2048 ? 2048 : bx;
-    hipLaunchKernelGGL(k_dequantize_peers, dim3(static_cast<unsigned>(bx), static_cast<unsigned>(n_peers)), dim3(256), 0,
-                       static_cast<hipStream_t>(stream), pp, n4, d_lookup, d_shift, n_bins);
-    return launch_status();
-}
-
-static int launch_quantize(const float* d_val, int k, const tplr_tensor_desc* d_desc, int n_tensors, int n_bins,
-                           float range_in_sigmas, int n_slices, double* d_work, uint8_t* d_codes, float* d_shift,
-                           float* d_scale, float* d_lookup, void* stream) {
-    const dim3 grid(static_cast<unsigned>(n_tensors) * n_slices), block(256);
-    hipStream_t st = static_cast<hipStream_t>(stream);
-    hipLaunchKernelGGL(k_quant_sum, grid, block, 0, st, d_val, k, d_desc, n_slices, d_work);
-    hipLaunchKernelGGL(k_quant_sumsq, grid, block, 0, st, d_val, k, d_desc, n_tensors, n_slices, d_work);
-    hipLaunchKernelGGL(k_quant_codes, grid, block, 0, st, d_val, k, d_desc, n_tensors, n_slices, n_bins, range_in_sigmas,
-                       d_codes, d_work);
-    hipLaunchKernelGGL(k_quant_tables, dim3(static_cast<unsigned>(n_tensors)), block, 0, st, d_desc, k, n_tensors,
-                       n_slices, n_bins, range_in_sigmas, d_work, d_shift, d_scale, d_lookup);
-    return launch_status();
-}
-
-static int check_quantize(const float* d_val, int k, const tplr_tensor_desc* d_desc, int n_tensors, int n_bins,
-                          int n_slices, const uint8_t* d_codes, const float* d_shift, const float* d_scale,
-                          const float* d_lookup) {
-    if (!d_val || !d_desc || !d_codes || !d_shift || !d_scale || !d_lookup || n_tensors < 1 || k < 4 || (k & 3) ||
-        n_bins < 1 || n_bins > 256 || n_slices < 1 || n_slices > 1024)
-        return TPLR_E_BADARG;
-    if ((reinterpret_cast<uintptr_t>(d_val) & 15) || (reinterpret_cast<uintptr_t>(d_codes) & 3)) return TPLR_E_BADARG;
-    if (static_cast<int64_t>(n_tensors) * n_slices > 0x7fffffff) return TPLR_E_TOOMANY;
-    return 0;
-}
-
-int tplr_quantize_batch(const float* d_val, int k, const tplr_tensor_desc* d_desc, int n_tensors, int n_bins,
-                        float range_in_sigmas, int n_slices, double* d_work, uint8_t* d_codes, float* d_shift,
-                        float* d_scale, float* d_lookup, void* stream) {
-    if (!d_work || (reinterpret_cast<uintptr_t>(d_work) & 7)) return TPLR_E_BADARG;
-    if (int s = check_quantize(d_val, k, d_desc, n_tensors, n_bins, n_slices, d_codes, d_shift, d_scale, d_lookup))
-        return s;
-    return launch_quantize(d_val, k, d_desc, n_tensors, n_bins, range_in_sigmas, n_slices, d_work, d_codes, d_shift,
-                           d_scale, d_lookup, stream);
-}
-
-int tplr_dequantize_batch(const uint8_t* d_codes, const float* d_lookup, const float* d_shift, int n_bins, int k,
-                          const tplr_tensor_desc* d_desc, int n_tensors, int64_t total_rows, float* d_val,
-                          void* stream) {
-    if (!d_codes || !d_lookup || !d_shift || !d_desc || !d_val || n_bins < 1 || n_bins > 256 || k < 4 || (k & 3) ||
-        n_tensors < 1 || total_rows < 0)
-        return TPLR_E_BADARG;
-    if ((reinterpret_cast<uintptr_t>(d_codes) & 3) || (reinterpret_cast<uintptr_t>(d_val) & 15)) return TPLR_E_BADARG;
-    if (total_rows == 0) return 0;
-    const int64_t n4 = total_rows * k / 4;
-    const int64_t blocks = (n4 + 255) / 256;
-    hipLaunchKernelGGL(k_dequantize_batch, dim3(static_cast<unsigned>(blocks < 65536 ? blocks : 65536)), dim3(256), 0,
-                       static_cast<hipStream_t>(stream), d_codes, d_lookup, d_shift, n_bins, k, d_desc, n_tensors, n4,
-                       d_val);
-    return launch_status();
-}
-
 int tplr_tensor_rnorm(const float* d_sumsq, const tplr_tensor_desc* d_desc, int n_tensors, float eps, float* d_factor,
                       void* stream) {
     if (!d_sumsq || !d_desc || !d_factor || n_tensors < 1) return TPLR_E_BADARG;
@@ -4448,63 +4144,6 @@ int tplr_calib_fill(void* d_dst, int64_t n_bytes, int pattern, void* stream) {
     else
         hipLaunchKernelGGL(k_calib_fill<2>, grid, block, 0, on, dst, n_bytes >> 4, 1.f);
     return launch_status();
-}
-
-// ---- the quantiser without a caller-provided workspace ----------------------------------------
-// The partial sums of tplr_quantize_batch live in a file-scope device array instead.  The array's
-// name is a host-side handle, not a device address: its address on the current device comes from
-// hipGetSymbolAddress, once per device, and only that pointer is handed to kernels.
-}  // extern "C"
-
-static __device__ __align__(256) double scratch[TPLR_STATIC_WORK_DOUBLES];
-
-namespace {
-constexpr int kMaxDevices = 64;
-std::mutex scratch_lock;
-double* scratch_ptr[kMaxDevices];  // per device: every GPU holds its own copy of the array
-
-// the array's address on the current device; nullptr with *status set when it cannot be had
-double* scratch_on_current_device(int* status) {
-    int dev = -1;
-    hipError_t e = hipGetDevice(&dev);
-    if (e != hipSuccess) {
-        *status = static_cast<int>(e);
-        return nullptr;
-    }
-    if (dev < 0 || dev >= kMaxDevices) {
-        *status = TPLR_E_TOOMANY;
-        return nullptr;
-    }
-    std::lock_guard<std::mutex> hold(scratch_lock);
-    if (!scratch_ptr[dev]) {
-        void* p = nullptr;
-        e = hipGetSymbolAddress(&p, HIP_SYMBOL(scratch));
-        if (e != hipSuccess || !p) {
-            *status = e != hipSuccess ? static_cast<int>(e) : TPLR_E_BADARG;
-            return nullptr;
-        }
-        scratch_ptr[dev] = static_cast<double*>(p);
-    }
-    return scratch_ptr[dev];
-}
-}  // namespace
-
-extern "C" {
-
-int64_t tplr_static_work_bytes(void) { return static_cast<int64_t>(TPLR_STATIC_WORK_DOUBLES) * 8; }
-
-int tplr_quantize_batch_static(const float* d_val, int k, const tplr_tensor_desc* d_desc, int n_tensors, int n_bins,
-                               float range_in_sigmas, int n_slices, uint8_t* d_codes, float* d_shift, float* d_scale,
-                               float* d_lookup, void* stream) {
-    if (int s = check_quantize(d_val, k, d_desc, n_tensors, n_bins, n_slices, d_codes, d_shift, d_scale, d_lookup))
-        return s;
-    const int64_t need = static_cast<int64_t>(n_tensors) * n_slices * (2 + 2 * static_cast<int64_t>(n_bins));
-    if (need > TPLR_STATIC_WORK_DOUBLES) return TPLR_E_WORKSPACE;
-    int status = 0;
-    double* work = scratch_on_current_device(&status);
-    if (!work) return status;
-    return launch_quantize(d_val, k, d_desc, n_tensors, n_bins, range_in_sigmas, n_slices, work, d_codes, d_shift,
-                           d_scale, d_lookup, stream);
 }
 
 }  // extern "C"

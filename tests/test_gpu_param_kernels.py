@@ -98,3 +98,29 @@ def test_vectors_transform_alike_in_both_forms(dev, n_vec, inverse):
     many = torch.zeros((16384 + 64 + n_vec, 64), device=dev)
     many[:n_vec] = x
     assert torch.equal(run(x), run(many)[:n_vec])
+
+
+@pytest.mark.parametrize("bins", [2, 4, 5, 8, 9, 256])
+@pytest.mark.parametrize("n", [4, 8, 1020, 1028, 65540, 270336])
+def test_quantiser_at_slice_and_bin_edges(dev, n, bins):
+    # the first value far out (values arrive in descending magnitude): the moments are taken about it
+    rng = np.random.default_rng(n + bins)
+    v = (rng.standard_t(3, n) * 1e-3 + 2e-4).astype(np.float32)
+    v[0] = 0.05
+    comp = tc.TopKCompressor(use_quantization=True, quantization_bins=bins, quantization_range=6)
+    q, (shift, scale, half, lut, _) = comp._quantize_values(torch.from_numpy(v).to(dev))
+    x = v.astype(np.float64)
+    # both figures are sums in double rounded once to fp32 (and a product and a quotient in fp32 for the scale)
+    assert abs(float(shift) - x.mean()) <= 2.0 ** -23 * abs(x.mean()) + 1e-12 * abs(x).max()
+    assert abs(scale / (6 * np.sqrt(((x - float(shift)) ** 2).sum() / (n - 1)) / bins) - 1) <= 2.0 ** -21
+    # with the device's own shift and scale every code and table entry is determined
+    c = v - np.float32(shift.item())
+    want = np.clip(np.rint(c / np.float32(scale) + np.float32(half)), 0, bins - 1).astype(np.uint8)
+    assert np.array_equal(q.cpu().numpy(), want)
+    for b in range(bins):
+        mine = c[want == b].astype(np.float64)
+        mean = mine.mean() if mine.size else 0.0
+        assert abs(float(lut[b]) - mean) <= 2.0 ** -23 * abs(mean) + 1e-12
+    const = torch.full((n,), 0.125, device=dev)
+    q, (shift, scale, _, _, _) = comp._quantize_values(const)
+    assert float(shift) == 0.125 and scale == 1.0 and (q == bins // 2).all()
