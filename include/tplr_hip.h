@@ -199,6 +199,12 @@ int tplr_scatter_rows(const uint8_t* d_idx12, const int64_t* d_idx64, const floa
                       int64_t n_rows, int64_t k_per_row, int64_t row_len, int reduce_mode,
                       float* d_out, int32_t* d_err, void* stream);
 
+/* TopKCompressor.decompress (src/tplr/compress.py:425-481) of one payload of packed rows, at most 64 entries each: as
+ * tplr_scatter_rows with TPLR_REDUCE_MEAN.  *flag (caller-zeroed, nullable, device or pinned host memory) becomes 1
+ * where an index lies outside its row; such entries are dropped. */
+int tplr_decompress_rows(const uint8_t* d_idx12, const float* d_val, int64_t n_rows, int k, int64_t row_len, float* d_out,
+                         int32_t* flag, void* stream);
+
 /* The same for P peers' flat payloads at once, without concatenating them: row g of d_out
  * (n_rows x row_len) takes the peers' entries for row g in peer order, peer p's values times
  * d_scale[t * n_peers + p], t the tensor of d_desc (chunk_begin = first row, as for the chunk
@@ -386,6 +392,11 @@ int tplr_dequantize_batch(const uint8_t* d_codes, const float* d_lookup, const f
 int tplr_dequantize_peers(const uint8_t* const* h_codes, int n_peers, int64_t n, const float* d_lookup,
                           const float* d_shift, int n_bins, float* const* h_out, void* stream);
 
+/* The same with peer p's lookup table and shift where they lie: h_lookup / h_shift are host arrays of n_peers device
+ * pointers (n_bins floats, one float). */
+int tplr_dequantize_lists(const uint8_t* const* h_codes, int n_peers, int64_t n, const float* const* h_lookup,
+                          const float* const* h_shift, int n_bins, float* const* h_out, void* stream);
+
 /* TopKCompressor._quantize_values (src/tplr/compress.py:582-621) for every parameter of a flat
  * payload (the reference runs it per parameter inside compress, :419-421): per tensor t,
  * shift = mean of its values, scale = range_in_sigmas * std / n_bins (1 when that is 0, NaN or
@@ -398,6 +409,11 @@ int tplr_dequantize_peers(const uint8_t* const* h_codes, int n_peers, int64_t n,
 int tplr_quantize_batch(const float* d_val, int k, const tplr_tensor_desc* d_desc, int n_tensors, int n_bins,
                         float range_in_sigmas, int n_slices, double* d_work, uint8_t* d_codes, float* d_shift,
                         float* d_scale, float* d_lookup, void* stream);
+
+/* The same for n values of one tensor (n a multiple of 4), d_work as for n_tensors = 1.  d_shift, d_scale and d_lookup may
+ * lie in pinned host memory. */
+int tplr_quantize(const float* d_val, int64_t n, int n_bins, float range_in_sigmas, int n_slices, double* d_work,
+                  uint8_t* d_codes, float* d_shift, float* d_scale, float* d_lookup, void* stream);
 
 /* The aggregate straight from quantised payloads, for a quantiser of at most four bins (templar runs
  * quantization_bins = 4, hparams/hparams.json) and chunks that are not transformed (use_dct = false): the

@@ -48,6 +48,7 @@ SIGNATURES = {
     "tplr_clip_scales_rows": (_i32, [_vp, _i32, _vp, _i32, _i32, _vp, _vp, _vp, _vp]),
     "tplr_decode_aggregate": (_i32, [_vp, _vp, _vp, _i32, _i32, _i64, _i64, _i32, _i32, _i32, _vp, _i64, _vp, _vp]),
     "tplr_scatter_rows": (_i32, [_vp, _vp, _vp, _i64, _i64, _i64, _i32, _vp, _vp, _vp]),
+    "tplr_decompress_rows": (_i32, [_vp, _vp, _i64, _i32, _i64, _vp, _vp, _vp]),
     "tplr_flat_update": (_i32, [_vp, _vp, _i64, C.c_float, _i32, _vp]),
     "tplr_aggregate_rows": (_i32, [_vp, _vp, _vp, _i32, _i32, _vp, _i32, _i64, _i64, _i32, _vp, _vp, _vp]),
     "tplr_decode_rows_batch": (_i32, [_vp, _vp, _vp, _i32, _i32, _vp, _i32, _i64, _i32, _i32, _vp, _vp]),
@@ -68,6 +69,8 @@ SIGNATURES = {
     "tplr_dequantize_batch": (_i32, [_vp, _vp, _vp, _i32, _i32, _vp, _i32, _i64, _vp, _vp]),
     "tplr_dequantize_peers": (_i32, [_vp, _i32, _i64, _vp, _vp, _i32, _vp, _vp]),
     "tplr_quantize_batch": (_i32, [_vp, _i32, _vp, _i32, _i32, C.c_float, _i32, _vp, _vp, _vp, _vp, _vp, _vp]),
+    "tplr_dequantize_lists": (_i32, [_vp, _i32, _i64, _vp, _vp, _i32, _vp, _vp]),
+    "tplr_quantize": (_i32, [_vp, _i64, _i32, C.c_float, _i32, _vp, _vp, _vp, _vp, _vp, _vp]),
     "tplr_tensor_rnorm": (_i32, [_vp, _vp, _i32, C.c_float, _vp, _vp]),
     "tplr_scale_batch": (_i32, [_vp, _i32, _i64, _vp, _vp]),
     "tplr_aggregate_sumsq_batch": (_i32, [_vp, _vp, _vp, _i32, _i32, _vp, _i32, _i64, _vp, _vp]),
@@ -100,6 +103,26 @@ def load():
             fn.argtypes = args
         _lib = lib
     return _lib
+
+
+_native = None
+
+
+def native():
+    """The host path of the per-parameter calls (csrc/tplr_native.cpp), bound to the loaded library's entry points."""
+    global _native
+    if _native is None:
+        import torch
+
+        lib = load()
+        try:
+            from . import _native as mod
+        except ImportError as e:
+            raise ImportError(f"templar_amd/_native is missing or does not load ({e}): build it with "
+                              "`python -c 'import __graft_entry__ as g; g.build()'`") from e
+        mod.bind({name: C.cast(getattr(lib, name), C.c_void_p).value for name in SIGNATURES}, TplrHipError, torch.float32)
+        _native = mod
+    return _native
 
 
 def check(status: int, what: str) -> None:

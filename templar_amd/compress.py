@@ -291,10 +291,18 @@ class ChunkingTransformer:
         return self.einsum_2d(x, b, d)
 
     # -- encode / decode ------------------------------------------------------------------
-    @torch.no_grad()
     def encode(self, x: torch.Tensor, *, use_dct: bool = False) -> torch.Tensor:
         """(R, C) -> (R/h, C/w, h, w), or (N,) -> (N/w, w); DCT-II per chunk when use_dct
         (reference :224-257).  Without use_dct the result is a view, as in the reference."""
+        if use_dct and self._fast64:
+            out = _lib.native().encode(x, self.shape_dict)
+            if out is not None:
+                return out
+        with torch.no_grad():
+            return self._encode(x, use_dct)
+
+    def _encode(self, x: torch.Tensor, use_dct: bool) -> torch.Tensor:
+        """encode of everything that is not a plain fp32 device tensor in chunks of 64."""
         if x.dim() > 1:
             n1 = self.shape_dict[x.shape[0]]
             n2 = self.shape_dict[x.shape[1]]
@@ -328,10 +336,18 @@ class ChunkingTransformer:
             return out if x.dtype == torch.float32 else out.to(x.dtype)
         return self.einsum_2d(rows, self._basis32(self.f_dict, n1, x.device))
 
-    @torch.no_grad()
     def decode(self, x: torch.Tensor, *, use_dct: bool = False) -> torch.Tensor:
         """(y, x, h, w) -> (y*h, x*w), or (x, w) -> (x*w,); inverse DCT per chunk when use_dct
         (reference :259-292)."""
+        if use_dct and self._fast64:
+            out = _lib.native().decode(x)
+            if out is not None:
+                return out
+        with torch.no_grad():
+            return self._decode(x, use_dct)
+
+    def _decode(self, x: torch.Tensor, use_dct: bool) -> torch.Tensor:
+        """decode of everything that is not a plain fp32 device tensor in chunks of 64."""
         if isinstance(x, LazyAggregate):
             if use_dct and not self._fast64:  # (the fused kernel is the orthonormal transform)
                 return self.decode(x.dense(), use_dct=True)
@@ -600,10 +616,20 @@ class TopKCompressor:
         """min(topk, last dim), at least 2, rounded down to even (reference :352-367)."""
         return _clamp_k(x.shape[-1], topk)
 
-    @torch.no_grad()
     def compress(self, x: torch.Tensor, topk: int):
         """Top-k by magnitude per chunk / row -> (packed idx, values, xshape, totalk[, qparams])
         (reference :385-423).  Values come out in descending-magnitude order."""
+        if self.use_quantization:
+            out = _lib.native().compress(x, topk, self.n_bins, self.range_in_sigmas)
+        else:
+            out = _lib.native().compress(x, topk, 0, 0)
+        if out is not None:
+            return out
+        with torch.no_grad():
+            return self._compress(x, topk)
+
+    def _compress(self, x: torch.Tensor, topk: int):
+        """compress of everything that is not a plain fp32 device tensor."""
         if _DT and isinstance(x, _DT):
             x = x.to_local()
         xshape = x.shape
@@ -626,11 +652,19 @@ class TopKCompressor:
             return idx, val, xshape, totalk, qparams
         return idx, val, xshape, totalk
 
-    @torch.no_grad()
     def decompress(self, p: torch.Tensor, idx: torch.Tensor, val: torch.Tensor, xshape: ShapeT, totalk: int,
                    quantize_params: QuantParamsT | None = None) -> torch.Tensor:
         """Scatter values back into a zero tensor of `xshape`, averaging duplicates
         (reference :425-481).  `p` only supplies device and dtype."""
+        out = _lib.native().decompress(p, idx, val, xshape, quantize_params if self.use_quantization else None)
+        if out is not None:
+            return out
+        with torch.no_grad():
+            return self._decompress(p, idx, val, xshape, quantize_params)
+
+    def _decompress(self, p: torch.Tensor, idx: torch.Tensor, val: torch.Tensor, xshape: ShapeT,
+                    quantize_params: QuantParamsT | None) -> torch.Tensor:
+        """decompress of everything that is not a plain payload on p's device, and of one with an index out of bounds."""
         if self.use_quantization and quantize_params is not None:
             val = self._dequantize_values(val, quantize_params)
         if idx.dtype not in (torch.uint8, torch.int64):
@@ -658,7 +692,6 @@ class TopKCompressor:
             out = _scatter_rows(idx.reshape(-1), val, n_rows, kk, row_len).reshape(xshape)
         return out if p.dtype == torch.float32 else out.to(p.dtype)
 
-    @torch.no_grad()
     def batch_decompress(self, p: torch.Tensor, idx: torch.Tensor | Sequence[torch.Tensor],
                          val: torch.Tensor | Sequence[torch.Tensor], xshape: ShapeT, totalk: int,
                          quantize_params: Sequence[QuantParamsT] | None = None, *,
@@ -668,6 +701,16 @@ class TopKCompressor:
         normalisation), then the coefficient-wise mean over the peers that sent each
         coefficient (reference :483-580).  With `defer=True` (an extension) the scatter is
         postponed so that ChunkingTransformer.decode() can run it fused with the inverse DCT."""
+        if not normalise and not defer and (quantize_params is None or not self.use_quantization):
+            out = _lib.native().aggregate(p, idx, val, xshape, block_norms, bool(clip_norm), False, False)
+            if out is not None:
+                return out
+        with torch.no_grad():
+            return self._batch_decompress(p, idx, val, xshape, quantize_params, block_norms, normalise, clip_norm, defer)
+
+    def _batch_decompress(self, p, idx, val, xshape: ShapeT, quantize_params, block_norms: torch.Tensor | None,
+                          normalise: bool, clip_norm: bool, defer: bool):
+        """batch_decompress of everything that is not a plain set of fp32 payloads of 64x64 chunks on p's device."""
         if quantize_params is not None and not isinstance(quantize_params, list):
             quantize_params = [quantize_params] * len(val)
         val_list = list(val) if isinstance(val, (list, tuple)) else [val]
@@ -742,25 +785,11 @@ class TopKCompressor:
     @torch.no_grad()
     def _quantize_values(self, val: torch.Tensor) -> tuple[torch.Tensor, QuantParamsT]:
         half = self.n_bins // 2
-        n = val.numel()
-        if (val.is_cuda and val.dtype == torch.float32 and n >= 4 and n % 4 == 0 and self.n_bins <= 256
-                and (val.data_ptr() % 16 == 0 or not val.is_contiguous())):  # (the kernel reads 16 bytes at a time)
-            # one launch (sums in double) instead of a dozen reductions and scatters; the scale is the
-            # only value that travels to the host, as in the reference (float(scale), :620)
-            lib = _lib.load()
-            dev = val.device
-            v = val.contiguous()
-            q = torch.empty(val.shape, dtype=torch.uint8, device=dev)
-            stats = torch.empty(2, dtype=torch.float32, device=dev)
-            lookup = torch.empty(self.n_bins, dtype=torch.float32, device=dev)
-            slices = max(1, min(256, n // 1024))  # one load per thread, a workgroup per compute unit
-            work = torch.empty(slices * (2 + 2 * self.n_bins), dtype=torch.float64, device=dev)
-            with _on(dev):
-                st = lib.tplr_quantize_batch(_ptr(v), 4, _ptr(_flat_desc(n // 4, dev)), 1, self.n_bins,
-                                             C.c_float(self.range_in_sigmas), slices, _ptr(work), _ptr(q),
-                                             _ptr(stats[0:1]), _ptr(stats[1:2]), _ptr(lookup), _stream(dev))
-            _lib.check(st, "tplr_quantize_batch")
-            return q, (stats[0], float(stats[1]), half, lookup, val.dtype)
+        # three launches (sums in double) instead of a dozen reductions and scatters; the scale is the only value that
+        # travels to the host, as in the reference (float(scale), :620)
+        out = _lib.native().quantize(val if val.is_contiguous() else val.contiguous(), self.n_bins, self.range_in_sigmas)
+        if out is not None:
+            return out
         shift = val.mean()
         centred = val - shift
         scale = self.range_in_sigmas * (centred.norm() / math.sqrt(centred.numel() - 1)) / self.n_bins
@@ -780,7 +809,7 @@ class TopKCompressor:
         if val.dtype != torch.uint8:
             return val
         if val.is_cuda:
-            fast = self._dequantize_peers([val], [qparams], val.device)
+            fast = _lib.native().dequantize([val], [qparams]) or self._dequantize_peers([val], [qparams], val.device)
             if fast is not None:
                 return fast[0]
         shift, _, _, lookup, orig_dtype = qparams
@@ -823,6 +852,10 @@ class TopKCompressor:
     def maybe_dequantize_values(self, vals: list[torch.Tensor], qparams: list[QuantParamsT],
                                 device: torch.device) -> list[torch.Tensor]:
         """Dequantise a list of per-peer values when all of them are uint8 (reference :646-696)."""
+        if type(vals) is list and type(qparams) is list and vals and vals[0].device == device:
+            fast = _lib.native().dequantize(vals, qparams)
+            if fast is not None:
+                return fast
         if not isinstance(vals, (list, tuple)):
             vals = [vals]
         if qparams is None or not all(v.dtype == torch.uint8 for v in vals):

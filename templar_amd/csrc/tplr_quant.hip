@@ -29,12 +29,13 @@ struct QuantSlice {
     int t, s;
 };
 
+// (`table` null: `single` is the one tensor)
 __device__ __forceinline__ QuantSlice quant_slice(const float* val, uint8_t* codes, const tplr_tensor_desc* table,
-                                                   int k, int S) {
+                                                   const tplr_tensor_desc& single, int k, int S) {
     QuantSlice qs;
     qs.t = blockIdx.x / S;
     qs.s = blockIdx.x - qs.t * S;
-    const tplr_tensor_desc d = table[qs.t];
+    const tplr_tensor_desc d = table ? table[qs.t] : single;
     const int64_t rows = static_cast<int64_t>(d.x_chunks) * d.y_chunks;
     const int64_t r0 = rows * qs.s / S, r1 = rows * (qs.s + 1) / S;
     qs.v = reinterpret_cast<const float4*>(val + (d.chunk_begin + r0) * k);
@@ -64,11 +65,12 @@ __device__ __forceinline__ void quant_shift_scale(const double* work, int t, int
 }
 
 __global__ __launch_bounds__(256) void k_quant_moments(const float* __restrict__ val, int k,
-                                                       const tplr_tensor_desc* __restrict__ table, int S,
+                                                       const tplr_tensor_desc* __restrict__ table,
+                                                       const tplr_tensor_desc single, int S,
                                                        double* __restrict__ work) {
     __shared__ double part[2][4];
     const int tid = threadIdx.x;
-    const QuantSlice qs = quant_slice(val, nullptr, table, k, S);
+    const QuantSlice qs = quant_slice(val, nullptr, table, single, k, S);
     const double first = static_cast<double>(qs.first);
     double s1 = 0.0, s2 = 0.0;
     for (int64_t i = tid; i < qs.n4; i += 256) {
@@ -90,11 +92,12 @@ __global__ __launch_bounds__(256) void k_quant_moments(const float* __restrict__
 // and this one 60 us (one parameter of 262 144 values: 19.3 us in 16 slices, now 5.5 in 256).
 template <int kBins>
 __global__ __launch_bounds__(256) void k_quant_codes(const float* __restrict__ val, int k,
-                                                     const tplr_tensor_desc* __restrict__ table, int T, int S, int n_bins,
+                                                     const tplr_tensor_desc* __restrict__ table,
+                                                     const tplr_tensor_desc single, int T, int S, int n_bins,
                                                      float range_in_sigmas, uint8_t* __restrict__ codes,
                                                      double* __restrict__ work) {
     const int tid = threadIdx.x;
-    const QuantSlice qs = quant_slice(val, codes, table, k, S);
+    const QuantSlice qs = quant_slice(val, codes, table, single, k, S);
     float shift, scale;
     quant_shift_scale(work, qs.t, S, qs.n, qs.first, n_bins, range_in_sigmas, shift, scale);
     double* out = work + 2 * static_cast<int64_t>(T) * S + static_cast<int64_t>(blockIdx.x) * 2 * n_bins;
@@ -163,7 +166,7 @@ __global__ __launch_bounds__(256) void k_quant_codes(const float* __restrict__ v
 
 // One wave per bin of tensor blockIdx.y (the slices' sums dealt over the lanes), and wave 0 of bin 0 the scalars.
 __global__ __launch_bounds__(64) void k_quant_tables(const float* __restrict__ val, const tplr_tensor_desc* __restrict__ table,
-                                                     int k, int T, int S, int n_bins, float range_in_sigmas,
+                                                     const tplr_tensor_desc single, int k, int T, int S, int n_bins, float range_in_sigmas,
                                                      const double* __restrict__ work, float* __restrict__ shift_out,
                                                      float* __restrict__ scale_out, float* __restrict__ lookup) {
     const int t = blockIdx.y, bin = blockIdx.x, lane = threadIdx.x;
@@ -174,7 +177,7 @@ __global__ __launch_bounds__(64) void k_quant_tables(const float* __restrict__ v
     cnt = wave_sum_f64(cnt);
     if (lane == 0) lookup[static_cast<int64_t>(t) * n_bins + bin] = cnt > 0.0 ? static_cast<float>(sum / cnt) : 0.f;  // :619
     if (bin == 0) {  // wave-uniform
-        const tplr_tensor_desc d = table[t];
+        const tplr_tensor_desc d = table ? table[t] : single;
         const int64_t n = static_cast<int64_t>(d.x_chunks) * d.y_chunks * k;
         float shift, scale;
         quant_shift_scale(work, t, S, n, n > 0 ? val[d.chunk_begin * k] : 0.f, n_bins, range_in_sigmas, shift, scale);
@@ -238,23 +241,50 @@ __global__ __launch_bounds__(256) void k_dequantize_peers(const DeqPtrs pp, int6
     }
 }
 
-static int launch_quantize(const float* d_val, int k, const tplr_tensor_desc* d_desc, int n_tensors, int n_bins,
+// The same with every peer's lookup and shift where they lie, up to kListPeers of them per launch.
+constexpr int kListPeers = 32;
+struct DeqLists {
+    const uint8_t* codes[kListPeers];
+    const float* lookup[kListPeers];
+    const float* shift[kListPeers];
+    float* out[kListPeers];
+};
+
+__global__ __launch_bounds__(256) void k_dequantize_lists(const DeqLists pp, int64_t n4, int n_bins) {
+    const int p = blockIdx.y;
+    const uchar4* q = reinterpret_cast<const uchar4*>(pp.codes[p]);
+    float4* o = reinterpret_cast<float4*>(pp.out[p]);
+    const float* lk = pp.lookup[p];
+    const float sh = *pp.shift[p];
+    const int64_t stride = static_cast<int64_t>(gridDim.x) * 256;
+    for (int64_t i = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x; i < n4; i += stride) {
+        const uchar4 c = q[i];
+        float4 r;
+        r.x = lk[c.x < n_bins ? c.x : n_bins - 1] + sh;
+        r.y = lk[c.y < n_bins ? c.y : n_bins - 1] + sh;
+        r.z = lk[c.z < n_bins ? c.z : n_bins - 1] + sh;
+        r.w = lk[c.w < n_bins ? c.w : n_bins - 1] + sh;
+        o[i] = r;
+    }
+}
+
+static int launch_quantize(const float* d_val, int k, const tplr_tensor_desc* d_desc, const tplr_tensor_desc& single, int n_tensors, int n_bins,
                            float range_in_sigmas, int n_slices, double* d_work, uint8_t* d_codes, float* d_shift,
                            float* d_scale, float* d_lookup, void* stream) {
     const dim3 grid(static_cast<unsigned>(n_tensors) * n_slices), block(256);
     hipStream_t st = static_cast<hipStream_t>(stream);
-    hipLaunchKernelGGL(k_quant_moments, grid, block, 0, st, d_val, k, d_desc, n_slices, d_work);
+    hipLaunchKernelGGL(k_quant_moments, grid, block, 0, st, d_val, k, d_desc, single, n_slices, d_work);
     hipLaunchKernelGGL(n_bins <= 4 ? k_quant_codes<4> : n_bins <= 8 ? k_quant_codes<8> : k_quant_codes<0>, grid, block, 0, st,
-                       d_val, k, d_desc, n_tensors, n_slices, n_bins, range_in_sigmas, d_codes, d_work);
+                       d_val, k, d_desc, single, n_tensors, n_slices, n_bins, range_in_sigmas, d_codes, d_work);
     hipLaunchKernelGGL(k_quant_tables, dim3(static_cast<unsigned>(n_bins), static_cast<unsigned>(n_tensors)), dim3(64), 0, st,
-                       d_val, d_desc, k, n_tensors, n_slices, n_bins, range_in_sigmas, d_work, d_shift, d_scale, d_lookup);
+                       d_val, d_desc, single, k, n_tensors, n_slices, n_bins, range_in_sigmas, d_work, d_shift, d_scale, d_lookup);
     return launch_status();
 }
 
 static int check_quantize(const float* d_val, int k, const tplr_tensor_desc* d_desc, int n_tensors, int n_bins,
                           int n_slices, const uint8_t* d_codes, const float* d_shift, const float* d_scale,
-                          const float* d_lookup) {
-    if (!d_val || !d_desc || !d_codes || !d_shift || !d_scale || !d_lookup || n_tensors < 1 || k < 4 || (k & 3) ||
+                          const float* d_lookup, bool one = false) {
+    if (!d_val || (!d_desc && !one) || !d_codes || !d_shift || !d_scale || !d_lookup || n_tensors < 1 || k < 4 || (k & 3) ||
         n_bins < 1 || n_bins > 256 || n_slices < 1 || n_slices > 1024)
         return TPLR_E_BADARG;
     if ((reinterpret_cast<uintptr_t>(d_val) & 15) || (reinterpret_cast<uintptr_t>(d_codes) & 3)) return TPLR_E_BADARG;
@@ -290,14 +320,54 @@ int tplr_dequantize_peers(const uint8_t* const* h_codes, int n_peers, int64_t n,
     return launch_status();
 }
 
+int tplr_dequantize_lists(const uint8_t* const* h_codes, int n_peers, int64_t n, const float* const* h_lookup,
+                          const float* const* h_shift, int n_bins, float* const* h_out, void* stream) {
+    if (!h_codes || !h_out || !h_lookup || !h_shift || n_peers < 1 || n < 0 || (n & 3) || n_bins < 1 || n_bins > 256)
+        return TPLR_E_BADARG;
+    if (n_peers > TPLR_MAX_PEERS) return TPLR_E_TOOMANY;
+    if (n == 0) return 0;
+    for (int p = 0; p < n_peers; ++p)
+        if (!h_codes[p] || !h_out[p] || !h_lookup[p] || !h_shift[p] || (reinterpret_cast<uintptr_t>(h_codes[p]) & 3) ||
+            (reinterpret_cast<uintptr_t>(h_out[p]) & 15))
+            return TPLR_E_BADARG;
+    const int64_t n4 = n >> 2;
+    int64_t bx = (n4 + 255) / 256;
+    bx = bx > 2048 ? 2048 : bx;
+    for (int p0 = 0; p0 < n_peers; p0 += kListPeers) {
+        DeqLists pp = {};
+        const int count = n_peers - p0 < kListPeers ? n_peers - p0 : kListPeers;
+        for (int p = 0; p < count; ++p) {
+            pp.codes[p] = h_codes[p0 + p];
+            pp.lookup[p] = h_lookup[p0 + p];
+            pp.shift[p] = h_shift[p0 + p];
+            pp.out[p] = h_out[p0 + p];
+        }
+        hipLaunchKernelGGL(k_dequantize_lists, dim3(static_cast<unsigned>(bx), static_cast<unsigned>(count)), dim3(256), 0,
+                           static_cast<hipStream_t>(stream), pp, n4, n_bins);
+    }
+    return launch_status();
+}
+
 int tplr_quantize_batch(const float* d_val, int k, const tplr_tensor_desc* d_desc, int n_tensors, int n_bins,
                         float range_in_sigmas, int n_slices, double* d_work, uint8_t* d_codes, float* d_shift,
                         float* d_scale, float* d_lookup, void* stream) {
     if (!d_work || (reinterpret_cast<uintptr_t>(d_work) & 7)) return TPLR_E_BADARG;
     if (int s = check_quantize(d_val, k, d_desc, n_tensors, n_bins, n_slices, d_codes, d_shift, d_scale, d_lookup))
         return s;
-    return launch_quantize(d_val, k, d_desc, n_tensors, n_bins, range_in_sigmas, n_slices, d_work, d_codes, d_shift,
+    return launch_quantize(d_val, k, d_desc, tplr_tensor_desc{}, n_tensors, n_bins, range_in_sigmas, n_slices, d_work, d_codes, d_shift,
                            d_scale, d_lookup, stream);
+}
+
+int tplr_quantize(const float* d_val, int64_t n, int n_bins, float range_in_sigmas, int n_slices, double* d_work,
+                  uint8_t* d_codes, float* d_shift, float* d_scale, float* d_lookup, void* stream) {
+    if (!d_work || (reinterpret_cast<uintptr_t>(d_work) & 7) || n < 4 || (n & 3)) return TPLR_E_BADARG;
+    if (int s = check_quantize(d_val, 4, nullptr, 1, n_bins, n_slices, d_codes, d_shift, d_scale, d_lookup, true)) return s;
+    if (n / 4 > 0x7fffffff) return TPLR_E_TOOMANY;
+    tplr_tensor_desc single = {};
+    single.x_chunks = static_cast<int32_t>(n / 4);  // rows of four values
+    single.y_chunks = 1;
+    return launch_quantize(d_val, 4, nullptr, single, 1, n_bins, range_in_sigmas, n_slices, d_work, d_codes, d_shift, d_scale,
+                           d_lookup, stream);
 }
 
 int tplr_dequantize_batch(const uint8_t* d_codes, const float* d_lookup, const float* d_shift, int n_bins, int k,
@@ -369,7 +439,7 @@ int tplr_quantize_batch_static(const float* d_val, int k, const tplr_tensor_desc
     int status = 0;
     double* work = scratch_on_current_device(&status);
     if (!work) return status;
-    return launch_quantize(d_val, k, d_desc, n_tensors, n_bins, range_in_sigmas, n_slices, work, d_codes, d_shift,
+    return launch_quantize(d_val, k, d_desc, tplr_tensor_desc{}, n_tensors, n_bins, range_in_sigmas, n_slices, work, d_codes, d_shift,
                            d_scale, d_lookup, stream);
 }
 

@@ -281,7 +281,7 @@ __global__ __launch_bounds__(256) void k_encode_rows(const tplr_tensor_desc* __r
 template <bool kVec>
 __global__ __launch_bounds__(256) void k_scatter_rows_packed(const uint8_t* __restrict__ idx12, const float* __restrict__ val,
                                                              int k, int row_len, int reduce_mode, float* __restrict__ out,
-                                                             int32_t* __restrict__ err) {
+                                                             int32_t* __restrict__ err, int32_t* __restrict__ flag) {
     __shared__ __align__(16) float acc[TPLR_MAX_ROW];
     const int tid = threadIdx.x, lane = tid & 63;
     const int64_t row = blockIdx.x;
@@ -298,6 +298,7 @@ __global__ __launch_bounds__(256) void k_scatter_rows_packed(const uint8_t* __re
     if (tid < 64) {
         if (me >= row_len) {
             if (err) atomicMax(err, me);
+            if (flag) *flag = 1;  // (pinned host memory: a plain store)
             me = -1;
         }
         if (me >= 0) acc[me] = __uint_as_float(static_cast<uint32_t>(lane));
@@ -456,6 +457,23 @@ int tplr_encode_rows_batch(const tplr_tensor_desc* d_desc, int n_tensors, int64_
     return launch_status();
 }
 
+static int scatter_packed(const uint8_t* d_idx12, const float* d_val, int64_t n_rows, int k, int row_len, int reduce_mode,
+                          float* d_out, int32_t* d_err, int32_t* flag, void* stream) {
+    const bool vec = (row_len & 3) == 0 && (reinterpret_cast<uintptr_t>(d_out) & 15) == 0;
+    hipLaunchKernelGGL(vec ? k_scatter_rows_packed<true> : k_scatter_rows_packed<false>, dim3(static_cast<unsigned>(n_rows)),
+                       dim3(256), 0, static_cast<hipStream_t>(stream), d_idx12, d_val, k, row_len, reduce_mode, d_out, d_err, flag);
+    return launch_status();
+}
+
+int tplr_decompress_rows(const uint8_t* d_idx12, const float* d_val, int64_t n_rows, int k, int64_t row_len, float* d_out,
+                         int32_t* flag, void* stream) {
+    if (!d_idx12 || !d_val || !d_out || n_rows < 0 || row_len < 1 || k < 2) return TPLR_E_BADARG;
+    if (k & 1) return TPLR_E_ODD;
+    if (k > 64 || row_len > TPLR_MAX_ROW || n_rows > 0x7fffffff) return TPLR_E_TOOMANY;
+    if (n_rows == 0) return 0;
+    return scatter_packed(d_idx12, d_val, n_rows, k, static_cast<int>(row_len), TPLR_REDUCE_MEAN, d_out, nullptr, flag, stream);
+}
+
 int tplr_scatter_rows(const uint8_t* d_idx12, const int64_t* d_idx64, const float* d_val, int64_t n_rows,
                       int64_t k_per_row, int64_t row_len, int reduce_mode, float* d_out, int32_t* d_err,
                       void* stream) {
@@ -466,13 +484,8 @@ int tplr_scatter_rows(const uint8_t* d_idx12, const int64_t* d_idx64, const floa
     if (row_len > TPLR_MAX_ROW) return TPLR_E_TOOMANY;
     if (n_rows == 0) return 0;
     if (d_idx12 && k_per_row <= 64) {
-        const int rl = static_cast<int>(row_len);
-        const dim3 grid(static_cast<unsigned>(n_rows)), block(256);
-        const bool vec = (rl & 3) == 0 && (reinterpret_cast<uintptr_t>(d_out) & 15) == 0;
-        hipLaunchKernelGGL(vec ? k_scatter_rows_packed<true> : k_scatter_rows_packed<false>, grid, block, 0,
-                           static_cast<hipStream_t>(stream), d_idx12, d_val, static_cast<int>(k_per_row), rl,
-                           reduce_mode, d_out, d_err);
-        return launch_status();
+        return scatter_packed(d_idx12, d_val, n_rows, static_cast<int>(k_per_row), static_cast<int>(row_len), reduce_mode, d_out,
+                              d_err, nullptr, stream);
     }
     hipLaunchKernelGGL(k_scatter_rows, dim3(static_cast<unsigned>(n_rows)), dim3(64), 0,
                        static_cast<hipStream_t>(stream), d_idx12, d_idx64, d_val, k_per_row,

@@ -124,3 +124,59 @@ def test_quantiser_at_slice_and_bin_edges(dev, n, bins):
     const = torch.full((n,), 0.125, device=dev)
     q, (shift, scale, _, _, _) = comp._quantize_values(const)
     assert float(shift) == 0.125 and scale == 1.0 and (q == bins // 2).all()
+
+
+def test_per_parameter_calls_agree_for_plain_and_converted_inputs(dev):
+    # plain tensors take the native host path, everything else is converted first: the same bits either way
+    from types import SimpleNamespace
+
+    params = [SimpleNamespace(requires_grad=True, shape=s, dtype=torch.float32, device=dev) for s in [(128, 192), (100, 60), (640,)]]
+    tr = tc.ChunkingTransformer(SimpleNamespace(named_parameters=lambda: ((str(i), p) for i, p in enumerate(params))), 64)
+    comp = tc.TopKCompressor(use_quantization=True, quantization_bins=4)
+    g = torch.Generator(device=dev).manual_seed(3)
+    for p in params:
+        x = torch.randn(p.shape, generator=g, device=dev)
+        wide = torch.randn(tuple(p.shape[:-1]) + (2 * p.shape[-1],), generator=g, device=dev)
+        wide[..., ::2] = x
+        results = []
+        for other in (x, torch.nn.Parameter(x.clone()), wide[..., ::2]):
+            enc = tr.encode(other, use_dct=True)
+            idx, q, xshape, totalk, qp = comp.compress(enc, 32)
+            dense = comp.decompress(x, idx, q, xshape, totalk, qp)
+            dec = tr.decode(dense, use_dct=True)
+            assert not dec.requires_grad and not enc.requires_grad
+            slow = tr.decode(comp.decompress(x, idx.reshape(1, -1), q, list(xshape), totalk, list(qp)), use_dct=True)
+            assert torch.equal(dec, slow)
+            results.append((idx, q, qp[0], torch.tensor(qp[1]), qp[3], dec))
+        for r in results[1:]:
+            assert all(torch.equal(a.reshape(-1), b.reshape(-1)) for a, b in zip(results[0], r))
+
+
+def test_decompress_names_the_index_outside_its_row(dev):
+    comp = tc.TopKCompressor()
+    idx = np.array([[1, 2, 3, 9], [4, 5, 11, 0]], np.int64)
+    val = torch.ones(2, 4, device=dev)
+    with pytest.raises(RuntimeError, match="index 11 is out of bounds for dimension -1 with size 9"):
+        comp.decompress(val, torch.from_numpy(orc.pack12(idx)).to(dev), val, (2, 9), 9)
+
+
+def test_quantisers_of_two_threads_do_not_meet(dev):
+    # each thread on a stream of its own: the scale travels through pinned memory of its own call
+    import threading
+
+    comp = tc.TopKCompressor(use_quantization=True, quantization_bins=4)
+    vals = [torch.randn(64 * 1024, device=dev) * (1 + 9 * t) for t in range(2)]
+    want = [comp._quantize_values(v)[1][1] for v in vals]
+    torch.cuda.synchronize()
+    wrong = []
+
+    def work(t):
+        with torch.cuda.stream(torch.cuda.Stream(dev)):
+            for _ in range(200):
+                if comp._quantize_values(vals[t])[1][1] != want[t]:
+                    wrong.append(t)
+
+    threads = [threading.Thread(target=work, args=(t,)) for t in range(2)]
+    [t.start() for t in threads]
+    [t.join() for t in threads]
+    assert not wrong
