@@ -339,8 +339,8 @@ class ChunkingTransformer:
     def decode(self, x: torch.Tensor, *, use_dct: bool = False) -> torch.Tensor:
         """(y, x, h, w) -> (y*h, x*w), or (x, w) -> (x*w,); inverse DCT per chunk when use_dct
         (reference :259-292)."""
-        if use_dct and self._fast64:
-            out = _lib.native().decode(x)
+        if self._fast64 or not use_dct:
+            out = _lib.native().decode(x, bool(use_dct))
             if out is not None:
                 return out
         with torch.no_grad():

@@ -15,6 +15,7 @@
 
 #include <ATen/core/Tensor.h>
 #include <ATen/ops/empty.h>
+#include <ATen/ops/empty_strided.h>
 #include <c10/hip/HIPFunctions.h>
 #include <c10/hip/HIPStream.h>
 #include <torch/csrc/Exceptions.h>
@@ -28,7 +29,7 @@ namespace {
 
 // ---- the library's entry points ---------------------------------------------------------------
 #define TPLR_NATIVE_ENTRIES(X)                                                                                       \
-    X(tplr_status_string) X(tplr_dct2d_fwd) X(tplr_dct2d_inv) X(tplr_dct1d) X(tplr_topk_pack) X(tplr_encode_topk_pack) \
+    X(tplr_status_string) X(tplr_dct2d_fwd) X(tplr_dct2d_inv_rows) X(tplr_dct2d_inv) X(tplr_dct1d) X(tplr_topk_pack) X(tplr_encode_topk_pack) \
     X(tplr_decode_aggregate) X(tplr_decompress_rows) X(tplr_clip_scales) X(tplr_peer_sumsq) X(tplr_quantize) X(tplr_dequantize_lists)
 #define X(name) decltype(&::name) p_##name = nullptr;
 TPLR_NATIVE_ENTRIES(X)
@@ -161,20 +162,37 @@ PyObject* encode(PyObject*, PyObject* const* args, Py_ssize_t n) {
     END_HANDLE_TH_ERRORS
 }
 
-// ---- decode(x, use_dct=True) ------------------------------------------------------------------
-PyObject* decode(PyObject*, PyObject* x_obj) {
+// ---- decode -----------------------------------------------------------------------------------
+// the (Y, X, 64, 64) view of a row-major (R, C) tensor, without gaps between its elements or with
+bool chunk_view(const at::Tensor& x) {
+    return x.dim() == 4 && x.size(2) == kEdge && x.size(3) == kEdge && x.stride(3) == 1 && x.stride(1) == kEdge &&
+           x.stride(2) >= x.size(1) * kEdge && (x.stride(0) == kEdge * x.stride(2) || x.size(0) == 1);
+}
+
+// decode(x, use_dct): chunks of 64x64 or rows of 64 back into their tensor
+PyObject* decode(PyObject*, PyObject* const* args, Py_ssize_t n) {
     HANDLE_TH_ERRORS
-    const at::Tensor* x = plain_f32(x_obj);
-    if (!x || x->numel() == 0 || !x->is_contiguous()) Py_RETURN_NONE;
+    if (n != 2) return PyErr_SetString(PyExc_TypeError, "decode(x, use_dct)"), nullptr;
+    const at::Tensor* x = plain_f32(args[0]);
+    if (!x || x->numel() == 0) Py_RETURN_NONE;
+    const bool view = chunk_view(*x);
+    if (args[1] != Py_True) {  // a change of shape: of a view of the tensor itself, the tensor
+        if (!view || x->requires_grad()) Py_RETURN_NONE;
+        return THPVariable_Wrap(x->as_strided({x->size(0) * kEdge, x->size(1) * kEdge}, {x->stride(2), 1}));
+    }
     Launch on(*x);
     if (x->dim() == 4 && x->size(2) == kEdge && x->size(3) == kEdge) {
         const int64_t R = x->size(0) * kEdge, C = x->size(1) * kEdge;
+        const bool aligned = x->stride(2) % 4 == 0 && reinterpret_cast<uintptr_t>(x->const_data_ptr()) % 16 == 0;
+        if (!x->is_contiguous() && !(view && aligned)) Py_RETURN_NONE;
         at::Tensor out = fresh({R, C}, c10::ScalarType::Float, *x);
-        if (int st = p_tplr_dct2d_inv(x->const_data_ptr<float>(), R, C, out.data_ptr<float>(), C, on.stream()))
-            return failed(st, "tplr_dct2d_inv");
+        const int st = x->is_contiguous()
+                           ? p_tplr_dct2d_inv(x->const_data_ptr<float>(), R, C, out.data_ptr<float>(), C, on.stream())
+                           : p_tplr_dct2d_inv_rows(x->const_data_ptr<float>(), x->stride(2), R, C, out.data_ptr<float>(), C, on.stream());
+        if (st) return failed(st, "tplr_dct2d_inv");
         return THPVariable_Wrap(std::move(out));
     }
-    if (x->dim() == 2 && x->size(1) == kEdge) {
+    if (x->dim() == 2 && x->size(1) == kEdge && x->is_contiguous()) {
         at::Tensor out = fresh({x->numel()}, c10::ScalarType::Float, *x);
         if (int st = p_tplr_dct1d(x->const_data_ptr<float>(), x->size(0), 1, out.data_ptr<float>(), on.stream()))
             return failed(st, "tplr_dct1d");
@@ -294,8 +312,7 @@ PyObject* compress(PyObject*, PyObject* const* args, Py_ssize_t n) {
     }
     if (bins && (bins < 1 || bins > 256 || rows * k % 4)) Py_RETURN_NONE;
     // the un-transformed chunk view of a row-major tensor, as encode(use_dct=False) returns it: select straight from it
-    const bool view = chunks && x->size(2) == kEdge && x->size(3) == kEdge && x->stride(3) == 1 && x->stride(1) == kEdge &&
-                      x->stride(2) >= x->size(1) * kEdge && (x->stride(0) == kEdge * x->stride(2) || x->size(0) == 1);
+    const bool view = chunk_view(*x);
     if (view ? k > 128 : !x->is_contiguous()) Py_RETURN_NONE;
     at::Tensor idx = fresh({rows * (k / 2) * 3}, c10::ScalarType::Byte, *x);
     at::Tensor val = chunks ? fresh({x->size(0), x->size(1), k}, c10::ScalarType::Float, *x)
@@ -336,10 +353,13 @@ struct Payloads {
 
 PyObject* scatter_chunks(const Payloads& pl, const float* scale, int64_t Y, int64_t X, bool rows, bool dct, const Launch& on) {
     const int64_t R = Y * kEdge, C = X * kEdge;
+    // the chunks come as the view of a row-major tensor that encode(use_dct=False) gives, which decode takes as it is:
+    // without the transform it has nothing to copy, with it the rows are as good to read as whole chunks
     at::Tensor out = rows ? fresh({R, C}, c10::ScalarType::Float, *pl.like)
-                          : fresh({Y, X, kEdge, kEdge}, c10::ScalarType::Float, *pl.like);
+                          : at::empty_strided({Y, X, kEdge, kEdge}, {kEdge * C, kEdge, C, 1},
+                                              at::TensorOptions().dtype(c10::ScalarType::Float).device(pl.like->device()));
     if (int st = p_tplr_decode_aggregate(pl.idx, pl.val, scale, pl.peers, static_cast<int>(pl.k), R, C, TPLR_REDUCE_MEAN, 0, dct,
-                                         out.data_ptr<float>(), rows ? C : 0, nullptr, on.stream()))
+                                         out.data_ptr<float>(), C, nullptr, on.stream()))
         return failed(st, "tplr_decode_aggregate");
     return THPVariable_Wrap(std::move(out));
 }
@@ -473,7 +493,7 @@ PyObject* decompress(PyObject*, PyObject* const* args, Py_ssize_t n) {
 PyMethodDef methods[] = {
     {"bind", reinterpret_cast<PyCFunction>(reinterpret_cast<void*>(bind)), METH_FASTCALL, nullptr},
     {"encode", reinterpret_cast<PyCFunction>(reinterpret_cast<void*>(encode)), METH_FASTCALL, nullptr},
-    {"decode", decode, METH_O, nullptr},
+    {"decode", reinterpret_cast<PyCFunction>(reinterpret_cast<void*>(decode)), METH_FASTCALL, nullptr},
     {"compress", reinterpret_cast<PyCFunction>(reinterpret_cast<void*>(compress)), METH_FASTCALL, nullptr},
     {"quantize", reinterpret_cast<PyCFunction>(reinterpret_cast<void*>(quantize)), METH_FASTCALL, nullptr},
     {"dequantize", reinterpret_cast<PyCFunction>(reinterpret_cast<void*>(dequantize)), METH_FASTCALL, nullptr},

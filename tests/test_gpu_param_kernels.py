@@ -180,3 +180,18 @@ def test_quantisers_of_two_threads_do_not_meet(dev):
     [t.start() for t in threads]
     [t.join() for t in threads]
     assert not wrong
+
+
+@pytest.mark.parametrize("Y,X", [(1, 1), (1, 3), (3, 1), (2, 5)])
+def test_decode_of_row_major_and_chunked_coefficients(dev, Y, X):
+    tr = tc.ChunkingTransformer(torch.nn.Linear(64 * X, 64 * Y, bias=False, device=dev), 64)
+    flat = torch.from_numpy(np.random.default_rng(Y * 7 + X).standard_normal((64 * Y, 64 * X + 64)).astype(np.float32)).to(dev)
+    for rows in (flat[:, :64 * X].contiguous(), flat[:, :64 * X]):  # without and with a gap between the rows
+        view = rows.reshape(Y, 64, X, 64).permute(0, 2, 1, 3) if rows.is_contiguous() else \
+            torch.as_strided(rows, (Y, X, 64, 64), (64 * rows.stride(0), 64, rows.stride(0), 1))
+        for use_dct in (True, False):
+            assert torch.equal(tr.decode(view, use_dct=use_dct), tr.decode(view.contiguous(), use_dct=use_dct))
+    # what decompress leaves is such a view: without the transform decode has nothing to copy
+    idx = torch.from_numpy(orc.pack12(np.tile(np.arange(4) * 1000, (Y * X, 1)))).to(dev)
+    dense = tc.TopKCompressor().decompress(rows, idx, torch.ones(Y, X, 4, device=dev), (Y, X, 64, 64), 4096)
+    assert dense.shape == (Y, X, 64, 64) and tr.decode(dense, use_dct=False).data_ptr() == dense.data_ptr()
