@@ -181,6 +181,20 @@ int tplr_decode_aggregate(const uint8_t* const* h_idx12, const float* const* h_v
                           int64_t R, int64_t C, int reduce_mode, int normalise, int use_dct,
                           float* d_out, int64_t ld_out, float* d_sumsq, void* stream);
 
+/* batch_decompress of one parameter without the transform (mean; src/tplr/compress.py:483-580), clip factors and all:
+ * d_norms (nullable) holds n_norms >= n_peers norms, peer p's factor is min(1, median of them all / (norm p + 1e-8)) and
+ * d_scale is scratch of n_norms floats; without d_norms d_scale (nullable) holds the n_peers factors themselves.  Output
+ * as tplr_decode_aggregate with use_dct == 0, and the same bits as tplr_clip_scales and that call. */
+int tplr_aggregate_param(const uint8_t* const* h_idx12, const float* const* h_val, const float* d_norms, int n_norms,
+                         float* d_scale, int n_peers, int k, int64_t R, int64_t C, float* d_out, int64_t ld_out,
+                         void* stream);
+
+/* decompress of one parameter from a quantiser's codes (:443-481 with :637-643): value = d_lookup[code] + *d_shift, a
+ * code past the table taken as its last.  k <= 64, d_out aligned to 16 bytes, ld_out a multiple of 4; output layout as
+ * tplr_decode_aggregate with use_dct == 0, and the same bits as tplr_dequantize_lists and that call. */
+int tplr_decompress_codes(const uint8_t* d_idx12, const uint8_t* d_codes, const float* d_lookup, const float* d_shift,
+                          int n_bins, int k, int64_t R, int64_t C, float* d_out, int64_t ld_out, void* stream);
+
 /* The same over a whole gradient set in ONE launch (the per-parameter loop of
  * src/tplr/neurons.py:309-367): every peer's payload is flat over the batch
  * (tplr_tensor_desc), results go to each descriptor's `dense` tensor ((R, C) with row stride

@@ -48,6 +48,8 @@ SIGNATURES = {
     "tplr_row_sumsq": (_i32, [_vp, _i32, _i32, _i64, _vp, _vp]),
     "tplr_clip_scales_rows": (_i32, [_vp, _i32, _vp, _i32, _i32, _vp, _vp, _vp, _vp]),
     "tplr_decode_aggregate": (_i32, [_vp, _vp, _vp, _i32, _i32, _i64, _i64, _i32, _i32, _i32, _vp, _i64, _vp, _vp]),
+    "tplr_aggregate_param": (_i32, [_vp, _vp, _vp, _i32, _vp, _i32, _i32, _i64, _i64, _vp, _i64, _vp]),
+    "tplr_decompress_codes": (_i32, [_vp, _vp, _vp, _vp, _i32, _i32, _i64, _i64, _vp, _i64, _vp]),
     "tplr_scatter_rows": (_i32, [_vp, _vp, _vp, _i64, _i64, _i64, _i32, _vp, _vp, _vp]),
     "tplr_decompress_rows": (_i32, [_vp, _vp, _i64, _i32, _i64, _vp, _vp, _vp]),
     "tplr_flat_update": (_i32, [_vp, _vp, _i64, C.c_float, _i32, _vp]),

@@ -30,7 +30,7 @@ namespace {
 // ---- the library's entry points ---------------------------------------------------------------
 #define TPLR_NATIVE_ENTRIES(X)                                                                                       \
     X(tplr_status_string) X(tplr_dct2d_fwd) X(tplr_dct2d_inv_rows) X(tplr_dct2d_inv) X(tplr_dct1d) X(tplr_topk_pack) X(tplr_encode_topk_pack) \
-    X(tplr_decode_aggregate) X(tplr_decompress_rows) X(tplr_clip_scales) X(tplr_peer_sumsq) X(tplr_quantize) X(tplr_dequantize_lists)
+    X(tplr_decode_aggregate) X(tplr_aggregate_param) X(tplr_decompress_codes) X(tplr_decompress_rows) X(tplr_clip_scales) X(tplr_peer_sumsq) X(tplr_quantize) X(tplr_dequantize_lists)
 #define X(name) decltype(&::name) p_##name = nullptr;
 TPLR_NATIVE_ENTRIES(X)
 #undef X
@@ -351,16 +351,26 @@ struct Payloads {
     const at::Tensor* like;
 };
 
-PyObject* scatter_chunks(const Payloads& pl, const float* scale, int64_t Y, int64_t X, bool rows, bool dct, const Launch& on) {
+// The coefficients as the (Y, X, 64, 64) view of a row-major tensor that encode(use_dct=False) gives, which decode takes
+// as it is: without the transform it has nothing to copy, with it the rows are as good to read as whole chunks.
+at::Tensor chunk_tensor(int64_t Y, int64_t X, const at::Tensor& like) {
+    return at::empty_strided({Y, X, kEdge, kEdge}, {kEdge * X * kEdge, kEdge, X * kEdge, 1},
+                             at::TensorOptions().dtype(c10::ScalarType::Float).device(like.device()));
+}
+
+// norms (n_norms of them) with scale as scratch, or scale (nullable) the factors themselves
+PyObject* scatter_chunks(const Payloads& pl, const float* norms, int64_t n_norms, float* scale, int64_t Y, int64_t X, bool rows,
+                         bool dct, const Launch& on) {
     const int64_t R = Y * kEdge, C = X * kEdge;
-    // the chunks come as the view of a row-major tensor that encode(use_dct=False) gives, which decode takes as it is:
-    // without the transform it has nothing to copy, with it the rows are as good to read as whole chunks
-    at::Tensor out = rows ? fresh({R, C}, c10::ScalarType::Float, *pl.like)
-                          : at::empty_strided({Y, X, kEdge, kEdge}, {kEdge * C, kEdge, C, 1},
-                                              at::TensorOptions().dtype(c10::ScalarType::Float).device(pl.like->device()));
-    if (int st = p_tplr_decode_aggregate(pl.idx, pl.val, scale, pl.peers, static_cast<int>(pl.k), R, C, TPLR_REDUCE_MEAN, 0, dct,
-                                         out.data_ptr<float>(), C, nullptr, on.stream()))
-        return failed(st, "tplr_decode_aggregate");
+    at::Tensor out = rows ? fresh({R, C}, c10::ScalarType::Float, *pl.like) : chunk_tensor(Y, X, *pl.like);
+    if (dct && norms)
+        if (int st = p_tplr_clip_scales(norms, static_cast<int>(n_norms), 0, scale, nullptr, on.stream()))
+            return failed(st, "tplr_clip_scales");
+    const int st = dct ? p_tplr_decode_aggregate(pl.idx, pl.val, scale, pl.peers, static_cast<int>(pl.k), R, C, TPLR_REDUCE_MEAN, 0,
+                                                 1, out.data_ptr<float>(), C, nullptr, on.stream())
+                       : p_tplr_aggregate_param(pl.idx, pl.val, norms, static_cast<int>(n_norms), scale, pl.peers,
+                                                static_cast<int>(pl.k), R, C, out.data_ptr<float>(), C, on.stream());
+    if (st) return failed(st, dct ? "tplr_decode_aggregate" : "tplr_aggregate_param");
     return THPVariable_Wrap(std::move(out));
 }
 
@@ -393,6 +403,8 @@ PyObject* aggregate(PyObject*, PyObject* const* args, Py_ssize_t n) {
     }
     Launch on(*like);
     at::Tensor scale;
+    const float* given = nullptr;
+    int64_t n_given = 0;
     if (clip) {
         if (args[4] != Py_None) {
             const at::Tensor* norms = plain_f32(args[4]);
@@ -400,10 +412,9 @@ PyObject* aggregate(PyObject*, PyObject* const* args, Py_ssize_t n) {
             if (!norms || norms->dim() != 1 || norms->numel() < P || norms->numel() > TPLR_MAX_PEERS || !norms->is_contiguous() ||
                 norms->device() != like->device())
                 Py_RETURN_NONE;
-            scale = fresh({norms->numel()}, c10::ScalarType::Float, *like);
-            if (int st = p_tplr_clip_scales(norms->const_data_ptr<float>(), static_cast<int>(norms->numel()), 0,
-                                            scale.data_ptr<float>(), nullptr, on.stream()))
-                return failed(st, "tplr_clip_scales");
+            n_given = norms->numel();
+            given = norms->const_data_ptr<float>();
+            scale = fresh({n_given}, c10::ScalarType::Float, *like);
         } else {
             const int64_t count = Y * X * pl.k;
             // about 32 K values per block, so that one large tensor still spreads over the device
@@ -417,7 +428,7 @@ PyObject* aggregate(PyObject*, PyObject* const* args, Py_ssize_t n) {
                 return failed(st, "tplr_clip_scales");
         }
     }
-    return scatter_chunks(pl, clip ? scale.const_data_ptr<float>() : nullptr, Y, X, rows, dct, on);
+    return scatter_chunks(pl, given, n_given, clip ? scale.data_ptr<float>() : nullptr, Y, X, rows, dct, on);
     END_HANDLE_TH_ERRORS
 }
 
@@ -459,6 +470,15 @@ PyObject* decompress(PyObject*, PyObject* const* args, Py_ssize_t n) {
             s->device() != like->device() || l->device() != like->device() ||
             reinterpret_cast<uintptr_t>(sent->const_data_ptr()) % 4 != 0)
             Py_RETURN_NONE;
+        if (chunks && k <= 64 && shape[0] * shape[1] <= 0xfffff0) {
+            at::Tensor out = chunk_tensor(shape[0], shape[1], *like);
+            const int64_t C = shape[1] * kEdge;
+            if (int st = p_tplr_decompress_codes(idx->const_data_ptr<uint8_t>(), sent->const_data_ptr<uint8_t>(),
+                                                 l->const_data_ptr<float>(), s->const_data_ptr<float>(), static_cast<int>(l->numel()),
+                                                 static_cast<int>(k), shape[0] * kEdge, C, out.data_ptr<float>(), C, on.stream()))
+                return failed(st, "tplr_decompress_codes");
+            return THPVariable_Wrap(std::move(out));
+        }
         values = fresh({count}, c10::ScalarType::Float, *like);
         const uint8_t* codes = sent->const_data_ptr<uint8_t>();
         const float *lookup = l->const_data_ptr<float>(), *shift = s->const_data_ptr<float>();
@@ -476,7 +496,7 @@ PyObject* decompress(PyObject*, PyObject* const* args, Py_ssize_t n) {
         pl.like = like;
         pl.idx[0] = idx->const_data_ptr<uint8_t>();
         pl.val[0] = val;
-        return scatter_chunks(pl, nullptr, shape[0], shape[1], false, false, on);
+        return scatter_chunks(pl, nullptr, 0, nullptr, shape[0], shape[1], false, false, on);
     }
     at::Tensor out = fresh(shape, c10::ScalarType::Float, *like);
     at::Tensor flag = at::empty({1}, at::TensorOptions().dtype(c10::ScalarType::Int).pinned_memory(true));

@@ -1,4 +1,6 @@
 """Kernels behind the reference's per-parameter calls, at the sizes where their tilings can go wrong."""
+import ctypes
+
 import numpy as np
 import pytest
 import torch
@@ -195,3 +197,71 @@ def test_decode_of_row_major_and_chunked_coefficients(dev, Y, X):
     idx = torch.from_numpy(orc.pack12(np.tile(np.arange(4) * 1000, (Y * X, 1)))).to(dev)
     dense = tc.TopKCompressor().decompress(rows, idx, torch.ones(Y, X, 4, device=dev), (Y, X, 64, 64), 4096)
     assert dense.shape == (Y, X, 64, 64) and tr.decode(dense, use_dct=False).data_ptr() == dense.data_ptr()
+
+
+def _payloads(dev, P, n, k, rng, repeats=False):
+    idx, val = [], []
+    for _ in range(P):
+        i = np.stack([rng.permutation(4096)[:k] for _ in range(n)]).astype(np.int64)
+        i[:, : k // 2] = np.arange(k // 2) * 61 % 4096  # shared by all peers (61 is odd: distinct)
+        if repeats:
+            i[n - 1, : max(2, k // 4)] = 4095
+        else:
+            for r in range(n):  # the other half distinct from it
+                rest = np.setdiff1d(rng.permutation(4096)[: 2 * k], i[r, : k // 2])
+                i[r, k // 2:] = rng.permutation(rest)[: k - k // 2]
+        idx.append(torch.from_numpy(orc.pack12(i)).to(dev))
+        val.append(torch.from_numpy(rng.standard_normal((n, k)).astype(np.float32)).to(dev))
+    return idx, val
+
+
+@pytest.mark.parametrize("repeats", [False, True])
+@pytest.mark.parametrize("P,k,Y,X", [(1, 2, 1, 1), (1, 64, 3, 5), (4, 32, 1, 9), (5, 32, 3, 3), (8, 64, 1, 1), (9, 2, 2, 3), (15, 32, 3, 5),
+                                     (16, 64, 2, 2), (17, 32, 1, 3), (24, 64, 3, 3), (25, 32, 2, 2), (3, 66, 2, 2)])
+def test_param_aggregate_is_the_two_launches(dev, P, k, Y, X, repeats):
+    """tplr_aggregate_param leaves the bits of tplr_clip_scales and tplr_decode_aggregate, in either layout."""
+    lib, rng, n = _lib.load(), np.random.default_rng(P * 100 + k), Y * X
+    idx, val = _payloads(dev, P, n, k, rng, repeats)
+    ptrs = lambda ts: (ctypes.c_void_p * P)(*[t.data_ptr() for t in ts])  # noqa: E731
+    ip, vp = ptrs(idx), ptrs(val)
+    stream = torch.cuda.current_stream(dev).cuda_stream
+    norms = rng.gamma(2.0, 1.0, P + 3).astype(np.float32)
+    cases = {"plain": norms[:P], "more": norms, "ties": np.round(norms[:P]) + 1.0, "nan": np.where(np.arange(P) == P // 2, np.nan, norms[:P]),
+             "inf": np.where(np.arange(P) == 0, np.inf, norms[:P]), "zero": np.zeros(P), "negative": norms[:P] - 2.0, "factors": None,
+             "none": None}
+    for name, given in cases.items():
+        for ld in (X * 64, 0):
+            scale = torch.from_numpy(norms[:P].copy()).to(dev) if name != "none" else None
+            got, want = torch.full((2, n * 4096), 7.0, device=dev)
+            gn, m = None, 0
+            if given is not None:
+                gn = torch.from_numpy(np.asarray(given, np.float32)).to(dev)
+                m = gn.numel()
+                scale = torch.empty(m, device=dev)
+            sp = scale.data_ptr() if scale is not None else None
+            _lib.check(lib.tplr_aggregate_param(ip, vp, gn.data_ptr() if m else None, m, sp, P, k, Y * 64, X * 64, got.data_ptr(), ld,
+                                                stream), "tplr_aggregate_param")
+            if m:
+                _lib.check(lib.tplr_clip_scales(gn.data_ptr(), m, 0, sp, None, stream), "tplr_clip_scales")
+            _lib.check(lib.tplr_decode_aggregate(ip, vp, sp, P, k, Y * 64, X * 64, 0, 0, 0, want.data_ptr(), ld, None, stream),
+                       "tplr_decode_aggregate")
+            same = (got.view(torch.int32) == want.view(torch.int32)) | (got.isnan() & want.isnan())
+            assert bool(same.all()), (name, ld)
+
+
+@pytest.mark.parametrize("bins,k,Y,X", [(1, 2, 1, 1), (4, 64, 3, 5), (8, 32, 1, 9), (255, 62, 2, 3), (256, 64, 5, 1)])
+def test_decompress_from_codes_is_the_two_launches(dev, bins, k, Y, X):
+    lib, rng, n = _lib.load(), np.random.default_rng(bins + k), Y * X
+    (idx,), _ = _payloads(dev, 1, n, k, rng)
+    codes = torch.from_numpy(rng.integers(0, 256, (n, k)).astype(np.uint8)).to(dev)  # codes past the table among them
+    lookup, shift = torch.randn(bins, device=dev), torch.randn((), device=dev)
+    stream = torch.cuda.current_stream(dev).cuda_stream
+    one = lambda t: (ctypes.c_void_p * 1)(t.data_ptr())  # noqa: E731
+    val = lookup[codes.long().clamp(max=bins - 1)] + shift
+    for ld in (X * 64, 0):
+        got, want = torch.full((2, n * 4096), 7.0, device=dev)
+        _lib.check(lib.tplr_decompress_codes(idx.data_ptr(), codes.data_ptr(), lookup.data_ptr(), shift.data_ptr(), bins, k, Y * 64,
+                                             X * 64, got.data_ptr(), ld, stream), "tplr_decompress_codes")
+        _lib.check(lib.tplr_decode_aggregate(one(idx), one(val), None, 1, k, Y * 64, X * 64, 0, 0, 0, want.data_ptr(), ld, None,
+                                             stream), "tplr_decode_aggregate")
+        assert torch.equal(got.view(torch.int32), want.view(torch.int32)), ld
