@@ -21,6 +21,7 @@
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/python_variable.h>
 
+#include <chrono>
 #include <vector>
 
 #include "../../include/tplr_hip.h"
@@ -81,6 +82,8 @@ at::Tensor fresh(at::IntArrayRef sizes, c10::ScalarType type, const at::Tensor& 
     return at::empty(sizes, at::TensorOptions().dtype(type).device(like.device()));
 }
 
+constexpr uint32_t kUnset = 0xffffffffu;  // as a float a NaN, which the quantiser's scale never is
+
 // launches go to the tensor's device and that device's current stream
 struct Launch {
     int before, here;
@@ -91,13 +94,26 @@ struct Launch {
         if (before != here) c10::hip::set_device(before);
     }
     void* stream() const { return c10::hip::getCurrentHIPStream(here).stream(); }
-    // wait for the stream, other Python threads running meanwhile
+    // other Python threads run meanwhile
+    struct Released {
+        PyThreadState* state = PyEval_SaveThread();
+        ~Released() { PyEval_RestoreThread(state); }
+    };
+    // wait for the stream
     void wait() const {
-        struct Released {
-            PyThreadState* state = PyEval_SaveThread();
-            ~Released() { PyEval_RestoreThread(state); }
-        } released;
+        Released released;
         c10::hip::getCurrentHIPStream(here).unwrap().synchronize();
+    }
+    // wait until a kernel of the stream has stored something else than kUnset in a word of pinned memory, which it does
+    // with a system-scope store; for the stream where half a millisecond does not bring it (work queued before, an error)
+    void wait_for(const uint32_t* word) const {
+        Released released;
+        const auto give_up = std::chrono::steady_clock::now() + std::chrono::microseconds(500);
+        while (__atomic_load_n(word, __ATOMIC_ACQUIRE) == kUnset)
+            if (std::chrono::steady_clock::now() > give_up) {
+                c10::hip::getCurrentHIPStream(here).unwrap().synchronize();
+                return;
+            }
     }
 };
 
@@ -210,15 +226,17 @@ PyObject* quantised(const at::Tensor& val, int64_t n_bins, double range, const L
     at::Tensor shift = fresh({}, c10::ScalarType::Float, val), lookup = fresh({n_bins}, c10::ScalarType::Float, val);
     // a workgroup per 1024 values (one load per thread), one per compute unit at most
     const int64_t slices = n / 1024 < 1 ? 1 : n / 1024 > 256 ? 256 : n / 1024;
-    at::Tensor work = fresh({slices * (2 + 2 * n_bins)}, c10::ScalarType::Double, val);
-    // the scale is the one figure that travels to the host (float(scale), src/tplr/compress.py:620): the kernel stores it
-    // in pinned memory, which the stream's end makes visible
+    at::Tensor work = fresh({slices * (2 + 2 * n_bins) + 1}, c10::ScalarType::Double, val);
+    // the scale is the one figure that travels to the host (float(scale), src/tplr/compress.py:620): the second launch
+    // stores it in pinned memory as it begins, and only that store is waited for
     at::Tensor scale = at::empty({1}, at::TensorOptions().dtype(c10::ScalarType::Float).pinned_memory(true));
+    uint32_t* const word = reinterpret_cast<uint32_t*>(scale.data_ptr<float>());
+    __atomic_store_n(word, kUnset, __ATOMIC_RELAXED);
     if (int st = p_tplr_quantize(val.const_data_ptr<float>(), n, static_cast<int>(n_bins), static_cast<float>(range),
                                  static_cast<int>(slices), work.data_ptr<double>(), codes.data_ptr<uint8_t>(),
                                  shift.data_ptr<float>(), scale.data_ptr<float>(), lookup.data_ptr<float>(), on.stream()))
         return failed(st, "tplr_quantize");
-    on.wait();
+    on.wait_for(word);
     return Py_BuildValue("(N(NdLNO))", THPVariable_Wrap(std::move(codes)), THPVariable_Wrap(std::move(shift)),
                          static_cast<double>(*scale.const_data_ptr<float>()), static_cast<long long>(n_bins / 2),
                          THPVariable_Wrap(std::move(lookup)), float32_dtype);

@@ -11,7 +11,8 @@
 
 namespace tplr {
 
-// Three launches over slices of every tensor: the moments, the codes with per-bin sums, the tables.  Partial sums are
+// Three launches over slices of every tensor: the moments, the codes with per-bin sums, the tables (of one tensor two: the
+// workgroup that finishes its codes last makes the table, which saves a launch of 4 us).  Partial sums are
 // carried in double, kept per (tensor, slice) in a caller-provided workspace and added in a fixed order by whoever
 // needs the total, so every workgroup of a tensor derives the same shift and scale.
 // Workspace layout (doubles): moments[T][S][2], then bins[T][S][2 * n_bins] (sums, counts).
@@ -64,12 +65,39 @@ __device__ __forceinline__ void quant_shift_scale(const double* work, int t, int
     scale = (sc == 0.f || sc != sc || __builtin_isinf(sc)) ? 1.0f : sc;                 // :599-600
 }
 
+// Doubles that another workgroup of the same launch reads: stored to and loaded from where the whole device sees them.
+// (Ordinary stores with a release and an acquire around them write back and invalidate an XCD's whole L2 per workgroup:
+// 20 us for 256 of them.)
+__device__ __forceinline__ void device_store(double* p, double x) {
+    __hip_atomic_store(p, x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ double device_load(const double* p) {
+    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// the mean of bin `bin` from the slices' sums and counts, dealt over the lanes of a wave (:619)
+__device__ __forceinline__ float quant_bin_mean(const double* bins, int S, int n_bins, int bin) {
+    double sum = 0.0, cnt = 0.0;
+    for (int s = threadIdx.x & 63; s < S; s += 64)
+        sum += device_load(bins + s * 2 * n_bins + bin), cnt += device_load(bins + s * 2 * n_bins + n_bins + bin);
+    sum = wave_sum_f64(sum);
+    cnt = wave_sum_f64(cnt);
+    return cnt > 0.0 ? static_cast<float>(sum / cnt) : 0.f;
+}
+
+// One tensor's results where its codes are made (k_quant_codes), instead of a launch of their own.
+struct QuantOne {
+    uint32_t* done;  // slices finished, zeroed by k_quant_moments; null: k_quant_tables follows
+    float *shift, *scale, *lookup;
+};
+
 __global__ __launch_bounds__(256) void k_quant_moments(const float* __restrict__ val, int k,
                                                        const tplr_tensor_desc* __restrict__ table,
                                                        const tplr_tensor_desc single, int S,
-                                                       double* __restrict__ work) {
+                                                       double* __restrict__ work, uint32_t* __restrict__ done) {
     __shared__ double part[2][4];
     const int tid = threadIdx.x;
+    if (done && blockIdx.x == 0 && tid == 0) *done = 0u;
     const QuantSlice qs = quant_slice(val, nullptr, table, single, k, S);
     const double first = static_cast<double>(qs.first);
     double s1 = 0.0, s2 = 0.0;
@@ -95,11 +123,16 @@ __global__ __launch_bounds__(256) void k_quant_codes(const float* __restrict__ v
                                                      const tplr_tensor_desc* __restrict__ table,
                                                      const tplr_tensor_desc single, int T, int S, int n_bins,
                                                      float range_in_sigmas, uint8_t* __restrict__ codes,
-                                                     double* __restrict__ work) {
+                                                     double* __restrict__ work, const QuantOne one) {
     const int tid = threadIdx.x;
     const QuantSlice qs = quant_slice(val, codes, table, single, k, S);
     float shift, scale;
     quant_shift_scale(work, qs.t, S, qs.n, qs.first, n_bins, range_in_sigmas, shift, scale);
+    if (one.done && blockIdx.x == 0 && tid == 0) {
+        *one.shift = shift;
+        // (the caller may be watching for it in pinned host memory while this launch goes on)
+        __hip_atomic_store(one.scale, scale, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    }
     double* out = work + 2 * static_cast<int64_t>(T) * S + static_cast<int64_t>(blockIdx.x) * 2 * n_bins;
     const float offset = static_cast<float>(n_bins / 2), top = static_cast<float>(n_bins - 1);
     auto code = [&](float x, float& c) {
@@ -140,8 +173,8 @@ __global__ __launch_bounds__(256) void k_quant_codes(const float* __restrict__ v
         }
         __syncthreads();
         if (tid < n_bins) {
-            out[tid] = (sums[0][tid] + sums[1][tid]) + (sums[2][tid] + sums[3][tid]);
-            out[n_bins + tid] = static_cast<double>(counts[0][tid] + counts[1][tid] + counts[2][tid] + counts[3][tid]);
+            device_store(out + tid, (sums[0][tid] + sums[1][tid]) + (sums[2][tid] + sums[3][tid]));
+            device_store(out + n_bins + tid, static_cast<double>(counts[0][tid] + counts[1][tid] + counts[2][tid] + counts[3][tid]));
         }
     } else {
         __shared__ double bin_sum[256];
@@ -160,22 +193,33 @@ __global__ __launch_bounds__(256) void k_quant_codes(const float* __restrict__ v
             atomicAdd(&bin_sum[q3], static_cast<double>(c3)), atomicAdd(&bin_cnt[q3], 1u);
         }
         __syncthreads();
-        if (tid < n_bins) out[tid] = bin_sum[tid], out[n_bins + tid] = static_cast<double>(bin_cnt[tid]);
+        if (tid < n_bins) device_store(out + tid, bin_sum[tid]), device_store(out + n_bins + tid, static_cast<double>(bin_cnt[tid]));
+    }
+    if (one.done) {  // uniform: the workgroup that finishes last, whichever that is, makes the table
+        __shared__ uint32_t before;
+        // every wave's sums have reached the device's memory before the workgroup's arrival is counted
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        __syncthreads();
+        if (tid == 0) before = __hip_atomic_fetch_add(one.done, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __syncthreads();
+        if (before == static_cast<uint32_t>(S) - 1u) {  // (so all have arrived, and the loads below are behind that)
+            const double* bins = work + 2 * static_cast<int64_t>(T) * S;
+            for (int bin = tid >> 6; bin < n_bins; bin += 4) {
+                const float mean = quant_bin_mean(bins, S, n_bins, bin);
+                if ((tid & 63) == 0) one.lookup[bin] = mean;
+            }
+        }
     }
 }
 
-// One wave per bin of tensor blockIdx.y (the slices' sums dealt over the lanes), and wave 0 of bin 0 the scalars.
+// One wave per bin of tensor blockIdx.y, and wave 0 of bin 0 the scalars.
 __global__ __launch_bounds__(64) void k_quant_tables(const float* __restrict__ val, const tplr_tensor_desc* __restrict__ table,
                                                      const tplr_tensor_desc single, int k, int T, int S, int n_bins, float range_in_sigmas,
                                                      const double* __restrict__ work, float* __restrict__ shift_out,
                                                      float* __restrict__ scale_out, float* __restrict__ lookup) {
     const int t = blockIdx.y, bin = blockIdx.x, lane = threadIdx.x;
-    const double* bins = work + 2 * static_cast<int64_t>(T) * S + static_cast<int64_t>(t) * S * 2 * n_bins;
-    double sum = 0.0, cnt = 0.0;
-    for (int s = lane; s < S; s += 64) sum += bins[s * 2 * n_bins + bin], cnt += bins[s * 2 * n_bins + n_bins + bin];
-    sum = wave_sum_f64(sum);
-    cnt = wave_sum_f64(cnt);
-    if (lane == 0) lookup[static_cast<int64_t>(t) * n_bins + bin] = cnt > 0.0 ? static_cast<float>(sum / cnt) : 0.f;  // :619
+    const float mean = quant_bin_mean(work + 2 * static_cast<int64_t>(T) * S + static_cast<int64_t>(t) * S * 2 * n_bins, S, n_bins, bin);
+    if (lane == 0) lookup[static_cast<int64_t>(t) * n_bins + bin] = mean;
     if (bin == 0) {  // wave-uniform
         const tplr_tensor_desc d = table ? table[t] : single;
         const int64_t n = static_cast<int64_t>(d.x_chunks) * d.y_chunks * k;
@@ -270,13 +314,14 @@ __global__ __launch_bounds__(256) void k_dequantize_lists(const DeqLists pp, int
 
 static int launch_quantize(const float* d_val, int k, const tplr_tensor_desc* d_desc, const tplr_tensor_desc& single, int n_tensors, int n_bins,
                            float range_in_sigmas, int n_slices, double* d_work, uint8_t* d_codes, float* d_shift,
-                           float* d_scale, float* d_lookup, void* stream) {
+                           float* d_scale, float* d_lookup, void* stream, uint32_t* done = nullptr) {
     const dim3 grid(static_cast<unsigned>(n_tensors) * n_slices), block(256);
     hipStream_t st = static_cast<hipStream_t>(stream);
-    hipLaunchKernelGGL(k_quant_moments, grid, block, 0, st, d_val, k, d_desc, single, n_slices, d_work);
+    const QuantOne one = {done, d_shift, d_scale, d_lookup};
+    hipLaunchKernelGGL(k_quant_moments, grid, block, 0, st, d_val, k, d_desc, single, n_slices, d_work, done);
     hipLaunchKernelGGL(n_bins <= 4 ? k_quant_codes<4> : n_bins <= 8 ? k_quant_codes<8> : k_quant_codes<0>, grid, block, 0, st,
-                       d_val, k, d_desc, single, n_tensors, n_slices, n_bins, range_in_sigmas, d_codes, d_work);
-    hipLaunchKernelGGL(k_quant_tables, dim3(static_cast<unsigned>(n_bins), static_cast<unsigned>(n_tensors)), dim3(64), 0, st,
+                       d_val, k, d_desc, single, n_tensors, n_slices, n_bins, range_in_sigmas, d_codes, d_work, one);
+    if (!done) hipLaunchKernelGGL(k_quant_tables, dim3(static_cast<unsigned>(n_bins), static_cast<unsigned>(n_tensors)), dim3(64), 0, st,
                        d_val, d_desc, single, k, n_tensors, n_slices, n_bins, range_in_sigmas, d_work, d_shift, d_scale, d_lookup);
     return launch_status();
 }
@@ -366,8 +411,9 @@ int tplr_quantize(const float* d_val, int64_t n, int n_bins, float range_in_sigm
     tplr_tensor_desc single = {};
     single.x_chunks = static_cast<int32_t>(n / 4);  // rows of four values
     single.y_chunks = 1;
+    uint32_t* done = reinterpret_cast<uint32_t*>(d_work + static_cast<int64_t>(n_slices) * (2 + 2 * n_bins));
     return launch_quantize(d_val, 4, nullptr, single, 1, n_bins, range_in_sigmas, n_slices, d_work, d_codes, d_shift, d_scale,
-                           d_lookup, stream);
+                           d_lookup, stream, done);
 }
 
 int tplr_dequantize_batch(const uint8_t* d_codes, const float* d_lookup, const float* d_shift, int n_bins, int k,

@@ -265,3 +265,28 @@ def test_decompress_from_codes_is_the_two_launches(dev, bins, k, Y, X):
         _lib.check(lib.tplr_decode_aggregate(one(idx), one(val), None, 1, k, Y * 64, X * 64, 0, 0, 0, want.data_ptr(), ld, None,
                                              stream), "tplr_decode_aggregate")
         assert torch.equal(got.view(torch.int32), want.view(torch.int32)), ld
+
+
+@pytest.mark.parametrize("n,bins,slices", [(4, 4, 1), (1020, 1, 1), (2052, 8, 2), (65536, 4, 64), (262144, 4, 256), (70000, 256, 68)])
+def test_quantiser_of_one_tensor_is_the_batch_of_one(dev, n, bins, slices):
+    """The table made by the workgroup that finishes last, and queued behind other work: the bits of the three launches."""
+    lib = _lib.load()
+    stream = torch.cuda.current_stream(dev).cuda_stream
+    v = torch.from_numpy(np.random.default_rng(n).standard_t(3, n).astype(np.float32)).to(dev)
+    desc = torch.tensor([0, 0, 0, (n // 4) | (1 << 32)], dtype=torch.int64, device=dev)  # rows of four values: n / 4 x 1 of them
+    size = slices * (2 + 2 * bins)
+    outs = []
+    for one in (True, False) * 3:
+        work = torch.full((size + 1,), -1.0, dtype=torch.float64, device=dev)
+        codes, out = torch.empty(n, dtype=torch.uint8, device=dev), torch.empty(2 + bins, device=dev)
+        ptr = [t.data_ptr() for t in (codes, out, out[1:], out[2:])]
+        if one:
+            _lib.check(lib.tplr_quantize(v.data_ptr(), n, bins, 6.0, slices, work.data_ptr(), *ptr, stream), "tplr_quantize")
+        else:
+            _lib.check(lib.tplr_quantize_batch(v.data_ptr(), 4, desc.data_ptr(), 1, bins, 6.0, slices, work.data_ptr(), *ptr, stream),
+                       "tplr_quantize_batch")
+        outs.append((codes, out))
+    for codes, out in outs[1:]:
+        assert torch.equal(codes, outs[0][0])
+        # the sums in LDS of more than eight bins are added in no fixed order: sums in double, one rounding to fp32
+        assert torch.equal(out, outs[0][1]) if bins <= 8 else torch.allclose(out, outs[0][1], rtol=2.0 ** -22, atol=1e-9)
