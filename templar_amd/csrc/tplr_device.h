@@ -882,4 +882,26 @@ __device__ __forceinline__ uint32_t load_idx12(BytePtr row, int j) {
     return (j & 1) ? (w >> 4) : (w & 0xfffu);
 }
 
+typedef uint16_t __attribute__((aligned(1))) unaligned_u16;
+using gu16 = __attribute__((address_space(1))) unaligned_u16;
+
+// Lane i's clip factor min(1, median / (norm_i + 1e-8)) of n <= 64 norms, lane i holding norm i: what k_clip_scales
+// makes of them (the lower of the two middle values; NaN as soon as one norm is NaN, :535, :553-556).
+__device__ __forceinline__ float lane_clip_factor(float mine, int n, int lane) {
+    // ranks in a total order without a branch: ascending, NaN after everything, ties by lane
+    const uint32_t b = __float_as_uint(mine + 0.0f);
+    const uint32_t key = mine != mine ? 0xffffffffu : b ^ ((b >> 31) ? 0xffffffffu : 0x80000000u);
+    uint32_t rank = 0;
+    for (int j = 0; j < n; ++j) {
+        const uint32_t other = __builtin_amdgcn_readlane(key, j);
+        rank += other < key || (other == key && j < lane) ? 1u : 0u;
+    }
+    const bool any_nan = __ballot(lane < n && mine != mine) != 0;
+    const uint64_t at = __ballot(lane < n && rank == static_cast<uint32_t>(n - 1) / 2);  // exactly one lane
+    float med = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, mine), __builtin_ctzll(at)));
+    if (any_nan) med = __builtin_nanf("");
+    const float f = med / (mine + 1e-8f);
+    return f > 1.0f ? 1.0f : f;
+}
+
 }  // namespace tplr

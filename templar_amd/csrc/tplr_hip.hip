@@ -463,8 +463,6 @@ struct PeerPtrs {
 
 __device__ __forceinline__ int tile_pos(uint32_t idx) { return (idx >> 6) * kLd + (idx & 63); }
 
-typedef uint16_t __attribute__((aligned(1))) unaligned_u16;
-using gu16 = __attribute__((address_space(1))) unaligned_u16;
 typedef uint32_t __attribute__((aligned(1))) unaligned_u32;
 using gu32 = __attribute__((address_space(1))) unaligned_u32;
 
@@ -576,6 +574,10 @@ __global__ __launch_bounds__((64 * aggregate_team<kUseDct, kUnits, kWideK, !kCod
     // floats per chunk, the sum of squares of the result and the sum of its elements
     const bool normalise = (options & 1) != 0;
     const bool with_sum = (options & 2) != 0;
+    // bit 2 (one tensor on the fast path without the transform): `scale` holds options >> 8 norms, at most 64, and every
+    // wave makes the clip factors from them itself - 3 us less than a launch of k_clip_scales in front
+    constexpr bool kFromNorms = kUnits > 0 && !kUseDct && !kCodes && !kSubtract;
+    const bool from_norms = kFromNorms && (options & 4) != 0;
     // per-chunk statistics of the result in registers (v: a column per lane); a chunk that is to be done
     // again on the exact path writes them there
     auto chunk_stats = [&](const float (&v)[64], int64_t g, bool skip) {
@@ -663,6 +665,11 @@ __global__ __launch_bounds__((64 * aggregate_team<kUseDct, kUnits, kWideK, !kCod
     const uint64_t my_val = kFast ? reinterpret_cast<uint64_t>(pp.val[pl]) : 0;
     float my_scale = out_scale;
     int t_scale = -1;  // tensor whose clip factors my_scale holds
+    if (from_norms) {  // wave-uniform
+        const int n = options >> 8;
+        my_scale = lane_clip_factor(scale[lane < n ? lane : 0], n, lane) * out_scale;
+        t_scale = 0;
+    }
     auto lane_bcast64 = [&](uint64_t mine, int i) -> uint64_t {
         const uint32_t lo = __builtin_amdgcn_readlane(static_cast<int>(static_cast<uint32_t>(mine)), i);
         const uint32_t hi = __builtin_amdgcn_readlane(static_cast<int>(static_cast<uint32_t>(mine >> 32)), i);
@@ -920,7 +927,9 @@ __global__ __launch_bounds__((64 * aggregate_team<kUseDct, kUnits, kWideK, !kCod
                     for (int j = lane; j < k; j += 64) ss += vrow[j] * vrow[j];
                     nrm = __builtin_sqrtf(wave_sum_f32(ss)) + 1e-8f;
                 }
-                const float sc = scale ? scale[static_cast<int64_t>(t_now) * P + p] : 1.0f;
+                const float sc = from_norms ? __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, my_scale), p))
+                                 : scale    ? scale[static_cast<int64_t>(t_now) * P + p]
+                                            : 1.0f;
 #pragma unroll 1
                 for (int j0 = 0; j0 < k; j0 += 64) {
                     const int j = j0 + lane;
@@ -4179,3 +4188,15 @@ int tplr_calib_fill(void* d_dst, int64_t n_bytes, int pattern, void* stream) {
 }
 
 }  // extern "C"
+
+int tplr::aggregate_from_norms(const uint8_t* const* h_idx12, const float* const* h_val, const float* d_norms, int n_norms,
+                               int n_peers, int k, int64_t R, int64_t C, float* d_out, int64_t ld_out, void* stream) {
+    tplr_tensor_desc single;
+    single.dense = d_out;
+    single.ld = ld_out;
+    single.chunk_begin = 0;
+    single.x_chunks = static_cast<int32_t>(C / 64);
+    single.y_chunks = static_cast<int32_t>(R / 64);
+    return launch_decode(h_idx12, h_val, d_norms, n_peers, k, nullptr, single, 1, (R / 64) * (C / 64), TPLR_REDUCE_MEAN,
+                         4 | n_norms << 8, 0, nullptr, stream);
+}

@@ -30,4 +30,9 @@ int persistent_grid(Kernel kernel, int64_t total, int threads = 64) {
     return static_cast<int>(need < g ? need : g);
 }
 
+// The persistent aggregate of one parameter (k <= 64, at most 24 peers, mean, no transform) with the clip factors made from
+// n_norms <= 64 norms inside the launch; the arguments checked by the caller (tplr_aggregate_param).
+int aggregate_from_norms(const uint8_t* const* h_idx12, const float* const* h_val, const float* d_norms, int n_norms, int n_peers,
+                         int k, int64_t R, int64_t C, float* d_out, int64_t ld_out, void* stream);
+
 }  // namespace tplr

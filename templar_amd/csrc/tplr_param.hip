@@ -13,12 +13,9 @@ constexpr int kParamPeers = 24;  // payloads of one launch
 constexpr int kParamNorms = 64;  // norms that one wave ranks
 // Chunks times peers up to which a chunk per workgroup is the faster way: beyond it the scatters, of which every wave
 // issues all and keeps a quarter, fill the compute units' LDS pipelines.  Clip factors and aggregate in us, this kernel
-// against k_clip_scales and k_decode_aggregate: 1024 chunks of 15 peers 9.1 : 12.3, 2048 of 20 16.7 : 17.5, 4096 of 5
-// 15.8 : 19.2, 16 384 of 1 48.1 : 54.4 - but 4096 of 15 22.9 : 22.7, 4096 of 20 28.3 : 25.5, 16 384 of 5 65 : 58.
-constexpr int64_t kParamWork = 49152;
-
-typedef uint16_t __attribute__((aligned(1))) unaligned_u16;
-using gu16 = __attribute__((address_space(1))) unaligned_u16;
+// against k_decode_aggregate that makes the factors itself: 1024 chunks of 15 peers 9.1 : 10.3, of 20 10.5 : 11.5, 4096
+// of 5 15.8 : 17.5, 16 384 of 1 48.2 : 53.5 - but 2048 of 15 13.9 : 13.5, of 20 16.7 : 14.8, 4096 of 15 22.9 : 20.6.
+constexpr int64_t kParamWork = 24576;
 
 struct ParamPeer {
     const uint8_t* idx;
@@ -27,25 +24,6 @@ struct ParamPeer {
 struct ParamPeers {
     ParamPeer peer[kParamPeers];  // those past the last repeat it: a wave fetches its peers' pointers without looking
 };
-
-// Lane i's clip factor min(1, median / (norm_i + 1e-8)) of n <= 64 norms, lane i holding norm i: what k_clip_scales
-// makes of them (the lower of the two middle values; NaN as soon as one norm is NaN, :535, :553-556).
-__device__ __forceinline__ float lane_clip_factor(float mine, int n, int lane) {
-    // ranks in a total order without a branch: ascending, NaN after everything, ties by lane
-    const uint32_t b = __float_as_uint(mine + 0.0f);
-    const uint32_t key = mine != mine ? 0xffffffffu : b ^ ((b >> 31) ? 0xffffffffu : 0x80000000u);
-    uint32_t rank = 0;
-    for (int j = 0; j < n; ++j) {
-        const uint32_t other = __builtin_amdgcn_readlane(key, j);
-        rank += other < key || (other == key && j < lane) ? 1u : 0u;
-    }
-    const bool any_nan = __ballot(lane < n && mine != mine) != 0;
-    const uint64_t at = __ballot(lane < n && rank == static_cast<uint32_t>(n - 1) / 2);  // exactly one lane
-    float med = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, mine), __builtin_ctzll(at)));
-    if (any_nan) med = __builtin_nanf("");
-    const float f = med / (mine + 1e-8f);
-    return f > 1.0f ? 1.0f : f;
-}
 
 // The aggregate of one parameter's chunks, without the transform.  A workgroup of four waves takes one chunk and wave w
 // its rows 16 w .. 16 w + 15.  What bounds it is the chain of one wave - payload, scatters in peer order, mean, stores -
@@ -247,6 +225,8 @@ extern "C" int tplr_aggregate_param(const uint8_t* const* h_idx12, const float* 
         }
         return launch_param<false>(pp, d_scale, d_norms, n_norms, n_peers, k, nullptr, nullptr, 0, C / 64, n, ld_out, d_out, stream);
     }
+    if (d_norms && n_peers <= kParamPeers && k <= 64 && n_norms <= kParamNorms)
+        return aggregate_from_norms(h_idx12, h_val, d_norms, n_norms, n_peers, k, R, C, d_out, ld_out, stream);
     if (d_norms)
         if (int s = tplr_clip_scales(d_norms, n_norms, 0, d_scale, nullptr, stream)) return s;
     return tplr_decode_aggregate(h_idx12, h_val, d_scale, n_peers, k, R, C, TPLR_REDUCE_MEAN, 0, 0, d_out, ld_out, nullptr, stream);

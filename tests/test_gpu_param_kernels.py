@@ -290,3 +290,27 @@ def test_quantiser_of_one_tensor_is_the_batch_of_one(dev, n, bins, slices):
         assert torch.equal(codes, outs[0][0])
         # the sums in LDS of more than eight bins are added in no fixed order: sums in double, one rounding to fp32
         assert torch.equal(out, outs[0][1]) if bins <= 8 else torch.allclose(out, outs[0][1], rtol=2.0 ** -22, atol=1e-9)
+
+
+@pytest.mark.parametrize("repeats", [False, True])
+@pytest.mark.parametrize("P,k", [(6, 64), (13, 32), (24, 64)])
+def test_large_param_aggregate_is_the_two_launches(dev, P, k, repeats):
+    """The same where the parameter is large for a chunk per workgroup: the persistent launch makes the factors itself."""
+    Y, X = 64, 130
+    assert Y * X * P > 24576
+    lib, n = _lib.load(), Y * X
+    idx, val = _payloads(dev, P, 65, k, np.random.default_rng(P), repeats)
+    idx = [i.reshape(65, -1).repeat(n // 65, 1).reshape(-1) for i in idx]  # the rows over and over
+    val = [v.repeat(n // 65, 1) for v in val]
+    ptrs = lambda ts: (ctypes.c_void_p * P)(*[t.data_ptr() for t in ts])  # noqa: E731
+    ip, vp = ptrs(idx), ptrs(val)
+    stream = torch.cuda.current_stream(dev).cuda_stream
+    norms = torch.rand(P + 2, device=dev) + 0.1
+    for m in (P, P + 2):
+        scale, (got, want) = torch.empty(m, device=dev), torch.full((2, n * 4096), 7.0, device=dev)
+        _lib.check(lib.tplr_aggregate_param(ip, vp, norms.data_ptr(), m, scale.data_ptr(), P, k, Y * 64, X * 64, got.data_ptr(), X * 64,
+                                            stream), "tplr_aggregate_param")
+        _lib.check(lib.tplr_clip_scales(norms.data_ptr(), m, 0, scale.data_ptr(), None, stream), "tplr_clip_scales")
+        _lib.check(lib.tplr_decode_aggregate(ip, vp, scale.data_ptr(), P, k, Y * 64, X * 64, 0, 0, 0, want.data_ptr(), X * 64, None,
+                                             stream), "tplr_decode_aggregate")
+        assert torch.equal(got.view(torch.int32), want.view(torch.int32)), m
