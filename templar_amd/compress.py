@@ -785,7 +785,7 @@ class TopKCompressor:
     @torch.no_grad()
     def _quantize_values(self, val: torch.Tensor) -> tuple[torch.Tensor, QuantParamsT]:
         half = self.n_bins // 2
-        # three launches (sums in double) instead of a dozen reductions and scatters; the scale is the only value that
+        # two launches (sums in double) instead of a dozen reductions and scatters; the scale is the only value that
         # travels to the host, as in the reference (float(scale), :620)
         out = _lib.native().quantize(val if val.is_contiguous() else val.contiguous(), self.n_bins, self.range_in_sigmas)
         if out is not None:
