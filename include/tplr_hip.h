@@ -105,10 +105,6 @@ int tplr_dct2d_fwd(const float* d_x, int64_t R, int64_t C, int64_t ld_x, float* 
  * einsum :222): d_coef (R/64, C/64, 64, 64) -> d_x (R, C), x[y,x] = F coef[y,x] F^T. */
 int tplr_dct2d_inv(const float* d_coef, int64_t R, int64_t C, float* d_x, int64_t ld_x, void* stream);
 
-/* The same from coefficients that lie as a row-major (R, C) tensor with row stride ld_coef (coefficient (b, d) of chunk
- * (y, x) at row 64 y + b, column 64 x + d): 16-byte aligned, ld_coef a multiple of 4. */
-int tplr_dct2d_inv_rows(const float* d_coef, int64_t ld_coef, int64_t R, int64_t C, float* d_x, int64_t ld_x, void* stream);
-
 /* 1-D tensors (src/tplr/compress.py:248-255, :283-290): n_vec rows of 64 floats,
  * each row r <- r @ F (inverse = 0) or r @ F^T (inverse = 1). */
 int tplr_dct1d(const float* d_in, int64_t n_vec, int inverse, float* d_out, void* stream);

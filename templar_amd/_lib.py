@@ -31,7 +31,6 @@ SIGNATURES = {
     "tplr_gather_host": (_i32, [_vp, _vp, _i64, _vp, _i32]),
     "tplr_dct2d_fwd": (_i32, [_vp, _i64, _i64, _i64, _vp, _vp]),
     "tplr_dct2d_inv": (_i32, [_vp, _i64, _i64, _vp, _i64, _vp]),
-    "tplr_dct2d_inv_rows": (_i32, [_vp, _i64, _i64, _i64, _vp, _i64, _vp]),
     "tplr_dct1d": (_i32, [_vp, _i64, _i32, _vp, _vp]),
     "tplr_dct2d_dense": (_i32, [_vp, _i64, _i64, _i32, _i32, _vp, _vp, _i32, _i32, _vp, _vp]),
     "tplr_topk_pack": (_i32, [_vp, _i64, _i64, _i32, _vp, _vp, _vp]),

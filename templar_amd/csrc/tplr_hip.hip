@@ -283,26 +283,14 @@ __global__ __launch_bounds__(64) void k_dct2d_fwd(const float* __restrict__ x, i
     tile_to_flat(tile, coef + chunk * 4096, lane);
 }
 
-// kRows: the coefficients lie as a row-major (R, C) tensor of row stride ld_coef - the (Y, X, 64, 64) view of one,
-// as decompress leaves it - instead of chunk after chunk
-template <bool kRows>
-__global__ __launch_bounds__(64) void k_dct2d_inv(const float* __restrict__ coef, int64_t ld_coef, int64_t X,
-                                                  int64_t n_chunks, float* __restrict__ x, int64_t ld) {
+__global__ __launch_bounds__(64) void k_dct2d_inv(const float* __restrict__ coef, int64_t X, int64_t n_chunks,
+                                                  float* __restrict__ x, int64_t ld) {
     __shared__ __align__(16) float tile[kTileFloats];
     const int lane = threadIdx.x;
     const int64_t chunk = xcd_contiguous(blockIdx.x, gridDim.x);
     if (chunk >= n_chunks) return;
     const int64_t y = chunk / X, xc = chunk - y * X;
-    if (kRows) {
-        const float* chunk0 = coef + (y * 64) * ld_coef + xc * 64;
-#pragma unroll
-        for (int c = 0; c < 16; ++c) {
-            const int q = c * 64 + lane, r = q >> 4, col = (q & 15) << 2;
-            *reinterpret_cast<float4*>(tile + r * kLd + col) = *reinterpret_cast<const float4*>(chunk0 + r * ld_coef + col);
-        }
-    } else {
-        flat_to_tile(coef + chunk * 4096, tile, lane);
-    }
+    flat_to_tile(coef + chunk * 4096, tile, lane);
     wave_lds_fence();
     float v[64];
     chunk_inverse<true, true>(v, tile, lane);
@@ -3291,18 +3279,7 @@ int tplr_dct2d_inv(const float* d_coef, int64_t R, int64_t C, float* d_x, int64_
     if (!ld_ok(ld_x)) return TPLR_E_TOOMANY;
     const int64_t n = (R / 64) * (C / 64);
     if (n == 0) return 0;
-    hipLaunchKernelGGL(k_dct2d_inv<false>, dim3(grid8(n)), dim3(64), 0, static_cast<hipStream_t>(stream), d_coef,
-                       int64_t{0}, C / 64, n, d_x, ld_x);
-    return launch_status();
-}
-
-int tplr_dct2d_inv_rows(const float* d_coef, int64_t ld_coef, int64_t R, int64_t C, float* d_x, int64_t ld_x, void* stream) {
-    if (int s = check_2d(d_x, d_coef, R, C)) return s;
-    if (ld_x < C || ld_coef < C || (ld_coef & 3) || (reinterpret_cast<uintptr_t>(d_coef) & 15)) return TPLR_E_BADARG;
-    if (!ld_ok(ld_x)) return TPLR_E_TOOMANY;
-    const int64_t n = (R / 64) * (C / 64);
-    if (n == 0) return 0;
-    hipLaunchKernelGGL(k_dct2d_inv<true>, dim3(grid8(n)), dim3(64), 0, static_cast<hipStream_t>(stream), d_coef, ld_coef,
+    hipLaunchKernelGGL(k_dct2d_inv, dim3(grid8(n)), dim3(64), 0, static_cast<hipStream_t>(stream), d_coef,
                        C / 64, n, d_x, ld_x);
     return launch_status();
 }

@@ -30,7 +30,7 @@ namespace {
 
 // ---- the library's entry points ---------------------------------------------------------------
 #define TPLR_NATIVE_ENTRIES(X)                                                                                       \
-    X(tplr_status_string) X(tplr_dct2d_fwd) X(tplr_dct2d_inv_rows) X(tplr_dct2d_inv) X(tplr_dct1d) X(tplr_topk_pack) X(tplr_encode_topk_pack) \
+    X(tplr_status_string) X(tplr_dct2d_fwd) X(tplr_dct2d_inv) X(tplr_dct1d) X(tplr_topk_pack) X(tplr_encode_topk_pack) \
     X(tplr_decode_aggregate) X(tplr_aggregate_param) X(tplr_decompress_codes) X(tplr_decompress_rows) X(tplr_clip_scales) X(tplr_peer_sumsq) X(tplr_quantize) X(tplr_dequantize_lists)
 #define X(name) decltype(&::name) p_##name = nullptr;
 TPLR_NATIVE_ENTRIES(X)
@@ -191,21 +191,17 @@ PyObject* decode(PyObject*, PyObject* const* args, Py_ssize_t n) {
     if (n != 2) return PyErr_SetString(PyExc_TypeError, "decode(x, use_dct)"), nullptr;
     const at::Tensor* x = plain_f32(args[0]);
     if (!x || x->numel() == 0) Py_RETURN_NONE;
-    const bool view = chunk_view(*x);
     if (args[1] != Py_True) {  // a change of shape: of a view of the tensor itself, the tensor
-        if (!view || x->requires_grad()) Py_RETURN_NONE;
+        if (!chunk_view(*x) || x->requires_grad()) Py_RETURN_NONE;
         return THPVariable_Wrap(x->as_strided({x->size(0) * kEdge, x->size(1) * kEdge}, {x->stride(2), 1}));
     }
     Launch on(*x);
     if (x->dim() == 4 && x->size(2) == kEdge && x->size(3) == kEdge) {
         const int64_t R = x->size(0) * kEdge, C = x->size(1) * kEdge;
-        const bool aligned = x->stride(2) % 4 == 0 && reinterpret_cast<uintptr_t>(x->const_data_ptr()) % 16 == 0;
-        if (!x->is_contiguous() && !(view && aligned)) Py_RETURN_NONE;
+        if (!x->is_contiguous()) Py_RETURN_NONE;
         at::Tensor out = fresh({R, C}, c10::ScalarType::Float, *x);
-        const int st = x->is_contiguous()
-                           ? p_tplr_dct2d_inv(x->const_data_ptr<float>(), R, C, out.data_ptr<float>(), C, on.stream())
-                           : p_tplr_dct2d_inv_rows(x->const_data_ptr<float>(), x->stride(2), R, C, out.data_ptr<float>(), C, on.stream());
-        if (st) return failed(st, "tplr_dct2d_inv");
+        if (int st = p_tplr_dct2d_inv(x->const_data_ptr<float>(), R, C, out.data_ptr<float>(), C, on.stream()))
+            return failed(st, "tplr_dct2d_inv");
         return THPVariable_Wrap(std::move(out));
     }
     if (x->dim() == 2 && x->size(1) == kEdge && x->is_contiguous()) {
@@ -369,11 +365,11 @@ struct Payloads {
     const at::Tensor* like;
 };
 
-// The coefficients as the (Y, X, 64, 64) view of a row-major tensor that encode(use_dct=False) gives, which decode takes
-// as it is: without the transform it has nothing to copy, with it the rows are as good to read as whole chunks.
+// The coefficients chunk after chunk, contiguous on every route: a caller may flatten them in place (view) or hand them
+// on as chunks, and what decode(use_dct=False) makes of them is a tensor of its own (a row-major layout would save that
+// copy, but share the storage).
 at::Tensor chunk_tensor(int64_t Y, int64_t X, const at::Tensor& like) {
-    return at::empty_strided({Y, X, kEdge, kEdge}, {kEdge * X * kEdge, kEdge, X * kEdge, 1},
-                             at::TensorOptions().dtype(c10::ScalarType::Float).device(like.device()));
+    return fresh({Y, X, kEdge, kEdge}, c10::ScalarType::Float, like);
 }
 
 // norms (n_norms of them) with scale as scratch, or scale (nullable) the factors themselves
@@ -381,13 +377,14 @@ PyObject* scatter_chunks(const Payloads& pl, const float* norms, int64_t n_norms
                          bool dct, const Launch& on) {
     const int64_t R = Y * kEdge, C = X * kEdge;
     at::Tensor out = rows ? fresh({R, C}, c10::ScalarType::Float, *pl.like) : chunk_tensor(Y, X, *pl.like);
+    const int64_t ld = rows ? C : 0;
     if (dct && norms)
         if (int st = p_tplr_clip_scales(norms, static_cast<int>(n_norms), 0, scale, nullptr, on.stream()))
             return failed(st, "tplr_clip_scales");
     const int st = dct ? p_tplr_decode_aggregate(pl.idx, pl.val, scale, pl.peers, static_cast<int>(pl.k), R, C, TPLR_REDUCE_MEAN, 0,
-                                                 1, out.data_ptr<float>(), C, nullptr, on.stream())
+                                                 1, out.data_ptr<float>(), ld, nullptr, on.stream())
                        : p_tplr_aggregate_param(pl.idx, pl.val, norms, static_cast<int>(n_norms), scale, pl.peers,
-                                                static_cast<int>(pl.k), R, C, out.data_ptr<float>(), C, on.stream());
+                                                static_cast<int>(pl.k), R, C, out.data_ptr<float>(), ld, on.stream());
     if (st) return failed(st, dct ? "tplr_decode_aggregate" : "tplr_aggregate_param");
     return THPVariable_Wrap(std::move(out));
 }
@@ -490,10 +487,10 @@ PyObject* decompress(PyObject*, PyObject* const* args, Py_ssize_t n) {
             Py_RETURN_NONE;
         if (chunks && k <= 64 && shape[0] * shape[1] <= 0xfffff0) {
             at::Tensor out = chunk_tensor(shape[0], shape[1], *like);
-            const int64_t C = shape[1] * kEdge;
             if (int st = p_tplr_decompress_codes(idx->const_data_ptr<uint8_t>(), sent->const_data_ptr<uint8_t>(),
                                                  l->const_data_ptr<float>(), s->const_data_ptr<float>(), static_cast<int>(l->numel()),
-                                                 static_cast<int>(k), shape[0] * kEdge, C, out.data_ptr<float>(), C, on.stream()))
+                                                 static_cast<int>(k), shape[0] * kEdge, shape[1] * kEdge, out.data_ptr<float>(), 0,
+                                                 on.stream()))
                 return failed(st, "tplr_decompress_codes");
             return THPVariable_Wrap(std::move(out));
         }

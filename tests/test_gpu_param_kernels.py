@@ -193,10 +193,50 @@ def test_decode_of_row_major_and_chunked_coefficients(dev, Y, X):
             torch.as_strided(rows, (Y, X, 64, 64), (64 * rows.stride(0), 64, rows.stride(0), 1))
         for use_dct in (True, False):
             assert torch.equal(tr.decode(view, use_dct=use_dct), tr.decode(view.contiguous(), use_dct=use_dct))
-    # what decompress leaves is such a view: without the transform decode has nothing to copy
-    idx = torch.from_numpy(orc.pack12(np.tile(np.arange(4) * 1000, (Y * X, 1)))).to(dev)
-    dense = tc.TopKCompressor().decompress(rows, idx, torch.ones(Y, X, 4, device=dev), (Y, X, 64, 64), 4096)
-    assert dense.shape == (Y, X, 64, 64) and tr.decode(dense, use_dct=False).data_ptr() == dense.data_ptr()
+
+
+@pytest.mark.parametrize("Y,X", [(1, 1), (1, 3), (3, 1), (2, 5), (40, 64)])
+@pytest.mark.parametrize("k,P", [(4, 1), (32, 3), (64, 15), (66, 2), (32, 25)])
+def test_dense_results_are_contiguous_on_every_route(dev, Y, X, k, P):
+    """Plain payloads, from codes, converted ones: contiguous chunks, and decode without the transform of them a copy."""
+    rng, n = np.random.default_rng(Y * 100 + X + k), Y * X
+    idx = torch.from_numpy(orc.pack12(np.stack([rng.permutation(4096)[:k] for _ in range(n)]).astype(np.int64))).to(dev)
+    vals = [torch.from_numpy(rng.standard_normal((Y, X, k)).astype(np.float32)).to(dev) for _ in range(P)]
+    shape, p = torch.Size((Y, X, 64, 64)), torch.empty(Y * 64, X * 64, device=dev)
+    tr = tc.ChunkingTransformer(torch.nn.Linear(64 * X, 64 * Y, bias=False, device=dev), 64)
+    plain, coder = tc.TopKCompressor(), tc.TopKCompressor(use_quantization=True, quantization_bins=4)
+    codes, qp = coder._quantize_values(vals[0])
+    norms = torch.rand(P, device=dev) + 0.5
+    groups = [[plain.decompress(p, idx, vals[0], shape, 4096), plain.decompress(p, idx, vals[0], list(shape), 4096)],
+              [coder.decompress(p, idx, codes, shape, 4096, qp), coder.decompress(p, idx, codes, shape, 4096, list(qp))]]
+    for kw in (dict(clip_norm=False), dict(block_norms=norms), dict()):
+        groups.append([plain.batch_decompress(p, [idx] * P, vals, shape, 4096, **kw),
+                       plain.batch_decompress(p, tuple([idx] * P), tuple(vals), list(shape), 4096, **kw)])
+    for same in groups:
+        for dense in same:
+            assert dense.shape == shape and dense.is_contiguous() and dense.view(-1).numel() == n * 4096
+            assert torch.equal(dense, same[0])
+            before, grad = dense.clone(), tr.decode(dense, use_dct=False)
+            assert torch.equal(grad, before.permute(0, 2, 1, 3).reshape(Y * 64, X * 64))
+            if X > 1:  # (a single column of chunks lies as the tensor does: the reference's rearrange is a view there too)
+                grad.mul_(0.5).add_(1.0)
+                assert torch.equal(dense, before)
+
+
+def test_parameter_of_more_columns_than_a_row_stride_holds(dev):
+    """Chunked results have no row stride, and so none of its limit of 2^23 floats."""
+    X = (1 << 17) + 2
+    shape, p = (1, X, 64, 64), torch.empty(1, device=dev)
+    idx = torch.from_numpy(orc.pack12(np.array([[5, 4094]]))).to(dev).repeat(X)
+    val = torch.arange(1.0, 2 * X + 1, device=dev).view(1, X, 2)
+    plain, coder = tc.TopKCompressor(), tc.TopKCompressor(use_quantization=True, quantization_bins=4)
+    codes, qp = torch.tensor([1, 3], dtype=torch.uint8, device=dev).expand(1, X, 2).contiguous(), \
+        (torch.tensor(0.5, device=dev), 1.0, 2, torch.arange(4.0, device=dev), torch.float32)
+    for call, want in ((lambda: plain.decompress(p, idx, val, shape, 4096), val),
+                       (lambda: plain.batch_decompress(p, [idx] * 2, [val] * 2, shape, 4096, clip_norm=False), val),
+                       (lambda: coder.decompress(p, idx, codes, shape, 4096, qp), torch.tensor([1.5, 3.5], device=dev))):
+        flat = call().view(X, 4096)
+        assert bool((flat[:, [5, 4094]] == want).all()) and int(torch.count_nonzero(flat)) == 2 * X
 
 
 def _payloads(dev, P, n, k, rng, repeats=False):
