@@ -11,6 +11,9 @@ inline int launch_status() {
     return e == hipSuccess ? 0 : static_cast<int>(e);
 }
 
+// workgroups of 256 threads in one launch, which has fewer than 2^32 threads
+constexpr int64_t kMaxGroups256 = 0xfffff0;
+
 inline unsigned grid8(int64_t n) { return static_cast<unsigned>(((n + 7) / 8) * 8); }
 
 // persistent grids: exactly one resident set of workgroups of `threads` threads (one wave, or a team of

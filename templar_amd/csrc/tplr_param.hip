@@ -241,7 +241,7 @@ extern "C" int tplr_decompress_codes(const uint8_t* d_idx12, const uint8_t* d_co
     if ((ld_out != 0 && ld_out < C) || (ld_out & 3) || (reinterpret_cast<uintptr_t>(d_out) & 15)) return TPLR_E_BADARG;
     const int64_t n = (R / 64) * (C / 64);
     if (n == 0) return 0;
-    if (n > 0xfffff0) return TPLR_E_TOOMANY;  // (a launch has fewer than 2^32 threads)
+    if (n > kMaxGroups256) return TPLR_E_TOOMANY;
     ParamPeers pp = {};
     for (ParamPeer& p : pp.peer) p = {d_idx12, d_codes};
     return launch_param<true>(pp, nullptr, nullptr, 0, 1, k, d_lookup, d_shift, n_bins, C / 64, n, ld_out, d_out, stream);

@@ -457,11 +457,16 @@ int tplr_encode_rows_batch(const tplr_tensor_desc* d_desc, int n_tensors, int64_
     return launch_status();
 }
 
+// (a workgroup of 256 per row, and a launch has fewer than 2^32 threads: more rows than kMaxGroups256 go in several)
 static int scatter_packed(const uint8_t* d_idx12, const float* d_val, int64_t n_rows, int k, int row_len, int reduce_mode,
                           float* d_out, int32_t* d_err, int32_t* flag, void* stream) {
     const bool vec = (row_len & 3) == 0 && (reinterpret_cast<uintptr_t>(d_out) & 15) == 0;
-    hipLaunchKernelGGL(vec ? k_scatter_rows_packed<true> : k_scatter_rows_packed<false>, dim3(static_cast<unsigned>(n_rows)),
-                       dim3(256), 0, static_cast<hipStream_t>(stream), d_idx12, d_val, k, row_len, reduce_mode, d_out, d_err, flag);
+    for (int64_t r = 0; r < n_rows; r += kMaxGroups256) {
+        const int64_t rows = n_rows - r < kMaxGroups256 ? n_rows - r : kMaxGroups256;
+        hipLaunchKernelGGL(vec ? k_scatter_rows_packed<true> : k_scatter_rows_packed<false>, dim3(static_cast<unsigned>(rows)),
+                           dim3(256), 0, static_cast<hipStream_t>(stream), d_idx12 + r * (k + (k >> 1)), d_val + r * k, k, row_len,
+                           reduce_mode, d_out + r * row_len, d_err, flag);
+    }
     return launch_status();
 }
 

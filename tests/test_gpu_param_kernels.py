@@ -84,6 +84,21 @@ def test_scatter_into_rows(dev, n, k, repeats):
     assert np.array_equal(got.cpu().numpy(), want)
 
 
+def test_scatter_into_more_rows_than_one_launch_takes(dev):
+    # a workgroup of 256 threads per row: 2^24 rows are 2^32 threads
+    n = (1 << 24) + 21
+    val = torch.arange(2.0 * n, device=dev).view(n, 2)  # (exact: below 2^26, rounded alike on both sides)
+    idx = torch.from_numpy(orc.pack12(np.array([[3, 1]]))).to(dev).repeat(n)
+    want = torch.zeros(n, 5, device=dev)
+    want[:, 3], want[:, 1] = val[:, 0], val[:, 1]
+    assert torch.equal(tc.TopKCompressor().decompress(val, idx, val, (n, 5), 5), want)
+    assert torch.equal(tc._scatter_rows(idx, val, n, 2, 5), want)
+    idx.view(-1, 3)[-1] = torch.from_numpy(orc.pack12(np.array([[3, 7]]))).to(dev)
+    for call in (lambda: tc._scatter_rows(idx, val, n, 2, 5), lambda: tc.TopKCompressor().decompress(val, idx, val, (n, 5), 5)):
+        with pytest.raises(RuntimeError, match="index 7 is out of bounds"):
+            call()
+
+
 @pytest.mark.parametrize("inverse", [0, 1])
 @pytest.mark.parametrize("n_vec", [1, 3, 4, 5, 32, 63, 16384, 16385])
 def test_vectors_transform_alike_in_both_forms(dev, n_vec, inverse):
