@@ -232,15 +232,15 @@ __global__ __launch_bounds__(64) void k_dct1d(const float* __restrict__ in, int6
 // scan of the table is a chain of dependent loads, and took longer than the rest of the launch.  The 25 norm vectors of
 // a 150M model (300 rows) take 7.8 us; a wave per 64 rows, every lane sorting a row of its own in registers, 10.1 us.
 template <bool kUseDct>
-__global__ __launch_bounds__(256) void k_encode_rows(const tplr_tensor_desc* __restrict__ table, int n_tensors, int k,
-                                                     uint8_t* __restrict__ idx12, float* __restrict__ val) {
+__global__ __launch_bounds__(256) void k_encode_rows(const tplr_tensor_desc* __restrict__ table, int n_tensors, int64_t first_group,
+                                                     int k, uint8_t* __restrict__ idx12, float* __restrict__ val) {
     constexpr int kPerWave = 4, kPerGroup = 64 / (4 * kPerWave);  // workgroups per group of 64 rows
     __shared__ __align__(16) float tile_all[4][kPerWave * kLd];
     const int lane = threadIdx.x & 63;
     const int wv = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
     float* const tile = tile_all[wv];
     // this workgroup's tensor and group of rows: tensor t has ceil(rows / 64) groups
-    int t = -1, grp = static_cast<int>(blockIdx.x / kPerGroup);
+    int t = -1, grp = static_cast<int>(first_group + blockIdx.x / kPerGroup);
     for (int t0 = 0; t0 < n_tensors && t < 0; t0 += 64) {  // (64 tensors a turn)
         const uint32_t groups = t0 + lane < n_tensors ? static_cast<uint32_t>((table[t0 + lane].x_chunks + 63) >> 6) : 0u;
         const uint32_t incl = wave_incl_scan_u32(groups);
@@ -446,14 +446,13 @@ int tplr_encode_rows_batch(const tplr_tensor_desc* d_desc, int n_tensors, int64_
     if (!d_desc || n_tensors < 1 || total_groups < 0 || !d_idx12 || !d_val || k < 2 || (k & 1) || k > 64)
         return TPLR_E_BADARG;
     if (total_groups == 0) return 0;
-    if (total_groups > 0x1fffffff) return TPLR_E_TOOMANY;
-    const dim3 grid(static_cast<unsigned>(total_groups * 4)), block(256);  // 16 rows each
-    if (use_dct)
-        hipLaunchKernelGGL(k_encode_rows<true>, grid, block, 0, static_cast<hipStream_t>(stream), d_desc, n_tensors, k,
-                           d_idx12, d_val);
-    else
-        hipLaunchKernelGGL(k_encode_rows<false>, grid, block, 0, static_cast<hipStream_t>(stream), d_desc, n_tensors, k,
-                           d_idx12, d_val);
+    if (total_groups > 0x7fffffff) return TPLR_E_TOOMANY;
+    constexpr int64_t kPiece = kMaxGroups256 / 4;  // groups of one launch: four workgroups of 256 threads each
+    for (int64_t g = 0; g < total_groups; g += kPiece) {
+        const int64_t count = total_groups - g < kPiece ? total_groups - g : kPiece;
+        hipLaunchKernelGGL(use_dct ? k_encode_rows<true> : k_encode_rows<false>, dim3(static_cast<unsigned>(count * 4)), dim3(256), 0,
+                           static_cast<hipStream_t>(stream), d_desc, n_tensors, g, k, d_idx12, d_val);
+    }
     return launch_status();
 }
 

@@ -99,6 +99,20 @@ def test_scatter_into_more_rows_than_one_launch_takes(dev):
             call()
 
 
+@pytest.mark.parametrize("use_dct", [True, False])
+def test_rows_of_a_set_of_more_groups_than_one_launch_takes(dev, use_dct):
+    # four workgroups of 256 threads per 64 rows: 2^22 groups are 2^32 threads; the same tensor over and over
+    rows, times = 1 << 16, (1 << 12) + 1
+    x = torch.randn(rows * 64, generator=torch.Generator(device=dev).manual_seed(5), device=dev)
+    want_i, want_v = tc.encode_compress_rows_batch(tc.RowBatch([x]), 2, use_dct=use_dct)
+    table = torch.tensor([[x.data_ptr(), 64, t * rows, rows | (1 << 32)] for t in range(times)], dtype=torch.int64, device=dev)
+    idx = torch.zeros(times, rows * 3, dtype=torch.uint8, device=dev)
+    val = torch.zeros(times, rows, 2, device=dev)
+    _lib.check(_lib.load().tplr_encode_rows_batch(table.data_ptr(), times, times * (rows // 64), 2, int(use_dct), idx.data_ptr(),
+                                                  val.data_ptr(), torch.cuda.current_stream(dev).cuda_stream), "tplr_encode_rows_batch")
+    assert bool((idx == want_i).all()) and bool((val == want_v).all())
+
+
 @pytest.mark.parametrize("inverse", [0, 1])
 @pytest.mark.parametrize("n_vec", [1, 3, 4, 5, 32, 63, 16384, 16385])
 def test_vectors_transform_alike_in_both_forms(dev, n_vec, inverse):
