@@ -226,11 +226,31 @@ __global__ __launch_bounds__(64) void k_dct1d(const float* __restrict__ in, int6
 }
 
 // The 1-D parameters of a set (norm vectors), every tensor a run of rows of 64 elements: transform,
-// top-k and pack of all of them in one launch, each tensor read where it lies.  A wave takes four rows of one tensor:
-// the transform and its scale exactly as k_dct1d applies them, then each row sorted across the lanes.
-// The tensor a workgroup belongs to is found with one load per lane and a prefix sum over the tensors' group counts: a
-// scan of the table is a chain of dependent loads, and took longer than the rest of the launch.  The 25 norm vectors of
-// a 150M model (300 rows) take 7.8 us; a wave per 64 rows, every lane sorting a row of its own in registers, 10.1 us.
+// top-k and pack of all of them in one launch, each tensor read where it lies.  Two forms, the same bits (of a NaN but
+// for its payload); the launcher's rule says where each is the faster one.
+//
+// The tensor that group `grp` of the set belongs to (tensor t has ceil(rows / 64) groups), `grp` becoming the group within
+// it: one load per lane and a prefix sum over the tensors' group counts - a scan of the table is a chain of dependent
+// loads, and took longer than the rest of the launch.  false where the set has no such group.
+__device__ __forceinline__ bool find_group(const tplr_tensor_desc* __restrict__ table, int n_tensors, int lane, int& t, int& grp) {
+    for (int t0 = 0; t0 < n_tensors; t0 += 64) {  // (64 tensors a turn)
+        const uint32_t groups = t0 + lane < n_tensors ? static_cast<uint32_t>((table[t0 + lane].x_chunks + 63) >> 6) : 0u;
+        const uint32_t incl = wave_incl_scan_u32(groups);
+        const uint64_t behind = __ballot(incl > static_cast<uint32_t>(grp));
+        if (behind) {
+            const int at = __builtin_ctzll(behind);
+            grp -= static_cast<int>(__builtin_amdgcn_readlane(incl - groups, at));
+            t = t0 + at;
+            return true;
+        }
+        grp -= static_cast<int>(__builtin_amdgcn_readlane(incl, 63));
+    }
+    return false;
+}
+
+// A wave takes four rows of one tensor: the transform and its scale exactly as k_dct1d applies them, then each row sorted
+// across the lanes.  What bounds it is the chain of one wave, which is short.  The 25 norm vectors of a 150M model (300
+// rows) take 8.3 us, in the other form 9.7 us.
 template <bool kUseDct>
 __global__ __launch_bounds__(256) void k_encode_rows(const tplr_tensor_desc* __restrict__ table, int n_tensors, int64_t first_group,
                                                      int k, uint8_t* __restrict__ idx12, float* __restrict__ val) {
@@ -239,21 +259,8 @@ __global__ __launch_bounds__(256) void k_encode_rows(const tplr_tensor_desc* __r
     const int lane = threadIdx.x & 63;
     const int wv = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
     float* const tile = tile_all[wv];
-    // this workgroup's tensor and group of rows: tensor t has ceil(rows / 64) groups
-    int t = -1, grp = static_cast<int>(first_group + blockIdx.x / kPerGroup);
-    for (int t0 = 0; t0 < n_tensors && t < 0; t0 += 64) {  // (64 tensors a turn)
-        const uint32_t groups = t0 + lane < n_tensors ? static_cast<uint32_t>((table[t0 + lane].x_chunks + 63) >> 6) : 0u;
-        const uint32_t incl = wave_incl_scan_u32(groups);
-        const uint64_t behind = __ballot(incl > static_cast<uint32_t>(grp));
-        if (behind) {
-            const int at = __builtin_ctzll(behind);
-            grp -= static_cast<int>(__builtin_amdgcn_readlane(incl - groups, at));
-            t = t0 + at;
-        } else {
-            grp -= static_cast<int>(__builtin_amdgcn_readlane(incl, 63));
-        }
-    }
-    if (t < 0) return;
+    int t, grp = static_cast<int>(first_group + blockIdx.x / kPerGroup);
+    if (!find_group(table, n_tensors, lane, t, grp)) return;
     const tplr_tensor_desc d = table[t];
     const int first = grp * 64 + (static_cast<int>(blockIdx.x % kPerGroup) * 4 + wv) * kPerWave;  // this wave's first row
     const int left = d.x_chunks - first;
@@ -265,6 +272,81 @@ __global__ __launch_bounds__(256) void k_encode_rows(const tplr_tensor_desc* __r
     for (int r = 0; r < kPerWave; ++r) {
         const Selected s = sort_row<false>(tile[r * kLd + lane], 0.f, true, false);
         if (r < left) emit_selected<false>(s, lane, k, row + r, idx12, val);
+    }
+}
+
+// A wave takes 64 rows of one tensor, a row per lane: every lane transforms its own, sorts its 64 coefficients in
+// registers with a bitonic network and writes its row's payload, the k leading indices and their values fetched back from
+// the tile.  No lane idles in the transform and the network needs no exchange between lanes; what bounds it is its stores,
+// 2.5 k of them a row and each to a line of its own, and that a short set leaves most SIMDs without a wave.
+template <bool kUseDct>
+__global__ __launch_bounds__(64) void k_encode_rows_lane(const tplr_tensor_desc* __restrict__ table, int n_tensors,
+                                                         int64_t first_group, int k, uint8_t* __restrict__ idx12,
+                                                         float* __restrict__ val) {
+    __shared__ __align__(16) float tile[64 * kLd];
+    const int lane = threadIdx.x;
+    int t, grp = static_cast<int>(first_group + blockIdx.x);
+    if (!find_group(table, n_tensors, lane, t, grp)) return;
+    const tplr_tensor_desc d = table[t];
+    const int left = d.x_chunks - grp * 64;  // rows from this group's first to the tensor's end
+    load_rows<64>((const gfloat*)d.dense + static_cast<int64_t>(grp) * 4096, left, tile, lane);
+    float w[64];
+    tile_rows_to_regs(w, tile, lane);
+    if (kUseDct) {  // (as transform_rows, with the result kept)
+        dct64_fwd(w);
+#pragma unroll
+        for (int d = 0; d < 64; ++d) w[d] *= 0.17677669529663687f;
+    }
+    wave_lds_fence();
+    regs_to_tile_rows(w, tile, lane);
+    // Keys (magnitude bits, 63 - index) ordered as unsigned 64-bit integers - held as doubles: for positive,
+    // normal, finite doubles the two orders are the same, and a compare-exchange is then one v_max_f64 and one
+    // v_min_f64.  One is added to the exponent field so that a zero magnitude is a normal double, and NaNs share
+    // a magnitude key just below where that addition would reach the doubles' own infinities and NaNs.
+    double key[64];
+#pragma unroll
+    for (int e = 0; e < 64; ++e) {
+        const uint32_t a = __builtin_bit_cast(uint32_t, w[e]) & 0x7fffffffu;
+        const uint32_t mag = (a > 0x7f800000u ? 0x7fdfffffu : a) + 0x00100000u;
+        key[e] = __builtin_bit_cast(double, (static_cast<uint64_t>(mag) << 32) | static_cast<uint32_t>(63 - e));
+    }
+    // bitonic sort, descending
+#pragma unroll
+    for (int size = 2; size <= 64; size <<= 1) {
+#pragma unroll
+        for (int stride = size >> 1; stride > 0; stride >>= 1) {
+#pragma unroll
+            for (int i = 0; i < 64; ++i) {
+                const int l = i ^ stride;
+                if (l > i) {
+                    const bool up = (i & size) != 0 && size < 64;  // this run ascends
+                    const double a = key[i], b = key[l];
+                    const double hi = __builtin_fmax(a, b), lo = __builtin_fmin(a, b);
+                    key[i] = up ? lo : hi;
+                    key[l] = up ? hi : lo;
+                }
+            }
+        }
+    }
+    wave_lds_fence();
+    if (lane >= left) return;
+    const int64_t row = d.chunk_begin + static_cast<int64_t>(grp) * 64 + lane;
+    float* vrow = val + row * k;
+    uint8_t* irow = idx12 + row * (k + (k >> 1));
+    const float* mine = tile + lane * kLd;
+#pragma unroll
+    for (int j = 0; j < 64; j += 2) {
+        if (j < k) {  // k is even
+            const uint32_t i0 = 63u - static_cast<uint32_t>(__builtin_bit_cast(uint64_t, key[j]));
+            const uint32_t i1 = 63u - static_cast<uint32_t>(__builtin_bit_cast(uint64_t, key[j + 1]));
+            vrow[j] = mine[i0];
+            vrow[j + 1] = mine[i1];
+            const uint32_t pair = i0 | (i1 << 12);
+            uint8_t* o = irow + 3 * (j >> 1);
+            o[0] = static_cast<uint8_t>(pair);
+            o[1] = static_cast<uint8_t>(pair >> 8);
+            o[2] = static_cast<uint8_t>(pair >> 16);
+        }
     }
 }
 
@@ -447,6 +529,23 @@ int tplr_encode_rows_batch(const tplr_tensor_desc* d_desc, int n_tensors, int64_
         return TPLR_E_BADARG;
     if (total_groups == 0) return 0;
     if (total_groups > 0x7fffffff) return TPLR_E_TOOMANY;
+    // Four rows a wave : a row a lane, in us.  With the transform 16 384 rows (256 groups) k = 2 10.5 : 8.8, k = 32 11.0 : 11.4;
+    // 24 576 rows k = 32 15.8 : 13.4, k = 48 16.2 : 17.6; 65 536 rows k = 2 32.5 : 9.6, k = 48 33.9 : 31.0, k = 64 34.7 : 38.7; 2^20
+    // rows k = 2 474 : 198, k = 48 489 : 473.  Few groups leave most compute units' instruction caches cold, which
+    // costs the four-row form more: 8 tensors of 16 rows k = 32 10.5 : 9.6, 16 groups 9.9 : 9.6 - but 32 groups 9.3 : 9.7, 25
+    // tensors of 12 rows 8.3 : 9.7, 8192 rows 7.9 : 10.2, a single row 6.1 : 8.6.  Without the transform 16 384 rows k = 2 7.2 : 7.5,
+    // 24 576 rows k = 2 9.2 : 7.7, k = 24 9.8 : 10.3, 65 536 rows k = 24 19.6 : 15.6, k = 32 19.9 : 20.1, 2^20 rows k = 24 243 : 265.
+    const int64_t n = total_groups;
+    const int most = !use_dct ? (n > 256 ? 24 : 0) : n >= 1024 ? 48 : n >= 384 ? 32 : n >= 256 ? 24 : n >= 2 && n <= 16 ? 32 : 0;
+    if (k <= most) {
+        constexpr int64_t kPiece = 4 * kMaxGroups256;  // groups of one launch: 64 threads each
+        for (int64_t g = 0; g < total_groups; g += kPiece) {
+            const int64_t count = total_groups - g < kPiece ? total_groups - g : kPiece;
+            hipLaunchKernelGGL(use_dct ? k_encode_rows_lane<true> : k_encode_rows_lane<false>, dim3(static_cast<unsigned>(count)), dim3(64),
+                               0, static_cast<hipStream_t>(stream), d_desc, n_tensors, g, k, d_idx12, d_val);
+        }
+        return launch_status();
+    }
     constexpr int64_t kPiece = kMaxGroups256 / 4;  // groups of one launch: four workgroups of 256 threads each
     for (int64_t g = 0; g < total_groups; g += kPiece) {
         const int64_t count = total_groups - g < kPiece ? total_groups - g : kPiece;

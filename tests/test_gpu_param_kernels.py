@@ -113,6 +113,29 @@ def test_rows_of_a_set_of_more_groups_than_one_launch_takes(dev, use_dct):
     assert bool((idx == want_i).all()) and bool((val == want_v).all())
 
 
+@pytest.mark.parametrize("use_dct", [True, False])
+@pytest.mark.parametrize("groups", [8, 16, 17, 255, 256, 257, 383, 384, 1023, 1024])
+def test_rows_of_a_set_alike_in_both_forms(dev, groups, use_dct):
+    # the launch changes form with the set's groups of 64 rows and with k, at k = 64 never: its leading entries are the others'
+    rows = [1, 63, 65, 64 * 70 + 1, 3] if groups > 80 else [1, 63, 65, 30, 3]
+    rows.append(64 * (groups - sum((r + 63) // 64 for r in rows)) - 5)
+    rng = np.random.default_rng(groups)
+    many = [rng.standard_normal(r * 64).astype(np.float32) for r in rows]
+    many[3][:640] = 0.0
+    many[3][640:1280] = rng.integers(-2, 3, 640)  # ties
+    many[4][70] = np.nan
+    if not use_dct:
+        many[4][[3, 90]] = np.inf, -np.inf
+    batch = tc.RowBatch([torch.from_numpy(m).to(dev) for m in many])
+    assert batch.total_groups == groups
+    idx64, val64 = tc.encode_compress_rows_batch(batch, 64, use_dct=use_dct)
+    for k in (2, 24, 26, 32, 34, 48, 50):
+        idx, val = tc.encode_compress_rows_batch(batch, k, use_dct=use_dct)
+        assert torch.equal(idx.view(-1, 3 * k // 2), idx64.view(-1, 96)[:, :3 * k // 2])
+        want = val64[:, :k]
+        assert bool(((val.view(torch.int32) == want.contiguous().view(torch.int32)) | (val.isnan() & want.isnan())).all())
+
+
 @pytest.mark.parametrize("inverse", [0, 1])
 @pytest.mark.parametrize("n_vec", [1, 3, 4, 5, 32, 63, 16384, 16385])
 def test_vectors_transform_alike_in_both_forms(dev, n_vec, inverse):
