@@ -2770,10 +2770,11 @@ __global__ __launch_bounds__(256) void k_tensor_stats(const float* __restrict__ 
 
 // The 1-D parameters of a set (rows of 64 elements) decoded where they lie: what k_aggregate_rows leaves for a
 // row, then the 64-point inverse transform and its scale exactly as k_dct1d applies them, written into the
-// row's tensor.  One wave per row, a handful of rows per parameter: every peer's entries of the row are
-// requested before the first is used (32 peers to a round), so a row waits for one memory round trip instead of one per
-// peer, and the row's transform runs on one lane (the same instruction sequence as on any lane of k_dct1d).  The 1056 rows
-// of a 1B model's norm vectors from 15 peers: 15.2 us; with the loads behind a branch per peer 22.2 us.
+// row's tensor.  One wave per row, a handful of rows per parameter: the row's transform runs on one lane (the same
+// instruction sequence as on any lane of k_dct1d), and the peers' entries are requested four peers at a time (32 peers to a
+// round), without a branch among them - behind a branch each every load is waited for by itself.  Eight tensors, k = 32, the
+// transform, in us, a branch per peer : four at a time : eight : 1056 rows from 15 peers 12.3 : 11.4 : 13.6, from one 6.6 :
+// 6.6 : 9.0; 65 536 rows from 15 201 : 153 : 174, from one 86 : 81 : 100 (units without a peer load and wait too).
 template <bool kUseDct>
 __global__ __launch_bounds__(64) void k_decode_rows64(const PeerPtrs pp, const float* __restrict__ scale, int P, int k,
                                                       const tplr_tensor_desc* __restrict__ table, int n_tensors,
@@ -2800,18 +2801,18 @@ __global__ __launch_bounds__(64) void k_decode_rows64(const PeerPtrs pp, const f
     const tplr_tensor_desc d = table[t];
     wave_lds_fence();
     const int64_t idx_stride = k + (k >> 1);
-    constexpr int kRound = 32;
+    constexpr int kRound = 32, kAtOnce = 4;
     const int le = lane < k ? lane : 0;
     for (int p0 = 0; p0 < P; p0 += kRound) {
         int me[kRound];
         float a[kRound];
 #pragma unroll
-        for (int h = 0; h < kRound; h += 8) {
-            if (p0 + h >= P) break;  // wave-uniform: eight peers are requested at a time
-            uint32_t raw[8];
-            float s[8];
+        for (int h = 0; h < kRound; h += kAtOnce) {
+            if (p0 + h >= P) break;  // wave-uniform
+            uint32_t raw[kAtOnce];
+            float s[kAtOnce];
 #pragma unroll
-            for (int i = 0; i < 8; ++i) {
+            for (int i = 0; i < kAtOnce; ++i) {
                 // (units without a peer read the last one's, lanes without an entry entry 0: behind a branch of its own
                 // every load would be waited for before the next is requested)
                 const int p = p0 + h + i < P ? p0 + h + i : P - 1;
@@ -2820,7 +2821,7 @@ __global__ __launch_bounds__(64) void k_decode_rows64(const PeerPtrs pp, const f
                 s[i] = scale ? scale[static_cast<int64_t>(t) * P + p] : 1.0f;
             }
 #pragma unroll
-            for (int i = 0; i < 8; ++i) {
+            for (int i = 0; i < kAtOnce; ++i) {
                 me[h + i] = p0 + h + i < P && lane < k ? static_cast<int>((le & 1) ? raw[i] >> 4 : raw[i] & 0xfffu) : -1;
                 a[h + i] *= s[i];
             }
