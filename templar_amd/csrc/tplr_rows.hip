@@ -33,9 +33,10 @@ __global__ __launch_bounds__(64) void k_topk_rows(const float* __restrict__ coef
 // has its share of it, ceil(n / 64) neighbouring elements in the leading registers of its 64: with 64 elements per lane
 // and the row in the first lanes, as it lies in memory, the lanes' maxima bound the k-th largest magnitude badly (a
 // row of 400 reaches seven lanes) and the select falls back to its bitwise search.  The registers past the share hold
-// zeros; a row with fewer than k non-zero values could select one of those in place of a later zero of its own, and is
-// then done again as it lies.  All of a row's loads are requested before the first is used.  1000 rows of 3000, k = 32:
-// 9.0 us (as rows of 4096, four loads at a time: 19.3 us).
+// zeros, one of which could be selected in place of a later zero of the row's own: a row with fewer than k values other
+// than zero (and denormals, for good measure) is therefore taken as it lies.  All of a row's loads are requested before the
+// first is used.  In us, k = 32: 1000 rows of 3000 7.3 (as rows of 4096, four loads at a time: 10.0), 1000 of 400 6.7 (15.9),
+// 10 000 of 400 all zeros 71 (66; selecting twice 123).
 template <bool kTwo>
 __global__ __launch_bounds__(64) void k_topk_rows_any(const float* __restrict__ coef, int64_t n_rows, int row_len,
                                                       int k, uint8_t* __restrict__ idx12, float* __restrict__ val) {
@@ -48,38 +49,34 @@ __global__ __launch_bounds__(64) void k_topk_rows_any(const float* __restrict__ 
     const __amdgpu_buffer_rsrc_t rs =
         __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(coef + row * row_len), 0, row_len * 4, 0x00020000);
     float w[64];
-#pragma unroll 1
-    for (int per = (row_len + 63) >> 6;; per = 64) {  // elements per lane; a second turn takes the row as it lies
-        // a word of padding every 32: lanes `per` elements apart meet in few banks whatever `per` is
-        auto pos = [](int e) { return e + (e >> 5); };
 #pragma unroll
-        for (int i = 0; i < 64; ++i)
-            w[i] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rs, lane * 4, i * 256, 0));
+    for (int i = 0; i < 64; ++i)
+        w[i] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rs, lane * 4, i * 256, 0));
+    // a word of padding every 32: lanes `per` elements apart meet in few banks whatever `per` is
+    auto pos = [](int e) { return e + (e >> 5); };
 #pragma unroll
-        for (int i = 0; i < 64; ++i) tile[pos(i * 64 + lane)] = w[i];
-        wave_lds_fence();
-        // (a lane's elements past its share are its neighbour's, read and dropped; the last lanes' lie past the tile)
-        const int first = lane * per;
+    for (int i = 0; i < 64; ++i) tile[pos(i * 64 + lane)] = w[i];
+    int normal = 0;
 #pragma unroll
-        for (int d = 0; d < 64; ++d) {
-            const int e = first + d < 4095 ? first + d : 4095;
-            w[d] = d < per ? tile[pos(e)] : 0.0f;
+    for (int i = 0; i < 64; i += 8)
+        if (normal < k) {  // wave-uniform: most rows have them in their first 512 elements
+#pragma unroll
+            for (int j = i; j < i + 8; ++j) normal += __popcll(__ballot(!(__builtin_fabsf(w[j]) < 1.17549435e-38f)));
         }
-        wave_lds_fence();
-        Selected s = select_topk<kTwo>(w, tile, cand, lane, k, 1.0f);
-        const uint32_t share = static_cast<uint32_t>(per);
-        bool wrong = lane < k && (s.idx0 & 63u) >= share;
-        s.idx0 = (s.idx0 >> 6) * share + (s.idx0 & 63u);
-        wrong = wrong || (lane < k && s.idx0 >= static_cast<uint32_t>(row_len));
-        if (kTwo && k > 64) {
-            wrong = wrong || (lane + 64 < k && (s.idx1 & 63u) >= share);
-            s.idx1 = (s.idx1 >> 6) * share + (s.idx1 & 63u);
-            wrong = wrong || (lane + 64 < k && s.idx1 >= static_cast<uint32_t>(row_len));
-        }
-        if (per < 64 && __ballot(wrong) != 0) continue;  // wave-uniform
-        emit_selected<kTwo>(s, lane, k, row, idx12, val);
-        return;
+    const int per = normal < k ? 64 : (row_len + 63) >> 6;  // elements per lane
+    wave_lds_fence();
+    // (a lane's elements past its share are its neighbour's, read and dropped; the last lanes' lie past the tile)
+    const int first = lane * per;
+#pragma unroll
+    for (int d = 0; d < 64; ++d) {
+        const int e = first + d < 4095 ? first + d : 4095;
+        w[d] = d < per ? tile[pos(e)] : 0.0f;
     }
+    wave_lds_fence();
+    Selected s = select_topk<kTwo>(w, tile, cand, lane, k, 1.0f);
+    s.idx0 = (s.idx0 >> 6) * static_cast<uint32_t>(per) + (s.idx0 & 63u);
+    if (kTwo) s.idx1 = (s.idx1 >> 6) * static_cast<uint32_t>(per) + (s.idx1 & 63u);
+    emit_selected<kTwo>(s, lane, k, row, idx12, val);
 }
 
 // Rows of at most 64 (kTwo: 128) elements, a 1-D parameter's: one (two) per lane, sorted as 64-bit keys (magnitude,
