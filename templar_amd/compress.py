@@ -622,7 +622,7 @@ class TopKCompressor:
         if self.use_quantization:
             out = _lib.native().compress(x, topk, self.n_bins, self.range_in_sigmas)
         else:
-            out = _lib.native().compress(x, topk, 0, 0)
+            out = _lib.native().compress(x, topk, None, None)
         if out is not None:
             return out
         with torch.no_grad():
@@ -784,6 +784,8 @@ class TopKCompressor:
     # -- statistical 8-bit quantiser (reference :582-696); payload-sized torch ops ----------
     @torch.no_grad()
     def _quantize_values(self, val: torch.Tensor) -> tuple[torch.Tensor, QuantParamsT]:
+        if self.n_bins < 1:
+            raise _lib.TplrHipError(f"a quantiser of {self.n_bins} bins")
         half = self.n_bins // 2
         # two launches (sums in double) instead of a dozen reductions and scatters; the scale is the only value that
         # travels to the host, as in the reference (float(scale), :620)

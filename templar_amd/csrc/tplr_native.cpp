@@ -307,24 +307,26 @@ PyObject* dequantize(PyObject*, PyObject* const* args, Py_ssize_t n) {
 }
 
 // ---- compress ---------------------------------------------------------------------------------
-// compress(x, topk, n_bins, range) -> (idx, val, xshape, totalk[, quant_params]); n_bins 0: no quantiser
+// compress(x, topk, n_bins, range) -> (idx, val, xshape, totalk[, quant_params]); n_bins None: no quantiser
 PyObject* compress(PyObject*, PyObject* const* args, Py_ssize_t n) {
     HANDLE_TH_ERRORS
-    int64_t topk, bins;
+    int64_t topk, bins = 0;
     if (n != 4) return PyErr_SetString(PyExc_TypeError, "compress(x, topk, n_bins, range)"), nullptr;
     const at::Tensor* x = plain_f32(args[0]);
-    if (!x || x->numel() == 0 || x->dim() < 1 || x->dim() == 3 || x->dim() > 4 || !to_int(args[1], topk) || !to_int(args[2], bins))
+    const bool coded = args[2] != Py_None;
+    if (!x || x->numel() == 0 || x->dim() < 1 || x->dim() == 3 || x->dim() > 4 || !to_int(args[1], topk) ||
+        (coded && !to_int(args[2], bins)))
         Py_RETURN_NONE;
     const bool chunks = x->dim() == 4;
     const int64_t totalk = chunks ? x->size(2) * x->size(3) : x->size(x->dim() - 1);
     const int64_t k = clamp_k(totalk, topk), rows = x->numel() / totalk;
     if (totalk > TPLR_MAX_ROW || k > totalk) Py_RETURN_NONE;
-    const double range = bins ? PyFloat_AsDouble(args[3]) : 0.0;
+    const double range = coded ? PyFloat_AsDouble(args[3]) : 0.0;
     if (PyErr_Occurred()) {
         PyErr_Clear();
         Py_RETURN_NONE;
     }
-    if (bins && (bins < 1 || bins > 256 || rows * k % 4)) Py_RETURN_NONE;
+    if (coded && (bins < 1 || bins > 256 || rows * k % 4)) Py_RETURN_NONE;
     // the un-transformed chunk view of a row-major tensor, as encode(use_dct=False) returns it: select straight from it
     const bool view = chunk_view(*x);
     if (view ? k > 128 : !x->is_contiguous()) Py_RETURN_NONE;
@@ -340,7 +342,7 @@ PyObject* compress(PyObject*, PyObject* const* args, Py_ssize_t n) {
     if (st) return failed(st, view ? "tplr_encode_topk_pack" : "tplr_topk_pack");
     PyObject* xshape = PyObject_GetAttrString(args[0], "shape");
     if (!xshape) return nullptr;
-    if (!bins)
+    if (!coded)
         return Py_BuildValue("(NNNL)", THPVariable_Wrap(std::move(idx)), THPVariable_Wrap(std::move(val)), xshape,
                              static_cast<long long>(totalk));
     PyObject* q = quantised(val, bins, range, on);

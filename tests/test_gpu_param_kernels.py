@@ -214,6 +214,18 @@ def test_decompress_names_the_index_outside_its_row(dev):
         comp.decompress(val, torch.from_numpy(orc.pack12(idx)).to(dev), val, (2, 9), 9)
 
 
+@pytest.mark.parametrize("bins", [0, -4])
+@pytest.mark.parametrize("shape", [(2, 3, 64, 64), (4, 100), (3, 50), (64,)])
+def test_quantiser_without_bins_is_refused(dev, bins, shape):
+    comp = tc.TopKCompressor(use_quantization=True, quantization_bins=bins)
+    x = torch.randn(shape, device=dev)
+    for other in (x, x.to(torch.bfloat16)):
+        with pytest.raises(RuntimeError, match=f"quantiser of {bins} bins"):
+            comp.compress(other, 10)
+    with pytest.raises(RuntimeError):
+        comp._quantize_values(x)
+
+
 def test_quantisers_of_two_threads_do_not_meet(dev):
     # each thread on a stream of its own: the scale travels through pinned memory of its own call
     import threading
