@@ -20,15 +20,22 @@ namespace tplr {
 // The moments are taken about the tensor's first value, where value - first is exact in double: sum (x - first) and
 // sum (x - first)^2 in one pass over the values give the mean and, about the rounded mean, the sum of squares of the
 // centred values (:594-597) - zero exactly for a constant tensor, as the reference's second pass has it, and otherwise
-// with the thirteen digits that are left of a double when the first value lies ten standard deviations out.
+// with the thirteen digits that are left of a double when the first value lies ten standard deviations out.  Where the
+// first value is not finite they are taken about zero: the mean of values with one infinity is that infinity (:594).
 struct QuantSlice {
     const float4* v;
     uchar4* q;
     int64_t n4;   // float4 groups in this slice
     int64_t n;    // values in the whole tensor
-    float first;  // the tensor's first value
+    float first;  // the tensor's first value, or zero
     int t, s;
 };
+
+// what the moments of n values from v[0] on are taken about
+__device__ __forceinline__ float quant_pivot(const float* v, int64_t n) {
+    const float x = n > 0 ? *v : 0.f;
+    return __builtin_fabsf(x) < __builtin_inff() ? x : 0.f;  // (NaN: zero)
+}
 
 // (`table` null: `single` is the one tensor)
 __device__ __forceinline__ QuantSlice quant_slice(const float* val, uint8_t* codes, const tplr_tensor_desc* table,
@@ -43,7 +50,7 @@ __device__ __forceinline__ QuantSlice quant_slice(const float* val, uint8_t* cod
     qs.q = codes ? reinterpret_cast<uchar4*>(codes + (d.chunk_begin + r0) * k) : nullptr;
     qs.n4 = (r1 - r0) * k >> 2;  // k is a multiple of 4
     qs.n = rows * k;
-    qs.first = rows > 0 ? val[d.chunk_begin * k] : 0.f;
+    qs.first = quant_pivot(val + d.chunk_begin * k, rows);
     return qs;
 }
 
@@ -224,7 +231,7 @@ __global__ __launch_bounds__(64) void k_quant_tables(const float* __restrict__ v
         const tplr_tensor_desc d = table ? table[t] : single;
         const int64_t n = static_cast<int64_t>(d.x_chunks) * d.y_chunks * k;
         float shift, scale;
-        quant_shift_scale(work, t, S, n, n > 0 ? val[d.chunk_begin * k] : 0.f, n_bins, range_in_sigmas, shift, scale);
+        quant_shift_scale(work, t, S, n, quant_pivot(val + d.chunk_begin * k, n), n_bins, range_in_sigmas, shift, scale);
         if (lane == 0) shift_out[t] = shift, scale_out[t] = scale;
     }
 }

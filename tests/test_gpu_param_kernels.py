@@ -214,6 +214,29 @@ def test_decompress_names_the_index_outside_its_row(dev):
         comp.decompress(val, torch.from_numpy(orc.pack12(idx)).to(dev), val, (2, 9), 9)
 
 
+@pytest.mark.parametrize("bins", [4, 256])
+@pytest.mark.parametrize("n", [4, 70000])
+@pytest.mark.parametrize("at,what", [(0, "inf"), (0, "-inf"), (0, "nan"), (3, "inf"), (-1, "-inf"), (-1, "nan")])
+def test_quantiser_of_values_that_are_not_finite(dev, bins, n, at, what):
+    # the reference's mean is the infinity (or NaN), and its scale, NaN, becomes one (:594-600); wherever it stands
+    v = torch.randn(n, device=dev)
+    v[at] = float(what)
+    comp = tc.TopKCompressor(use_quantization=True, quantization_bins=bins)
+    q, (shift, scale, half, lut, _) = comp._quantize_values(v)
+    b = tc.TensorBatch([torch.empty(64, 64, device=dev) for _ in range(2)])
+    pair = torch.randn(2, 4, device=dev)
+    pair[1, at] = float(what)
+    _, shifts, scales, _ = tc.quantize_batch(b, pair, 4, bins)
+    for got, sc in ((shift, scale), (shifts[1], float(scales[1]))):
+        assert float(got) == float(what) or (what == "nan" and bool(got.isnan()))
+        assert sc == 1.0
+    assert bool(torch.isfinite(shifts[0])) and float(scales[0]) != 1.0
+    # a finite value lies infinitely far below an infinite mean, or above (codes of NaN are not defined)
+    if what != "nan":
+        finite = torch.isfinite(v)
+        assert bool((q[finite] == (0 if what == "inf" else bins - 1)).all())
+
+
 @pytest.mark.parametrize("bins", [0, -4])
 @pytest.mark.parametrize("shape", [(2, 3, 64, 64), (4, 100), (3, 50), (64,)])
 def test_quantiser_without_bins_is_refused(dev, bins, shape):
