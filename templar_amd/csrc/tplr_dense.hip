@@ -62,6 +62,8 @@ __global__ __launch_bounds__(256, 3) void k_dense2d(const float* __restrict__ in
         const int y = static_cast<int>(static_cast<unsigned>(chunk) / static_cast<unsigned>(X));
         return static_cast<int64_t>(y) * h * C + static_cast<int64_t>(chunk - y * X) * w;
     };
+    // (T past the chunk's columns is zero times Bh: kept at zero where Bh holds an infinity)
+    const bool last_in = 16 * (kNT - 1) + l16 < w;
     // this lane's place in a load: column `col` of row i * kStep + wv * kPerInstr + sub of a chunk
     const int col = lane % (16 * kNS), sub = lane / (16 * kNS);
     float pre[kStack][kLoads];
@@ -133,7 +135,8 @@ __global__ __launch_bounds__(256, 3) void k_dense2d(const float* __restrict__ in
 #pragma unroll
                 for (int n = 0; n < kNT; ++n)
 #pragma unroll
-                    for (int r = 0; r < 4; ++r) st[(c * kRowsPer + 16 * mt + 4 * lq + r) * kLt + 16 * n + l16] = acc[n][r];
+                    for (int r = 0; r < 4; ++r)
+                        st[(c * kRowsPer + 16 * mt + 4 * lq + r) * kLt + 16 * n + l16] = n + 1 < kNT || last_in ? acc[n][r] : 0.f;
             }
         }
         __syncthreads();

@@ -39,6 +39,23 @@ def test_dense_transform_at_tile_edges(dev, h, w, Y, X):
         assert (np.abs(got - ref) <= tol).all(), (in_chunked, out_chunked)
 
 
+@pytest.mark.parametrize("h,w", [(2, 1), (7, 3), (17, 18), (60, 50), (63, 63), (64, 49), (1, 50)])
+def test_dense_contraction_with_an_infinite_matrix(dev, h, w):
+    # an infinity in either matrix reaches the results that depend on it, and no padding of the tiles turns it into NaN
+    rng = np.random.default_rng(h + w)
+    x, b, d = (rng.random(s).astype(np.float32) + 0.5 for s in ((3, 2, h, w), (h, h), (w, w)))
+    b[h // 2, h - 1] = np.inf
+    d2 = d.copy()
+    d2[w - 1, 0] = -np.inf
+    tr = tc.ChunkingTransformer(torch.nn.Linear(1, 1, bias=False), 64)
+    for second in (d, d2):
+        with np.errstate(invalid="ignore"):
+            want = b.T.astype(np.float64) @ x.astype(np.float64) @ second
+        got = tr.einsum_2d(*(torch.from_numpy(a).to(dev) for a in (x, b, second))).cpu().numpy()
+        assert np.array_equal(np.isnan(got), np.isnan(want))
+        assert np.allclose(got, want, rtol=1e-4, equal_nan=True)
+
+
 def _rows(kind, n_rows, n, rng):
     if kind == "normal":
         return rng.standard_normal((n_rows, n)).astype(np.float32)
