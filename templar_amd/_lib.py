@@ -110,21 +110,48 @@ def load():
 _native = None
 
 
+class _NotBuilt:
+    """In place of the native path where it does not load.  What works on host tensors is torch's own and needs nothing
+    built: those are not served, which leaves them to it; a device tensor raises."""
+
+    def __init__(self, error: Exception):
+        self._error = error
+
+    def __bool__(self) -> bool:
+        return False
+
+    def __getattr__(self, name: str):
+        return self._serve
+
+    def _serve(self, first, *_):
+        t = first[0] if isinstance(first, list) and first else first
+        if getattr(t, "is_cuda", False):
+            raise self._error
+        return None
+
+
 def native():
     """The host path of the per-parameter calls (csrc/tplr_native.cpp), bound to the loaded library's entry points."""
     global _native
     if _native is None:
-        import torch
-
-        lib = load()
         try:
-            from . import _native as mod
-        except ImportError as e:
-            raise ImportError(f"templar_amd/_native is missing or does not load ({e}): build it with "
-                              "`python -c 'import __graft_entry__ as g; g.build()'`") from e
-        mod.bind({name: C.cast(getattr(lib, name), C.c_void_p).value for name in SIGNATURES}, TplrHipError, torch.float32)
-        _native = mod
+            _native = _bind_native()
+        except (ImportError, OSError, AttributeError) as e:
+            return _NotBuilt(e)  # (not kept: it may be built yet)
     return _native
+
+
+def _bind_native():
+    import torch
+
+    lib = load()
+    try:
+        from . import _native as mod
+    except ImportError as e:
+        raise ImportError(f"templar_amd/_native is missing or does not load ({e}): build it with "
+                          "`python -c 'import __graft_entry__ as g; g.build()'`") from e
+    mod.bind({name: C.cast(getattr(lib, name), C.c_void_p).value for name in SIGNATURES}, TplrHipError, torch.float32)
+    return mod
 
 
 def check(status: int, what: str) -> None:

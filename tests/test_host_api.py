@@ -121,6 +121,36 @@ def test_encode_decode_without_dct_is_a_view():
         tr.encode(x, use_dct=True)
 
 
+def test_host_tensors_need_nothing_built(monkeypatch):
+    """What torch alone does on host tensors works, and what needs a device says so, without either library."""
+    def missing():
+        raise ImportError("not built")
+
+    monkeypatch.setattr(_lib, "load", missing)
+    monkeypatch.setattr(_lib, "_native", None)
+    tr = tc.ChunkingTransformer(torch.nn.Linear(128, 64), 64)
+    x = torch.rand(64, 128)
+    chunks = tr.encode(x)
+    assert torch.equal(tr.decode(chunks), x) and torch.equal(tr.decode(chunks.contiguous()), x)
+    assert torch.equal(tr.decode(tr.encode(x[0])), x[0])
+    comp = tc.TopKCompressor(use_quantization=True, quantization_bins=16)
+    codes, qp = comp._quantize_values(x)
+    assert torch.allclose(comp._dequantize_values(codes, qp), x, atol=qp[1])
+    out = comp.maybe_dequantize_values([codes, codes], [qp, qp], x.device)
+    assert torch.equal(out[0], out[1]) and torch.equal(out[0], comp._dequantize_values(codes, qp))
+    idx, val = torch.zeros(3, dtype=torch.uint8), torch.zeros(1, 2)
+    for call in (lambda: tr.encode(x, use_dct=True), lambda: tr.decode(chunks, use_dct=True), lambda: comp.compress(x, 32),
+                 lambda: comp.decompress(x, idx, val, (1, 64), 64), lambda: comp.batch_decompress(x, [idx], [val], (1, 64), 64)):
+        with pytest.raises(RuntimeError, match="HIP device only"):
+            call()
+    # a device tensor does not go unserved silently
+    assert not _lib.native()
+    on_device = type("OnDevice", (), {"is_cuda": True})()
+    for call in (lambda: _lib.native().encode(on_device, {}), lambda: _lib.native().dequantize([on_device], [qp])):
+        with pytest.raises(ImportError, match="not built"):
+            call()
+
+
 def test_clamp_topk():
     c = tc.TopKCompressor()
     for last in (1, 2, 3, 10, 64, 100, 4096):
