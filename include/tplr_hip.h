@@ -424,7 +424,8 @@ int tplr_quantize_batch(const float* d_val, int k, const tplr_tensor_desc* d_des
                         float range_in_sigmas, int n_slices, double* d_work, uint8_t* d_codes, float* d_shift,
                         float* d_scale, float* d_lookup, void* stream);
 
-/* The same for n values of one tensor (n a multiple of 4) in two launches, d_work as for n_tensors = 1 and one double more.
+/* The same for n values of one tensor (n a multiple of 4), with up to eight bins in two launches; d_work as for n_tensors = 1
+ * and one double more.
  * d_shift, d_scale and d_lookup may lie in pinned host memory; *d_scale is stored with system scope as the second launch
  * begins, so that a host that watches it need not wait for the codes. */
 int tplr_quantize(const float* d_val, int64_t n, int n_bins, float range_in_sigmas, int n_slices, double* d_work,

@@ -11,8 +11,10 @@
 
 namespace tplr {
 
-// Three launches over slices of every tensor: the moments, the codes with per-bin sums, the tables (of one tensor two: the
-// workgroup that finishes its codes last makes the table, which saves a launch of 4 us).  Partial sums are
+// Three launches over slices of every tensor: the moments, the codes with per-bin sums, the tables.  Of one tensor with up to
+// eight bins two: the workgroup that finishes its codes last makes the table, which saves a launch of 4 us.  With more bins
+// that workgroup would read up to a megabyte by itself, its lanes 4 KB apart: of 262 144 values a whole call with 256 bins
+// takes 98.9 us that way and 17.6 us with a wave per bin, with 64 bins 32.9 and 17.6.  Partial sums are
 // carried in double, kept per (tensor, slice) in a caller-provided workspace and added in a fixed order by whoever
 // needs the total, so every workgroup of a tensor derives the same shift and scale.
 // Workspace layout (doubles): moments[T][S][2], then bins[T][S][2 * n_bins] (sums, counts).
@@ -94,8 +96,8 @@ __device__ __forceinline__ float quant_bin_mean(const double* bins, int S, int n
 
 // One tensor's results where its codes are made (k_quant_codes), instead of a launch of their own.
 struct QuantOne {
-    uint32_t* done;  // slices finished, zeroed by k_quant_moments; null: k_quant_tables follows
-    float *shift, *scale, *lookup;
+    uint32_t* done;  // slices finished, zeroed by k_quant_moments; null: k_quant_tables makes the table
+    float *shift, *scale, *lookup;  // null: k_quant_tables stores all
 };
 
 __global__ __launch_bounds__(256) void k_quant_moments(const float* __restrict__ val, int k,
@@ -135,7 +137,7 @@ __global__ __launch_bounds__(256) void k_quant_codes(const float* __restrict__ v
     const QuantSlice qs = quant_slice(val, codes, table, single, k, S);
     float shift, scale;
     quant_shift_scale(work, qs.t, S, qs.n, qs.first, n_bins, range_in_sigmas, shift, scale);
-    if (one.done && blockIdx.x == 0 && tid == 0) {
+    if (one.scale && blockIdx.x == 0 && tid == 0) {
         *one.shift = shift;
         // (the caller may be watching for it in pinned host memory while this launch goes on)
         __hip_atomic_store(one.scale, scale, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
@@ -219,7 +221,7 @@ __global__ __launch_bounds__(256) void k_quant_codes(const float* __restrict__ v
     }
 }
 
-// One wave per bin of tensor blockIdx.y, and wave 0 of bin 0 the scalars.
+// One wave per bin of tensor blockIdx.y, and bin 0's the scalars (null: they are stored already).
 __global__ __launch_bounds__(64) void k_quant_tables(const float* __restrict__ val, const tplr_tensor_desc* __restrict__ table,
                                                      const tplr_tensor_desc single, int k, int T, int S, int n_bins, float range_in_sigmas,
                                                      const double* __restrict__ work, float* __restrict__ shift_out,
@@ -227,7 +229,7 @@ __global__ __launch_bounds__(64) void k_quant_tables(const float* __restrict__ v
     const int t = blockIdx.y, bin = blockIdx.x, lane = threadIdx.x;
     const float mean = quant_bin_mean(work + 2 * static_cast<int64_t>(T) * S + static_cast<int64_t>(t) * S * 2 * n_bins, S, n_bins, bin);
     if (lane == 0) lookup[static_cast<int64_t>(t) * n_bins + bin] = mean;
-    if (bin == 0) {  // wave-uniform
+    if (bin == 0 && scale_out) {  // wave-uniform
         const tplr_tensor_desc d = table ? table[t] : single;
         const int64_t n = static_cast<int64_t>(d.x_chunks) * d.y_chunks * k;
         float shift, scale;
@@ -319,17 +321,21 @@ __global__ __launch_bounds__(256) void k_dequantize_lists(const DeqLists pp, int
     }
 }
 
+// `one`: a single tensor (its descriptor `single`) with d_shift and d_scale stored early
 static int launch_quantize(const float* d_val, int k, const tplr_tensor_desc* d_desc, const tplr_tensor_desc& single, int n_tensors, int n_bins,
                            float range_in_sigmas, int n_slices, double* d_work, uint8_t* d_codes, float* d_shift,
-                           float* d_scale, float* d_lookup, void* stream, uint32_t* done = nullptr) {
+                           float* d_scale, float* d_lookup, void* stream, bool one = false) {
     const dim3 grid(static_cast<unsigned>(n_tensors) * n_slices), block(256);
     hipStream_t st = static_cast<hipStream_t>(stream);
-    const QuantOne one = {done, d_shift, d_scale, d_lookup};
+    uint32_t* done = one && n_bins <= 8 ? reinterpret_cast<uint32_t*>(d_work + static_cast<int64_t>(n_slices) * (2 + 2 * n_bins)) : nullptr;
+    const QuantOne results = {done, one ? d_shift : nullptr, one ? d_scale : nullptr, one ? d_lookup : nullptr};
     hipLaunchKernelGGL(k_quant_moments, grid, block, 0, st, d_val, k, d_desc, single, n_slices, d_work, done);
     hipLaunchKernelGGL(n_bins <= 4 ? k_quant_codes<4> : n_bins <= 8 ? k_quant_codes<8> : k_quant_codes<0>, grid, block, 0, st,
-                       d_val, k, d_desc, single, n_tensors, n_slices, n_bins, range_in_sigmas, d_codes, d_work, one);
-    if (!done) hipLaunchKernelGGL(k_quant_tables, dim3(static_cast<unsigned>(n_bins), static_cast<unsigned>(n_tensors)), dim3(64), 0, st,
-                       d_val, d_desc, single, k, n_tensors, n_slices, n_bins, range_in_sigmas, d_work, d_shift, d_scale, d_lookup);
+                       d_val, k, d_desc, single, n_tensors, n_slices, n_bins, range_in_sigmas, d_codes, d_work, results);
+    if (!done)
+        hipLaunchKernelGGL(k_quant_tables, dim3(static_cast<unsigned>(n_bins), static_cast<unsigned>(n_tensors)), dim3(64), 0, st,
+                           d_val, d_desc, single, k, n_tensors, n_slices, n_bins, range_in_sigmas, d_work, one ? nullptr : d_shift,
+                           one ? nullptr : d_scale, d_lookup);
     return launch_status();
 }
 
@@ -418,9 +424,8 @@ int tplr_quantize(const float* d_val, int64_t n, int n_bins, float range_in_sigm
     tplr_tensor_desc single = {};
     single.x_chunks = static_cast<int32_t>(n / 4);  // rows of four values
     single.y_chunks = 1;
-    uint32_t* done = reinterpret_cast<uint32_t*>(d_work + static_cast<int64_t>(n_slices) * (2 + 2 * n_bins));
     return launch_quantize(d_val, 4, nullptr, single, 1, n_bins, range_in_sigmas, n_slices, d_work, d_codes, d_shift, d_scale,
-                           d_lookup, stream, done);
+                           d_lookup, stream, true);
 }
 
 int tplr_dequantize_batch(const uint8_t* d_codes, const float* d_lookup, const float* d_shift, int n_bins, int k,
