@@ -20,6 +20,7 @@
 #include <c10/hip/HIPStream.h>
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/python_variable.h>
+#include <torch/csrc/utils/object_ptr.h>
 
 #include <chrono>
 #include <vector>
@@ -290,19 +291,17 @@ PyObject* dequantize(PyObject*, PyObject* const* args, Py_ssize_t n) {
     }
     const int64_t count = first->numel();
     if (count == 0 || count % 4 || bins < 1 || bins > 256) Py_RETURN_NONE;
-    PyObject* list = PyList_New(P);
+    THPObjectPtr list(PyList_New(P));  // (an allocation that throws releases the ones before it)
     if (!list) return nullptr;
     for (Py_ssize_t p = 0; p < P; ++p) {
         at::Tensor o = fresh(THPVariable_Unpack(PyList_GET_ITEM(args[0], p)).sizes(), c10::ScalarType::Float, *first);
         out[p] = o.data_ptr<float>();
-        PyList_SET_ITEM(list, p, THPVariable_Wrap(std::move(o)));
+        PyList_SET_ITEM(list.get(), p, THPVariable_Wrap(std::move(o)));
     }
     Launch on(*first);
-    if (int st = p_tplr_dequantize_lists(codes, static_cast<int>(P), count, lookup, shift, static_cast<int>(bins), out, on.stream())) {
-        Py_DECREF(list);
+    if (int st = p_tplr_dequantize_lists(codes, static_cast<int>(P), count, lookup, shift, static_cast<int>(bins), out, on.stream()))
         return failed(st, "tplr_dequantize_lists");
-    }
-    return list;
+    return list.release();
     END_HANDLE_TH_ERRORS
 }
 
@@ -340,20 +339,15 @@ PyObject* compress(PyObject*, PyObject* const* args, Py_ssize_t n) {
                         : p_tplr_topk_pack(x->const_data_ptr<float>(), rows, totalk, static_cast<int>(k), idx.data_ptr<uint8_t>(),
                                            val.data_ptr<float>(), on.stream());
     if (st) return failed(st, view ? "tplr_encode_topk_pack" : "tplr_topk_pack");
-    PyObject* xshape = PyObject_GetAttrString(args[0], "shape");
+    THPObjectPtr xshape(PyObject_GetAttrString(args[0], "shape"));
     if (!xshape) return nullptr;
     if (!coded)
-        return Py_BuildValue("(NNNL)", THPVariable_Wrap(std::move(idx)), THPVariable_Wrap(std::move(val)), xshape,
+        return Py_BuildValue("(NNOL)", THPVariable_Wrap(std::move(idx)), THPVariable_Wrap(std::move(val)), xshape.get(),
                              static_cast<long long>(totalk));
-    PyObject* q = quantised(val, bins, range, on);
-    if (!q) {
-        Py_DECREF(xshape);
-        return nullptr;
-    }
-    PyObject* out = Py_BuildValue("(NONLO)", THPVariable_Wrap(std::move(idx)), PyTuple_GET_ITEM(q, 0), xshape,
-                                  static_cast<long long>(totalk), PyTuple_GET_ITEM(q, 1));
-    Py_DECREF(q);
-    return out;
+    THPObjectPtr q(quantised(val, bins, range, on));
+    if (!q) return nullptr;
+    return Py_BuildValue("(NOOLO)", THPVariable_Wrap(std::move(idx)), PyTuple_GET_ITEM(q.get(), 0), xshape.get(),
+                         static_cast<long long>(totalk), PyTuple_GET_ITEM(q.get(), 1));
     END_HANDLE_TH_ERRORS
 }
 

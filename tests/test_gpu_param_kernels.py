@@ -223,6 +223,32 @@ def test_per_parameter_calls_agree_for_plain_and_converted_inputs(dev):
             assert all(torch.equal(a.reshape(-1), b.reshape(-1)) for a, b in zip(results[0], r))
 
 
+def test_running_out_of_memory_leaves_nothing_allocated(dev):
+    comp = tc.TopKCompressor(use_quantization=True, quantization_bins=4)
+    qp = (torch.tensor(0.5, device=dev), 1.0, 2, torch.arange(4.0, device=dev), torch.float32)
+    codes = [torch.zeros(1 << 25, dtype=torch.uint8, device=dev)] * 16  # 16 results of 128 MiB each
+    x = torch.zeros(1 << 19, 64, device=dev)  # 128 MiB of values, 32 MiB of codes and 48 MiB of indices
+    torch.cuda.synchronize()
+    torch.cuda.empty_cache()
+    before = torch.cuda.memory_allocated(dev)
+    total = torch.cuda.get_device_properties(dev).total_memory
+    try:
+        torch.cuda.set_per_process_memory_fraction((torch.cuda.memory_reserved(dev) + (1 << 30)) / total, dev)
+        for _ in range(2):
+            with pytest.raises(torch.OutOfMemoryError):
+                comp.maybe_dequantize_values(codes, [qp] * 16, dev)
+            assert torch.cuda.memory_allocated(dev) == before
+            torch.cuda.empty_cache()
+        torch.cuda.set_per_process_memory_fraction((torch.cuda.memory_reserved(dev) + (180 << 20)) / total, dev)
+        with pytest.raises(torch.OutOfMemoryError):
+            comp.compress(x, 64)
+        assert torch.cuda.memory_allocated(dev) == before
+    finally:
+        torch.cuda.set_per_process_memory_fraction(1.0, dev)
+        torch.cuda.empty_cache()
+    assert comp.maybe_dequantize_values(codes[:2], [qp] * 2, dev)[1].numel() == 1 << 25
+
+
 def test_decompress_names_the_index_outside_its_row(dev):
     comp = tc.TopKCompressor()
     idx = np.array([[1, 2, 3, 9], [4, 5, 11, 0]], np.int64)
