@@ -702,7 +702,7 @@ class TopKCompressor:
         coefficient (reference :483-580).  With `defer=True` (an extension) the scatter is
         postponed so that ChunkingTransformer.decode() can run it fused with the inverse DCT."""
         if not normalise and not defer and (quantize_params is None or not self.use_quantization):
-            out = _lib.native().aggregate(p, idx, val, xshape, block_norms, bool(clip_norm), False, False)
+            out = _lib.native().aggregate(p, idx, val, xshape, block_norms, bool(clip_norm))
             if out is not None:
                 return out
         with torch.no_grad():

@@ -30,9 +30,10 @@
 namespace {
 
 // ---- the library's entry points ---------------------------------------------------------------
-#define TPLR_NATIVE_ENTRIES(X)                                                                                       \
-    X(tplr_status_string) X(tplr_dct2d_fwd) X(tplr_dct2d_inv) X(tplr_dct1d) X(tplr_topk_pack) X(tplr_encode_topk_pack) \
-    X(tplr_decode_aggregate) X(tplr_aggregate_param) X(tplr_decompress_codes) X(tplr_decompress_rows) X(tplr_clip_scales) X(tplr_peer_sumsq) X(tplr_quantize) X(tplr_dequantize_lists)
+#define TPLR_NATIVE_ENTRIES(X)                                                                            \
+    X(tplr_status_string) X(tplr_dct2d_fwd) X(tplr_dct2d_inv) X(tplr_dct1d) X(tplr_topk_pack)                \
+    X(tplr_encode_topk_pack) X(tplr_aggregate_param) X(tplr_decompress_codes) X(tplr_decompress_rows)        \
+    X(tplr_clip_scales) X(tplr_peer_sumsq) X(tplr_quantize) X(tplr_dequantize_lists)
 #define X(name) decltype(&::name) p_##name = nullptr;
 TPLR_NATIVE_ENTRIES(X)
 #undef X
@@ -369,34 +370,26 @@ at::Tensor chunk_tensor(int64_t Y, int64_t X, const at::Tensor& like) {
 }
 
 // norms (n_norms of them) with scale as scratch, or scale (nullable) the factors themselves
-PyObject* scatter_chunks(const Payloads& pl, const float* norms, int64_t n_norms, float* scale, int64_t Y, int64_t X, bool rows,
-                         bool dct, const Launch& on) {
-    const int64_t R = Y * kEdge, C = X * kEdge;
-    at::Tensor out = rows ? fresh({R, C}, c10::ScalarType::Float, *pl.like) : chunk_tensor(Y, X, *pl.like);
-    const int64_t ld = rows ? C : 0;
-    if (dct && norms)
-        if (int st = p_tplr_clip_scales(norms, static_cast<int>(n_norms), 0, scale, nullptr, on.stream()))
-            return failed(st, "tplr_clip_scales");
-    const int st = dct ? p_tplr_decode_aggregate(pl.idx, pl.val, scale, pl.peers, static_cast<int>(pl.k), R, C, TPLR_REDUCE_MEAN, 0,
-                                                 1, out.data_ptr<float>(), ld, nullptr, on.stream())
-                       : p_tplr_aggregate_param(pl.idx, pl.val, norms, static_cast<int>(n_norms), scale, pl.peers,
-                                                static_cast<int>(pl.k), R, C, out.data_ptr<float>(), ld, on.stream());
-    if (st) return failed(st, dct ? "tplr_decode_aggregate" : "tplr_aggregate_param");
+PyObject* scatter_chunks(const Payloads& pl, const float* norms, int64_t n_norms, float* scale, int64_t Y, int64_t X, const Launch& on) {
+    at::Tensor out = chunk_tensor(Y, X, *pl.like);
+    if (int st = p_tplr_aggregate_param(pl.idx, pl.val, norms, static_cast<int>(n_norms), scale, pl.peers, static_cast<int>(pl.k),
+                                        Y * kEdge, X * kEdge, out.data_ptr<float>(), 0, on.stream()))
+        return failed(st, "tplr_aggregate_param");
     return THPVariable_Wrap(std::move(out));
 }
 
-// aggregate(p, idx list, val list, xshape, block_norms | None, clip, as_rows, use_dct): the payloads of P peers on p's
-// device, scatter-mean with the clip factors min(1, median / (norm + 1e-8)) of the given norms, or of the values' own
-// -> (Y, X, 64, 64) coefficients, or with as_rows / use_dct the (R, C) tensor
+// aggregate(p, idx list, val list, xshape, block_norms | None, clip): the payloads of P peers on p's device, scatter-mean
+// with the clip factors min(1, median / (norm + 1e-8)) of the given norms, or of the values' own -> (Y, X, 64, 64)
+// coefficients
 PyObject* aggregate(PyObject*, PyObject* const* args, Py_ssize_t n) {
     HANDLE_TH_ERRORS
-    if (n != 8) return PyErr_SetString(PyExc_TypeError, "aggregate(p, idx, val, xshape, norms, clip, as_rows, use_dct)"), nullptr;
+    if (n != 6) return PyErr_SetString(PyExc_TypeError, "aggregate(p, idx, val, xshape, norms, clip)"), nullptr;
     const at::Tensor* like = plain_f32(args[0]);
     if (!like || !PyList_Check(args[1]) || !PyList_Check(args[2])) Py_RETURN_NONE;
     int64_t Y, X;
     const Py_ssize_t P = PyList_GET_SIZE(args[2]);
     if (P < 1 || P > TPLR_MAX_PEERS || PyList_GET_SIZE(args[1]) != P || !chunk_shape(args[3], Y, X)) Py_RETURN_NONE;
-    const bool clip = args[5] == Py_True, dct = args[7] == Py_True, rows = dct || args[6] == Py_True;
+    const bool clip = args[5] == Py_True;
     Payloads pl;
     pl.peers = static_cast<int>(P);
     pl.k = 0;
@@ -439,7 +432,7 @@ PyObject* aggregate(PyObject*, PyObject* const* args, Py_ssize_t n) {
                 return failed(st, "tplr_clip_scales");
         }
     }
-    return scatter_chunks(pl, given, n_given, clip ? scale.data_ptr<float>() : nullptr, Y, X, rows, dct, on);
+    return scatter_chunks(pl, given, n_given, clip ? scale.data_ptr<float>() : nullptr, Y, X, on);
     END_HANDLE_TH_ERRORS
 }
 
@@ -507,7 +500,7 @@ PyObject* decompress(PyObject*, PyObject* const* args, Py_ssize_t n) {
         pl.like = like;
         pl.idx[0] = idx->const_data_ptr<uint8_t>();
         pl.val[0] = val;
-        return scatter_chunks(pl, nullptr, 0, nullptr, shape[0], shape[1], false, false, on);
+        return scatter_chunks(pl, nullptr, 0, nullptr, shape[0], shape[1], on);
     }
     at::Tensor out = fresh(shape, c10::ScalarType::Float, *like);
     at::Tensor flag = at::empty({1}, at::TensorOptions().dtype(c10::ScalarType::Int).pinned_memory(true));
