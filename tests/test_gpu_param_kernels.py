@@ -292,6 +292,27 @@ def test_quantiser_without_bins_is_refused(dev, bins, shape):
         comp._quantize_values(x)
 
 
+@pytest.mark.parametrize("bins", [4, 256])
+def test_quantiser_queued_behind_other_work(dev, bins):
+    # the host watches for the scale for half a millisecond, and then waits for the stream
+    comp = tc.TopKCompressor(use_quantization=True, quantization_bins=bins)
+    v = torch.randn(262144, device=dev)
+    codes, (shift, scale, _, lookup, _) = comp._quantize_values(v)
+    a = torch.randn(4096, 4096, device=dev)
+    torch.mm(a, a)
+    torch.cuda.synchronize()
+    for _ in range(3):
+        events = [torch.cuda.Event(enable_timing=True) for _ in range(2)]
+        events[0].record()
+        for _ in range(8):
+            torch.mm(a, a)
+        events[1].record()
+        late = comp._quantize_values(v)
+        assert events[1].query() and events[0].elapsed_time(events[1]) > 2.0
+        assert torch.equal(late[0], codes) and torch.equal(late[1][0], shift) and late[1][1] == scale
+        assert torch.equal(late[1][3], lookup) if bins <= 8 else torch.allclose(late[1][3], lookup, rtol=2.0 ** -22, atol=1e-9)
+
+
 def test_quantisers_of_two_threads_do_not_meet(dev):
     # each thread on a stream of its own: the scale travels through pinned memory of its own call
     import threading
@@ -439,7 +460,7 @@ def test_decompress_from_codes_is_the_two_launches(dev, bins, k, Y, X):
 
 @pytest.mark.parametrize("n,bins,slices", [(4, 4, 1), (1020, 1, 1), (2052, 8, 2), (65536, 4, 64), (262144, 4, 256), (70000, 256, 68)])
 def test_quantiser_of_one_tensor_is_the_batch_of_one(dev, n, bins, slices):
-    """The table made by the workgroup that finishes last, and queued behind other work: the bits of the three launches."""
+    """The table made by the workgroup that finishes last, or past eight bins by a launch: the bits of the batch's launches."""
     lib = _lib.load()
     stream = torch.cuda.current_stream(dev).cuda_stream
     v = torch.from_numpy(np.random.default_rng(n).standard_t(3, n).astype(np.float32)).to(dev)
