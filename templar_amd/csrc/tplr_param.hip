@@ -11,11 +11,13 @@ namespace tplr {
 
 constexpr int kParamPeers = 24;  // payloads of one launch
 constexpr int kParamNorms = 64;  // norms that one wave ranks
-// Chunks times peers up to which a chunk per workgroup is the faster way: beyond it the scatters, of which every wave
-// issues all and keeps a quarter, fill the compute units' LDS pipelines.  Clip factors and aggregate in us, this kernel
-// against k_decode_aggregate that makes the factors itself: 1024 chunks of 15 peers 9.1 : 10.3, of 20 10.5 : 11.5, 4096
-// of 5 15.8 : 17.5, 16 384 of 1 48.2 : 53.5 - but 2048 of 15 13.9 : 13.5, of 20 16.7 : 14.8, 4096 of 15 22.9 : 20.6.
-constexpr int64_t kParamWork = 24576;
+// Chunks times peers up to which a chunk per workgroup is the faster way, into chunked results and into rows: beyond it
+// the scatters, of which every wave issues all and keeps a quarter, fill the compute units' LDS pipelines; and the
+// persistent kernel's teams store rows of 1 KB together, but no such rows into chunks.  Clip factors and aggregate in us, this
+// kernel against k_decode_aggregate that makes the factors itself, chunked: 1024 chunks of 15 peers 8.9 : 11.5, of 20
+// (k = 64) 10.7 : 13.3, 4096 of 5 15.2 : 18.7, of 15 22.1 : 22.5, 16 384 of 4 58.7 : 62.5 - but 2048 of 20 (k = 64) 17.0 : 16.5, 4096
+// of 20 28.9 : 27.1.  Into rows: 1024 of 15 9.2 : 10.7, 4096 of 5 15.9 : 18.4 - but 2048 of 15 14.1 : 12.8, of 12 13.2 : 12.5.
+constexpr int64_t kParamWorkChunks = 61440, kParamWorkRows = 24576;
 
 struct ParamPeer {
     const uint8_t* idx;
@@ -33,8 +35,9 @@ struct ParamPeers {
 // LDS, the last wave the clip factors with them (made from the norms: cheaper than a launch); then each walks all entries in peer order and keeps those of its own rows.  One instruction adds one peer's entries: an
 // exchange that leaves a mark in the slot until the sum is written back, as in k_decode_aggregate, tells of a repeated
 // index in a peer's row, and the wave then does its rows again with every entry in its turn (exact).
-// Measured, clip factors included: 2048 x 2048, 15 peers of k = 32 12.3 -> 9.1 us; 8192 x 2048 from one peer's codes,
-// k = 64, 19.8 -> 13.5 us.  Its compute units' LDS pipelines are what fills up first (three LDS instructions a step).
+// Measured, clip factors included, chunked: 2048 x 2048, 15 peers of k = 32 8.9 us (two launches of the general kernels
+// 12.3); 8192 x 2048 from one peer's codes, k = 64, 12.1 us (19.8).  Its compute units' LDS pipelines are what fills up
+// first (three LDS instructions a step).
 // kUnits: peers staged (the launcher rounds up); kCodes: values are a quantiser's codes, lookup[code] + shift (:637-643).
 template <int kUnits, bool kCodes>
 __global__ __launch_bounds__(256) void k_aggregate_param(const ParamPeers pp, const float* __restrict__ factors,
@@ -213,7 +216,7 @@ extern "C" int tplr_aggregate_param(const uint8_t* const* h_idx12, const float* 
     const int64_t n = (R / 64) * (C / 64);
     if (n == 0) return 0;
     if (C / 64 > 0x7fffffff || R / 64 > 0x7fffffff || ld_out > (int64_t{1} << 23)) return TPLR_E_TOOMANY;
-    if (n_peers <= kParamPeers && k <= 64 && n_norms <= kParamNorms && n * n_peers <= kParamWork && (ld_out & 3) == 0 &&
+    if (n_peers <= kParamPeers && k <= 64 && n_norms <= kParamNorms && n * n_peers <= (ld_out ? kParamWorkRows : kParamWorkChunks) && (ld_out & 3) == 0 &&
         (reinterpret_cast<uintptr_t>(d_out) & 15) == 0) {
         ParamPeers pp = {};
         for (int p = 0; p < n_peers; ++p) {

@@ -497,11 +497,11 @@ def test_large_param_aggregate_is_the_two_launches(dev, P, k, repeats):
     ip, vp = ptrs(idx), ptrs(val)
     stream = torch.cuda.current_stream(dev).cuda_stream
     norms = torch.rand(P + 2, device=dev) + 0.1
-    for m in (P, P + 2):
+    for m, ld in ((P, X * 64), (P + 2, X * 64), (P, 0), (P + 2, 0)):
         scale, (got, want) = torch.empty(m, device=dev), torch.full((2, n * 4096), 7.0, device=dev)
-        _lib.check(lib.tplr_aggregate_param(ip, vp, norms.data_ptr(), m, scale.data_ptr(), P, k, Y * 64, X * 64, got.data_ptr(), X * 64,
+        _lib.check(lib.tplr_aggregate_param(ip, vp, norms.data_ptr(), m, scale.data_ptr(), P, k, Y * 64, X * 64, got.data_ptr(), ld,
                                             stream), "tplr_aggregate_param")
         _lib.check(lib.tplr_clip_scales(norms.data_ptr(), m, 0, scale.data_ptr(), None, stream), "tplr_clip_scales")
-        _lib.check(lib.tplr_decode_aggregate(ip, vp, scale.data_ptr(), P, k, Y * 64, X * 64, 0, 0, 0, want.data_ptr(), X * 64, None,
+        _lib.check(lib.tplr_decode_aggregate(ip, vp, scale.data_ptr(), P, k, Y * 64, X * 64, 0, 0, 0, want.data_ptr(), ld, None,
                                              stream), "tplr_decode_aggregate")
-        assert torch.equal(got.view(torch.int32), want.view(torch.int32)), m
+        assert torch.equal(got.view(torch.int32), want.view(torch.int32)), (m, ld)
