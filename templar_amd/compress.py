@@ -13,7 +13,8 @@ place of `tplr.compress`:
 
 All tensor arithmetic of the codec runs in the HIP library on the tensor's device and on
 torch's current stream; nothing here synchronises except where the reference does
-(`pack_12bit_indices` reads back the range-check flag, as the reference's `.item()` does).
+(`pack_12bit_indices` reads back the range-check flag, as the reference's `.item()` does, `decompress` and
+`batch_decompress` of rows other than 64x64 chunks whether an index lay outside its row, and the quantiser its scale).
 Only the basis construction at start-up and the small statistical quantiser use torch ops.
 The two fused entry points `encode_compress` and `batch_decompress_decode` do what the
 callers' back-to-back `encode`+`compress` and `batch_decompress`+`decode` do, in one kernel
