@@ -193,9 +193,11 @@ PyObject* decode(PyObject*, PyObject* const* args, Py_ssize_t n) {
     if (n != 2) return PyErr_SetString(PyExc_TypeError, "decode(x, use_dct)"), nullptr;
     const at::Tensor* x = plain_f32(args[0]);
     if (!x || x->numel() == 0) Py_RETURN_NONE;
-    if (args[1] != Py_True) {  // a change of shape: of a view of the tensor itself, the tensor
-        if (!chunk_view(*x) || x->requires_grad()) Py_RETURN_NONE;
-        return THPVariable_Wrap(x->as_strided({x->size(0) * kEdge, x->size(1) * kEdge}, {x->stride(2), 1}));
+    if (args[1] != Py_True) {  // a change of shape: of a view of the tensor itself, the tensor; of whole chunks a copy
+        if (x->requires_grad()) Py_RETURN_NONE;
+        if (chunk_view(*x)) return THPVariable_Wrap(x->as_strided({x->size(0) * kEdge, x->size(1) * kEdge}, {x->stride(2), 1}));
+        if (x->dim() != 4 || !x->is_contiguous()) Py_RETURN_NONE;
+        return THPVariable_Wrap(x->permute({0, 2, 1, 3}).reshape({x->size(0) * x->size(2), x->size(1) * x->size(3)}));
     }
     Launch on(*x);
     if (x->dim() == 4 && x->size(2) == kEdge && x->size(3) == kEdge) {
