@@ -1,5 +1,6 @@
 """Kernels behind the reference's per-parameter calls, at the sizes where their tilings can go wrong."""
 import ctypes
+import gc
 
 import numpy as np
 import pytest
@@ -224,6 +225,10 @@ def test_per_parameter_calls_agree_for_plain_and_converted_inputs(dev):
 
 
 def test_running_out_of_memory_leaves_nothing_allocated(dev):
+    # The limits hold whatever ran before: what is left to the garbage collector (the frames behind pytest.raises, say) goes
+    # first, or its memory would come back in between, and room is counted from what is allocated, since the free rest of
+    # reserved segments serves requests as well.
+    gc.collect()
     comp = tc.TopKCompressor(use_quantization=True, quantization_bins=4)
     qp = (torch.tensor(0.5, device=dev), 1.0, 2, torch.arange(4.0, device=dev), torch.float32)
     codes = [torch.zeros(1 << 25, dtype=torch.uint8, device=dev)] * 16  # 16 results of 128 MiB each
@@ -233,13 +238,13 @@ def test_running_out_of_memory_leaves_nothing_allocated(dev):
     before = torch.cuda.memory_allocated(dev)
     total = torch.cuda.get_device_properties(dev).total_memory
     try:
-        torch.cuda.set_per_process_memory_fraction((torch.cuda.memory_reserved(dev) + (1 << 30)) / total, dev)
+        torch.cuda.set_per_process_memory_fraction((before + (1 << 30)) / total, dev)
         for _ in range(2):
             with pytest.raises(torch.OutOfMemoryError):
                 comp.maybe_dequantize_values(codes, [qp] * 16, dev)
             assert torch.cuda.memory_allocated(dev) == before
             torch.cuda.empty_cache()
-        torch.cuda.set_per_process_memory_fraction((torch.cuda.memory_reserved(dev) + (180 << 20)) / total, dev)
+        torch.cuda.set_per_process_memory_fraction((before + (180 << 20)) / total, dev)
         with pytest.raises(torch.OutOfMemoryError):
             comp.compress(x, 64)
         assert torch.cuda.memory_allocated(dev) == before
