@@ -6,6 +6,7 @@
 #include <string.h>
 
 #include "../../include/tplr_hip.h"
+#include "tplr_chunk.h"
 #include "tplr_device.h"
 #include "tplr_launch.h"
 
@@ -77,193 +78,6 @@ __global__ __launch_bounds__(256) void k_unpack12(const uint8_t* __restrict__ in
 }
 
 // =========================================================================================
-// chunk loaders / storers for the (R, C) row-major side: lane = column
-// =========================================================================================
-// Chunk rows through buffer instructions: one resource descriptor per chunk (scalar base,
-// byte range for bounds checking), the row offset r*ld in a scalar register and lane*4 as the
-// only vector operand, so addressing costs no vector ALU work.  ld*4*63 must fit in 31 bits.
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t chunk_rsrc(const void* chunk0, int64_t ld) {
-    return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(chunk0), 0, static_cast<int>((63 * ld + 64) * 4),
-                                             0x00020000);
-}
-
-template <int kRow0 = 0, int kRow1 = 64>
-__device__ __forceinline__ void load_chunk_rows(float (&v)[64], const void* chunk0, int64_t ld, int lane) {
-    const __amdgpu_buffer_rsrc_t rs = chunk_rsrc(chunk0, ld);
-    const int ld4 = static_cast<int>(ld) * 4;
-#pragma unroll
-    for (int r = kRow0; r < kRow1; ++r)
-        v[r] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rs, lane * 4, r * ld4, 2));
-}
-
-// drop (wave-uniform): the stores are issued against a range of zero bytes, whose bounds check
-// discards them - the instruction stream stays the same for a chunk that must not be written
-__device__ __forceinline__ void store_chunk_rows(const float (&v)[64], void* chunk0, int64_t ld, int lane,
-                                                 bool drop = false) {
-    const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(
-        chunk0, 0, drop ? 0 : static_cast<int>((63 * ld + 64) * 4), 0x00020000);
-    const int ld4 = static_cast<int>(ld) * 4;
-#pragma unroll
-    for (int r = 0; r < 64; ++r)
-        __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(int, v[r]), rs, lane * 4, r * ld4, 2);
-}
-
-__device__ __forceinline__ void load_chunk_cols(float (&v)[64], const float* __restrict__ x, int64_t ld,
-                                                int64_t y, int64_t xc, int lane) {
-    load_chunk_rows(v, x + (y * 64) * ld + xc * 64, ld, lane);
-}
-
-__device__ __forceinline__ void store_chunk_cols(const float (&v)[64], float* __restrict__ x, int64_t ld,
-                                                 int64_t y, int64_t xc, int lane) {
-    store_chunk_rows(v, x + (y * 64) * ld + xc * 64, ld, lane);
-}
-
-// forward 2-D transform of the chunk held column-per-lane; result row-per-lane:
-// v[d] = coef[lane][d], and the tile is left free
-// registers column-per-lane (v[r] = M[r][lane]) -> registers row-per-lane (w[c] = M[lane][c])
-// through a 32-row staging buffer: rows 0..31 go first and lanes 0..31 pick theirs up, then rows
-// 32..63 for lanes 32..63.  Half the LDS of a whole-chunk tile, which is what lets twice as many
-// waves stay resident.
-__device__ __forceinline__ void transpose_via_half(const float (&v)[64], float (&w)[64], float* buf, int lane) {
-#pragma unroll
-    for (int half = 0; half < 2; ++half) {
-#pragma unroll
-        for (int r = 0; r < kHalfRows; ++r) buf[r * kLd + lane] = v[half * kHalfRows + r];
-        wave_lds_fence();
-        if ((lane >> 5) == half) tile_rows_to_regs(w, buf, lane & 31);
-        wave_lds_fence();
-    }
-}
-
-// Forward 2-D transform of a chunk held column-per-lane (v[r] = X[r][lane]); the result is
-// row-per-lane: w[d] = 32 * coef[lane][d] with the transform, X[lane][d] without.
-template <bool kUseDct>
-__device__ __forceinline__ void chunk_forward(float (&v)[64], float (&w)[64], float* buf, int lane) {
-    if (kUseDct) dct64_fwd(v);  // along rows k: v[b] = sum_k X[k][lane] F[k][b]
-    transpose_via_half(v, w, buf, lane);
-    if (kUseDct) dct64_fwd(w);  // along columns l: w[d] = sum_l T[lane][l] F[l][d]
-}
-
-// inverse: tile holds coef rows; result column-per-lane v[k] = x[k][lane]
-// (the tile must hold the coefficients times 2^-5: the two passes multiply by 32; kScaleInput
-// applies that factor here for callers whose tile holds plain coefficients)
-template <bool kUseDct, bool kScaleInput = false>
-__device__ __forceinline__ void chunk_inverse(float (&v)[64], float* tile, int lane) {
-    if (kUseDct) {
-        tile_rows_to_regs(v, tile, lane);
-        if (kScaleInput) {
-#pragma unroll
-            for (int d = 0; d < 64; ++d) v[d] *= kDctPow2Scale;
-        }
-        dct64_inv(v);  // along d: v[l] = sum_d Y[lane][d] F[l][d]
-        wave_lds_fence();
-        regs_to_tile_rows(v, tile, lane);
-        wave_lds_fence();
-    }
-    tile_cols_to_regs(v, tile, lane);
-    if (kUseDct) dct64_inv(v);  // along b: v[k] = sum_b Z[b][lane] F[k][b]
-}
-
-// -----------------------------------------------------------------------------------------
-// Persistent kernels walk a contiguous range of the batch's chunk list.  A cursor keeps the
-// current tensor's descriptor and the chunk's (y, x) position in wave-uniform registers.
-// -----------------------------------------------------------------------------------------
-struct Cursor {
-    const tplr_tensor_desc* table;
-    int n_tensors;
-    int t;
-    gfloat* base;
-    int64_t ld;
-    int64_t begin, end;  // chunk ids covered by tensor t
-    int X;
-    int64_t y;
-    int xc;
-};
-
-// descriptor fields are the same for every lane: move them to scalar registers so that chunk
-// rows are addressed as scalar base + 32-bit lane offset
-__device__ __forceinline__ int64_t uniform64(int64_t x) {
-    const uint32_t lo = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(x));
-    const uint32_t hi = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(static_cast<uint64_t>(x) >> 32));
-    return static_cast<int64_t>((static_cast<uint64_t>(hi) << 32) | lo);
-}
-
-__device__ __forceinline__ void cursor_take(Cursor& c, const tplr_tensor_desc& d) {
-    c.base = (gfloat*)uniform64(reinterpret_cast<int64_t>(d.dense));
-    c.ld = uniform64(d.ld);
-    c.begin = uniform64(d.chunk_begin);
-    c.X = __builtin_amdgcn_readfirstlane(d.x_chunks);
-    c.end = c.begin + static_cast<int64_t>(c.X) * __builtin_amdgcn_readfirstlane(d.y_chunks);
-}
-
-__device__ __forceinline__ void cursor_seek(Cursor& c, const tplr_tensor_desc* table, const tplr_tensor_desc& single,
-                                            int n_tensors, int64_t g) {
-    c.table = table;
-    c.n_tensors = n_tensors;
-    c.t = 0;
-    if (table) {
-        int lo = 0, hi = n_tensors;  // last tensor whose chunk_begin <= g and that is not empty
-        while (hi - lo > 1) {
-            const int mid = (lo + hi) >> 1;
-            if (table[mid].chunk_begin <= g)
-                lo = mid;
-            else
-                hi = mid;
-        }
-        c.t = lo;
-        cursor_take(c, table[lo]);
-    } else {
-        cursor_take(c, single);
-    }
-    const int64_t local = g - c.begin;
-    c.y = local / c.X;
-    c.xc = static_cast<int>(local - c.y * c.X);
-}
-
-// advance to chunk g (= previous chunk + 1)
-__device__ __forceinline__ void cursor_next(Cursor& c, int64_t g) {
-    if (++c.xc == c.X) {
-        c.xc = 0;
-        ++c.y;
-    }
-    while (g >= c.end && c.t + 1 < c.n_tensors) {  // batch mode only: single tensors never get here
-        ++c.t;
-        cursor_take(c, c.table[c.t]);
-        c.y = 0;
-        c.xc = 0;
-    }
-}
-
-// the contiguous slice of [0, total) that workgroup `bid` of a grid of G (multiple of 8) owns;
-// workgroups b, b+8, b+16, ... run on the same XCD and take neighbouring slices
-// `align` > 1 (a power of two): where slices are long (64 items and more), the boundaries between the
-// slices of one XCD fall on multiples of `align` counted from -`first`, i.e. on absolute multiples when
-// [0, total) stands for the items first .. first + total - 1 of a longer list
-__device__ __forceinline__ void my_range(int64_t total, int64_t& g0, int64_t& g1, int align = 1, int64_t first = 0) {
-    const int64_t bid = blockIdx.x, S = gridDim.x >> 3;
-    const int64_t xcd = bid & 7, slot = bid >> 3;
-    const int64_t per = (total + 7) >> 3;
-    const int64_t xb = xcd * per;
-    int64_t xe = xb + per;
-    xe = xe > total ? total : xe;
-    const int64_t len = xe > xb ? xe - xb : 0;
-    g0 = xb + len * slot / S;
-    g1 = xb + len * (slot + 1) / S;
-    if (align > 1 && len >= 64 * S) {
-        if (slot > 0) g0 = ((g0 + first) & ~static_cast<int64_t>(align - 1)) - first;
-        if (slot + 1 < S) g1 = ((g1 + first) & ~static_cast<int64_t>(align - 1)) - first;
-        g0 = g0 < xb ? xb : g0;
-        g1 = g1 < xb ? xb : g1;
-    }
-}
-
-template <int kRow0 = 0, int kRow1 = 64>
-__device__ __forceinline__ void load_chunk_cols(float (&v)[64], const Cursor& c, int lane) {
-    load_chunk_rows<kRow0, kRow1>(v, (const void*)(c.base + (c.y * 64) * c.ld + static_cast<int64_t>(c.xc) * 64),
-                                  c.ld, lane);
-}
-
-// =========================================================================================
 // standalone transforms
 // =========================================================================================
 __global__ __launch_bounds__(64) void k_dct2d_fwd(const float* __restrict__ x, int64_t ld, int64_t X,
@@ -295,136 +109,6 @@ __global__ __launch_bounds__(64) void k_dct2d_inv(const float* __restrict__ coef
     float v[64];
     chunk_inverse<true, true>(v, tile, lane);
     store_chunk_cols(v, x, ld, y, xc, lane);
-}
-
-// the wave's issue priority (0 .. 3; the instruction takes an immediate, hence the ladder); `level` is wave-uniform
-__device__ __forceinline__ void set_wave_priority(int level) {
-    if (level == 0) __builtin_amdgcn_s_setprio(0);
-    else if (level == 1) __builtin_amdgcn_s_setprio(1);
-    else if (level == 2) __builtin_amdgcn_s_setprio(2);
-    else __builtin_amdgcn_s_setprio(3);
-}
-
-// Persistent fused encode: every wave walks its slice of the chunk list.  The kernel is bound by
-// vector-ALU issue and by the latencies between its phases, so it is shaped for residency -
-// 8.5 KB + 1 KB of LDS and a register budget that admits three to four waves per SIMD - and
-// leaves the overlap of one wave's row loads with the other waves' arithmetic to the hardware.
-// The three waves of a SIMD pass its issue slots round: the arbiter alone serves the oldest wave first, so
-// that the workgroups dispatched last run behind all the way and the launch waits for them.  Each wave
-// therefore steps through the priority levels 0, 1, 2 chunk by chunk, the three dispatch layers of a full
-// grid one step apart, and changes level once its rows are requested (4 % off the launch; the level
-// values, the direction and a change at another phase or every other chunk matter less than 1 %).
-// kEf: the miner's momentum update rides on the load (src/tplr/neurons.py:151-152): the chunk of
-// the error-feedback tensor becomes ef * decay + grad (two roundings, as mul_ then add_), is
-// written back in place and is what gets encoded.
-// Without the transform the kernel waits more than it computes, and workgroups of two waves that take alternate
-// chunks and meet at a barrier before they request their rows (512 contiguous bytes per row at the same moment) are
-// 6 % faster; with the transform, where the vector ALU is the bound, any team is slower (8 % with four waves).
-// kEf also writes every chunk back, and rows written together are served sooner: teams of four without the
-// transform (8 % off the two-launch miner step against single waves), of two with it (4 %).
-template <bool kUseDct, bool kEf = false>
-constexpr int encode_team() { return kUseDct ? (kEf ? 2 : 1) : (kEf ? 4 : 2); }
-
-template <bool kTwo, bool kUseDct, bool kEf = false>
-__global__ __launch_bounds__((64 * encode_team<kUseDct, kEf>()), 3) void k_encode_topk_pack(const tplr_tensor_desc* __restrict__ table,
-                                                            const tplr_tensor_desc single, int n_tensors,
-                                                            int64_t total, int k, uint8_t* __restrict__ idx12,
-                                                            float* __restrict__ val,
-                                                            const tplr_tensor_desc* __restrict__ grad_table,
-                                                            float decay) {
-    constexpr int T = encode_team<kUseDct, kEf>();
-    __shared__ __align__(16) float buf_all[T][kHalfFloats];
-    __shared__ uint64_t cand_all[T][kCandCap];
-    const int wv = T > 1 ? __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6)) : 0;  // wave of the team
-    float* const buf = buf_all[wv];
-    uint64_t* const cand = cand_all[wv];
-    const int lane = threadIdx.x & 63;
-    int64_t g0, g1;
-    my_range(total, g0, g1, T);
-    if (g0 >= g1) return;
-    // T > 1: [g0, g1) becomes this wave's share of the team's range, every T-th chunk; every wave of the team arrives
-    // at `team_steps` barriers
-    const int64_t team_steps = (g1 - g0 + T - 1) / T;
-    g0 += wv;
-    const int64_t my_steps = g0 < g1 ? (g1 - 1 - g0) / T + 1 : 0;
-    if constexpr (T > 1) {
-        if (my_steps == 0) {  // wave-uniform: a team with fewer chunks than waves
-            for (int64_t i = 0; i < team_steps; ++i) __builtin_amdgcn_s_barrier();
-            return;
-        }
-    }
-    Cursor c, cg;
-    cursor_seek(c, table, single, n_tensors, g0);
-    if (kEf) cursor_seek(cg, grad_table, single, n_tensors, g0);
-#if TPLR_DCT_MATRIX_CORES
-    float ca[16] = {};
-    if (kUseDct) load_dct4_operand(ca, lane);
-#endif
-    int turn = static_cast<int>(blockIdx.x * 3u / gridDim.x);  // the dispatch layer of a full grid; wave-uniform
-    for (int64_t g = g0; g < g1; g += T) {
-        float v[64], w[64];
-        if constexpr (T > 1) __builtin_amdgcn_s_barrier();  // the team asks for its rows together
-        load_chunk_cols(v, c, lane);
-        if (kEf) {
-            load_chunk_cols(w, cg, lane);
-#pragma unroll
-            for (int r = 0; r < 64; ++r) {
-                const float m = v[r] * decay;
-                v[r] = m + w[r];
-            }
-            store_chunk_cols(v, (float*)c.base, c.ld, c.y, c.xc, lane);
-            if (g + T < g1) {
-#pragma unroll
-                for (int s = 1; s <= T; ++s) cursor_next(cg, g + s);
-            }
-        }
-        if (g + T < g1) {
-#pragma unroll
-            for (int s = 1; s <= T; ++s) cursor_next(c, g + s);
-        }
-        // Untransformed gradients often differ in scale from row to row or column to column;
-        // the select's threshold statistic is then taken in both directions.  (Coefficients of
-        // the transform are mixed across both and one direction is as good as two.)
-        set_wave_priority(turn);
-        turn = turn == 2 ? 0 : turn + 1;
-        uint32_t c1 = 0, c2 = 0;
-        if (!kUseDct) lane_stats<kTwo>(v, c1, c2);
-#if TPLR_DCT_MATRIX_CORES
-        if (kUseDct) dct64_fwd_matrix(v, ca);
-        transpose_via_half(v, w, buf, lane);
-        if (kUseDct) dct64_fwd_matrix(w, ca);
-#else
-        chunk_forward<kUseDct>(v, w, buf, lane);
-#endif
-        const Selected s =
-            select_topk<kTwo, !kUseDct>(w, buf, cand, lane, k, kUseDct ? kDctPow2Scale : 1.0f, c1, c2);
-        emit_selected<kTwo>(s, lane, k, g, idx12, val);
-    }
-    if constexpr (T > 1) {
-        for (int64_t i = my_steps; i < team_steps; ++i) __builtin_amdgcn_s_barrier();
-    }
-}
-
-// Measurement aid: the memory side of the encode alone - the same grid, chunk ranges and row loads, nothing else
-// (the 64 values of a lane are added up so that the loads are not dropped, and the sum never leaves the wave).
-__global__ __launch_bounds__(64, 3) void k_calib_encode(const tplr_tensor_desc* __restrict__ table,
-                                                        const tplr_tensor_desc single, int n_tensors, int64_t total,
-                                                        float* __restrict__ sink) {
-    const int lane = threadIdx.x;
-    int64_t g0, g1;
-    my_range(total, g0, g1);
-    if (g0 >= g1) return;
-    Cursor c;
-    cursor_seek(c, table, single, n_tensors, g0);
-    float s = 0.0f;
-    for (int64_t g = g0; g < g1; ++g) {
-        float v[64];
-        load_chunk_cols(v, c, lane);
-        if (g + 1 < g1) cursor_next(c, g + 1);
-#pragma unroll
-        for (int r = 0; r < 64; ++r) s += v[r];
-    }
-    if (__float_as_uint(s) == 0x7fedcba9u && sink) sink[0] = s;  // (a NaN pattern no sum produces)
 }
 
 // body(Index<0>{}) ... body(Index<N - 1>{}): a loop whose counter is a constant in the body, so that
@@ -3176,20 +2860,6 @@ __global__ __launch_bounds__(256, 2) void k_fill_lds(uint32_t word, uint32_t* __
 // =========================================================================================
 using namespace tplr;
 
-// kTeam: waves per workgroup of the kernel (encode_team<> of its instantiation)
-template <int kTeam = 1, typename Kernel>
-static int launch_encode_as(Kernel kernel, const tplr_tensor_desc* d_desc, const tplr_tensor_desc& single,
-                            int n_tensors, int64_t total, int k, uint8_t* d_idx12, float* d_val, void* stream,
-                            const tplr_tensor_desc* d_grad_desc = nullptr, float decay = 0.f) {
-    static int resident = 0;  // workgroups
-    if (resident == 0) resident = persistent_grid(kernel, int64_t{1} << 40, 64 * kTeam);
-    const int64_t need = (((total + kTeam - 1) / kTeam + 7) / 8) * 8;  // workgroups that have a chunk each, in eights
-    const dim3 grid(static_cast<unsigned>(need < resident ? need : resident)), block(64 * kTeam);
-    hipLaunchKernelGGL(kernel, grid, block, 0, static_cast<hipStream_t>(stream), d_desc, single, n_tensors, total, k,
-                       d_idx12, d_val, d_grad_desc, decay);
-    return launch_status();
-}
-
 // kTeam: waves per workgroup of the kernel (aggregate_team<> of its instantiation)
 template <int kTeam = 1, typename Kernel>
 static int launch_decode_as(Kernel kernel, const PeerPtrs& pp, const float* d_scale, int n_peers, int k,
@@ -3254,15 +2924,6 @@ int tplr_unpack12(const uint8_t* d_packed, int64_t n, int64_t* d_idx, void* stre
 
 // (tplr_pack12_host, tplr_unpack12_host and tplr_gather_host touch host memory only: tplr_host.cpp)
 
-static int check_2d(const void* a, const void* b, int64_t R, int64_t C) {
-    if (!a || !b || R < 0 || C < 0) return TPLR_E_BADARG;
-    if ((R % 64) || (C % 64)) return TPLR_E_SHAPE;
-    return 0;
-}
-
-// chunk rows are addressed with 32-bit byte offsets (63 rows * ld * 4 bytes)
-static inline bool ld_ok(int64_t ld) { return ld > 0 && ld <= (int64_t{1} << 23); }
-
 int tplr_dct2d_fwd(const float* d_x, int64_t R, int64_t C, int64_t ld_x, float* d_coef, void* stream) {
     if (int s = check_2d(d_x, d_coef, R, C)) return s;
     if (ld_x < C) return TPLR_E_BADARG;
@@ -3283,65 +2944,6 @@ int tplr_dct2d_inv(const float* d_coef, int64_t R, int64_t C, float* d_x, int64_
     hipLaunchKernelGGL(k_dct2d_inv, dim3(grid8(n)), dim3(64), 0, static_cast<hipStream_t>(stream), d_coef,
                        C / 64, n, d_x, ld_x);
     return launch_status();
-}
-
-static int launch_encode(const tplr_tensor_desc* d_desc, const tplr_tensor_desc& single, int n_tensors,
-                         int64_t total, int k, int use_dct, uint8_t* d_idx12, float* d_val, void* stream) {
-    if (k > 32) {
-        if (use_dct)
-            return launch_encode_as(k_encode_topk_pack<true, true>, d_desc, single, n_tensors, total, k, d_idx12, d_val, stream);
-        return launch_encode_as<encode_team<false>()>(k_encode_topk_pack<true, false>, d_desc, single, n_tensors, total, k, d_idx12, d_val, stream);
-    }
-    if (use_dct)
-        return launch_encode_as(k_encode_topk_pack<false, true>, d_desc, single, n_tensors, total, k, d_idx12, d_val, stream);
-    return launch_encode_as<encode_team<false>()>(k_encode_topk_pack<false, false>, d_desc, single, n_tensors, total, k, d_idx12, d_val, stream);
-}
-
-int tplr_encode_topk_pack(const float* d_x, int64_t R, int64_t C, int64_t ld_x, int k, int use_dct,
-                          uint8_t* d_idx12, float* d_val, void* stream) {
-    if (int s = check_2d(d_x, d_val, R, C)) return s;
-    if (!d_idx12 || ld_x < C || k < 2 || (k & 1) || k > kCandCap) return TPLR_E_BADARG;
-    const int64_t n = (R / 64) * (C / 64);
-    if (n == 0) return 0;
-    if (C / 64 > 0x7fffffff || R / 64 > 0x7fffffff || !ld_ok(ld_x)) return TPLR_E_TOOMANY;
-    tplr_tensor_desc single;
-    single.dense = const_cast<float*>(d_x);
-    single.ld = ld_x;
-    single.chunk_begin = 0;
-    single.x_chunks = static_cast<int32_t>(C / 64);
-    single.y_chunks = static_cast<int32_t>(R / 64);
-    return launch_encode(nullptr, single, 1, n, k, use_dct, d_idx12, d_val, stream);
-}
-
-int tplr_encode_topk_pack_batch(const tplr_tensor_desc* d_desc, int n_tensors, int64_t total_chunks, int k,
-                                int use_dct, uint8_t* d_idx12, float* d_val, void* stream) {
-    if (!d_desc || n_tensors < 1 || total_chunks < 0 || !d_idx12 || !d_val || k < 2 || (k & 1) || k > kCandCap)
-        return TPLR_E_BADARG;
-    if (total_chunks == 0) return 0;
-    tplr_tensor_desc none = {};
-    return launch_encode(d_desc, none, n_tensors, total_chunks, k, use_dct, d_idx12, d_val, stream);
-}
-
-int tplr_ef_encode_topk_pack_batch(const tplr_tensor_desc* d_ef_desc, const tplr_tensor_desc* d_grad_desc,
-                                   int n_tensors, int64_t total_chunks, float decay, int k, int use_dct,
-                                   uint8_t* d_idx12, float* d_val, void* stream) {
-    if (!d_ef_desc || !d_grad_desc || n_tensors < 1 || total_chunks < 0 || !d_idx12 || !d_val || k < 2 || (k & 1) ||
-        k > kCandCap)
-        return TPLR_E_BADARG;
-    if (total_chunks == 0) return 0;
-    tplr_tensor_desc none = {};
-    if (k > 32) {
-        if (use_dct)
-            return launch_encode_as<encode_team<true, true>()>(k_encode_topk_pack<true, true, true>, d_ef_desc, none, n_tensors, total_chunks, k,
-                                    d_idx12, d_val, stream, d_grad_desc, decay);
-        return launch_encode_as<encode_team<false, true>()>(k_encode_topk_pack<true, false, true>, d_ef_desc, none, n_tensors, total_chunks, k,
-                                d_idx12, d_val, stream, d_grad_desc, decay);
-    }
-    if (use_dct)
-        return launch_encode_as<encode_team<true, true>()>(k_encode_topk_pack<false, true, true>, d_ef_desc, none, n_tensors, total_chunks, k,
-                                d_idx12, d_val, stream, d_grad_desc, decay);
-    return launch_encode_as<encode_team<false, true>()>(k_encode_topk_pack<false, false, true>, d_ef_desc, none, n_tensors, total_chunks, k,
-                            d_idx12, d_val, stream, d_grad_desc, decay);
 }
 
 int tplr_ef_step_batch(const tplr_tensor_desc* d_ef_desc, const tplr_tensor_desc* d_grad_desc, int n_tensors,
@@ -4114,19 +3716,6 @@ int tplr_calib_aggregate(const uint8_t* const* h_idx12, const float* const* h_va
         hipLaunchKernelGGL(k_calib_aggregate<4>, grid, dim3(64), 0, on, pp, n_peers, k, d_desc, n_tensors, total_chunks);
     else
         hipLaunchKernelGGL(k_calib_aggregate<2>, grid, dim3(64), 0, on, pp, n_peers, k, d_desc, n_tensors, total_chunks);
-    return launch_status();
-}
-
-int tplr_calib_encode(const tplr_tensor_desc* d_desc, int n_tensors, int64_t total_chunks, void* stream) {
-    if (!d_desc || n_tensors < 1 || total_chunks < 0) return TPLR_E_BADARG;
-    if (total_chunks == 0) return 0;
-    static int resident = 0;
-    if (resident == 0) resident = persistent_grid(k_encode_topk_pack<false, true>, int64_t{1} << 40);  // the grid it stands in for
-    const int64_t need = ((total_chunks + 7) / 8) * 8;
-    tplr_tensor_desc none = {};
-    hipLaunchKernelGGL(k_calib_encode, dim3(static_cast<unsigned>(need < resident ? need : resident)), dim3(64), 0,
-                       static_cast<hipStream_t>(stream), d_desc, none, n_tensors, total_chunks,
-                       static_cast<float*>(nullptr));
     return launch_status();
 }
 

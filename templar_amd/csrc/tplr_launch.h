@@ -4,6 +4,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include "../../include/tplr_hip.h"
+
 namespace tplr {
 
 inline int launch_status() {
@@ -15,6 +17,15 @@ inline int launch_status() {
 constexpr int64_t kMaxGroups256 = 0xfffff0;
 
 inline unsigned grid8(int64_t n) { return static_cast<unsigned>(((n + 7) / 8) * 8); }
+
+inline int check_2d(const void* a, const void* b, int64_t R, int64_t C) {
+    if (!a || !b || R < 0 || C < 0) return TPLR_E_BADARG;
+    if ((R % 64) || (C % 64)) return TPLR_E_SHAPE;
+    return 0;
+}
+
+// chunk rows are addressed with 32-bit byte offsets (63 rows * ld * 4 bytes)
+inline bool ld_ok(int64_t ld) { return ld > 0 && ld <= (int64_t{1} << 23); }
 
 // persistent grids: exactly one resident set of workgroups of `threads` threads (one wave, or a team of
 // waves), as the occupancy calculator reports it for the kernel at hand (registers or LDS bound it); a
