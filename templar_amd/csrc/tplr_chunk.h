@@ -218,12 +218,13 @@ __device__ __forceinline__ int find_tensor(const tplr_tensor_desc* __restrict__ 
     int lo = 0, len = n_tensors;
     while (len > 1) {  // wave-uniform
         const int step = (len + 7) >> 3;
+        uint32_t begin[8];
+#pragma unroll
+        for (int i = 1; i < 8; ++i)  // (past the end the last one: a load behind a branch would be waited for there)
+            begin[i] = static_cast<uint32_t>(table[lo + (i * step < len ? i * step : len - 1)].chunk_begin);
         int k = 0;
 #pragma unroll
-        for (int i = 1; i < 8; ++i) {
-            const int at = i * step < len ? i * step : 0;
-            k += at != 0 && static_cast<uint32_t>(table[lo + at].chunk_begin) <= g ? step : 0;
-        }
+        for (int i = 1; i < 8; ++i) k += i * step < len && begin[i] <= g ? step : 0;
         lo += k;
         len = len - k < step ? len - k : step;
     }
@@ -232,8 +233,12 @@ __device__ __forceinline__ int find_tensor(const tplr_tensor_desc* __restrict__ 
 
 __device__ __forceinline__ Place place_of(const tplr_tensor_desc* __restrict__ table, const tplr_tensor_desc& single, int n_tensors,
                                           int64_t g) {
-    const int t = table ? find_tensor(table, n_tensors, static_cast<uint32_t>(g)) : 0;  // wave-uniform branch
-    const tplr_tensor_desc& d = table ? table[t] : single;
+    tplr_tensor_desc d = single;
+    int t = 0;
+    if (table) {  // wave-uniform
+        t = find_tensor(table, n_tensors, static_cast<uint32_t>(g));
+        d = table[t];
+    }
     const int64_t ld = uniform64(d.ld), begin = uniform64(d.chunk_begin);
     const uint32_t X = __builtin_amdgcn_readfirstlane(d.x_chunks);
     const uint32_t local = static_cast<uint32_t>(g - begin), y = local / X, xc = local - y * X;

@@ -1,0 +1,279 @@
+// Decode of payloads with the transform, a chunk per wave: aggregate, evaluation update, outer step.
+#include <hip/hip_runtime.h>
+#include <stdint.h>
+
+#include <type_traits>
+
+#include "../../include/tplr_hip.h"
+#include "tplr_chunk.h"
+#include "tplr_device.h"
+#include "tplr_launch.h"
+
+namespace tplr {
+
+// ---- half a chunk in LDS: 32 rows of 64 floats, without padding.  Row r's sixteen quads of columns are permuted by r mod 16,
+// so that a row per lane (16 bytes at a time) and a column per lane (4 bytes) both reach all banks.
+constexpr int kHalfWords = 32 * 64;
+// where coefficient e = 64 row + column of the chunk lies, counted over both halves
+__device__ __forceinline__ uint32_t half_pos(uint32_t e) { return e ^ ((e >> 4) & 0x3cu); }
+
+__device__ __forceinline__ void half_rows_to_regs(float (&w)[64], const float* tile, int row) {  // row: 0 .. 31
+    const float4* r4 = reinterpret_cast<const float4*>(tile + row * 64);
+#pragma unroll
+    for (int c = 0; c < 16; ++c) {
+        const float4 t = r4[c ^ (row & 15)];
+        w[4 * c] = t.x, w[4 * c + 1] = t.y, w[4 * c + 2] = t.z, w[4 * c + 3] = t.w;
+    }
+}
+__device__ __forceinline__ void regs_to_half_rows(const float (&w)[64], float* tile, int row) {
+    float4* r4 = reinterpret_cast<float4*>(tile + row * 64);
+#pragma unroll
+    for (int c = 0; c < 16; ++c) r4[c ^ (row & 15)] = make_float4(w[4 * c], w[4 * c + 1], w[4 * c + 2], w[4 * c + 3]);
+}
+// v[32 half + r] = row r, column `lane`
+template <int kHalf>
+__device__ __forceinline__ void half_cols_to_regs(float (&v)[64], const float* tile, int lane) {
+#pragma unroll
+    for (int r = 0; r < 32; ++r) v[32 * kHalf + r] = tile[r * 64 + (lane ^ ((r & 15) << 2))];
+}
+
+// Up to fifteen peers' payloads into chunks, through the inverse transform: the aggregate of k_decode_aggregate (same bits), and
+// with kSubtract dst - result and its guard against results that are not finite.
+//
+// A wave takes one chunk, a workgroup four neighbouring ones, and ends: the hardware puts the next chunk where one has
+// ended, so that loads, arithmetic and stores of a compute unit's waves overlap whatever their pace, and a set's last round
+// is as full as the others.  What that needs is waves: the chunk goes through LDS in halves of 32 rows (9 KB a wave),
+// scattered, averaged and read into registers one after the other, and three waves fit a SIMD where k_decode_aggregate has
+// two, its next chunks' payloads in the registers of the third.  Against that stand the payload's way from memory, which
+// nothing hides here, and a chain of LDS round trips per peer and half.
+// Subtracting, what bounds it is the loads and stores (1520 us alone) and this form is the faster one throughout.  In us, before
+// and now: one peer, the 294 144 chunks of a 1B set 1722 -> 1545, a 150M model's 39 648 274 -> 225; eight peers of k = 64 1890 -> 1725,
+// fifteen 2222 -> 1915; one 2048 x 2048 tensor from four 19 -> 15.  The team stores together (1544, each wave by itself 1570).
+// Not subtracting, payloads not in any cache: one peer 972 -> 940 and 154 -> 138; for more see decode_chunks_serves.
+constexpr int kChunkPeers = 15;  // what four bits count
+struct ChunkPeers {
+    const uint8_t* idx[kChunkPeers];
+    const float* val[kChunkPeers];  // (those past the last repeat it)
+};
+
+template <int kUnits, bool kSubtract>
+__global__ __launch_bounds__(256, 3) void k_decode_chunk(const ChunkPeers pp, const float* __restrict__ scale, int P, int k,
+                                                       const tplr_tensor_desc* __restrict__ table, const tplr_tensor_desc single,
+                                                       int n_tensors, int64_t first, int64_t end, int mean, int with_sum,
+                                                       float* __restrict__ stats, int32_t* __restrict__ guard) {
+    constexpr int T = 4;
+    constexpr int kCntWords = kUnits > 1 ? kHalfWords / 8 : 4;  // four bits a coefficient
+    constexpr uint32_t kMark = 0xffffffffu;  // (a NaN: a sum has these bits only if a peer sent them)
+    __shared__ __align__(16) float tile_all[T][kHalfWords];
+    __shared__ __align__(16) uint32_t cnt_all[T][kCntWords];
+    const int wv = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
+    float* const tile = tile_all[wv];
+    uint32_t* const cnt = cnt_all[wv];
+    const int lane = threadIdx.x & 63;
+    const int64_t g = first + xcd_contiguous(blockIdx.x, gridDim.x) * T + wv;
+    if (g >= end) return;  // wave-uniform
+
+    // ---- the payload: lane j holds entry j of every peer (lanes without one reload entry 0 and stay out of it)
+    const bool lane_on = lane < k;
+    const int le = lane_on ? lane : 0;
+    const int64_t at_idx = uniform64(g * (k + (k >> 1))), at_val = uniform64(g * k);
+    const uint32_t io = 3u * (static_cast<uint32_t>(le) >> 1) + (le & 1);
+    uint32_t pos[kUnits];
+    float val[kUnits];
+#pragma unroll
+    for (int u = 0; u < kUnits; ++u) {
+        pos[u] = *(const gu16*)((const gbyte*)pp.idx[u] + at_idx + io);
+        val[u] = ((const gfloat*)pp.val[u] + at_val)[le];
+    }
+    const Place at = place_of(table, single, n_tensors, g);
+    const int pl = lane < P ? lane : P - 1;
+    // (the transform below is 32x the orthonormal one: its input carries the exact 2^-5)
+    const float sc = (scale ? scale[static_cast<int64_t>(at.t) * P + pl] : 1.0f) * kDctPow2Scale;
+    auto factor_of = [&](int p) { return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, sc), p)); };
+#pragma unroll
+    for (int u = 0; u < kUnits; ++u) {
+        const uint32_t e = (le & 1) ? pos[u] >> 4 : pos[u] & 0xfffu;
+        pos[u] = lane_on && u < P ? half_pos(e) << 2 : 0xffffu;  // in bytes; the last of them in neither half
+        val[u] *= factor_of(u);
+    }
+
+    auto clear = [&] {
+#pragma unroll
+        for (int q = 0; q < 8; ++q) reinterpret_cast<float4*>(tile)[q * 64 + lane] = make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma unroll
+        for (int q = 0; q < kCntWords / 256; ++q) reinterpret_cast<uint4*>(cnt)[q * 64 + lane] = make_uint4(0u, 0u, 0u, 0u);
+        wave_lds_fence();
+    };
+    // sums of half a chunk with every entry in its turn, then counts, then means
+    auto exact_half = [&](uint32_t half) __attribute__((always_inline)) {
+        float4 total[8];
+#pragma unroll 1
+        for (int phase = 0; phase < 2; ++phase) {
+            clear();
+#pragma unroll 1
+            for (int p = 0; p < P; ++p) {
+                const uint32_t w = *(const gu16*)((const gbyte*)pp.idx[p] + at_idx + io);
+                const uint32_t e = half_pos((le & 1) ? w >> 4 : w & 0xfffu);
+                float x = ((const gfloat*)pp.val[p] + at_val)[le] * factor_of(p);
+                if (phase) x = 1.0f;
+                const bool here = lane_on && (e >> 11) == half;
+                const int me = here ? static_cast<int>(e & 2047u) : -1;
+                int rank = 0;  // among the earlier lanes that name the same coefficient; one rank per turn
+                for (int i = 0; i < 63; ++i) {
+                    const int other = __shfl(me, i);
+                    rank += (i < lane && other == me && here) ? 1 : 0;
+                }
+                const int turns = static_cast<int>(wave_max_u32(static_cast<uint32_t>(rank)));
+                for (int r = 0; r <= turns; ++r) {
+                    if (here && rank == r) tile[me] = tile[me] + x;
+                    wave_lds_fence();
+                }
+            }
+            if (phase == 0) {
+#pragma unroll
+                for (int q = 0; q < 8; ++q) total[q] = reinterpret_cast<const float4*>(tile)[q * 64 + lane];
+                wave_lds_fence();
+            }
+        }
+#pragma unroll
+        for (int q = 0; q < 8; ++q) {
+            float4 n = reinterpret_cast<const float4*>(tile)[q * 64 + lane];
+            auto one = [&](float s, float c) { return mean && c > 1.0f ? s / c : s; };
+            n.x = one(total[q].x, n.x), n.y = one(total[q].y, n.y), n.z = one(total[q].z, n.z), n.w = one(total[q].w, n.w);
+            reinterpret_cast<float4*>(tile)[q * 64 + lane] = n;
+        }
+        wave_lds_fence();
+    };
+    // the coefficients of one half into the tile
+    auto gather_half = [&](auto ht) __attribute__((always_inline)) {
+        constexpr uint32_t half = decltype(ht)::value;
+        clear();
+        uint32_t seen = 0;
+#pragma unroll
+        for (int u = 0; u < kUnits; ++u) {
+            if ((pos[u] >> 13) == half) {
+                float* const t = reinterpret_cast<float*>(reinterpret_cast<char*>(tile) + (pos[u] & 8191u));
+                const uint32_t old = __hip_atomic_exchange(reinterpret_cast<uint32_t*>(t), kMark, __ATOMIC_RELAXED,
+                                                           __HIP_MEMORY_SCOPE_WAVEFRONT);
+                // (one peer sends a coefficient once, or the exact path has it)
+                if constexpr (kUnits > 1)
+                    __hip_atomic_fetch_add(&cnt[(pos[u] >> 5) & 255u], 1u << (pos[u] & 28u), __ATOMIC_RELAXED,
+                                           __HIP_MEMORY_SCOPE_WAVEFRONT);
+                seen = seen > old ? seen : old;
+                *t = __uint_as_float(old) + val[u];
+            }
+        }
+        wave_lds_fence();
+        if (__builtin_expect(__ballot(seen == kMark) != 0, 0)) {  // wave-uniform
+            exact_half(half);
+        } else if (kUnits > 1 && mean) {
+            // a lane scans the counters of half a row and divides the coefficients that several peers sent, one per trip;
+            // bit 4 j + q of m: the counter of its coefficient 8 q + j is at least two
+            const uint4 w = reinterpret_cast<const uint4*>(cnt)[lane];
+            auto multi = [](uint32_t c) { return ((c >> 1) | (c >> 2) | (c >> 3)) & 0x11111111u; };
+            uint32_t m = multi(w.x) | multi(w.y) << 1 | multi(w.z) << 2 | multi(w.w) << 3;
+            while (m) {
+                const int b = __builtin_ctz(m);
+                m &= m - 1;
+                const uint32_t w01 = (b & 1) ? w.y : w.x, w23 = (b & 1) ? w.w : w.z;
+                const uint32_t n = (((b & 2) ? w23 : w01) >> (b & 28)) & 15u;
+                float* const t = &tile[lane * 32 + (b & 3) * 8 + (b >> 2)];
+                *t = *t / static_cast<float>(n);
+            }
+            wave_lds_fence();
+        }
+    };
+
+    float v[64], before[64];
+    {
+        float w[64];
+        gather_half(std::integral_constant<uint32_t, 0>{});
+        if (lane < 32) half_rows_to_regs(w, tile, lane & 31);
+        wave_lds_fence();
+        gather_half(std::integral_constant<uint32_t, 1>{});
+        if (lane >= 32) half_rows_to_regs(w, tile, lane & 31);
+        wave_lds_fence();
+        dct64_inv(w);  // along d: w[l] = sum_d Y[lane][d] F[l][d]
+        if (lane < 32) regs_to_half_rows(w, tile, lane & 31);
+        wave_lds_fence();
+        half_cols_to_regs<0>(v, tile, lane);
+        wave_lds_fence();
+        if (lane >= 32) regs_to_half_rows(w, tile, lane & 31);
+        wave_lds_fence();
+        half_cols_to_regs<1>(v, tile, lane);
+    }
+    // (the destination's rows arrive during the second pass)
+    if constexpr (kSubtract) load_chunk_rows(before, (const void*)at.chunk0, at.ld, lane);
+    dct64_inv(v);  // along b: v[k] = sum_b Z[b][lane] F[k][b]
+    if (stats) {  // wave-uniform
+        float ss = 0.f, sm = 0.f;
+#pragma unroll
+        for (int r = 0; r < 64; ++r) ss = __builtin_fmaf(v[r], v[r], ss);
+        ss = wave_sum_f32(ss);
+        if (with_sum) {
+#pragma unroll
+            for (int r = 0; r < 64; ++r) sm += v[r];
+            sm = wave_sum_f32(sm);
+            if (lane == 0) stats[2 * g] = ss, stats[2 * g + 1] = sm;
+        } else if (lane == 0) {
+            stats[g] = ss;
+        }
+    }
+    bool drop = false;
+    if constexpr (kSubtract) {
+        if (guard) {  // wave-uniform
+            float z = 0.f;
+#pragma unroll
+            for (int r = 0; r < 64; ++r) z = __builtin_fmaf(v[r], 0.0f, z);
+            drop = __ballot(z != z) != 0;
+            if (drop && lane == 0) guard[at.t] = 1;
+        }
+#pragma unroll
+        for (int r = 0; r < 64; ++r) v[r] = before[r] - v[r];
+    }
+    // (a bare barrier: nothing is handed over, and a wave that has ended is not waited for)
+    if constexpr (kSubtract) __builtin_amdgcn_s_barrier();
+    store_chunk_rows(v, (void*)at.chunk0, at.ld, lane, drop);
+}
+
+template <int kUnits, bool kSubtract>
+static int launch_chunks(const ChunkPeers& pp, const float* d_scale, int n_peers, int k, const tplr_tensor_desc* d_desc,
+                      const tplr_tensor_desc& single, int n_tensors, int64_t total, int mean, int with_sum, float* d_stats,
+                      int32_t* d_guard, void* stream) {
+    constexpr int64_t piece = kMaxGroups256 * 4;  // chunks of one launch
+    for (int64_t first = 0; first < total; first += piece) {
+        const int64_t end = total - first < piece ? total : first + piece;
+        hipLaunchKernelGGL((k_decode_chunk<kUnits, kSubtract>), dim3(grid8((end - first + 3) / 4)), dim3(256), 0,
+                           static_cast<hipStream_t>(stream), pp, d_scale, n_peers, k, d_desc, single, n_tensors, first, end, mean,
+                           with_sum, d_stats, d_guard);
+    }
+    return launch_status();
+}
+
+// Without the subtraction, payloads coming from memory, in us k_decode_aggregate against this form (k = 32 / 64): 1024 chunks of
+// four peers 11.9 : 9.3 / 12.2 : 9.4, of fifteen 14.0 : 11.6 / 15.3 : 12.3; 4096 of four 23.9 : 21.9 / 24.5 : 22.8, of fifteen 27.5 : 27.1 /
+// 29.6 : 28.6; 8192 of four 40.2 : 37.9 / 41.6 : 39.4, of fifteen 46.9 : 47.5 / 50.8 : 50.4; but 16 384 of two 66.9 : 67.0 / 69.5 : 68.6, of eight
+// 72.5 : 76.2 / 75.1 : 80.5, 294 144 of two 980 : 1032 / 1074 : 1062, of fifteen 1216 : 1344 / 1255 : 1364.  (Between, where the other's rounds come out
+// badly, this one is ahead for a few peers: 39 648 of four 162 : 157 / 169 : 164.)
+bool decode_chunks_serves(int n_peers, int k, int64_t total, bool subtract) {
+    return n_peers <= kChunkPeers && k <= 64 && (subtract || n_peers == 1 || total <= 8192);
+}
+
+int decode_chunks(const uint8_t* const* h_idx12, const float* const* h_val, const float* d_scale, int n_peers, int k,
+                  const tplr_tensor_desc* d_desc, const tplr_tensor_desc& single, int n_tensors, int64_t total, bool subtract,
+                  bool mean, bool with_sum, float* d_stats, int32_t* d_guard, void* stream) {
+    ChunkPeers pp;
+    for (int u = 0; u < kChunkPeers; ++u) {
+        pp.idx[u] = h_idx12[u < n_peers ? u : n_peers - 1];
+        pp.val[u] = h_val[u < n_peers ? u : n_peers - 1];
+    }
+    auto launch = n_peers == 1    ? subtract ? launch_chunks<1, true> : launch_chunks<1, false>
+                  : n_peers == 2  ? subtract ? launch_chunks<2, true> : launch_chunks<2, false>
+                  : n_peers <= 4  ? subtract ? launch_chunks<4, true> : launch_chunks<4, false>
+                  : n_peers <= 8  ? subtract ? launch_chunks<8, true> : launch_chunks<8, false>
+                  : n_peers <= 12 ? subtract ? launch_chunks<12, true> : launch_chunks<12, false>
+                                  : subtract ? launch_chunks<15, true> : launch_chunks<15, false>;
+    return launch(pp, d_scale, n_peers, k, d_desc, single, n_tensors, total, mean, with_sum, d_stats, d_guard, stream);
+}
+
+}  // namespace tplr

@@ -191,10 +191,8 @@ struct Counters {
 // offset) plus one lane-constant offset and each clip factor is a scalar; the whole payload of
 // a chunk sits in 2 * kUnits registers and is requested a whole transform pass before it is used.
 // Generic path (kUnits == 0): any k and peer count, entries loaded where they are used.
-// kSubtract (fast path with the transform only): the destination receives destination - result
-// instead of the result (the error-feedback update of src/tplr/neurons.py:171); its rows are
-// requested before the second pass and arrive during it (without the transform, codes through wide loads:
-// requested when the chunk leaves the tile, before it is read out).  With `guard` (one int per tensor, zeroed by the
+// kSubtract (codes through wide loads): the destination receives destination - result; its rows are requested when the
+// chunk leaves the tile, before it is read out.  With `guard` (one int per tensor, zeroed by the
 // caller) a chunk whose result holds a NaN or an infinity is not subtracted - its destination keeps its
 // bits - and guard[tensor] becomes 1: the validator's check of the decoded gradient before
 // p.data.sub_ (neurons/validator.py:3646-3660).
@@ -239,7 +237,7 @@ __global__ __launch_bounds__((64 * aggregate_team<kUseDct, kUnits, kWideK, !kCod
                                                             const float* __restrict__ deq,
                                                             int32_t* __restrict__ guard) {
     static_assert(!kCodes || (kUnits > 0 && !kUseDct), "codes are served by the fast path without the transform");
-    static_assert(!(kCodes && kSubtract) || kWideK > 0, "the subtraction from codes: the wide-load pipeline only");
+    static_assert(!kSubtract || kWideK > 0, "the subtraction: the wide-load pipeline only");
     static_assert(kWideK == 0 || (kCodes && kStrided && (kWideK == 32 || kWideK == 64)), "wide loads: codes, equally spaced payloads");
     // this launch covers the chunks first .. first + total - 1 of the batch
     // options: bit 0 = per-peer, per-chunk normalisation (generic instantiation); bit 1 = `sumsq` takes two
@@ -979,13 +977,6 @@ __global__ __launch_bounds__((64 * aggregate_team<kUseDct, kUnits, kWideK, !kCod
             asm volatile("" : "+v"(my_units));
             // the register with the next unit's entry, on its way from another lane
             uint32_t held = group_entry(cur[0], from4);
-            // kSubtract: the destination's rows are requested here and arrive during the pass where the
-            // registers for that exist (up to 8 peers' payload in flight); with more peers they are fetched
-            // after the pass, sixteen rows at a time, two such groups in flight (kLateRows)
-            constexpr bool kLateRows = kSubtract && kUnits > 8;
-            float before[kSubtract && !kLateRows ? 64 : 1];
-            if constexpr (kSubtract && !kLateRows)
-                load_chunk_rows(before, (const void*)uniform64(reinterpret_cast<int64_t>(o0.chunk0)), uniform64(o0.ld), lane);
             // along b: v[k] = sum_b Z[b][lane] F[k][b]
             dct64_inv_hooked(v, [&](auto tag) {
                 constexpr int h = decltype(tag)::value;
@@ -1024,18 +1015,7 @@ __global__ __launch_bounds__((64 * aggregate_team<kUseDct, kUnits, kWideK, !kCod
                     }
                 }
             });
-            bool tripped = false;
-            // (kSubtract: the statistics are those of the decoded values, not of the difference)
-            if constexpr (kSubtract) chunk_stats(v, g, skip0);
-            if constexpr (kSubtract) {
-                // (a chunk that is to be done again on the exact path holds claim marks: it is tested there)
-                if (!skip0) tripped = guard_trips(v, o0.t);
-                if constexpr (!kLateRows) {
-#pragma unroll
-                    for (int r = 0; r < 64; ++r) v[r] = before[r] - v[r];
-                }
-            }
-            if constexpr (!kSubtract) chunk_stats(v, g, skip0);
+            chunk_stats(v, g, skip0);
             // (the loop-carried destination may have been parked in vector registers: make it
             // scalar again, or every store becomes a loop over distinct descriptors)
             const bool skip1 = g + T < g1 && __ballot(repeat == kClaimMark) != 0;  // wave-uniform, false for top-k payloads
@@ -1048,37 +1028,11 @@ __global__ __launch_bounds__((64 * aggregate_team<kUseDct, kUnits, kWideK, !kCod
             MeanState ms;
             mean_begin(ms);
             // a chunk that is to be done again is not stored: its descriptor gets a range of zero bytes
-            if constexpr (kLateRows) {
-                void* chunk0 = (void*)uniform64(reinterpret_cast<int64_t>(o0.chunk0));
-                const int64_t ld0 = uniform64(o0.ld);
-                const __amdgpu_buffer_rsrc_t rd = chunk_rsrc(chunk0, ld0);
-                const __amdgpu_buffer_rsrc_t wr = __builtin_amdgcn_make_buffer_rsrc(
-                    chunk0, 0, (skip0 || tripped) ? 0 : static_cast<int>((63 * ld0 + 64) * 4), 0x00020000);
-                const int ld4 = static_cast<int>(ld0) * 4;
-                float b[2][16];
-                auto fetch = [&](auto qt) {
-                    constexpr int q = decltype(qt)::value;
-#pragma unroll
-                    for (int i = 0; i < 16; ++i)
-                        b[q & 1][i] = __builtin_bit_cast(
-                            float, __builtin_amdgcn_raw_buffer_load_b32(rd, lane * 4, (q * 16 + i) * ld4, 0));
-                };
-                fetch(Index<0>{});
-                fetch(Index<1>{});
-                static_for<4>([&](auto qt) {
-                    constexpr int q = decltype(qt)::value;
-#pragma unroll
-                    for (int i = 0; i < 16; ++i)
-                        __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(int, b[q & 1][i] - v[q * 16 + i]), wr,
-                                                              lane * 4, (q * 16 + i) * ld4, 2);
-                    if constexpr (q + 2 < 4) fetch(Index<q + 2>{});
-                    mean_trip(ms);
-                });
-            } else {
+            {
                 const int64_t ld0 = uniform64(o0.ld);
                 const __amdgpu_buffer_rsrc_t wr = __builtin_amdgcn_make_buffer_rsrc(
                     (void*)uniform64(reinterpret_cast<int64_t>(o0.chunk0)), 0,
-                    (skip0 || tripped) ? 0 : static_cast<int>((63 * ld0 + 64) * 4), 0x00020000);
+                    skip0 ? 0 : static_cast<int>((63 * ld0 + 64) * 4), 0x00020000);
                 const int ld4 = static_cast<int>(ld0) * 4;
                 // (sixteen groups of four: 1.2 % faster than eight of eight in teams; thirty-two of two 13 % slower)
                 static_for<16>([&](auto qt) {
@@ -2989,13 +2943,9 @@ static int subtract_decoded(const uint8_t* d_idx12, const float* d_val, const fl
                            total_chunks, d_factor, d_guard);
         return launch_status();
     }
-    PeerPtrs pp;
-    for (int p = 0; p < TPLR_MAX_PEERS; ++p) pp.idx[p] = nullptr, pp.val[p] = nullptr;
-    pp.idx[0] = d_idx12;
-    pp.val[0] = d_val;
     // (one peer: the factor table (n_tensors, 1) is the aggregate's clip-factor table)
-    return launch_decode_as<4>(k_decode_aggregate<true, 8, 4, true, true>, pp, d_factor, 1, k, d_desc, none, n_tensors,
-                            total_chunks, TPLR_REDUCE_MEAN, 0, nullptr, stream, 0, 0, nullptr, d_guard);
+    return decode_chunks(&d_idx12, &d_val, d_factor, 1, k, d_desc, none, n_tensors, total_chunks, true, true, false, nullptr, d_guard,
+                      stream);
 }
 
 int tplr_ef_subtract_batch(const uint8_t* d_idx12, const float* d_val, int k, const tplr_tensor_desc* d_ef_desc,
@@ -3016,37 +2966,13 @@ int tplr_outer_step_batch(const uint8_t* const* h_idx12, const float* const* h_v
     if (!h_idx12 || !h_val || !d_param_desc || n_peers < 1 || n_tensors < 1 || total_chunks < 0 || k < 4 || (k & 1))
         return TPLR_E_BADARG;
     if ((d_chunk_stats == nullptr) != (d_tensor_stats == nullptr)) return TPLR_E_BADARG;
-    if (k > 64 || n_peers > 15) return TPLR_E_TOOMANY;  // the register-resident path with 4-bit counters
-    PeerPtrs pp;
-    for (int p = 0; p < TPLR_MAX_PEERS; ++p) {
-        pp.idx[p] = p < n_peers ? h_idx12[p] : nullptr;
-        pp.val[p] = p < n_peers ? h_val[p] : nullptr;
-        if (p < n_peers && (!pp.idx[p] || !pp.val[p])) return TPLR_E_BADARG;
-    }
+    if (k > 64 || n_peers > 15) return TPLR_E_TOOMANY;  // 4-bit counters
+    for (int p = 0; p < n_peers; ++p)
+        if (!h_idx12[p] || !h_val[p]) return TPLR_E_BADARG;
     if (total_chunks > 0) {
-        auto apart = [](const void* a, const void* b) {
-            return static_cast<int64_t>(reinterpret_cast<intptr_t>(a) - reinterpret_cast<intptr_t>(b));
-        };
-        const int64_t si = n_peers > 1 ? apart(pp.idx[1], pp.idx[0]) : 0;
-        const int64_t sv4 = n_peers > 1 ? apart(pp.val[1], pp.val[0]) : 0;
-        bool strided = true;
-        for (int p = 1; p < n_peers; ++p)
-            strided = strided && apart(pp.idx[p], pp.idx[0]) == p * si && apart(pp.val[p], pp.val[0]) == p * sv4;
-        tplr_tensor_desc none = {};
-        const int options = d_chunk_stats ? 2 : 0;
-        int st;
-        if (n_peers <= 8 && strided)
-            st = launch_decode_as<4>(k_decode_aggregate<true, 8, 4, true, true>, pp, d_factor, n_peers, k, d_param_desc, none,
-                                  n_tensors, total_chunks, TPLR_REDUCE_MEAN, options, d_chunk_stats, stream, si, sv4 / 4,
-                                  nullptr, d_nonfinite);
-        else if (strided)
-            st = launch_decode_as<4>(k_decode_aggregate<true, 16, 4, true, true>, pp, d_factor, n_peers, k, d_param_desc,
-                                  none, n_tensors, total_chunks, TPLR_REDUCE_MEAN, options, d_chunk_stats, stream, si,
-                                  sv4 / 4, nullptr, d_nonfinite);
-        else
-            st = launch_decode_as<4>(k_decode_aggregate<true, 16, 4, true, false>, pp, d_factor, n_peers, k, d_param_desc,
-                                  none, n_tensors, total_chunks, TPLR_REDUCE_MEAN, options, d_chunk_stats, stream, 0, 0,
-                                  nullptr, d_nonfinite);
+        const tplr_tensor_desc none = {};
+        const int st = decode_chunks(h_idx12, h_val, d_factor, n_peers, k, d_param_desc, none, n_tensors, total_chunks, true, true, true,
+                                     d_chunk_stats, d_nonfinite, stream);
         if (st) return st;
     }
     if (d_tensor_stats)
@@ -3132,6 +3058,9 @@ static int launch_decode(const uint8_t* const* h_idx12, const float* const* h_va
         pp.val[p] = p < n_peers ? h_val[p] : nullptr;
         if (p < n_peers && (!pp.idx[p] || !pp.val[p])) return TPLR_E_BADARG;
     }
+    if (use_dct && !d_deq && !(normalise & 1) && decode_chunks_serves(n_peers, k, total, false))
+        return decode_chunks(h_idx12, h_val, d_scale, n_peers, k, d_desc, single, n_tensors, total, false, reduce_mode == TPLR_REDUCE_MEAN,
+                          (normalise & 2) != 0, d_sumsq, nullptr, stream);
     // register-resident fast path: k <= 64 and at most 24 peers; 4-bit counters up to 15 peers, 5-bit beyond
     const int units = (k > 64 || (normalise & 1)) ? 0 : n_peers <= 8 ? 8 : n_peers <= 15 ? 16 : n_peers <= 24 ? 24 : 0;
     // equally spaced payloads (one staged buffer per window): scalar addressing

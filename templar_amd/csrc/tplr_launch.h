@@ -44,6 +44,15 @@ int persistent_grid(Kernel kernel, int64_t total, int threads = 64) {
     return static_cast<int>(need < g ? need : g);
 }
 
+// The aggregate with the transform, a chunk per wave, where that is the way to go (mean: as the reference, otherwise the sum;
+// with_sum: d_stats takes two floats a chunk, otherwise the sum of squares alone), subtract: dst - result, chunks whose
+// result is not finite left and their tensors flagged in d_guard.  single: the tensor where d_desc is null.  The arguments
+// checked by the caller.
+bool decode_chunks_serves(int n_peers, int k, int64_t total, bool subtract);
+int decode_chunks(const uint8_t* const* h_idx12, const float* const* h_val, const float* d_scale, int n_peers, int k,
+                  const tplr_tensor_desc* d_desc, const tplr_tensor_desc& single, int n_tensors, int64_t total, bool subtract,
+                  bool mean, bool with_sum, float* d_stats, int32_t* d_guard, void* stream);
+
 // The persistent aggregate of one parameter (k <= 64, at most 24 peers, mean, no transform) with the clip factors made from
 // n_norms <= 64 norms inside the launch; the arguments checked by the caller (tplr_aggregate_param).
 int aggregate_from_norms(const uint8_t* const* h_idx12, const float* const* h_val, const float* d_norms, int n_norms, int n_peers,

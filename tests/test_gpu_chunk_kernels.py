@@ -1,0 +1,117 @@
+"""Kernels that take one chunk per wave: sets of any make-up, and payloads at the edges of their peer counts."""
+import ctypes
+
+import numpy as np
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+from oracle import codec as orc  # noqa: E402  (the checker)
+import templar_amd.compress as tc  # noqa: E402
+from templar_amd import _lib  # noqa: E402
+
+
+@pytest.fixture(scope="module")
+def dev():
+    assert torch.cuda.is_available(), "these tests need an MI355X"
+    return torch.device("cuda:0")
+
+
+def _randn(shape, rng, dev):
+    return torch.empty(shape, device=dev).copy_(torch.from_numpy(rng.standard_normal(shape).astype(np.float32)))
+
+
+def _sizes(n, rng):
+    """(rows, columns) of n tensors of 0 .. 3 chunks, an empty one first, last and in between."""
+    out = [(64 * int(rng.integers(0, 3)), 64 * int(rng.integers(1, 3))) for _ in range(n)]
+    out[0] = out[-1] = (0, 64)
+    out[n // 2] = (64, 192)
+    return out
+
+
+@pytest.mark.parametrize("k", [2, 32, 34, 64, 128])
+@pytest.mark.parametrize("n", [1, 3, 8, 9, 64, 65, 513])
+def test_untransformed_sets_of_any_make_up(dev, n, k):
+    rng = np.random.default_rng(n)
+    x = [_randn(s, rng, dev) for s in _sizes(n, rng)]
+    batch = tc.TensorBatch(x)
+    idx, val = tc.encode_compress_batch(batch, k, use_dct=False)
+    want = [orc.topk_rows(orc.encode2d(t.cpu().numpy(), use_dct=False).reshape(-1, 4096), k) for t in x if t.numel()]
+    assert np.array_equal(idx.cpu().numpy(), np.concatenate([orc.pack12(i) for i, _ in want]))
+    assert np.array_equal(val.cpu().numpy(), np.concatenate([v for _, v in want]))
+    ef = [0.5 * t for t in x]
+    own, prev = tc.TensorBatch([t.clone() for t in ef]), tc.TensorBatch([t - 0.475 * t for t in x])
+    i2, v2 = torch.empty_like(idx), torch.empty_like(val)
+    st = _lib.load().tplr_ef_encode_topk_pack_batch(
+        ctypes.c_void_p(own.table.data_ptr()), ctypes.c_void_p(prev.table.data_ptr()), n, batch.total_chunks, 0.95, k, 0,
+        ctypes.c_void_p(i2.data_ptr()), ctypes.c_void_p(v2.data_ptr()), ctypes.c_void_p(torch.cuda.current_stream().cuda_stream))
+    assert st == 0
+    for got, e, g in zip(own.tensors, ef, prev.tensors):
+        assert torch.equal(got, e * 0.95 + g)
+    i3, v3 = tc.encode_compress_batch(own, k, use_dct=False)
+    assert torch.equal(i2, i3) and torch.equal(v2, v3)
+
+
+def _payloads(dev, batch, P, k, rng, repeat):
+    """P payloads that share half of their coefficients; `repeat`: some rows name one twice."""
+    n = batch.total_chunks
+    shared = np.stack([rng.permutation(4096)[: k // 2] for _ in range(n)])
+    idxs, vals = [], []
+    for _ in range(P):
+        own = np.stack([rng.permutation(np.setdiff1d(rng.permutation(4096)[: 3 * k], s))[: k - k // 2] for s in shared])
+        idx = rng.permuted(np.concatenate([shared, own], 1), axis=1)
+        if repeat:
+            idx[:: max(1, n // 3), -1] = idx[:: max(1, n // 3), 0]
+        idxs.append(torch.from_numpy(orc.pack12(idx)).to(dev))
+        vals.append(torch.from_numpy(rng.standard_normal((n, k)).astype(np.float32)).to(dev))
+    return idxs, vals
+
+
+# (the last: two chunks and more for every wave that could be resident at a time)
+@pytest.mark.parametrize("shapes,repeat", [([(64, 64)], False), ([(64, 64)], True), ([(0, 64), (128, 192), (64, 64), (64, 320), (0, 64)], False),
+                                           ([(0, 64), (128, 192), (64, 64), (64, 320), (0, 64)], True),
+                                           ([(2048, 8192), (2048, 320)], False)])
+@pytest.mark.parametrize("P,k", [(1, 64), (2, 32), (3, 32), (4, 64), (5, 64), (6, 16), (7, 4), (8, 34), (9, 32), (12, 64), (13, 4),
+                                 (15, 32), (15, 64)])
+def test_payloads_with_the_transform(dev, shapes, P, k, repeat):
+    rng = np.random.default_rng(1000 * P + k)
+    params = [_randn(s, rng, dev) for s in shapes]
+    before = [p.clone() for p in params]
+    out = tc.TensorBatch([torch.full_like(p, 7.0) for p in params])
+    batch = tc.TensorBatch(params)
+    idxs, vals = _payloads(dev, batch, P, k, rng, repeat)
+    scale = torch.from_numpy(rng.uniform(0.5, 1.0, (len(batch), P)).astype(np.float32)).to(dev)
+    n = batch.total_chunks
+    lib, stream = _lib.load(), ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    ptr = lambda t: ctypes.c_void_p(t.data_ptr())  # noqa: E731
+    lists = [(ctypes.c_void_p * P)(*[t.data_ptr() for t in ts]) for ts in (idxs, vals)]
+    flags = torch.zeros(len(batch), dtype=torch.int32, device=dev)
+    chunk_stats, stats = torch.zeros(2 * n, device=dev), torch.zeros(4 * len(batch), device=dev)
+    assert lib.tplr_decode_aggregate_batch(*lists, ptr(scale), P, k, ptr(out.table), len(batch), n, 0, 0, 1, None, stream) == 0
+    assert lib.tplr_outer_step_batch(*lists, ptr(scale), P, k, ptr(batch.table), len(batch), n, ptr(chunk_stats), ptr(stats), ptr(flags),
+                                     stream) == 0
+    assert not bool(flags.any())
+    for t in range(len(batch)):
+        if params[t].numel() == 0:
+            continue
+        # the step subtracts exactly what the aggregate leaves
+        assert torch.equal(params[t], before[t] - out.tensors[t]), t
+        if params[t].numel() <= 1 << 20:
+            sl = [batch.payload_slice(t, i, v, k) for i, v in zip(idxs, vals)]
+            Y, X = batch.xshape(t)[:2]
+            coef = orc.batch_decompress([i.cpu().numpy() for i, _ in sl],
+                                        [(v * scale[t, p]).cpu().numpy().reshape(Y, X, k) for p, (_, v) in enumerate(sl)],
+                                        batch.xshape(t), 4096, clip_norm=False)
+            want = orc.decode2d(coef)
+            assert np.abs(out.tensors[t].cpu().numpy() - want).max() <= 1e-5 * np.abs(want).max()
+    ss = torch.stack([o.double().square().sum() for o in out.tensors if o.numel()])
+    got = torch.stack([stats[4 * t + 3].double() for t in range(len(batch)) if params[t].numel()])
+    assert bool((got - ss).abs().le(4e-5 * ss).all())
+    # a chunk whose result is not finite is left as it is, and its tensor flagged
+    last = max(t for t in range(len(batch)) if params[t].numel())
+    vals[P - 1][-1, 0] = float("nan")
+    kept = params[last].clone()
+    assert lib.tplr_outer_step_batch(*lists, ptr(scale), P, k, ptr(batch.table), len(batch), n, None, None, ptr(flags), stream) == 0
+    assert flags.cpu().tolist() == [int(t == last) for t in range(len(batch))]
+    assert torch.equal(params[last][-64:, -64:], kept[-64:, -64:])
