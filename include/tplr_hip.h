@@ -371,6 +371,19 @@ int tplr_outer_step_codes_batch(const uint8_t* const* h_idx12, const uint8_t* co
                                 int n_tensors, int64_t total_chunks, float* d_chunk_stats, float* d_tensor_stats,
                                 int32_t* d_nonfinite, void* stream);
 
+/* The small launches around an update of a whole set.
+ * tplr_outer_factors: d_factor[t][p] = d_scale[t][p] * lr, the table an outer step takes; NaN for all peers of a tensor
+ * with a factor that is not finite and positive, and for every tensor where d_bad (one int, nullable) is not zero - such
+ * tensors are left as they are and flagged.
+ * tplr_update_factors: d_factor[t] = alpha * min(1, d_clip[t] / (norm_t + 1e-8)), norm_t from n_partials partial sums of
+ * squares (tplr_segment_sumsq of one peer); n_partials 0: alpha * d_clip[t].
+ * tplr_outer_stats: the (n_tensors, 4) figures of lr * gradient that an outer step leaves -> those of the gradient. */
+int tplr_outer_factors(const float* d_scale, int n_tensors, int n_peers, float lr, const int32_t* d_bad, float* d_factor,
+                       void* stream);
+int tplr_update_factors(const float* d_partials, int n_partials, const float* d_clip, float alpha, int n_tensors,
+                        float* d_factor, void* stream);
+int tplr_outer_stats(float* d_stats, int n_tensors, float lr, void* stream);
+
 /* ---- validator side: checks on the packed index streams ------------------------------
  * For up to 32 peers whose flat payloads share one row layout (d_desc: n_tensors descriptors, of
  * which only chunk_begin, x_chunks and y_chunks are read; a parameter of n rows that are not

@@ -1260,33 +1260,41 @@ def apply_decoded_batch(params: TensorBatch, idx12: torch.Tensor, val: torch.Ten
         raise RuntimeError(f"flat payload mismatch: {idx12.numel()} index bytes / {val.numel()} values for {n} chunks, k={k}")
     if k > _CH:
         raise NotImplementedError(f"top-{k}: the fused update handles k up to {_CH}")
+    factor = None
     if clip_norm is not None:
         if clip is not None:
             raise ValueError("give clip_norm or clip, not both")
         if clip_norm.numel() != T:
             raise IndexError(f"{clip_norm.numel()} clip norms for {T} parameters")
-        slices = max(1, min(64, 4096 // T))
+        # (a workgroup of 1024 threads per parameter and slice: about a thousand, each with a few loads a thread. A 1B set,
+        # k = 32, in eight slices 13 us, in thirty-five 24; one of 14 small parameters 3.6, in 64 slices 6.3)
+        slices = max(1, min(64, 1024 // T, n * k // (2048 * T)))
         ss = torch.empty((T, 1, slices), dtype=torch.float32, device=dev)
+        clip_norm = clip_norm.to(device=dev, dtype=torch.float32).reshape(T).contiguous()
+        factor = torch.empty(T, dtype=torch.float32, device=dev)
         vp = (C.c_void_p * 1)(val.data_ptr())
         with _on(dev):
             _lib.check(lib.tplr_segment_sumsq(vp, 1, k, _ptr(params.table), T, slices, _ptr(ss), _stream(dev)),
                        "tplr_segment_sumsq")
-        norm = ss.reshape(T, slices).sum(dim=1).sqrt()
-        clip = (clip_norm.to(device=dev, dtype=torch.float32).reshape(T) / (norm + 1e-8)).clamp(max=1)
-    factor = None
-    if clip is not None or alpha != 1.0:
+            _lib.check(lib.tplr_update_factors(_ptr(ss), slices, _ptr(clip_norm), float(alpha), T, _ptr(factor), _stream(dev)),
+                       "tplr_update_factors")
+    elif clip is not None:
+        if clip.numel() != T:
+            raise IndexError(f"{clip.numel()} clip factors for {T} parameters")
+        clip = clip.to(device=dev, dtype=torch.float32).reshape(T).contiguous()
+        factor = torch.empty(T, dtype=torch.float32, device=dev)
+        with _on(dev):
+            _lib.check(lib.tplr_update_factors(None, 0, _ptr(clip), float(alpha), T, _ptr(factor), _stream(dev)),
+                       "tplr_update_factors")
+    elif alpha != 1.0:
         factor = torch.full((T,), float(alpha), dtype=torch.float32, device=dev)
-        if clip is not None:
-            if clip.numel() != T:
-                raise IndexError(f"{clip.numel()} clip factors for {T} parameters")
-            factor = factor * clip.to(device=dev, dtype=torch.float32).reshape(T)
     flags = None if on_nonfinite == "ignore" else torch.zeros(T, dtype=torch.int32, device=dev)
     with _on(dev):
         st = lib.tplr_apply_decoded_batch(_ptr(idx12), _ptr(val), _ptr(factor), k, _ptr(params.table), T, n, int(use_dct),
                                           _ptr(flags), _stream(dev))
     _lib.check(st, "tplr_apply_decoded_batch")
     if on_nonfinite == "raise":
-        bad = torch.nonzero(flags).reshape(-1).tolist()  # synchronises, as the reference's isnan().any() does
+        bad = [t for t, flag in enumerate(flags.tolist()) if flag]  # synchronises, as the reference's isnan().any() does
         if bad:
             raise ValueError(f"Invalid gradient: the decoded gradient of parameter {bad[0]} contains NaN/Inf "
                              f"({len(bad)} of {T} parameters affected; their non-finite chunks were not applied)")
@@ -1333,21 +1341,18 @@ def outer_step_batch(params: TensorBatch, idxs: Sequence[torch.Tensor], vals: Se
     fused = use_dct and 4 <= k <= _CH and P <= 15
     flagged = list(range(T))
     if fused:
-        sound = (torch.isfinite(scale) & (scale > 0)).all(dim=1, keepdim=True)
-        factor = torch.where(sound, scale * float(lr), torch.full_like(scale, float("nan"))).contiguous()
+        factor = torch.empty_like(scale)
         flags = torch.zeros(T, dtype=torch.int32, device=dev)
         per_chunk = torch.empty((max(n, 1), 2), dtype=torch.float32, device=dev) if stats else None
         ip = (C.c_void_p * P)(*[i.data_ptr() for i in idxs])
         vp = (C.c_void_p * P)(*[v.data_ptr() for v in vals])
         with _on(dev):
-            st = lib.tplr_outer_step_batch(ip, vp, _ptr(factor), P, k, _ptr(params.table), T, n, _ptr(per_chunk), _ptr(out),
-                                           _ptr(flags), _stream(dev))
-        _lib.check(st, "tplr_outer_step_batch")
-        if stats:  # the launch's figures are those of lr * grad
-            out[:, 0] /= abs(float(lr))
-            out[:, 1] /= float(lr)
-            out[:, 3] /= float(lr) * float(lr)
-        flagged = torch.nonzero(flags).reshape(-1).tolist()  # the call's one synchronisation
+            _lib.check(lib.tplr_outer_factors(_ptr(scale), T, P, float(lr), None, _ptr(factor), _stream(dev)), "tplr_outer_factors")
+            _lib.check(lib.tplr_outer_step_batch(ip, vp, _ptr(factor), P, k, _ptr(params.table), T, n, _ptr(per_chunk), _ptr(out),
+                                                 _ptr(flags), _stream(dev)), "tplr_outer_step_batch")
+            if stats:  # the launch's figures are those of lr * grad
+                _lib.check(lib.tplr_outer_stats(_ptr(out), T, float(lr), _stream(dev)), "tplr_outer_stats")
+        flagged = [t for t, flag in enumerate(flags.tolist()) if flag]  # the call's one synchronisation
     skipped = []
     for t in flagged:  # the reference's own sequence, one parameter at a time
         y, x = params.xshape(t)[:2]
@@ -1925,33 +1930,31 @@ def outer_step_codes_batch(params: TensorBatch, idxs: Sequence[torch.Tensor], co
     slices = max(1, min(64, 8192 // (T * P)))
     ss = torch.empty((T, P, slices), dtype=torch.float32, device=dev)
     scale = torch.empty((T, P), dtype=torch.float32, device=dev)
-    bad = torch.zeros(1, dtype=torch.int32, device=dev)
+    flags = torch.zeros(T + 1, dtype=torch.int32, device=dev)  # one per parameter, and the largest code outside its quantiser
+    bad = flags[T:]
+    factor = torch.empty((T, P), dtype=torch.float32, device=dev)
+    out = torch.zeros((T, 4), dtype=torch.float32, device=dev) if stats else None
+    per_chunk = torch.empty((max(n, 1), 2), dtype=torch.float32, device=dev) if stats else None
     with _on(dev):
         _lib.check(lib.tplr_code_sumsq(cp, P, k, _ptr(params.table), T, slices, n_bins, _ptr(deq), _ptr(ss), _ptr(bad),
                                        _stream(dev)), "tplr_code_sumsq")
         _lib.check(lib.tplr_clip_scales_batch(_ptr(ss), T, P, slices, _ptr(scale), None, _stream(dev)),
                    "tplr_clip_scales_batch")
-    if validate:
-        worst = int(bad.item())
-        if worst:
-            raise IndexError(f"index {worst} is out of bounds for dimension 0 with size {n_bins}")
-    sound = (torch.isfinite(scale) & (scale > 0)).all(dim=1, keepdim=True)
-    factor = torch.where(sound, scale * float(lr), torch.full_like(scale, float("nan"))).contiguous()
-    flags = torch.zeros(T, dtype=torch.int32, device=dev)
-    out = torch.zeros((T, 4), dtype=torch.float32, device=dev) if stats else None
-    per_chunk = torch.empty((max(n, 1), 2), dtype=torch.float32, device=dev) if stats else None
-    with _on(dev):
+        # (with a code that is refused below all factors are NaN: nothing is written)
+        _lib.check(lib.tplr_outer_factors(_ptr(scale), T, P, float(lr), _ptr(bad) if validate else None, _ptr(factor), _stream(dev)),
+                   "tplr_outer_factors")
         st = lib.tplr_outer_step_codes_batch(ip, cp, _ptr(deq), _ptr(factor), P, k, _ptr(params.table), T, n,
                                              _ptr(per_chunk), _ptr(out), _ptr(flags), _stream(dev))
+        if stats and st == 0:  # the launch's figures are those of lr * grad
+            _lib.check(lib.tplr_outer_stats(_ptr(out), T, float(lr), _stream(dev)), "tplr_outer_stats")
+    found = flags.tolist()  # the call's one synchronisation
+    if validate and found[T]:
+        raise IndexError(f"index {found[T]} is out of bounds for dimension 0 with size {n_bins}")
     if st == _lib.TPLR_E_SHAPE:  # the payloads are not a staged window
         return outer_step_batch(params, idxs, dequantised(), k, lr, use_dct=False, stats=stats)
     _lib.check(st, "tplr_outer_step_codes_batch")
-    if stats:  # the launch's figures are those of lr * grad
-        out[:, 0] /= abs(float(lr))
-        out[:, 1] /= float(lr)
-        out[:, 3] /= float(lr) * float(lr)
     skipped = []
-    for t in torch.nonzero(flags).reshape(-1).tolist():  # the reference's own sequence, one parameter at a time
+    for t in [t for t in range(T) if found[t]]:  # the reference's own sequence, one parameter at a time
         y, x = params.xshape(t)[:2]
         b, rows = params.offsets[t], params.payload_rows(t)
         ti = [i[b * (k // 2) * 3:(b + rows) * (k // 2) * 3].contiguous() for i in idxs]

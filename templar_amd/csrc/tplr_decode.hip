@@ -276,4 +276,72 @@ int decode_chunks(const uint8_t* const* h_idx12, const float* const* h_val, cons
     return launch(pp, d_scale, n_peers, k, d_desc, single, n_tensors, total, mean, with_sum, d_stats, d_guard, stream);
 }
 
+// What the updates' launches multiply their values by, and what an outer step reports, where a chain of elementwise launches of
+// 4-5 us each would stand around a launch of one or two milliseconds.
+//
+// Per tensor the peers' factors times lr; NaN, which keeps every chunk of the tensor as it is and flags it, where one of them
+// is not finite and positive (nothing then vouches for the gradient), or where `bad` names a code outside its quantiser.
+__global__ __launch_bounds__(64) void k_outer_factors(const float* __restrict__ scale, int P, float lr,
+                                                      const int32_t* __restrict__ bad, float* __restrict__ factor) {
+    const int64_t row = static_cast<int64_t>(blockIdx.x) * P;
+    bool unsound = bad && *bad != 0;
+    for (int p = threadIdx.x; p < P; p += 64) {
+        const float f = scale[row + p];
+        unsound = unsound || !(f > 0.f) || __builtin_isinf(f);
+    }
+    const bool keep = __ballot(unsound) != 0;
+    for (int p = threadIdx.x; p < P; p += 64) factor[row + p] = keep ? __builtin_nanf("") : scale[row + p] * lr;
+}
+
+// factor_t = alpha * min(1, clip_t / (norm_t + 1e-8)), the norm from n_partials partial sums of squares (added in double);
+// without partial sums alpha * clip_t
+__global__ __launch_bounds__(64) void k_update_factors(const float* __restrict__ partials, int n_partials,
+                                                       const float* __restrict__ clip, float alpha, int n_tensors,
+                                                       float* __restrict__ factor) {
+    const int t = blockIdx.x * 64 + threadIdx.x;
+    if (t >= n_tensors) return;
+    float f = clip[t];
+    if (n_partials > 0) {
+        double ss = 0.0;
+        for (int i = 0; i < n_partials; ++i) ss += static_cast<double>(partials[static_cast<int64_t>(t) * n_partials + i]);
+        f = f / (static_cast<float>(__builtin_sqrt(ss)) + 1e-8f);
+        f = f > 1.0f ? 1.0f : f;  // clamp(max=1); NaN propagates as in torch.clamp
+    }
+    factor[t] = alpha * f;
+}
+
+// figures of lr * gradient {norm, mean, all finite, sum of squares} -> those of the gradient
+__global__ __launch_bounds__(64) void k_outer_stats(float4* __restrict__ stats, int n_tensors, float lr) {
+    const int t = blockIdx.x * 64 + threadIdx.x;
+    if (t >= n_tensors) return;
+    float4 v = stats[t];
+    v.x /= __builtin_fabsf(lr), v.y /= lr, v.w /= lr * lr;
+    stats[t] = v;
+}
+
 }  // namespace tplr
+
+using namespace tplr;
+
+extern "C" int tplr_outer_factors(const float* d_scale, int n_tensors, int n_peers, float lr, const int32_t* d_bad, float* d_factor,
+                                  void* stream) {
+    if (!d_scale || !d_factor || n_tensors < 1 || n_peers < 1) return TPLR_E_BADARG;
+    hipLaunchKernelGGL(k_outer_factors, dim3(static_cast<unsigned>(n_tensors)), dim3(64), 0, static_cast<hipStream_t>(stream), d_scale,
+                       n_peers, lr, d_bad, d_factor);
+    return launch_status();
+}
+
+extern "C" int tplr_update_factors(const float* d_partials, int n_partials, const float* d_clip, float alpha, int n_tensors,
+                                   float* d_factor, void* stream) {
+    if (!d_clip || !d_factor || n_tensors < 1 || n_partials < 0 || (n_partials > 0 && !d_partials)) return TPLR_E_BADARG;
+    hipLaunchKernelGGL(k_update_factors, dim3((static_cast<unsigned>(n_tensors) + 63) / 64), dim3(64), 0, static_cast<hipStream_t>(stream),
+                       d_partials, n_partials, d_clip, alpha, n_tensors, d_factor);
+    return launch_status();
+}
+
+extern "C" int tplr_outer_stats(float* d_stats, int n_tensors, float lr, void* stream) {
+    if (!d_stats || n_tensors < 1 || (reinterpret_cast<uintptr_t>(d_stats) & 15)) return TPLR_E_BADARG;
+    hipLaunchKernelGGL(k_outer_stats, dim3((static_cast<unsigned>(n_tensors) + 63) / 64), dim3(64), 0, static_cast<hipStream_t>(stream),
+                       reinterpret_cast<float4*>(d_stats), n_tensors, lr);
+    return launch_status();
+}

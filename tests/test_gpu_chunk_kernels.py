@@ -115,3 +115,33 @@ def test_payloads_with_the_transform(dev, shapes, P, k, repeat):
     assert lib.tplr_outer_step_batch(*lists, ptr(scale), P, k, ptr(batch.table), len(batch), n, None, None, ptr(flags), stream) == 0
     assert flags.cpu().tolist() == [int(t == last) for t in range(len(batch))]
     assert torch.equal(params[last][-64:, -64:], kept[-64:, -64:])
+
+
+@pytest.mark.parametrize("T,P", [(1, 1), (3, 20), (65, 64), (130, 65), (7, 128)])
+def test_factors_of_updates(dev, T, P):
+    rng = np.random.default_rng(T)
+    lib, stream = _lib.load(), ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    ptr = lambda t: ctypes.c_void_p(t.data_ptr())  # noqa: E731
+    scale = torch.from_numpy(rng.uniform(0.1, 1.0, (T, P)).astype(np.float32)).to(dev)
+    for t, bad in zip(range(1, T), [0.0, -1.0, float("nan"), float("inf"), float("-inf")]):
+        scale[t, P - 1 - t % P] = bad
+    want = torch.where((torch.isfinite(scale) & (scale > 0)).all(1, keepdim=True), scale * 0.4, float("nan"))
+    got = torch.empty_like(scale)
+    for code in (None, torch.zeros(1, dtype=torch.int32, device=dev), torch.full((1,), 9, dtype=torch.int32, device=dev)):
+        assert lib.tplr_outer_factors(ptr(scale), T, P, 0.4, None if code is None else ptr(code), ptr(got), stream) == 0
+        refused = code is not None and int(code)
+        assert torch.equal(got.isnan(), torch.ones_like(want, dtype=torch.bool) if refused else want.isnan())
+        assert refused or torch.equal(got.nan_to_num(-1.0), want.nan_to_num(-1.0))
+    # one peer's: the norm from P partial sums
+    ss, clip = scale.nan_to_num(1.0, 1.0, 1.0).abs(), torch.from_numpy(rng.uniform(0.0, 2.0 * P**0.5, T).astype(np.float32)).to(dev)
+    clip[T // 2] = float("nan")
+    f = torch.empty(T, device=dev)
+    assert lib.tplr_update_factors(ptr(ss), P, ptr(clip), -0.5, T, ptr(f), stream) == 0
+    torch.testing.assert_close(f.double(), -0.5 * (clip.double() / (ss.double().sum(1).sqrt() + 1e-8)).clamp(max=1), rtol=3e-7, atol=0,
+                               equal_nan=True)  # (three roundings of a single precision)
+    assert lib.tplr_update_factors(None, 0, ptr(clip), -0.5, T, ptr(f), stream) == 0
+    torch.testing.assert_close(f, -0.5 * clip, rtol=0, atol=0, equal_nan=True)
+    stats = torch.from_numpy(rng.uniform(1.0, 2.0, (T, 4)).astype(np.float32)).to(dev)
+    want = stats / torch.tensor([0.4, -0.4, 1.0, 0.4 * 0.4], device=dev)
+    assert lib.tplr_outer_stats(ptr(stats), T, -0.4, stream) == 0
+    torch.testing.assert_close(stats, want, rtol=3e-7, atol=0)
