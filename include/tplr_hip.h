@@ -371,6 +371,9 @@ int tplr_outer_step_codes_batch(const uint8_t* const* h_idx12, const uint8_t* co
                                 int n_tensors, int64_t total_chunks, float* d_chunk_stats, float* d_tensor_stats,
                                 int32_t* d_nonfinite, void* stream);
 
+/* The chunks (R/64, C/64, 64, 64) of a tensor -> the (R, C) tensor, both 16-byte aligned: decode without the transform. */
+int tplr_unchunk(const float* d_chunks, int64_t R, int64_t C, float* d_out, void* stream);
+
 /* The small launches around an update of a whole set.
  * tplr_outer_factors: d_factor[t][p] = d_scale[t][p] * lr, the table an outer step takes; NaN for all peers of a tensor
  * with a factor that is not finite and positive, and for every tensor where d_bad (one int, nullable) is not zero - such

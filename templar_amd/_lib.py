@@ -66,6 +66,7 @@ SIGNATURES = {
     "tplr_apply_decoded_batch": (_i32, [_vp, _vp, _vp, _i32, _vp, _i32, _i64, _i32, _vp, _vp]),
     "tplr_outer_step_codes_batch": (_i32, [_vp, _vp, _vp, _vp, _i32, _i32, _vp, _i32, _i64, _vp, _vp, _vp, _vp]),
     "tplr_outer_step_batch": (_i32, [_vp, _vp, _vp, _i32, _i32, _vp, _i32, _i64, _vp, _vp, _vp, _vp]),
+    "tplr_unchunk": (_i32, [_vp, _i64, _i64, _vp, _vp]),
     "tplr_outer_factors": (_i32, [_vp, _i32, _i32, C.c_float, _vp, _vp, _vp]),
     "tplr_update_factors": (_i32, [_vp, _i32, _vp, C.c_float, _i32, _vp, _vp]),
     "tplr_outer_stats": (_i32, [_vp, _i32, C.c_float, _vp]),

@@ -246,4 +246,64 @@ __device__ __forceinline__ Place place_of(const tplr_tensor_desc* __restrict__ t
     return Place{base + static_cast<int64_t>(y) * 64 * ld + static_cast<int64_t>(xc) * 64, ld, t};
 }
 
+// ---- half a chunk in LDS: 32 rows of 64 floats, without padding.  Row r's sixteen quads of columns are permuted by r mod 16,
+// so that a row per lane (16 bytes at a time) and a column per lane (4 bytes) both reach all banks.
+constexpr int kHalfWords = 32 * 64;
+// where coefficient e = 64 row + column of the chunk lies, counted over both halves
+__device__ __forceinline__ uint32_t half_pos(uint32_t e) { return e ^ ((e >> 4) & 0x3cu); }
+
+__device__ __forceinline__ void half_rows_to_regs(float (&w)[64], const float* tile, int row) {  // row: 0 .. 31
+    const float4* r4 = reinterpret_cast<const float4*>(tile + row * 64);
+#pragma unroll
+    for (int c = 0; c < 16; ++c) {
+        const float4 t = r4[c ^ (row & 15)];
+        w[4 * c] = t.x, w[4 * c + 1] = t.y, w[4 * c + 2] = t.z, w[4 * c + 3] = t.w;
+    }
+}
+__device__ __forceinline__ void regs_to_half_rows(const float (&w)[64], float* tile, int row) {
+    float4* r4 = reinterpret_cast<float4*>(tile + row * 64);
+#pragma unroll
+    for (int c = 0; c < 16; ++c) r4[c ^ (row & 15)] = make_float4(w[4 * c], w[4 * c + 1], w[4 * c + 2], w[4 * c + 3]);
+}
+// v[32 half + r] = row r, column `lane`
+template <int kHalf>
+__device__ __forceinline__ void half_cols_to_regs(float (&v)[64], const float* tile, int lane) {
+#pragma unroll
+    for (int r = 0; r < 32; ++r) v[32 * kHalf + r] = tile[r * 64 + (lane ^ ((r & 15) << 2))];
+}
+
+// Where several peers sent a coefficient, its sum over its count: a lane scans the counters of half a row - four bits each,
+// or eight - and divides, one coefficient per trip of a lane-divergent loop.
+__device__ __forceinline__ void half_means4(float* tile, const uint32_t* cnt, int lane) {
+    // bit 4 j + q of m: the counter of the lane's coefficient 8 q + j is at least two
+    const uint4 w = reinterpret_cast<const uint4*>(cnt)[lane];
+    auto multi = [](uint32_t c) { return ((c >> 1) | (c >> 2) | (c >> 3)) & 0x11111111u; };
+    uint32_t m = multi(w.x) | multi(w.y) << 1 | multi(w.z) << 2 | multi(w.w) << 3;
+    while (m) {
+        const int b = __builtin_ctz(m);
+        m &= m - 1;
+        const uint32_t w01 = (b & 1) ? w.y : w.x, w23 = (b & 1) ? w.w : w.z;
+        const uint32_t n = (((b & 2) ? w23 : w01) >> (b & 28)) & 15u;
+        float* const t = &tile[lane * 32 + (b & 3) * 8 + (b >> 2)];
+        *t = *t / static_cast<float>(n);
+    }
+}
+__device__ __forceinline__ void half_means8(float* tile, const uint32_t* cnt, int lane) {  // counts up to 31
+    // bit 8 j + q of m: that of coefficient 4 q + j
+    uint32_t m = 0;
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+        const uint4 w = reinterpret_cast<const uint4*>(cnt)[lane * 2 + h];
+        auto multi = [](uint32_t c) { return ((c >> 1) | (c >> 2) | (c >> 3) | (c >> 4)) & 0x01010101u; };
+        m |= (multi(w.x) | multi(w.y) << 1 | multi(w.z) << 2 | multi(w.w) << 3) << (4 * h);
+    }
+    while (m) {
+        const int b = __builtin_ctz(m);
+        m &= m - 1;
+        const int at = lane * 32 + (b & 7) * 4 + (b >> 3);
+        const uint32_t n = reinterpret_cast<const uint8_t*>(cnt)[at];
+        tile[at] = tile[at] / static_cast<float>(n);
+    }
+}
+
 }  // namespace tplr

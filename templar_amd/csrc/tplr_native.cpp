@@ -16,6 +16,7 @@
 #include <ATen/core/Tensor.h>
 #include <ATen/ops/empty.h>
 #include <ATen/ops/empty_strided.h>
+#include <c10/core/impl/LocalDispatchKeySet.h>
 #include <c10/hip/HIPFunctions.h>
 #include <c10/hip/HIPStream.h>
 #include <torch/csrc/Exceptions.h>
@@ -33,7 +34,7 @@ namespace {
 #define TPLR_NATIVE_ENTRIES(X)                                                                            \
     X(tplr_status_string) X(tplr_dct2d_fwd) X(tplr_dct2d_inv) X(tplr_dct1d) X(tplr_topk_pack)                \
     X(tplr_encode_topk_pack) X(tplr_aggregate_param) X(tplr_decompress_codes) X(tplr_decompress_rows)        \
-    X(tplr_clip_scales) X(tplr_peer_sumsq) X(tplr_quantize) X(tplr_dequantize_lists)
+    X(tplr_clip_scales) X(tplr_peer_sumsq) X(tplr_quantize) X(tplr_dequantize_lists) X(tplr_unchunk)
 #define X(name) decltype(&::name) p_##name = nullptr;
 TPLR_NATIVE_ENTRIES(X)
 #undef X
@@ -79,6 +80,17 @@ const at::Tensor* plain(PyObject* o, c10::ScalarType type) {
 }
 
 const at::Tensor* plain_f32(PyObject* o) { return plain(o, c10::ScalarType::Float); }
+
+// An operation on this tensor would be plain dispatch to the device: no tangent, no transform (vmap, jvp), tracer or mode would
+// see it.  For what has been torch's own operation: a launch in its place is invisible to those.
+bool nobody_else(const at::Tensor& t) {
+    using c10::DispatchKey;
+    const c10::DispatchKeySet plain_keys({DispatchKey::Dense, DispatchKey::CUDA, DispatchKey::AutogradCUDA, DispatchKey::ADInplaceOrView,
+                                          DispatchKey::AutocastCUDA, DispatchKey::BackendSelect});
+    const c10::DispatchKeySet usual = plain_keys | c10::default_included_set;
+    const c10::impl::LocalDispatchKeySet tls = c10::impl::tls_local_dispatch_key_set();
+    return (t.key_set() - usual).empty() && (tls.included_ - usual).empty() && !t._fw_grad(0).defined();
+}
 
 at::Tensor fresh(at::IntArrayRef sizes, c10::ScalarType type, const at::Tensor& like) {
     return at::empty(sizes, at::TensorOptions().dtype(type).device(like.device()));
@@ -197,6 +209,16 @@ PyObject* decode(PyObject*, PyObject* const* args, Py_ssize_t n) {
         if (x->requires_grad()) Py_RETURN_NONE;
         if (chunk_view(*x)) return THPVariable_Wrap(x->as_strided({x->size(0) * kEdge, x->size(1) * kEdge}, {x->stride(2), 1}));
         if (x->dim() != 4 || !x->is_contiguous()) Py_RETURN_NONE;
+        // (one column of chunks is the tensor already: a view)
+        if (x->size(1) > 1 && x->size(2) == kEdge && x->size(3) == kEdge && nobody_else(*x) &&
+            reinterpret_cast<uintptr_t>(x->const_data_ptr()) % 16 == 0) {
+            const int64_t R = x->size(0) * kEdge, C = x->size(1) * kEdge;
+            Launch on(*x);
+            at::Tensor out = fresh({R, C}, c10::ScalarType::Float, *x);
+            const int st = p_tplr_unchunk(x->const_data_ptr<float>(), R, C, out.data_ptr<float>(), on.stream());
+            if (st == 0) return THPVariable_Wrap(std::move(out));
+            if (st != TPLR_E_TOOMANY) return failed(st, "tplr_unchunk");
+        }
         return THPVariable_Wrap(x->permute({0, 2, 1, 3}).reshape({x->size(0) * x->size(2), x->size(1) * x->size(3)}));
     }
     Launch on(*x);

@@ -145,3 +145,74 @@ def test_factors_of_updates(dev, T, P):
     want = stats / torch.tensor([0.4, -0.4, 1.0, 0.4 * 0.4], device=dev)
     assert lib.tplr_outer_stats(ptr(stats), T, -0.4, stream) == 0
     torch.testing.assert_close(stats, want, rtol=3e-7, atol=0)
+
+
+@pytest.mark.parametrize("repeat", [False, True])
+@pytest.mark.parametrize("P,k", [(1, 64), (2, 2), (3, 32), (4, 64), (5, 64), (8, 32), (9, 34), (12, 64), (13, 16), (15, 64), (16, 64), (20, 64),
+                                 (21, 32), (24, 64)])
+@pytest.mark.parametrize("Y,X", [(47, 48), (64, 128)])  # more than a resident round of workgroups per chunk, and the last of the rows'
+def test_parameter_of_a_chunk_per_wave(dev, Y, X, P, k, repeat):
+    n, rng = Y * X, np.random.default_rng(100 * P + k)
+    unit = tc.TensorBatch([torch.empty(64, 64 * 41, device=dev)])
+    idx, val = _payloads(dev, unit, P, k, rng, repeat)
+    over = -(-n // 41)  # the payload rows over and over
+    idx = [i.repeat(over)[: n * k * 3 // 2].contiguous() for i in idx]
+    val = [v.repeat(over, 1)[:n].contiguous() for v in val]
+    val[-1][3, 0], val[0][5, 1] = float("inf"), float("nan")
+    lib, stream = _lib.load(), ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    ptr = lambda t: ctypes.c_void_p(t.data_ptr())  # noqa: E731
+    lists = [(ctypes.c_void_p * P)(*[t.data_ptr() for t in ts]) for ts in (idx, val)]
+    norms = torch.from_numpy(rng.gamma(2.0, 1.0, P).astype(np.float32)).to(dev)
+    scale, scratch = torch.empty(P, device=dev), torch.empty(P, device=dev)
+    assert lib.tplr_clip_scales(ptr(norms), P, 0, ptr(scale), None, stream) == 0
+    for factors in ("norms", "factors", "none"):
+        for ld in (X * 64, X * 64 + 12, 0):
+            got, want = torch.full((2, n * 4096 + 12 * 64 * Y), 7.0, device=dev)
+            given = ptr(norms) if factors == "norms" else None
+            own = {"norms": ptr(scratch), "factors": ptr(scale), "none": None}[factors]
+            assert lib.tplr_aggregate_param(*lists, given, P if given else 0, own, P, k, Y * 64, X * 64, ptr(got), ld, stream) == 0
+            assert lib.tplr_decode_aggregate(*lists, None if factors == "none" else ptr(scale), P, k, Y * 64, X * 64, 0, 0, 0, ptr(want), ld,
+                                             None, stream) == 0
+            same = (got.view(torch.int32) == want.view(torch.int32)) | (got.isnan() & want.isnan())
+            assert bool(same.all()), (factors, ld)
+
+
+def _decoder(shape, dev):
+    from types import SimpleNamespace
+
+    p = SimpleNamespace(requires_grad=True, shape=shape, dtype=torch.float32, device=dev)
+    return tc.ChunkingTransformer(SimpleNamespace(named_parameters=lambda: [("p", p)]), 64)
+
+
+@pytest.mark.parametrize("Y,X", [(1, 1), (3, 1), (1, 2), (5, 3), (2, 4), (7, 5), (1, 65), (130, 9)])
+def test_untransformed_decode(dev, Y, X):
+    tr, base = _decoder((Y * 64, X * 64), dev), torch.randn(Y * X * 4096 + 8, device=dev)
+    for at in (0, 1, 4):  # aligned for wide loads or not
+        x = base[at: at + Y * X * 4096].view(Y, X, 64, 64)
+        out = tr.decode(x, use_dct=False)
+        assert out.is_contiguous() and torch.equal(out, x.permute(0, 2, 1, 3).reshape(Y * 64, X * 64))
+        assert (out.data_ptr() == x.data_ptr()) == (X == 1)
+
+
+def test_untransformed_decode_under_transforms_and_modes(dev):
+    from torch.utils._python_dispatch import TorchDispatchMode
+
+    tr, x = _decoder((128, 192), dev), torch.randn(4, 2, 3, 64, 64, device=dev)
+    want = torch.stack([tr.decode(c, use_dct=False) for c in x])
+    assert torch.equal(torch.func.vmap(lambda c: tr.decode(c, use_dct=False))(x), want)
+    out, tangent = torch.func.jvp(lambda c: tr.decode(c, use_dct=False), (x[0],), (x[1],))
+    assert torch.equal(out, want[0]) and torch.equal(tangent, want[1])
+    with torch.autograd.forward_ad.dual_level():
+        dual = torch.autograd.forward_ad.make_dual(x[0], x[2])
+        out, tangent = torch.autograd.forward_ad.unpack_dual(tr.decode(dual, use_dct=False))
+        assert torch.equal(out, want[0]) and torch.equal(tangent, want[2])
+    seen = []
+
+    class Log(TorchDispatchMode):
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            seen.append(str(func))
+            return func(*args, **(kwargs or {}))
+
+    with Log():
+        assert tr.decode(x[0], use_dct=False).shape == (128, 192)
+    assert any("permute" in s for s in seen)
