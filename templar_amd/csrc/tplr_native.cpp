@@ -89,7 +89,7 @@ bool nobody_else(const at::Tensor& t) {
                                           DispatchKey::AutocastCUDA, DispatchKey::BackendSelect});
     const c10::DispatchKeySet usual = plain_keys | c10::default_included_set;
     const c10::impl::LocalDispatchKeySet tls = c10::impl::tls_local_dispatch_key_set();
-    return (t.key_set() - usual).empty() && (tls.included_ - usual).empty() && !t._fw_grad(0).defined();
+    return ((t.key_set() | tls.included_).raw_repr() & ~usual.raw_repr()) == 0 && !t._fw_grad(0).defined();
 }
 
 at::Tensor fresh(at::IntArrayRef sizes, c10::ScalarType type, const at::Tensor& like) {
