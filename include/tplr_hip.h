@@ -218,6 +218,10 @@ int tplr_scatter_rows(const uint8_t* d_idx12, const int64_t* d_idx64, const floa
  * where an index lies outside its row; such entries are dropped. */
 int tplr_decompress_rows(const uint8_t* d_idx12, const float* d_val, int64_t n_rows, int k, int64_t row_len, float* d_out,
                          int32_t* flag, void* stream);
+/* n_words words of pinned host memory, each written by a system-scope store of its own: 0 where all packed indices of one
+ * n_words-th of the n_rows x k lie below row_len, else 1. */
+int tplr_check_rows(const uint8_t* d_idx12, int64_t n_rows, int k, int64_t row_len, uint32_t* words, int n_words,
+                    void* stream);
 
 /* The same for P peers' flat payloads at once, without concatenating them: row g of d_out
  * (n_rows x row_len) takes the peers' entries for row g in peer order, peer p's values times

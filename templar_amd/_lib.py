@@ -51,6 +51,7 @@ SIGNATURES = {
     "tplr_decompress_codes": (_i32, [_vp, _vp, _vp, _vp, _i32, _i32, _i64, _i64, _vp, _i64, _vp]),
     "tplr_scatter_rows": (_i32, [_vp, _vp, _vp, _i64, _i64, _i64, _i32, _vp, _vp, _vp]),
     "tplr_decompress_rows": (_i32, [_vp, _vp, _i64, _i32, _i64, _vp, _vp, _vp]),
+    "tplr_check_rows": (_i32, [_vp, _i64, _i32, _i64, _vp, _i32, _vp]),
     "tplr_flat_update": (_i32, [_vp, _vp, _i64, C.c_float, _i32, _vp]),
     "tplr_aggregate_rows": (_i32, [_vp, _vp, _vp, _i32, _i32, _vp, _i32, _i64, _i64, _i32, _vp, _vp, _vp]),
     "tplr_decode_rows_batch": (_i32, [_vp, _vp, _vp, _i32, _i32, _vp, _i32, _i64, _i32, _i32, _vp, _vp]),

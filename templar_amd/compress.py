@@ -296,7 +296,7 @@ class ChunkingTransformer:
         """(R, C) -> (R/h, C/w, h, w), or (N,) -> (N/w, w); DCT-II per chunk when use_dct
         (reference :224-257).  Without use_dct the result is a view, as in the reference."""
         if use_dct and self._fast64:
-            out = _lib.native().encode(x, self.shape_dict)
+            out = _lib.native().encode(x, self.shape_dict, self.f_dict)
             if out is not None:
                 return out
         with torch.no_grad():
@@ -341,7 +341,7 @@ class ChunkingTransformer:
         """(y, x, h, w) -> (y*h, x*w), or (x, w) -> (x*w,); inverse DCT per chunk when use_dct
         (reference :259-292)."""
         if self._fast64 or not use_dct:
-            out = _lib.native().decode(x, bool(use_dct))
+            out = _lib.native().decode(x, bool(use_dct), self.b_dict)
             if out is not None:
                 return out
         with torch.no_grad():

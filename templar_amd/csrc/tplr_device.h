@@ -884,6 +884,8 @@ __device__ __forceinline__ uint32_t load_idx12(BytePtr row, int j) {
 
 typedef uint16_t __attribute__((aligned(1))) unaligned_u16;
 using gu16 = __attribute__((address_space(1))) unaligned_u16;
+typedef uint32_t __attribute__((aligned(1))) unaligned_u32;
+using gu32 = __attribute__((address_space(1))) unaligned_u32;
 
 // Lane i's clip factor min(1, median / (norm_i + 1e-8)) of n <= 64 norms, lane i holding norm i: what k_clip_scales
 // makes of them (the lower of the two middle values; NaN as soon as one norm is NaN, :535, :553-556).

@@ -135,9 +135,6 @@ struct PeerPtrs {
 
 __device__ __forceinline__ int tile_pos(uint32_t idx) { return (idx >> 6) * kLd + (idx & 63); }
 
-typedef uint32_t __attribute__((aligned(1))) unaligned_u32;
-using gu32 = __attribute__((address_space(1))) unaligned_u32;
-
 // The fast scatter adds one peer's entries with a plain read-add-write per wave instruction, which is
 // only right when the instruction's destinations are distinct.  A top-k selection has no repeats,
 // but payloads come from other machines: so the read is an exchange that leaves a marker in the

@@ -34,7 +34,8 @@ namespace {
 #define TPLR_NATIVE_ENTRIES(X)                                                                            \
     X(tplr_status_string) X(tplr_dct2d_fwd) X(tplr_dct2d_inv) X(tplr_dct1d) X(tplr_topk_pack)                \
     X(tplr_encode_topk_pack) X(tplr_aggregate_param) X(tplr_decompress_codes) X(tplr_decompress_rows)        \
-    X(tplr_clip_scales) X(tplr_peer_sumsq) X(tplr_quantize) X(tplr_dequantize_lists) X(tplr_unchunk)
+    X(tplr_clip_scales) X(tplr_peer_sumsq) X(tplr_quantize) X(tplr_dequantize_lists) X(tplr_unchunk)                \
+    X(tplr_check_rows) X(tplr_dct2d_dense)
 #define X(name) decltype(&::name) p_##name = nullptr;
 TPLR_NATIVE_ENTRIES(X)
 #undef X
@@ -158,32 +159,54 @@ bool chunk_shape(PyObject* o, int64_t& Y, int64_t& X) {
            to_int(PyTuple_GET_ITEM(o, 3), w) && h == kEdge && w == kEdge && Y > 0 && X > 0;
 }
 
+// The (edge, edge) basis of a chunk edge, plain and on the tensor's device, or nullptr.
+const float* basis_of(PyObject* bases, int64_t edge, const at::Tensor& x) {
+    PyObject* key = PyLong_FromLongLong(edge);
+    PyObject* found = key ? PyDict_GetItemWithError(bases, key) : nullptr;
+    Py_XDECREF(key);
+    const at::Tensor* b = found ? plain_f32(found) : nullptr;
+    PyErr_Clear();
+    return b && b->dim() == 2 && b->size(0) == edge && b->size(1) == edge && b->is_contiguous() && b->device() == x.device()
+               ? b->const_data_ptr<float>()
+               : nullptr;
+}
+
 // ---- encode(x, use_dct=True) ------------------------------------------------------------------
-// encode(x, shape_dict): the 64-point transforms of a registered 2-D or 1-D parameter
+// encode(x, shape_dict, bases): the transforms of a registered 2-D parameter, or of a 1-D one in chunks of 64
 PyObject* encode(PyObject*, PyObject* const* args, Py_ssize_t n) {
     HANDLE_TH_ERRORS
-    if (n != 2) return PyErr_SetString(PyExc_TypeError, "encode(x, shape_dict)"), nullptr;
+    if (n != 3) return PyErr_SetString(PyExc_TypeError, "encode(x, shape_dict, bases)"), nullptr;
     const at::Tensor* x = plain_f32(args[0]);
-    if (!x || !PyDict_Check(args[1]) || x->numel() == 0 || x->dim() < 1 || x->dim() > 2) Py_RETURN_NONE;
+    if (!x || !PyDict_Check(args[1]) || !PyDict_Check(args[2]) || x->numel() == 0 || x->dim() < 1 || x->dim() > 2) Py_RETURN_NONE;
+    int64_t edges[2] = {0, 0};
     for (int64_t d = 0; d < x->dim(); ++d) {
         PyObject* key = PyLong_FromLongLong(x->size(d));
         PyObject* edge = key ? PyDict_GetItemWithError(args[1], key) : nullptr;
         Py_XDECREF(key);
-        int64_t e = 0;
-        if (!edge || !to_int(edge, e) || e != kEdge) {
+        if (!edge || !to_int(edge, edges[d])) {
             PyErr_Clear();
             Py_RETURN_NONE;
         }
     }
     Launch on(*x);
     if (x->dim() == 1) {
-        if (!x->is_contiguous()) Py_RETURN_NONE;
+        if (!x->is_contiguous() || edges[0] != kEdge) Py_RETURN_NONE;
         at::Tensor out = fresh({x->size(0) / kEdge, kEdge}, c10::ScalarType::Float, *x);
         if (int st = p_tplr_dct1d(x->const_data_ptr<float>(), x->size(0) / kEdge, 0, out.data_ptr<float>(), on.stream()))
             return failed(st, "tplr_dct1d");
         return THPVariable_Wrap(std::move(out));
     }
-    const int64_t R = x->size(0), C = x->size(1);
+    const int64_t R = x->size(0), C = x->size(1), h = edges[0], w = edges[1];
+    if (h != kEdge || w != kEdge) {
+        if (h < 1 || w < 1 || h > kEdge || w > kEdge || R % h || C % w || !x->is_contiguous()) Py_RETURN_NONE;
+        const float *bh = basis_of(args[2], h, *x), *bw = basis_of(args[2], w, *x);
+        if (!bh || !bw) Py_RETURN_NONE;
+        at::Tensor out = fresh({R / h, C / w, h, w}, c10::ScalarType::Float, *x);
+        if (int st = p_tplr_dct2d_dense(x->const_data_ptr<float>(), R, C, static_cast<int>(h), static_cast<int>(w), bh, bw, 0, 1,
+                                        out.data_ptr<float>(), on.stream()))
+            return failed(st, "tplr_dct2d_dense");
+        return THPVariable_Wrap(std::move(out));
+    }
     if (x->stride(1) != 1 || x->stride(0) < C) Py_RETURN_NONE;
     at::Tensor out = fresh({R / kEdge, C / kEdge, kEdge, kEdge}, c10::ScalarType::Float, *x);
     if (int st = p_tplr_dct2d_fwd(x->const_data_ptr<float>(), R, C, x->stride(0), out.data_ptr<float>(), on.stream()))
@@ -199,10 +222,10 @@ bool chunk_view(const at::Tensor& x) {
            x.stride(2) >= x.size(1) * kEdge && (x.stride(0) == kEdge * x.stride(2) || x.size(0) == 1);
 }
 
-// decode(x, use_dct): chunks of 64x64 or rows of 64 back into their tensor
+// decode(x, use_dct, bases): chunks or rows of 64 back into their tensor
 PyObject* decode(PyObject*, PyObject* const* args, Py_ssize_t n) {
     HANDLE_TH_ERRORS
-    if (n != 2) return PyErr_SetString(PyExc_TypeError, "decode(x, use_dct)"), nullptr;
+    if (n != 3) return PyErr_SetString(PyExc_TypeError, "decode(x, use_dct, bases)"), nullptr;
     const at::Tensor* x = plain_f32(args[0]);
     if (!x || x->numel() == 0) Py_RETURN_NONE;
     if (args[1] != Py_True) {  // a change of shape: of a view of the tensor itself, the tensor; of whole chunks a copy
@@ -228,6 +251,16 @@ PyObject* decode(PyObject*, PyObject* const* args, Py_ssize_t n) {
         at::Tensor out = fresh({R, C}, c10::ScalarType::Float, *x);
         if (int st = p_tplr_dct2d_inv(x->const_data_ptr<float>(), R, C, out.data_ptr<float>(), C, on.stream()))
             return failed(st, "tplr_dct2d_inv");
+        return THPVariable_Wrap(std::move(out));
+    }
+    if (x->dim() == 4 && x->size(2) <= kEdge && x->size(3) <= kEdge && x->is_contiguous() && PyDict_Check(args[2])) {
+        const int64_t h = x->size(2), w = x->size(3), R = x->size(0) * h, C = x->size(1) * w;
+        const float *bh = basis_of(args[2], h, *x), *bw = basis_of(args[2], w, *x);
+        if (!bh || !bw) Py_RETURN_NONE;
+        at::Tensor out = fresh({R, C}, c10::ScalarType::Float, *x);
+        if (int st = p_tplr_dct2d_dense(x->const_data_ptr<float>(), R, C, static_cast<int>(h), static_cast<int>(w), bh, bw, 1, 0,
+                                        out.data_ptr<float>(), on.stream()))
+            return failed(st, "tplr_dct2d_dense");
         return THPVariable_Wrap(std::move(out));
     }
     if (x->dim() == 2 && x->size(1) == kEdge && x->is_contiguous()) {
@@ -527,13 +560,24 @@ PyObject* decompress(PyObject*, PyObject* const* args, Py_ssize_t n) {
         return scatter_chunks(pl, nullptr, 0, nullptr, shape[0], shape[1], on);
     }
     at::Tensor out = fresh(shape, c10::ScalarType::Float, *like);
-    at::Tensor flag = at::empty({1}, at::TensorOptions().dtype(c10::ScalarType::Int).pinned_memory(true));
-    *flag.data_ptr<int32_t>() = 0;
-    if (int st = p_tplr_decompress_rows(idx->const_data_ptr<uint8_t>(), val, count / k, static_cast<int>(k), row_len,
-                                        out.data_ptr<float>(), flag.data_ptr<int32_t>(), on.stream()))
-        return failed(st, "tplr_decompress_rows");
-    on.wait();  // (the reference's scatter raises on an index outside its row as well)
-    if (*flag.const_data_ptr<int32_t>() != 0) Py_RETURN_NONE;
+    // (the reference's scatter raises on an index outside its row as well.)  The check is a launch ahead of the scatter, a
+    // workgroup per 32 K entries, and only its words are waited for.
+    const int64_t n_words = count >> 15 < 1 ? 1 : count >> 15 > 64 ? 64 : count >> 15;
+    at::Tensor seen = at::empty({n_words}, at::TensorOptions().dtype(c10::ScalarType::Int).pinned_memory(true));
+    uint32_t* const words = reinterpret_cast<uint32_t*>(seen.data_ptr<int32_t>());
+    for (int64_t i = 0; i < n_words; ++i) __atomic_store_n(words + i, kUnset, __ATOMIC_RELAXED);
+    if (int st = p_tplr_check_rows(idx->const_data_ptr<uint8_t>(), count / k, static_cast<int>(k), row_len, words,
+                                   static_cast<int>(n_words), on.stream()))
+        return failed(st, "tplr_check_rows");
+    const int st = p_tplr_decompress_rows(idx->const_data_ptr<uint8_t>(), val, count / k, static_cast<int>(k), row_len,
+                                          out.data_ptr<float>(), nullptr, on.stream());
+    bool outside = false;
+    for (int64_t i = 0; i < n_words; ++i) {  // (all of them: the memory is given back behind this)
+        on.wait_for(words + i);
+        outside |= __atomic_load_n(words + i, __ATOMIC_ACQUIRE) != 0;
+    }
+    if (st) return failed(st, "tplr_decompress_rows");
+    if (outside) Py_RETURN_NONE;
     return THPVariable_Wrap(std::move(out));
     END_HANDLE_TH_ERRORS
 }

@@ -216,3 +216,25 @@ def test_untransformed_decode_under_transforms_and_modes(dev):
     with Log():
         assert tr.decode(x[0], use_dct=False).shape == (128, 192)
     assert any("permute" in s for s in seen)
+
+
+@pytest.mark.parametrize("n_rows,k", [(1, 2), (1, 6), (5, 6), (3, 64), (1025, 64), (4099, 34)])
+@pytest.mark.parametrize("n_words", [1, 3, 64])
+def test_check_of_indices(dev, n_rows, k, n_words):
+    rng, lib = np.random.default_rng(n_rows), _lib.load()
+    pairs = n_rows * k // 2
+    for where in (None, 0, pairs - 1, int(rng.integers(0, pairs))):
+        for length, worst in ((4095, 4095), (100, 100), (1, 1)):
+            idx = rng.integers(0, length, (n_rows, k))
+            if where is not None:
+                idx.reshape(-1)[2 * where + int(rng.integers(0, 2))] = worst
+            for shift in (0, 1):  # payload bytes that do not begin on a word
+                buf = torch.zeros(pairs * 3 + 1, dtype=torch.uint8, device=dev)
+                buf[shift: shift + pairs * 3] = torch.from_numpy(orc.pack12(idx)).to(dev)
+                words = torch.full((n_words,), -1, dtype=torch.int32).pin_memory()
+                assert lib.tplr_check_rows(buf.data_ptr() + shift, n_rows, k, length, words.data_ptr(), n_words,
+                                           torch.cuda.current_stream().cuda_stream) == 0
+                torch.cuda.synchronize()
+                want = [int(where is not None and pairs * i // n_words <= where < pairs * (i + 1) // n_words) for i in range(n_words)]
+                assert words.tolist() == want
+    assert lib.tplr_check_rows(buf.data_ptr(), n_rows, k, 4097, words.data_ptr(), n_words, None) == _lib.TPLR_E_TOOMANY
