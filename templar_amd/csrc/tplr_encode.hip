@@ -18,9 +18,9 @@ namespace tplr {
 // therefore steps through the priority levels 0, 1, 2 chunk by chunk, the three dispatch layers of a full
 // grid one step apart, and changes level once its rows are requested (4 % off the launch; the level
 // values, the direction and a change at another phase or every other chunk matter less than 1 %).
-// Every other encode is k_encode_chunk's, below; this form is for sets with the transform, where what counts is that a wave
-// has nothing to wait for: 868 us for the 115 tensors of a 1B set (k = 32), against 900 with a look-up of its tensor in
-// every wave (1000 cycles of latency at three waves per SIMD); without that look-up the other form takes 854.
+// Every other encode is k_encode_chunk's, below; this form is for sets with the transform that fit one round of waves or
+// fill many (see walks), where what counts is that a wave has nothing to wait for: 879 us for the 115 tensors of a 1B set
+// (k = 32), against 928 with a look-up of its tensor in every wave at three waves per SIMD.
 template <bool kTwo>
 __global__ __launch_bounds__(64, 3) void k_encode_topk_pack(const tplr_tensor_desc* __restrict__ table, int n_tensors, int64_t total,
                                                             int k, uint8_t* __restrict__ idx12, float* __restrict__ val) {
@@ -77,7 +77,7 @@ __global__ __launch_bounds__(64, 3) void k_calib_encode(const tplr_tensor_desc* 
     if (__float_as_uint(s) == 0x7fedcba9u && sink) sink[0] = s;  // (a NaN pattern no sum produces)
 }
 
-// One chunk per wave, kTeam neighbouring chunks per workgroup.  Without the transform it is bound by memory and by the
+// One chunk per wave, kTeam neighbouring chunks per workgroup (with the transform single waves).  Without the transform it is bound by memory and by the
 // latencies of the select: four waves per SIMD (128 registers, a few of the rare exact search's spilled; 10 KB of LDS a wave
 // is just what sixteen waves of a compute unit may have); with it by vector-ALU issue, three waves.  Workgroups are
 // short-lived: the hardware puts the next chunk where one has ended, so no wave waits for a slower one, and a wave's loads
@@ -88,14 +88,14 @@ __global__ __launch_bounds__(64, 3) void k_calib_encode(const tplr_tensor_desc* 
 // kEf: the miner's momentum update rides on the load (src/tplr/neurons.py:151-152): the chunk of
 // the error-feedback tensor becomes ef * decay + grad (two roundings, as mul_ then add_), is
 // written back in place and is what gets encoded.  Rows written together are served sooner: teams of four there.
-template <bool kEf>
-constexpr int encode_team() { return kEf ? 4 : 2; }
+template <bool kUseDct, bool kEf>
+constexpr int encode_team() { return kEf ? 4 : kUseDct ? 1 : 2; }
 
 template <bool kTwo, bool kUseDct, bool kEf>
-__global__ __launch_bounds__((64 * encode_team<kEf>()), kUseDct || kEf ? 3 : 4) void k_encode_chunk(
+__global__ __launch_bounds__((64 * encode_team<kUseDct, kEf>()), kUseDct || kEf ? 3 : 4) void k_encode_chunk(
     const tplr_tensor_desc* __restrict__ table, const tplr_tensor_desc single, int n_tensors, int64_t first, int64_t end, int k,
     uint8_t* __restrict__ idx12, float* __restrict__ val, const tplr_tensor_desc* __restrict__ grad_table, float decay) {
-    constexpr int T = encode_team<kEf>();
+    constexpr int T = encode_team<kUseDct, kEf>();
     __shared__ __align__(16) float buf_all[T][kHalfFloats];
     __shared__ uint64_t cand_all[T][kCandCap];
     const int wv = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));  // wave of the team
@@ -140,7 +140,7 @@ template <bool kTwo, bool kUseDct, bool kEf = false>
 static int launch_chunks(const tplr_tensor_desc* d_desc, const tplr_tensor_desc& single, int n_tensors, int64_t total, int k,
                          uint8_t* d_idx12, float* d_val, void* stream, const tplr_tensor_desc* d_grad_desc = nullptr,
                          float decay = 0.f) {
-    constexpr int T = encode_team<kEf>();
+    constexpr int T = encode_team<kUseDct, kEf>();
     constexpr int64_t piece = kMaxGroups256 * T;  // chunks of one launch
     for (int64_t first = 0; first < total; first += piece) {
         const int64_t end = total - first < piece ? total : first + piece;
@@ -151,10 +151,24 @@ static int launch_chunks(const tplr_tensor_desc* d_desc, const tplr_tensor_desc&
     return launch_status();
 }
 
+// A set with the transform: ranges of the chunk list for one resident round of waves, or a chunk per wave?  The ranges differ
+// by a chunk, which the whole device waits for - with a handful of chunks a wave that is most of the last round - where the
+// other looks up every chunk's tensor.  In us, ranges against a chunk per wave (k = 32 / 64): 2560 chunks 16.6 : 18.1 / 18.4 : 19.6; 5120
+// 28.3 : 27.6 / 32.2 : 30.5; 10 240 43.7 : 40.7 / 51.7 : 47.8; 15 360 57.4 : 56.5 / 67.9 : 65.0; 20 480 72.7 : 75.5 / 88.4 : 80.7; 61 440 194 : 195 / 223 :
+// 219; 294 144 879 : 928 / 1015 : 1040.
 template <bool kTwo>
-static int launch_walk(const tplr_tensor_desc* d_desc, int n_tensors, int64_t total, int k, uint8_t* d_idx12, float* d_val,
-                       void* stream) {
-    static const int resident = persistent_grid(k_encode_topk_pack<kTwo>, int64_t{1} << 40);
+static bool walks(int64_t total, int& resident) {
+    static const int waves = persistent_grid(k_encode_topk_pack<kTwo>, int64_t{1} << 40);
+    resident = waves;
+    return total <= waves || total > static_cast<int64_t>(waves) * (kTwo ? 20 : 5);
+}
+
+template <bool kTwo>
+static int launch_set(const tplr_tensor_desc* d_desc, int n_tensors, int64_t total, int k, uint8_t* d_idx12, float* d_val,
+                      void* stream) {
+    int resident;
+    if (!walks<kTwo>(total, resident))
+        return launch_chunks<kTwo, true>(d_desc, tplr_tensor_desc{}, n_tensors, total, k, d_idx12, d_val, stream);
     const int64_t need = ((total + 7) / 8) * 8;
     hipLaunchKernelGGL(k_encode_topk_pack<kTwo>, dim3(static_cast<unsigned>(need < resident ? need : resident)), dim3(64), 0,
                        static_cast<hipStream_t>(stream), d_desc, n_tensors, total, k, d_idx12, d_val);
@@ -192,8 +206,8 @@ extern "C" int tplr_encode_topk_pack_batch(const tplr_tensor_desc* d_desc, int n
     if (total_chunks == 0) return 0;
     const tplr_tensor_desc none = {};
     if (use_dct)
-        return k > 32 ? launch_walk<true>(d_desc, n_tensors, total_chunks, k, d_idx12, d_val, stream)
-                      : launch_walk<false>(d_desc, n_tensors, total_chunks, k, d_idx12, d_val, stream);
+        return k > 32 ? launch_set<true>(d_desc, n_tensors, total_chunks, k, d_idx12, d_val, stream)
+                      : launch_set<false>(d_desc, n_tensors, total_chunks, k, d_idx12, d_val, stream);
     return k > 32 ? launch_chunks<true, false>(d_desc, none, n_tensors, total_chunks, k, d_idx12, d_val, stream)
                   : launch_chunks<false, false>(d_desc, none, n_tensors, total_chunks, k, d_idx12, d_val, stream);
 }

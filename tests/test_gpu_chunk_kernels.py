@@ -53,6 +53,20 @@ def test_untransformed_sets_of_any_make_up(dev, n, k):
     assert torch.equal(i2, i3) and torch.equal(v2, v3)
 
 
+@pytest.mark.parametrize("k", [32, 64])
+@pytest.mark.parametrize("chunks", [3071, 3073, 6000])  # a round of resident waves, and past it: the launch changes form
+def test_transformed_sets_alike_in_both_forms(dev, chunks, k):
+    gen = torch.Generator(device=dev).manual_seed(chunks)
+    rest = chunks - 2 * 7 * 17
+    x = [torch.randn(s, device=dev, generator=gen) for s in [(64 * 7, 64 * 17), (64, 64 * rest), (64 * 17, 64 * 7)]]
+    batch = tc.TensorBatch(x)
+    idx, val = tc.encode_compress_batch(batch, k, use_dct=True)
+    for t, one in enumerate(x):  # each tensor by itself takes a chunk per wave
+        si, sv = batch.payload_slice(t, idx, val, k)
+        i1, v1, _, _ = tc.encode_compress(one, k, use_dct=True)
+        assert torch.equal(si, i1) and torch.equal(sv.reshape(-1), v1.reshape(-1))
+
+
 def _payloads(dev, batch, P, k, rng, repeat):
     """P payloads that share half of their coefficients; `repeat`: some rows name one twice."""
     n = batch.total_chunks
