@@ -1426,91 +1426,55 @@ __global__ __launch_bounds__((64 * aggregate_team<kUseDct, kUnits, kWideK, !kCod
 // the k selected values go back into a cleared tile exactly as the one-peer decode adds them (0 + value * 2^-5),
 // through the inverse transform, and the difference is stored.  Two waves per SIMD (a whole tile, 64 more
 // registers): the launch moves 14 GB and is bound by that.
-// Workgroups are teams of four (two) waves, as in the aggregate: wave w takes every fourth chunk of the team's range,
-// the team reads rows of 1 KB at the same moment and meets at a barrier before it stores them (6 % off the launch).
-// (at k = 64 the select's instantiation is at the register limit: teams of four are 2 % slower than single
-// waves there, teams of two 4.5 % faster)
+// A wave takes one chunk and ends, so that the next one's loads begin where this one's stores go out; as one resident round of
+// waves on ranges of the chunk list, each waiting for its rows with one other wave on its SIMD, the launch took, in us, k = 32 / 64:
+// 1B set 2747 / 2661, now 2415 / 2480; a 72B block 2031 / 1957, now 1787 / 1822; a 150M model 435 / 432, now 344 / 352.
+// The two waves of a team take neighbouring chunks and meet at a barrier before they store them (teams of four: 2417 / 2508).
+constexpr int kEfTeam = 2;
 template <bool kTwo>
-constexpr int ef_team() { return kTwo ? 2 : 4; }
-template <bool kTwo>
-__global__ __launch_bounds__(64 * ef_team<kTwo>(), 2) void k_ef_step(const tplr_tensor_desc* __restrict__ table,
+__global__ __launch_bounds__(64 * kEfTeam, 2) void k_ef_step(const tplr_tensor_desc* __restrict__ table,
                                                    const tplr_tensor_desc* __restrict__ grad_table, int n_tensors,
-                                                   int64_t total, int k, float decay, uint8_t* __restrict__ idx12,
+                                                   int64_t first, int64_t end, int k, float decay, uint8_t* __restrict__ idx12,
                                                    float* __restrict__ val) {
-    constexpr int T = ef_team<kTwo>();
+    constexpr int T = kEfTeam;
     __shared__ __align__(16) float tile_all[T][kTileFloats];
     __shared__ uint64_t cand_all[T][kCandCap];
-    const int wv = T > 1 ? __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6)) : 0;
+    const int wv = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
     float* const tile = tile_all[wv];
     uint64_t* const cand = cand_all[wv];
-    int64_t g0, g1;
-    my_range(total, g0, g1, T);
-    if (g0 >= g1) return;
-    const int64_t team_steps = (g1 - g0 + T - 1) / T;
-    g0 += wv;
-    const int64_t my_steps = g0 < g1 ? (g1 - 1 - g0) / T + 1 : 0;
-    if (my_steps == 0) {  // wave-uniform: a team with fewer chunks than waves
-        if constexpr (T > 1) {
-            for (int64_t i = 0; i < team_steps; ++i) __builtin_amdgcn_s_barrier();
-        }
-        return;
+    const int lane = threadIdx.x & 63;
+    const int64_t g = first + xcd_contiguous(blockIdx.x, gridDim.x) * T + wv;
+    if (g >= end) return;  // wave-uniform
+    const Place at = place_of(table, tplr_tensor_desc{}, n_tensors, g);
+    const Place from = place_of(grad_table, tplr_tensor_desc{}, n_tensors, g);
+    float e[64], v[64], w[64];
+    load_chunk_rows(e, (const void*)at.chunk0, at.ld, lane);
+    load_chunk_rows(w, (const void*)from.chunk0, from.ld, lane);
+#pragma unroll
+    for (int r = 0; r < 64; ++r) {
+        const float m = e[r] * decay;
+        e[r] = m + w[r];
+        v[r] = e[r];
     }
-    Cursor c, cg;
-    tplr_tensor_desc none = {};
-    cursor_seek(c, table, none, n_tensors, g0);
-    cursor_seek(cg, grad_table, none, n_tensors, g0);
-    for (int64_t g = g0; g < g1; g += T) {
-        // (lane-derived addresses are formed per chunk from a copy of the lane id the optimiser cannot see
-        // through: hoisted out of the loop they would be spilled)
-        int lane = threadIdx.x & 63;
-        asm volatile("" : "+v"(lane));
-        float e[64], v[64], w[64];
-        load_chunk_cols(e, c, lane);
-        load_chunk_cols(w, cg, lane);
+    chunk_forward<true>(v, w, tile, lane);
+    const Selected s = select_topk<kTwo, false>(w, tile, cand, lane, k, kDctPow2Scale, 0, 0);
+    emit_selected<kTwo>(s, lane, k, g, idx12, val);
+    // the payload's reconstruction
+    {
+        const float4 z = make_float4(0.f, 0.f, 0.f, 0.f);
+        float4* row = reinterpret_cast<float4*>(tile + lane * kLd);
 #pragma unroll
-        for (int r = 0; r < 64; ++r) {
-            const float m = e[r] * decay;
-            e[r] = m + w[r];
-            v[r] = e[r];
-        }
-        gfloat* const dst = c.base + (c.y * 64) * c.ld + static_cast<int64_t>(c.xc) * 64;
-        const int64_t ld = c.ld;
-        if (g + T < g1) {
-#pragma unroll
-            for (int s = 1; s <= T; ++s) {
-                cursor_next(cg, g + s);
-                cursor_next(c, g + s);
-            }
-        }
-        // the two waves of a SIMD take turns chunk by chunk, as in the aggregate: two priority levels up on every
-        // other chunk, opposite chunks in the two dispatch layers, one more level from the stores to the next
-        // chunk's requests (3 % off the launch)
-        const int turn = ((((g - g0) / T) & 1) != 0) != (blockIdx.x * 2 >= gridDim.x) ? 2 : 0;  // wave-uniform
-        set_wave_priority(turn);
-        chunk_forward<true>(v, w, tile, lane);
-        const Selected s = select_topk<kTwo, false>(w, tile, cand, lane, k, kDctPow2Scale, 0, 0);
-        emit_selected<kTwo>(s, lane, k, g, idx12, val);
-        // the payload's reconstruction
-        {
-            const float4 z = make_float4(0.f, 0.f, 0.f, 0.f);
-            float4* row = reinterpret_cast<float4*>(tile + lane * kLd);
-#pragma unroll
-            for (int q = 0; q < 16; ++q) row[q] = z;
-        }
-        wave_lds_fence();
-        if (lane < k) tile[tile_pos(s.idx0)] = 0.0f + s.val0 * kDctPow2Scale;
-        wave_lds_fence();
-        chunk_inverse<true>(v, tile, lane);
-        wave_lds_fence();
-#pragma unroll
-        for (int r = 0; r < 64; ++r) v[r] = e[r] - v[r];
-        if constexpr (T > 1) __builtin_amdgcn_s_barrier();  // the team stores together
-        set_wave_priority(turn + 1);
-        store_chunk_rows(v, (void*)uniform64(reinterpret_cast<int64_t>(dst)), uniform64(ld), lane);
+        for (int q = 0; q < 16; ++q) row[q] = z;
     }
-    if constexpr (T > 1) {
-        for (int64_t i = my_steps; i < team_steps; ++i) __builtin_amdgcn_s_barrier();
-    }
+    wave_lds_fence();
+    if (lane < k) tile[tile_pos(s.idx0)] = 0.0f + s.val0 * kDctPow2Scale;
+    wave_lds_fence();
+    chunk_inverse<true>(v, tile, lane);
+    wave_lds_fence();
+#pragma unroll
+    for (int r = 0; r < 64; ++r) v[r] = e[r] - v[r];
+    __builtin_amdgcn_s_barrier();  // the team stores together; a wave that has ended is not waited for
+    store_chunk_rows(v, (void*)at.chunk0, at.ld, lane);
 }
 
 // ef <- ef - (the payload's entries) for chunks that are not transformed (use_dct = 0): the
@@ -2835,6 +2799,19 @@ static int launch_decode_as(Kernel kernel, const PeerPtrs& pp, const float* d_sc
     return launch_status();
 }
 
+template <bool kTwo>
+static int launch_ef(const tplr_tensor_desc* d_ef_desc, const tplr_tensor_desc* d_grad_desc, int n_tensors, int64_t total,
+                     float decay, int k, uint8_t* d_idx12, float* d_val, void* stream) {
+    constexpr int T = kEfTeam;
+    constexpr int64_t piece = kMaxGroups256 * T;  // chunks of one launch
+    for (int64_t first = 0; first < total; first += piece) {
+        const int64_t end = total - first < piece ? total : first + piece;
+        hipLaunchKernelGGL(k_ef_step<kTwo>, dim3(grid8((end - first + T - 1) / T)), dim3(64 * T), 0, static_cast<hipStream_t>(stream),
+                           d_ef_desc, d_grad_desc, n_tensors, first, end, k, decay, d_idx12, d_val);
+    }
+    return launch_status();
+}
+
 extern "C" {
 
 int tplr_version(void) { return 100; }
@@ -2903,24 +2880,8 @@ int tplr_ef_step_batch(const tplr_tensor_desc* d_ef_desc, const tplr_tensor_desc
         return TPLR_E_BADARG;
     if (k > 64) return TPLR_E_TOOMANY;
     if (total_chunks == 0) return 0;
-    if (k > 32) {
-        constexpr int kT = ef_team<true>();
-        const int64_t teams = (((total_chunks + kT - 1) / kT + 7) / 8) * 8;  // workgroups that have a chunk each, in eights
-        static int resident = 0;
-        if (resident == 0) resident = persistent_grid(k_ef_step<true>, int64_t{1} << 40, 64 * kT);
-        hipLaunchKernelGGL(k_ef_step<true>, dim3(static_cast<unsigned>(teams < resident ? teams : resident)), dim3(64 * kT), 0,
-                           static_cast<hipStream_t>(stream), d_ef_desc, d_grad_desc, n_tensors, total_chunks, k, decay,
-                           d_idx12, d_val);
-    } else {
-        static int resident = 0;
-        constexpr int kT = ef_team<false>();
-        const int64_t teams = (((total_chunks + kT - 1) / kT + 7) / 8) * 8;
-        if (resident == 0) resident = persistent_grid(k_ef_step<false>, int64_t{1} << 40, 64 * kT);
-        hipLaunchKernelGGL(k_ef_step<false>, dim3(static_cast<unsigned>(teams < resident ? teams : resident)), dim3(64 * kT), 0,
-                           static_cast<hipStream_t>(stream), d_ef_desc, d_grad_desc, n_tensors, total_chunks, k, decay,
-                           d_idx12, d_val);
-    }
-    return launch_status();
+    return k > 32 ? launch_ef<true>(d_ef_desc, d_grad_desc, n_tensors, total_chunks, decay, k, d_idx12, d_val, stream)
+                  : launch_ef<false>(d_ef_desc, d_grad_desc, n_tensors, total_chunks, decay, k, d_idx12, d_val, stream);
 }
 
 // dst <- dst - decode(decompress(payload)), every value of tensor t times d_factor[t] first (d_factor nullable)
