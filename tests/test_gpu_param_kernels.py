@@ -1,6 +1,8 @@
 """Kernels behind the reference's per-parameter calls, at the sizes where their tilings can go wrong."""
 import ctypes
-import gc
+import os
+import subprocess
+import sys
 
 import numpy as np
 import pytest
@@ -224,34 +226,49 @@ def test_per_parameter_calls_agree_for_plain_and_converted_inputs(dev):
             assert all(torch.equal(a.reshape(-1), b.reshape(-1)) for a, b in zip(results[0], r))
 
 
-def test_running_out_of_memory_leaves_nothing_allocated(dev):
-    # The limits hold whatever ran before: what is left to the garbage collector (the frames behind pytest.raises, say) goes
-    # first, or its memory would come back in between, and room is counted from what is allocated, since the free rest of
-    # reserved segments serves requests as well.
-    gc.collect()
-    comp = tc.TopKCompressor(use_quantization=True, quantization_bins=4)
-    qp = (torch.tensor(0.5, device=dev), 1.0, 2, torch.arange(4.0, device=dev), torch.float32)
-    codes = [torch.zeros(1 << 25, dtype=torch.uint8, device=dev)] * 16  # 16 results of 128 MiB each
-    x = torch.zeros(1 << 19, 64, device=dev)  # 128 MiB of values, 32 MiB of codes and 48 MiB of indices
+# (a process of its own: the limits bound what the allocator takes from the device, and the free rests of segments that other
+# tests keep partly in use would serve the requests whatever the limit)
+OUT_OF_MEMORY = """
+import torch
+import templar_amd.compress as tc
+
+dev = torch.device("cuda:0")
+comp = tc.TopKCompressor(use_quantization=True, quantization_bins=4)
+qp = (torch.tensor(0.5, device=dev), 1.0, 2, torch.arange(4.0, device=dev), torch.float32)
+codes = [torch.zeros(1 << 25, dtype=torch.uint8, device=dev)] * 16  # 16 results of 128 MiB each
+x = torch.zeros(1 << 19, 64, device=dev)  # 128 MiB of values, 32 MiB of codes and 48 MiB of indices
+total = torch.cuda.get_device_properties(dev).total_memory
+before = torch.cuda.memory_allocated(dev)
+
+
+def refused(call, mib):
     torch.cuda.synchronize()
     torch.cuda.empty_cache()
-    before = torch.cuda.memory_allocated(dev)
-    total = torch.cuda.get_device_properties(dev).total_memory
+    room = torch.cuda.memory_reserved(dev) + (mib << 20)
+    assert room - before < (mib + 40) << 20  # (two pools, segments of 20 MiB at most for what is small)
+    torch.cuda.set_per_process_memory_fraction(room / total, dev)
     try:
-        torch.cuda.set_per_process_memory_fraction((before + (1 << 30)) / total, dev)
-        for _ in range(2):
-            with pytest.raises(torch.OutOfMemoryError):
-                comp.maybe_dequantize_values(codes, [qp] * 16, dev)
-            assert torch.cuda.memory_allocated(dev) == before
-            torch.cuda.empty_cache()
-        torch.cuda.set_per_process_memory_fraction((before + (180 << 20)) / total, dev)
-        with pytest.raises(torch.OutOfMemoryError):
-            comp.compress(x, 64)
-        assert torch.cuda.memory_allocated(dev) == before
-    finally:
-        torch.cuda.set_per_process_memory_fraction(1.0, dev)
-        torch.cuda.empty_cache()
-    assert comp.maybe_dequantize_values(codes[:2], [qp] * 2, dev)[1].numel() == 1 << 25
+        call()
+    except torch.OutOfMemoryError:
+        pass
+    else:
+        raise SystemExit("was not refused")
+    assert torch.cuda.memory_allocated(dev) == before
+
+
+for _ in range(2):
+    refused(lambda: comp.maybe_dequantize_values(codes, [qp] * 16, dev), 1024)
+refused(lambda: comp.compress(x, 64), 180)
+torch.cuda.set_per_process_memory_fraction(1.0, dev)
+assert comp.maybe_dequantize_values(codes[:2], [qp] * 2, dev)[1].numel() == 1 << 25
+print("nothing left")
+"""
+
+
+def test_running_out_of_memory_leaves_nothing_allocated():
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    run = subprocess.run([sys.executable, "-c", OUT_OF_MEMORY], cwd=root, capture_output=True, text=True, timeout=100)
+    assert run.returncode == 0 and "nothing left" in run.stdout, run.stderr[-2000:] + run.stdout
 
 
 def test_decompress_names_the_index_outside_its_row(dev):
