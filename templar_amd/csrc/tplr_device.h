@@ -412,35 +412,42 @@ __device__ __forceinline__ void filter_masks(const float (&v)[64], float thr, ui
     mlo = lo;
 }
 
-// Exact masks: strictly-greater and equal to key t (integer compares on canonical keys).
+// Exact masks: strictly-greater and equal to key t.  By signs of differences, as count_ge: 128 comparisons would leave their
+// results in scalar registers that are not there.
 __device__ __forceinline__ void exact_masks(const float (&v)[64], uint32_t t, uint32_t& ghi, uint32_t& glo,
                                             uint32_t& ehi, uint32_t& elo) {
-    uint32_t gh = 0, gl = 0, eh = 0, el = 0;
+    const uint32_t at = t < 0x7f800001u ? t : 0x7f800001u;  // (all NaNs alike, just past the infinity)
+    // (a copy the optimiser cannot see through, or two calls in a row keep the 64 magnitudes in registers of their own)
+    uint32_t magnitude = 0x7fffffffu;
+    asm volatile("" : "+s"(magnitude));
+    uint32_t g[2] = {0, 0}, ge[2] = {0, 0};
 #pragma unroll
     for (int d = 0; d < 64; ++d) {
-        const uint32_t key = mag_key(__float_as_uint(v[d]));
-        const uint32_t g = key > t ? 1u : 0u;
-        const uint32_t e = key == t ? 1u : 0u;
-        if (d < 32) {
-            gh = (gh << 1) | g;
-            eh = (eh << 1) | e;
-        } else {
-            gl = (gl << 1) | g;
-            el = (el << 1) | e;
-        }
+        const uint32_t a = __float_as_uint(v[d]) & magnitude, x = a < 0x7f800001u ? a : 0x7f800001u;
+        g[d >> 5] = __builtin_amdgcn_alignbit(g[d >> 5], at - x, 31);
+        ge[d >> 5] = __builtin_amdgcn_alignbit(ge[d >> 5], at - 1u - x, 31);
     }
-    ghi = gh;
-    glo = gl;
-    ehi = eh;
-    elo = el;
+    ghi = g[0], glo = g[1];
+    ehi = ge[0] & ~g[0], elo = ge[1] & ~g[1];
 }
 
-// (inlined on purpose: a call would force the register-resident chunk through scratch memory)
+// How many of the chunk's keys are at least c?  The sign of c - 1 - |x| says it of one of them; three instructions each and no
+// comparison, whose results the scheduler would gather by the dozen in scalar registers.  Without transform, k = 128, a chunk of
+// noise in this search: one 2048 x 2048 tensor 30.0 us, with comparisons and the magnitudes kept over the passes 56.5 (spilled) at four
+// waves per SIMD, 35.4 at three; one of 0.5 % values other than zero, k = 32 38.7 : 66 : 46.  (Inlined on purpose: a call would force
+// the register-resident chunk through scratch memory.)
 __device__ __forceinline__ uint32_t count_ge(const float (&v)[64], uint32_t c) {
-    uint32_t n = 0;
+    const uint32_t below = (c < 0x7f800001u ? c : 0x7f800001u) - 1u;  // (past the infinity there are only NaNs, all alike)
+    // (a copy as above, for a caller's loop)
+    uint32_t magnitude = 0x7fffffffu;
+    asm volatile("" : "+s"(magnitude));
+    uint32_t m0 = 0, m1 = 0;
 #pragma unroll
-    for (int d = 0; d < 64; ++d) n += mag_key(__float_as_uint(v[d])) >= c ? 1u : 0u;
-    return wave_sum_u32(n);
+    for (int d = 0; d < 32; ++d) {
+        m0 = __builtin_amdgcn_alignbit(m0, below - (__float_as_uint(v[d]) & magnitude), 31);
+        m1 = __builtin_amdgcn_alignbit(m1, below - (__float_as_uint(v[d + 32]) & magnitude), 31);
+    }
+    return wave_sum_u32(__popc(m0) + __popc(m1));
 }
 
 // keep only the first `keep` set bits (in d order = from bit 31 of hi down) of a mask pair

@@ -78,7 +78,7 @@ __global__ __launch_bounds__(64, 3) void k_calib_encode(const tplr_tensor_desc* 
 }
 
 // One chunk per wave, kTeam neighbouring chunks per workgroup (with the transform single waves).  Without the transform it is bound by memory and by the
-// latencies of the select: four waves per SIMD (128 registers, a few of the rare exact search's spilled; 10 KB of LDS a wave
+// latencies of the select: four waves per SIMD (112 registers, the exact search's among them; 10 KB of LDS a wave
 // is just what sixteen waves of a compute unit may have); with it by vector-ALU issue, three waves.  Workgroups are
 // short-lived: the hardware puts the next chunk where one has ended, so no wave waits for a slower one, and a wave's loads
 // overlap the others' arithmetic.  As one resident round of waves that walk ranges of the chunk list, with 4096 chunks over
