@@ -119,16 +119,18 @@ struct Launch {
         Released released;
         c10::hip::getCurrentHIPStream(here).unwrap().synchronize();
     }
-    // wait until a kernel of the stream has stored something else than kUnset in a word of pinned memory, which it does
-    // with a system-scope store; for the stream where half a millisecond does not bring it (work queued before, an error)
-    void wait_for(const uint32_t* word) const {
+    // wait until kernels of the stream have stored something else than kUnset in each of n words of pinned memory, which they do
+    // with system-scope stores; for the stream where half a millisecond does not bring them (work queued before, an error).
+    // The interpreter is given up once for all of them: beside a busy thread it comes back a switch interval later.
+    void wait_for(const uint32_t* words, int64_t n) const {
         Released released;
         const auto give_up = std::chrono::steady_clock::now() + std::chrono::microseconds(500);
-        while (__atomic_load_n(word, __ATOMIC_ACQUIRE) == kUnset)
-            if (std::chrono::steady_clock::now() > give_up) {
-                c10::hip::getCurrentHIPStream(here).unwrap().synchronize();
-                return;
-            }
+        for (int64_t i = 0; i < n; ++i)
+            while (__atomic_load_n(words + i, __ATOMIC_ACQUIRE) == kUnset)
+                if (std::chrono::steady_clock::now() > give_up) {
+                    c10::hip::getCurrentHIPStream(here).unwrap().synchronize();
+                    return;
+                }
     }
 };
 
@@ -291,7 +293,7 @@ PyObject* quantised(const at::Tensor& val, int64_t n_bins, double range, const L
                                  static_cast<int>(slices), work.data_ptr<double>(), codes.data_ptr<uint8_t>(),
                                  shift.data_ptr<float>(), scale.data_ptr<float>(), lookup.data_ptr<float>(), on.stream()))
         return failed(st, "tplr_quantize");
-    on.wait_for(word);
+    on.wait_for(word, 1);
     return Py_BuildValue("(N(NdLNO))", THPVariable_Wrap(std::move(codes)), THPVariable_Wrap(std::move(shift)),
                          static_cast<double>(*scale.const_data_ptr<float>()), static_cast<long long>(n_bins / 2),
                          THPVariable_Wrap(std::move(lookup)), float32_dtype);
@@ -571,11 +573,9 @@ PyObject* decompress(PyObject*, PyObject* const* args, Py_ssize_t n) {
         return failed(st, "tplr_check_rows");
     const int st = p_tplr_decompress_rows(idx->const_data_ptr<uint8_t>(), val, count / k, static_cast<int>(k), row_len,
                                           out.data_ptr<float>(), nullptr, on.stream());
+    on.wait_for(words, n_words);  // (all of them: the memory is given back behind this)
     bool outside = false;
-    for (int64_t i = 0; i < n_words; ++i) {  // (all of them: the memory is given back behind this)
-        on.wait_for(words + i);
-        outside |= __atomic_load_n(words + i, __ATOMIC_ACQUIRE) != 0;
-    }
+    for (int64_t i = 0; i < n_words; ++i) outside |= words[i] != 0;
     if (st) return failed(st, "tplr_decompress_rows");
     if (outside) Py_RETURN_NONE;
     return THPVariable_Wrap(std::move(out));

@@ -3,6 +3,8 @@ import ctypes
 import os
 import subprocess
 import sys
+import threading
+import time
 
 import numpy as np
 import pytest
@@ -277,6 +279,34 @@ def test_decompress_names_the_index_outside_its_row(dev):
     val = torch.ones(2, 4, device=dev)
     with pytest.raises(RuntimeError, match="index 11 is out of bounds for dimension -1 with size 9"):
         comp.decompress(val, torch.from_numpy(orc.pack12(idx)).to(dev), val, (2, 9), 9)
+
+
+def test_decompress_of_many_rows_waits_once_for_the_interpreter(dev):
+    # 64 words tell whether the indices lie in their rows.  Beside a busy thread every release of the interpreter may cost a switch
+    # interval; the call releases it once for all words, and the rest of it another time at most.
+    comp, interval = tc.TopKCompressor(), sys.getswitchinterval()
+    x = torch.randn(32768, 100, device=dev)
+    sent = comp.compress(x, 64)
+    comp.decompress(x, *sent)
+    stop = threading.Event()
+
+    def busy():
+        while not stop.is_set():
+            pass
+
+    thread, took = threading.Thread(target=busy), []
+    sys.setswitchinterval(0.01)
+    thread.start()
+    try:
+        for _ in range(40):
+            t = time.perf_counter()
+            comp.decompress(x, *sent)
+            took.append(time.perf_counter() - t)
+    finally:
+        stop.set()
+        thread.join()
+        sys.setswitchinterval(interval)
+    assert sum(t > 0.025 for t in took) <= 1, took
 
 
 @pytest.mark.parametrize("bins", [4, 256])
