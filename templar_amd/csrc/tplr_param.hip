@@ -22,10 +22,11 @@ constexpr int kParamNorms = 64;  // norms that one wave ranks
 //    12.3.  One or two peers' few entries leave it ahead into chunks beyond: 4096 of one 13.0 : 13.6, of two 13.4 : 13.8; 59 136 of
 //    one 169 : 173.
 //  - Into chunks a wave per chunk stays ahead of the teams: 4096 of twenty (k = 64) 26.6 : 21.3, payloads from memory 27.8 :
-//    22.1; 16 384 of four 60 : 54 / 65 : 60, 59 136 of fifteen 272 : 240 / 291 : 254.
+//    22.1; 16 384 of four 60 : 54 / 65 : 60, 59 136 of fifteen 272 : 240 / 291 : 254 (of five 218 : 196, but 228 : 245).
 //  - Into rows up to 8192: 8192 of four 33 : 21 / 33 : 22, of fifteen 37.6 : 28.0 / 40.7 : 39.1; but the teams store rows of 1 KB
-//    together: 16 384 of fifteen 60.5 : 71.4 / 66.4 : 79.0, 59 136 of ten 228 : 243 / 255 : 240.
-constexpr int64_t kFourWaveFewPeers = 61440, kRowChunks = 8192;  // chunks times peers; chunks
+//    together: 16 384 of fifteen 60.5 : 71.4 / 66.4 : 79.0, 59 136 of ten 228 : 243 / 255 : 240.  Of one or two peers
+//    the chunks by themselves stay ahead for longer: 12 288 of one 46.5 : 30.2, of two 46.7 : 30.8, 24 576 of one 95 : 85.
+constexpr int64_t kFourWaveFewPeers = 61440, kFewPeersRows = 24576, kRowChunks = 8192;  // chunks times peers, twice; chunks
 
 struct ParamPeer {
     const uint8_t* idx;
@@ -418,7 +419,8 @@ extern "C" int tplr_aggregate_param(const uint8_t* const* h_idx12, const float* 
     const int64_t n = (R / 64) * (C / 64);
     if (n == 0) return 0;
     if (C / 64 > 0x7fffffff || R / 64 > 0x7fffffff || ld_out > (int64_t{1} << 23)) return TPLR_E_TOOMANY;
-    if (n_peers <= kParamPeers && k <= 64 && n_norms <= kParamNorms && n <= (ld_out ? kRowChunks : kMaxGroups256) &&
+    const bool few = n_peers <= 2 && n * n_peers <= (ld_out ? kFewPeersRows : kFourWaveFewPeers);
+    if (n_peers <= kParamPeers && k <= 64 && n_norms <= kParamNorms && (few || n <= (ld_out ? kRowChunks : kMaxGroups256)) &&
         (ld_out & 3) == 0 && (reinterpret_cast<uintptr_t>(d_out) & 15) == 0) {
         ParamPeers pp = {};
         for (int p = 0; p < n_peers; ++p) {
@@ -428,7 +430,7 @@ extern "C" int tplr_aggregate_param(const uint8_t* const* h_idx12, const float* 
             const int u = p < n_peers ? p : n_peers - 1;
             pp.peer[p] = {h_idx12[u], h_val[u]};
         }
-        if (n <= four_wave_round(n_peers) || (!ld_out && n_peers <= 2 && n * n_peers <= kFourWaveFewPeers))
+        if (n <= four_wave_round(n_peers) || (few && !ld_out))
             return launch_param<false>(pp, d_scale, d_norms, n_norms, n_peers, k, nullptr, nullptr, 0, C / 64, n, ld_out, d_out, stream);
         return launch_chunk(pp, d_scale, d_norms, n_norms, n_peers, k, C / 64, n, ld_out, d_out, stream);
     }

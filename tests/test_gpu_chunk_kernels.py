@@ -161,10 +161,13 @@ def test_factors_of_updates(dev, T, P):
     torch.testing.assert_close(stats, want, rtol=3e-7, atol=0)
 
 
+_PEERS = [(1, 64), (2, 2), (3, 32), (4, 64), (5, 64), (8, 32), (9, 34), (12, 64), (13, 16), (15, 64), (16, 64), (20, 64), (21, 32), (24, 64)]
+
+
+# (47 x 48: more than a resident round of workgroups per chunk; 64 x 128: the last of the rows, and of one or two peers past it)
 @pytest.mark.parametrize("repeat", [False, True])
-@pytest.mark.parametrize("P,k", [(1, 64), (2, 2), (3, 32), (4, 64), (5, 64), (8, 32), (9, 34), (12, 64), (13, 16), (15, 64), (16, 64), (20, 64),
-                                 (21, 32), (24, 64)])
-@pytest.mark.parametrize("Y,X", [(47, 48), (64, 128)])  # more than a resident round of workgroups per chunk, and the last of the rows'
+@pytest.mark.parametrize("Y,X,P,k", [(*s, *p) for s in ((47, 48), (64, 128)) for p in _PEERS] +
+                         [(128, 192, 1, 32), (129, 191, 1, 64), (96, 128, 2, 64), (97, 127, 2, 32)])
 def test_parameter_of_a_chunk_per_wave(dev, Y, X, P, k, repeat):
     n, rng = Y * X, np.random.default_rng(100 * P + k)
     unit = tc.TensorBatch([torch.empty(64, 64 * 41, device=dev)])
