@@ -964,6 +964,7 @@ class TensorBatch:
             begin += x * y
         self.tensors = list(tensors)  # keeps the storage alive
         self.total_chunks = begin
+        self.max_chunks = max(b - a for a, b in zip(self.offsets, self.offsets[1:] + [begin]))
         self.device = dev
         self.desc = desc  # host copy of the table
         self.table = torch.from_numpy(desc.view(np.uint8).copy()).to(dev)
@@ -1228,6 +1229,16 @@ def aggregate_mean_normalised_batch(out: TensorBatch, idxs: Sequence[torch.Tenso
     return factor
 
 
+def _value_slices(batch: TensorBatch, k: int) -> int:
+    """Slices of a parameter's values in tplr_segment_sumsq, a workgroup of 1024 threads each: about a thousand of them, each
+    with a few loads a thread; more where the largest parameter's would be longer than 512 KB.  A 1B set, k = 32, in eight 13 us,
+    in thirty-five 24; one of 14 small parameters in one 3.6, in 64 6.3.  A parameter of 16 000 chunks beside 600 of one,
+    k = 64: in one 72 us, in six 26."""
+    T = len(batch)
+    return max(1, min(64, max(min(1024 // T, batch.total_chunks * k // (2048 * T)),
+                              min(4096 // T, batch.max_chunks * k // 131072))))
+
+
 @torch.no_grad()
 def apply_decoded_batch(params: TensorBatch, idx12: torch.Tensor, val: torch.Tensor, k: int, *, alpha: float = 1.0,
                         clip: torch.Tensor | None = None, clip_norm: torch.Tensor | None = None,
@@ -1266,9 +1277,7 @@ def apply_decoded_batch(params: TensorBatch, idx12: torch.Tensor, val: torch.Ten
             raise ValueError("give clip_norm or clip, not both")
         if clip_norm.numel() != T:
             raise IndexError(f"{clip_norm.numel()} clip norms for {T} parameters")
-        # (a workgroup of 1024 threads per parameter and slice: about a thousand, each with a few loads a thread. A 1B set,
-        # k = 32, in eight slices 13 us, in thirty-five 24; one of 14 small parameters 3.6, in 64 slices 6.3)
-        slices = max(1, min(64, 1024 // T, n * k // (2048 * T)))
+        slices = _value_slices(params, k)
         ss = torch.empty((T, 1, slices), dtype=torch.float32, device=dev)
         clip_norm = clip_norm.to(device=dev, dtype=torch.float32).reshape(T).contiguous()
         factor = torch.empty(T, dtype=torch.float32, device=dev)
@@ -1814,10 +1823,14 @@ def dequantised_tables(quant_params: Sequence[Sequence[QuantParamsT]], dev: torc
     return deq.contiguous(), n_bins
 
 
-def _code_slices(T: int, P: int, n: int, k: int) -> int:
-    """Slices of a parameter's codes in tplr_code_sumsq, a workgroup each per peer: no smaller than 8 KB on average.  20 peers,
-    k = 64: a 1B set in three 67 us, in four 63, in eight 68; 14 small parameters in one 5, in 29 15."""
-    return max(1, min(64, 9600 // (T * P), n * k // (8192 * T)))
+def _code_slices(batch: TensorBatch, P: int, k: int) -> int:
+    """Slices of a parameter's codes in tplr_code_sumsq, a workgroup each per peer: no smaller than 8 KB on average, but the
+    largest parameter's no larger than 64 KB.  20 peers, k = 64: a 1B set in three 67 us, in four 63, in eight 68; 14 small
+    parameters in one 5, in 29 15.  A parameter of 16 000 chunks beside 100 of one, one peer: in
+    one 35 us, in fifteen 8."""
+    T = len(batch)
+    by_size = max(batch.total_chunks * k // (8192 * T), batch.max_chunks * k // 65536)
+    return max(1, min(64, 9600 // (T * P), by_size))
 
 
 @torch.no_grad()
@@ -1868,7 +1881,7 @@ def batch_decompress_decode_codes_batch(out: TensorBatch, idxs: Sequence[torch.T
     bad = torch.zeros(1, dtype=torch.int32, device=dev) if validate else None
     with _on(dev):
         if clip_norm or validate:
-            slices = _code_slices(T, P, n, k)
+            slices = _code_slices(out, P, k)
             ss = torch.empty((T, P, slices), dtype=torch.float32, device=dev)
             _lib.check(lib.tplr_code_sumsq(cp, P, k, _ptr(out.table), T, slices, n_bins, _ptr(deq), _ptr(ss), _ptr(bad),
                                            _stream(dev)), "tplr_code_sumsq")
@@ -1933,7 +1946,7 @@ def outer_step_codes_batch(params: TensorBatch, idxs: Sequence[torch.Tensor], co
         return outer_step_batch(params, idxs, dequantised(), k, lr, use_dct=False, stats=stats)
     ip = (C.c_void_p * P)(*[i.data_ptr() for i in idxs])
     cp = (C.c_void_p * P)(*[c.data_ptr() for c in codes])
-    slices = _code_slices(T, P, n, k)
+    slices = _code_slices(params, P, k)
     ss = torch.empty((T, P, slices), dtype=torch.float32, device=dev)
     scale = torch.empty((T, P), dtype=torch.float32, device=dev)
     flags = torch.zeros(T + 1, dtype=torch.int32, device=dev)  # one per parameter, and the largest code outside its quantiser

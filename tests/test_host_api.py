@@ -356,3 +356,25 @@ def test_quantiser_tables_round_through_the_senders_dtype():
     assert torch.equal(deq[0, 0], tcp.dequantize(codes, qp32)) and torch.equal(deq[0, 1], want16.float())
     with pytest.raises(ValueError, match="different sizes"):
         tc._qparam_tables([qp32, (shift, 1.0, 4, torch.randn(8), torch.float32)], torch.device("cpu"))
+
+
+@pytest.mark.parametrize("small", [0, 3, 13, 100, 600, 2000])
+@pytest.mark.parametrize("large", [1, 64, 16000, 59136])
+def test_a_large_parameter_beside_small_ones_is_summed_in_slices(small, large):
+    class Batch:
+        total_chunks, max_chunks = large + small, large
+
+        def __len__(self):
+            return small + 1
+
+    T = small + 1
+    for k in (2, 32, 64):
+        s = tc._value_slices(Batch(), k)
+        # a workgroup's part of the largest parameter stays below 1 MB, unless there are 64 or the launch has its 4096
+        assert 1 <= s <= 64 and (large * k * 4 < s << 20 or s >= min(64, 4096 // T)), (k, s)
+        assert s * T <= max(T, 4096)
+        for P in (1, 6, 20):
+            s = tc._code_slices(Batch(), P, k)
+            # (codes: 128 KB, and the launch 9600)
+            assert 1 <= s <= 64 and (large * k < s << 17 or s >= min(64, 9600 // (T * P))), (P, k, s)
+            assert s * T * P <= max(T * P, 9600)
