@@ -272,12 +272,14 @@ __global__ __launch_bounds__(64) void k_update_factors(const float* __restrict__
     factor[t] = alpha * f;
 }
 
-// figures of lr * gradient {norm, mean, all finite, sum of squares} -> those of the gradient
+// figures of lr * gradient {norm, mean, all finite, sum of squares} -> those of the gradient, each rounded once (lr^2 in single
+// precision would be rounded itself, and is zero from 1e-23 down)
 __global__ __launch_bounds__(64) void k_outer_stats(float4* __restrict__ stats, int n_tensors, float lr) {
     const int t = blockIdx.x * 64 + threadIdx.x;
     if (t >= n_tensors) return;
     float4 v = stats[t];
-    v.x /= __builtin_fabsf(lr), v.y /= lr, v.w /= lr * lr;
+    v.x /= __builtin_fabsf(lr), v.y /= lr;
+    v.w = static_cast<float>(v.w / (static_cast<double>(lr) * lr));
     stats[t] = v;
 }
 

@@ -155,10 +155,12 @@ def test_factors_of_updates(dev, T, P):
                                equal_nan=True)  # (three roundings of a single precision)
     assert lib.tplr_update_factors(None, 0, ptr(clip), -0.5, T, ptr(f), stream) == 0
     torch.testing.assert_close(f, -0.5 * clip, rtol=0, atol=0, equal_nan=True)
-    stats = torch.from_numpy(rng.uniform(1.0, 2.0, (T, 4)).astype(np.float32)).to(dev)
-    want = stats / torch.tensor([0.4, -0.4, 1.0, 0.4 * 0.4], device=dev)
-    assert lib.tplr_outer_stats(ptr(stats), T, -0.4, stream) == 0
-    torch.testing.assert_close(stats, want, rtol=3e-7, atol=0)
+    for lr, squares in ((-0.4, 0.16), (0.7, 0.49), (1e-23, 1e-30)):
+        lr = float(np.float32(lr))
+        stats = torch.from_numpy(rng.uniform(1.0, 2.0, (T, 4)).astype(np.float32) * np.float32([abs(lr), lr, 1.0, squares])).to(dev)
+        want = stats.cpu().double() / torch.tensor([abs(lr), lr, 1.0, lr * lr], dtype=torch.float64)
+        assert lib.tplr_outer_stats(ptr(stats), T, lr, stream) == 0
+        assert torch.equal(stats.cpu(), want.float())  # the quotients, rounded once
 
 
 _PEERS = [(1, 64), (2, 2), (3, 32), (4, 64), (5, 64), (8, 32), (9, 34), (12, 64), (13, 16), (15, 64), (16, 64), (20, 64), (21, 32), (24, 64)]
