@@ -87,22 +87,25 @@ __global__ __launch_bounds__(64, 3) void k_calib_encode(const tplr_tensor_desc* 
 // chunks without it, k = 32 795 -> 750, k = 64 841 -> 790; its miner step of two launches, k = 64 with four-bin codes 3436 -> 3165.
 // kEf: the miner's momentum update rides on the load (src/tplr/neurons.py:151-152): the chunk of
 // the error-feedback tensor becomes ef * decay + grad (two roundings, as mul_ then add_), is
-// written back in place and is what gets encoded.  Rows written together are served sooner: teams of four there.
+// written back in place and is what gets encoded.  Rows written together are served sooner: teams of four there, but single waves
+// (of the same kernel) while there are fewer chunks than SIMDs, which then share no compute unit's LDS and fetches: with the
+// transform 64 chunks 10.2 -> 8.6 us / 11.4 -> 9.7, 768 12.3 -> 11.7 / 13.2 -> 12.6; 2048 23.3 : 24.4, 4096 40.4 : 42.2.
 template <bool kUseDct, bool kEf>
 constexpr int encode_team() { return kEf ? 4 : kUseDct ? 1 : 2; }
 
 template <bool kTwo, bool kUseDct, bool kEf>
 __global__ __launch_bounds__((64 * encode_team<kUseDct, kEf>()), kUseDct || kEf ? 3 : 4) void k_encode_chunk(
     const tplr_tensor_desc* __restrict__ table, const tplr_tensor_desc single, int n_tensors, int64_t first, int64_t end, int k,
-    uint8_t* __restrict__ idx12, float* __restrict__ val, const tplr_tensor_desc* __restrict__ grad_table, float decay) {
+    uint8_t* __restrict__ idx12, float* __restrict__ val, const tplr_tensor_desc* __restrict__ grad_table, float decay, int team) {
     constexpr int T = encode_team<kUseDct, kEf>();
+    // team: waves of this launch's workgroups, at most T (with the momentum update; otherwise T)
     __shared__ __align__(16) float buf_all[T][kHalfFloats];
     __shared__ uint64_t cand_all[T][kCandCap];
     const int wv = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));  // wave of the team
     float* const buf = buf_all[wv];
     uint64_t* const cand = cand_all[wv];
     const int lane = threadIdx.x & 63;
-    const int64_t g = first + xcd_contiguous(blockIdx.x, gridDim.x) * T + wv;
+    const int64_t g = first + xcd_contiguous(blockIdx.x, gridDim.x) * (kEf ? team : T) + wv;
     if (g >= end) return;  // wave-uniform; the waves of a team never wait for one another
     const Place at = place_of(table, single, n_tensors, g);
     float v[64], w[64];
@@ -140,13 +143,14 @@ template <bool kTwo, bool kUseDct, bool kEf = false>
 static int launch_chunks(const tplr_tensor_desc* d_desc, const tplr_tensor_desc& single, int n_tensors, int64_t total, int k,
                          uint8_t* d_idx12, float* d_val, void* stream, const tplr_tensor_desc* d_grad_desc = nullptr,
                          float decay = 0.f) {
-    constexpr int T = encode_team<kUseDct, kEf>();
-    constexpr int64_t piece = kMaxGroups256 * T;  // chunks of one launch
+    constexpr int kSimds = 1024;
+    const int team = kEf && total < kSimds ? 1 : encode_team<kUseDct, kEf>();
+    const int64_t piece = kMaxGroups256 * team;  // chunks of one launch
     for (int64_t first = 0; first < total; first += piece) {
         const int64_t end = total - first < piece ? total : first + piece;
-        hipLaunchKernelGGL((k_encode_chunk<kTwo, kUseDct, kEf>), dim3(grid8((end - first + T - 1) / T)), dim3(64 * T), 0,
+        hipLaunchKernelGGL((k_encode_chunk<kTwo, kUseDct, kEf>), dim3(grid8((end - first + team - 1) / team)), dim3(64 * team), 0,
                            static_cast<hipStream_t>(stream), d_desc, single, n_tensors, first, end, k, d_idx12, d_val, d_grad_desc,
-                           decay);
+                           decay, team);
     }
     return launch_status();
 }

@@ -67,6 +67,24 @@ def test_transformed_sets_alike_in_both_forms(dev, chunks, k):
         assert torch.equal(si, i1) and torch.equal(sv.reshape(-1), v1.reshape(-1))
 
 
+@pytest.mark.parametrize("use_dct", [True, False])
+@pytest.mark.parametrize("k", [32, 64])
+@pytest.mark.parametrize("chunks", [5, 1023, 1024, 1029])  # single waves, and teams of four from a chunk for every SIMD on
+def test_momentum_update_and_encode(dev, chunks, k, use_dct):
+    gen = torch.Generator(device=dev).manual_seed(chunks)
+    shapes = [(64, 64 * 2), (64, 64 * (chunks - 3)), (64, 64)]
+    ef, grad = ([torch.randn(s, device=dev, generator=gen) for s in shapes] for _ in range(2))
+    want = [e * 0.9 + g for e, g in zip(ef, grad)]
+    own, from_ = tc.TensorBatch(ef), tc.TensorBatch(grad)
+    idx, val = torch.empty(chunks * k * 3 // 2, dtype=torch.uint8, device=dev), torch.empty(chunks, k, device=dev)
+    ptr = lambda t: ctypes.c_void_p(t.data_ptr())  # noqa: E731
+    assert _lib.load().tplr_ef_encode_topk_pack_batch(ptr(own.table), ptr(from_.table), 3, chunks, 0.9, k, int(use_dct), ptr(idx), ptr(val),
+                                                      ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)) == 0
+    assert all(torch.equal(e, w) for e, w in zip(ef, want))
+    i2, v2 = tc.encode_compress_batch(own, k, use_dct=use_dct)
+    assert torch.equal(idx, i2) and torch.equal(val, v2)
+
+
 def _payloads(dev, batch, P, k, rng, repeat):
     """P payloads that share half of their coefficients; `repeat`: some rows name one twice."""
     n = batch.total_chunks
