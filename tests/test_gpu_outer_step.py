@@ -271,6 +271,43 @@ def test_outer_step_from_codes_leaves_a_poisoned_parameter_alone(dev):
     assert all(torch.equal(a, b) for a, b in zip(params, start))
 
 
+@pytest.mark.parametrize("P,k,bins,code", [(20, 64, 4, 9), (20, 64, 3, 3), (15, 32, 4, 255), (24, 32, 4, 4)])
+def test_outer_step_from_codes_refuses_without_writing(dev, P, k, bins, code):
+    # a code past the quantiser's bins, known only once the update is in flight: nothing is written, in sets of several chunks a
+    # wave, with rows that name an index twice (their chunks are done again on a path of their own)
+    shapes = [(64 * 60, 64 * 60), (64, 64), (64 * 50, 64 * 64), (64 * 7, 64 * 9)]
+    start = [torch.randn(s, device=dev) for s in shapes]
+    params = [s.clone() for s in start]
+    batch = tc.TensorBatch(params)
+    T, n = len(batch), batch.total_chunks
+    gen = torch.Generator(device=dev).manual_seed(P)
+    stage = tc.PayloadStage(batch, k, P, quantized=True)
+    idxs, codes = [], []
+    for p in range(P):
+        i12, c = stage.regions(p)
+        idx = torch.rand((n, 512), device=dev, generator=gen).topk(k, dim=1).indices * 8 + 3
+        idx[p::7, 1] = idx[p::7, 0]
+        i12.copy_(tc.pack_12bit_indices(idx.reshape(-1)))
+        c.copy_(torch.randint(0, bins, c.shape, device=dev, generator=gen, dtype=torch.uint8))
+        idxs.append(i12)
+        codes.append(c)
+    lut = torch.linspace(-1.5, 1.5, bins, device=dev)
+    one = (torch.zeros((), device=dev), 1.0, bins // 2, lut, torch.float32)
+    qps = [[one] * P for _ in range(T)]
+    for tensor, entry in ((0, 0), (T - 1, -1)):
+        flat = codes[P - 1].view(-1)
+        at = batch.offsets[tensor] * k if entry == 0 else n * k - 1
+        kept = flat[at].clone()
+        flat[at] = code
+        for stats in (True, False):
+            with pytest.raises(IndexError):
+                tc.outer_step_codes_batch(batch, idxs, codes, qps, k, 0.4, stats=stats)
+            assert all(torch.equal(a.view(torch.int32), b.view(torch.int32)) for a, b in zip(params, start))
+        flat[at] = kept
+    _, skipped = tc.outer_step_codes_batch(batch, idxs, codes, qps, k, 0.4)
+    assert skipped == [] and not any(torch.equal(a, b) for a, b in zip(params, start))
+
+
 def test_outer_step_seeded_sweep(dev):
     # twenty draws of shapes, peer counts, k, learning rates and layouts, each against the oracle
     rng = np.random.default_rng(2024)
