@@ -281,6 +281,27 @@ def test_decompress_names_the_index_outside_its_row(dev):
         comp.decompress(val, torch.from_numpy(orc.pack12(idx)).to(dev), val, (2, 9), 9)
 
 
+@pytest.mark.parametrize("k", [2, 32, 64])
+def test_scatter_of_rows_flags_an_index_outside_its_row(dev, k):
+    # tplr_decompress_rows by itself: the flag is set where an index lies outside its row, that entry is dropped
+    lib, stream = _lib.load(), ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    rng, n, length = np.random.default_rng(k), 517, 100
+    idx = np.stack([rng.permutation(length)[:k] for _ in range(n)])
+    val = rng.standard_normal((n, k)).astype(np.float32)
+    dv = torch.from_numpy(val).to(dev)
+    for where in (None, (0, 0), (n - 1, k - 1), (200, k // 2)):
+        sent, kept = idx.copy(), val.copy()
+        if where:
+            sent[where], kept[where] = length + 7, 0.0
+        di, out = torch.from_numpy(orc.pack12(sent)).to(dev), torch.full((n, length), 7.0, device=dev)
+        flag = torch.zeros(1, dtype=torch.int32, device=dev)
+        assert lib.tplr_decompress_rows(di.data_ptr(), dv.data_ptr(), n, k, length, out.data_ptr(), flag.data_ptr(), stream) == 0
+        assert bool(flag.item()) == (where is not None)
+        want = np.zeros((n, length), np.float32)
+        np.put_along_axis(want, idx, kept, 1)
+        assert np.array_equal(out.cpu().numpy(), want)
+
+
 def test_decompress_of_many_rows_waits_once_for_the_interpreter(dev):
     # 64 words tell whether the indices lie in their rows.  Beside a busy thread every release of the interpreter may cost a switch
     # interval; the call releases it once for all words, and the rest of it another time at most.
