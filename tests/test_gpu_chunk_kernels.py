@@ -53,18 +53,26 @@ def test_untransformed_sets_of_any_make_up(dev, n, k):
     assert torch.equal(i2, i3) and torch.equal(v2, v3)
 
 
-@pytest.mark.parametrize("k", [32, 64])
-@pytest.mark.parametrize("chunks", [3071, 3073, 6000])  # a round of resident waves, and past it: the launch changes form
-def test_transformed_sets_alike_in_both_forms(dev, chunks, k):
-    gen = torch.Generator(device=dev).manual_seed(chunks)
-    rest = chunks - 2 * 7 * 17
-    x = [torch.randn(s, device=dev, generator=gen) for s in [(64 * 7, 64 * 17), (64, 64 * rest), (64 * 17, 64 * 7)]]
+# Sets with the transform are walked by one resident round of waves up to a chunk for each, and again from five rounds (k <= 32) or
+# twenty on; between, every wave takes one chunk, as all of them do for a single tensor.
+@pytest.mark.parametrize("rounds,over,k", [(1, -1, 32), (1, 1, 32), (1, 0, 64), (2, 0, 64), (5, 0, 32), (5, 1, 32), (5, 1, 34), (7, 5, 32),
+                                           (20, 0, 64), (20, 1, 64)])
+def test_transformed_sets_alike_in_both_forms(dev, rounds, over, k):
+    resident = torch.cuda.get_device_properties(dev).multi_processor_count * 12  # three waves a SIMD
+    chunks = rounds * resident + over
+    rng, gen = np.random.default_rng(chunks), torch.Generator(device=dev).manual_seed(chunks)
+    small = [_sizes(n, rng) for n in (150, 150)]  # of 0 to 4 chunks: a wave's range crosses several
+    rest = chunks - sum(r * c // 4096 for s in small for r, c in s) - 7 * 17
+    shapes = [*small[0], (64 * 7, 64 * 17), (64, 64 * (rest // 2)), *small[1], (64 * (rest - rest // 2), 64)]
+    x = [torch.randn(s, device=dev, generator=gen) for s in shapes]
     batch = tc.TensorBatch(x)
+    assert batch.total_chunks == chunks
     idx, val = tc.encode_compress_batch(batch, k, use_dct=True)
-    for t, one in enumerate(x):  # each tensor by itself takes a chunk per wave
-        si, sv = batch.payload_slice(t, idx, val, k)
-        i1, v1, _, _ = tc.encode_compress(one, k, use_dct=True)
-        assert torch.equal(si, i1) and torch.equal(sv.reshape(-1), v1.reshape(-1))
+    for t, one in enumerate(x):
+        if one.numel():
+            si, sv = batch.payload_slice(t, idx, val, k)
+            i1, v1, _, _ = tc.encode_compress(one, k, use_dct=True)
+            assert torch.equal(si, i1) and torch.equal(sv.reshape(-1), v1.reshape(-1)), t
 
 
 @pytest.mark.parametrize("use_dct", [True, False])
@@ -100,7 +108,7 @@ def _payloads(dev, batch, P, k, rng, repeat):
     return idxs, vals
 
 
-# (the last: two chunks and more for every wave that could be resident at a time)
+# (the last: more chunks than waves that can be resident at a time)
 @pytest.mark.parametrize("shapes,repeat", [([(64, 64)], False), ([(64, 64)], True), ([(0, 64), (128, 192), (64, 64), (64, 320), (0, 64)], False),
                                            ([(0, 64), (128, 192), (64, 64), (64, 320), (0, 64)], True),
                                            ([(2048, 8192), (2048, 320)], False)])
@@ -147,6 +155,46 @@ def test_payloads_with_the_transform(dev, shapes, P, k, repeat):
     assert lib.tplr_outer_step_batch(*lists, ptr(scale), P, k, ptr(batch.table), len(batch), n, None, None, ptr(flags), stream) == 0
     assert flags.cpu().tolist() == [int(t == last) for t in range(len(batch))]
     assert torch.equal(params[last][-64:, -64:], kept[-64:, -64:])
+
+
+def _crowded(dev, n, k, seed, repeat):
+    """A payload of n rows whose entries lie among 256 coefficients of the chunk (so that peers meet in them); `repeat`: every fifth
+    row names one twice."""
+    gen = torch.Generator(device=dev).manual_seed(seed)
+    idx = torch.rand((n, 256), device=dev, generator=gen).topk(k, dim=1).indices * 16 + 5
+    if repeat:
+        idx[::5, k - 1] = idx[::5, 0]
+    return tc.pack_12bit_indices(idx.reshape(-1)), torch.randn((n, k), device=dev, generator=gen)
+
+
+@pytest.mark.parametrize("staged", [False, True])
+@pytest.mark.parametrize("repeat", [False, True])
+@pytest.mark.parametrize("P,k", [(2, 64), (3, 32), (4, 2), (7, 64), (8, 32), (9, 32), (12, 64), (15, 32), (15, 64)])
+def test_aggregates_with_the_transform_alike_in_both_forms(dev, P, k, repeat, staged):
+    # Up to 8192 chunks a wave takes one (k_decode_chunk), beyond resident waves take several in turn (k_decode_aggregate): the same
+    # payload rows give the same bits, chunks on the exact path and chunks that are not finite among them.
+    shapes = [(64 * 40, 64 * 100), (0, 64), (64 * 33, 64 * 64), (64, 64 * 2080)]
+    extra = (64, 64)
+    n = sum(r * c // 4096 for r, c in shapes)
+    assert n == 8192
+    pays = [_crowded(dev, n + 1, k, 10 * P + p, repeat) for p in range(P)]
+    pays[P - 1][1][77, 0], pays[0][1][8000, 1], pays[P // 2][1][4100, 0] = float("nan"), float("inf"), float("-inf")
+    if staged:
+        ib, vb = (torch.stack([p[i].reshape(-1) for p in pays]) for i in (0, 1))
+        pays = [(ib[p], vb[p].view(n + 1, k)) for p in range(P)]
+    scale = torch.rand((len(shapes) + 1, P), device=dev) + 0.5
+    got = []
+    for last in ([], [extra]):
+        out = tc.TensorBatch([torch.full(s, 7.0, device=dev) for s in shapes + last])
+        m = out.total_chunks
+        ss = torch.zeros(m, device=dev)
+        tc.batch_decompress_decode_batch(out, [i[: m * k * 3 // 2] for i, _ in pays], [v[:m] for _, v in pays], k,
+                                         scale=scale[: len(out)].contiguous(), use_dct=True, sumsq=ss)
+        got.append((out.tensors, ss))
+    for a, b in zip(got[0][0], got[1][0]):
+        assert bool(((a.view(torch.int32) == b.view(torch.int32)) | (a.isnan() & b.isnan())).all())
+    a, b = got[0][1], got[1][1][:n]
+    assert bool(((a == b) | (a.isnan() & b.isnan()) | ((a - b).abs() <= 1e-5 * a)).all())
 
 
 @pytest.mark.parametrize("T,P", [(1, 1), (3, 20), (65, 64), (130, 65), (7, 128)])

@@ -52,9 +52,11 @@ def test_whole_set_encode_twice(dev):
         assert torch.equal(snaps[0][0], snaps[1][0]) and torch.equal(snaps[0][1].view(torch.int32), snaps[1][1].view(torch.int32))
 
 
-@pytest.mark.parametrize("P,use_dct", [(15, True), (15, False), (30, True), (30, False), (3, True)])
-def test_aggregate_twice(dev, P, use_dct):
-    shapes = [(2048, 2048), (512, 1024), (64, 64), (3072, 768), (768, 3072)]
+@pytest.mark.parametrize("P,use_dct,large", [(15, True, False), (15, False, False), (30, True, False), (30, False, False), (3, True, False),
+                                             (15, True, True), (3, True, True)])
+def test_aggregate_twice(dev, P, use_dct, large):
+    # (large: more than 8192 chunks, of which a wave takes several)
+    shapes = [(2048, 2048), (512, 1024), (64, 64), (3072, 768), (768, 3072)] + [(4096, 6144)] * large
     grads = [workloads.student_t3(s, 60 + i, row_scale=True, device=dev) for i, s in enumerate(shapes)]
     k = 32
     idxs, vals = _payloads(dev, grads, k, P, use_dct)
@@ -111,8 +113,8 @@ def test_aggregate_does_not_depend_on_what_lds_held(dev, P, k, use_dct):
     from templar_amd import _lib
     lib = _lib.load()
     stream = torch.cuda.current_stream(dev).cuda_stream
-    # (several chunks per wave: a wave's first chunk is scattered serially and never touches those slots)
-    shapes = [(4096, 4096), (2048, 4096), (64, 64)]
+    # (several chunks per wave, which takes more than 8192: a wave's first chunk is scattered serially and never touches those slots)
+    shapes = [(4096, 6144), (2048, 4096), (64, 64)]
     grads = [workloads.student_t3(s, 700 + i, row_scale=True, device=dev) for i, s in enumerate(shapes)]
     idxs, vals = _payloads(dev, grads, k, P, use_dct)
     outs = [torch.empty_like(g) for g in grads]

@@ -161,13 +161,15 @@ def test_staged_window_gives_the_same_bits_as_separate_payloads(dev, P, k, use_d
 
 
 @pytest.mark.parametrize("P,k,use_dct,window", [(15, 32, True, False), (15, 32, True, True), (15, 32, False, False),
-                                                (15, 32, False, True), (20, 64, True, True), (31, 32, True, False)])
+                                                (15, 32, False, True), (20, 64, True, True), (31, 32, True, False),
+                                                (4, 64, True, False), (8, 32, True, True), (9, 32, True, False)])
 def test_whole_set_aggregate_with_repeats_in_some_rows(dev, P, k, use_dct, window):
-    # enough chunks that every wave walks several, a repeat planted in every 5th row: marked rows in the
-    # middle of a wave's range, at its first and at its last chunk; the other rows go the fast way
-    shapes = [(64 * 70, 64 * 48), (64 * 33, 64 * 64), (64, 64), (64 * 50, 64 * 40)]
+    # enough chunks that every wave walks several (more than 8192: up to there a wave takes one), a repeat planted in every
+    # 5th row: marked rows in the middle of a wave's range, at its first and at its last chunk; the other rows go the fast way
+    shapes = [(64 * 70, 64 * 60), (64 * 33, 64 * 64), (64, 64), (64 * 50, 64 * 40)]
     counts = [(s[0] // 64) * (s[1] // 64) for s in shapes]
     n = sum(counts)
+    assert n > 8192
     idxs, vals = peers_with_repeats(P, 1, n, k, 77 + P + k, every=5)
     di, dv = on_device(idxs, vals, dev)
     if window:
