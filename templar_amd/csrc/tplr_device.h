@@ -431,16 +431,18 @@ __device__ __forceinline__ void exact_masks(const float (&v)[64], uint32_t t, ui
     ehi = ge[0] & ~g[0], elo = ge[1] & ~g[1];
 }
 
-// How many of the chunk's keys are at least c?  The sign of c - 1 - |x| says it of one of them; three instructions each and no
-// comparison, whose results the scheduler would gather by the dozen in scalar registers.  Without transform, k = 128, a chunk of
-// noise in this search: one 2048 x 2048 tensor 30.0 us, with comparisons and the magnitudes kept over the passes 56.5 (spilled) at four
-// waves per SIMD, 35.4 at three; one of 0.5 % values other than zero, k = 32 38.7 : 66 : 46.  (Inlined on purpose: a call would force
-// the register-resident chunk through scratch memory.)
+// How many of the chunk's keys are at least c?  The sign of c - 1 - |x| says it of one of them; no comparison, whose results the
+// scheduler would gather by the dozen in scalar registers.  In a caller's loop the optimiser forms the 64 magnitudes once, ahead of
+// it, and keeps them in 64 registers more; without kSpare they are formed anew each time.  Without transform (four waves per SIMD,
+// 128 registers), k = 128, a chunk of noise in this search: one 2048 x 2048 tensor 30.0 us, with the magnitudes kept and comparisons
+// 56.5 (spilled), at three waves per SIMD 35.4; one of 0.5 % values other than zero, k = 32 38.7 : 66 : 46.  With registers to spare
+// keeping them is faster: 4000 rows of 4096 with 0.5 %, k = 32, 62 against 73.  (Inlined on purpose: a call would force the
+// register-resident chunk through scratch memory.)
+template <bool kSpare>
 __device__ __forceinline__ uint32_t count_ge(const float (&v)[64], uint32_t c) {
     const uint32_t below = (c < 0x7f800001u ? c : 0x7f800001u) - 1u;  // (past the infinity there are only NaNs, all alike)
-    // (a copy as above, for a caller's loop)
     uint32_t magnitude = 0x7fffffffu;
-    asm volatile("" : "+s"(magnitude));
+    if constexpr (!kSpare) asm volatile("" : "+s"(magnitude));
     uint32_t m0 = 0, m1 = 0;
 #pragma unroll
     for (int d = 0; d < 32; ++d) {
@@ -671,7 +673,7 @@ __device__ __forceinline__ void sort128_desc_u32(uint32_t& e0, uint32_t& e1) {
 // kOther: `o1`, `o2` are a second set of lane statistics of the same chunk, e.g. taken over the
 // columns: data whose rows differ in scale put most candidates into a few lanes and one direction
 // alone passes far too many of them; the threshold is then the larger of the two directions'.
-template <bool kTwo, bool kOther = false>
+template <bool kTwo, bool kOther = false, bool kSpare = true>
 __device__ __forceinline__ Selected select_topk(const float (&w)[64], float* buf, uint64_t* cand, int lane, int k,
                                                 float out_scale, uint32_t o1 = 0, uint32_t o2 = 0) {
     uint32_t mhi = 0, mlo = 0, cnt = 0, incl = 0, total = 0;
@@ -692,7 +694,7 @@ __device__ __forceinline__ Selected select_topk(const float (&w)[64], float* buf
             // Exact search for the k-th largest key, from the bits t0 and the maximum share.
             const uint32_t vmax = wave_max_u32(kTwo ? (mag_key(b1) > mag_key(b2) ? mag_key(b1) : mag_key(b2)) : mag_key(b1));
             uint32_t t = mag_key(t0);
-            uint32_t n_ge = count_ge(w, t);
+            uint32_t n_ge = count_ge<kSpare>(w, t);
             if (n_ge > static_cast<uint32_t>(kCandCap)) {
                 const uint32_t diff = t ^ vmax;
                 const int top = diff ? 31 - __builtin_clz(diff) : -1;
@@ -700,7 +702,7 @@ __device__ __forceinline__ Selected select_topk(const float (&w)[64], float* buf
 #pragma nounroll
                 for (int bit = top; bit >= 0; --bit) {
                     const uint32_t c = t | (1u << bit);
-                    const uint32_t n = count_ge(w, c);
+                    const uint32_t n = count_ge<kSpare>(w, c);
                     if (n >= static_cast<uint32_t>(k)) {
                         t = c;
                         n_ge = n;

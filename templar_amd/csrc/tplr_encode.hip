@@ -134,7 +134,7 @@ __global__ __launch_bounds__((64 * encode_team<kUseDct, kEf>()), kUseDct || kEf 
 #else
     chunk_forward<kUseDct>(v, w, buf, lane);
 #endif
-    const Selected s = select_topk<kTwo, !kUseDct>(w, buf, cand, lane, k, kUseDct ? kDctPow2Scale : 1.0f, c1, c2);
+    const Selected s = select_topk<kTwo, !kUseDct, kUseDct || kEf>(w, buf, cand, lane, k, kUseDct ? kDctPow2Scale : 1.0f, c1, c2);
     emit_selected<kTwo>(s, lane, k, g, idx12, val);
 }
 
