@@ -53,8 +53,26 @@ SETS = {
     "nodct": dict(args=["--no-dct"], workload="cfg3_llama1b", chunks=294144, k=32, P=15, dct=False, name="cfg3_llama1b_no_transform",
                   what="the 1B gradient set, k = 32, chunks not transformed", phases=["encode", "aggregate"]),
 }
-COUNTED = {"copy", "encode", "aggregate", "calib", "outer"}   # phases whose HBM traffic is counted
-WITH_SQ = {"encode", "aggregate"}
+COUNTED = {"copy", "encode", "aggregate", "calib", "outer", "miner"}   # phases whose HBM traffic is counted
+WITH_SQ = {"encode", "aggregate", "outer", "miner"}
+
+
+def kernel_of(S, phase):
+    """The kernel that a phase of a set is about, as its name stands in a trace; the tests hold these against the library."""
+    two, dct = ("true" if f else "false" for f in (S["k"] > 32, S["dct"]))
+    if phase == "encode":  # (a set of this size: walked by resident waves with the transform, a chunk per wave without it)
+        return f"k_encode_topk_pack<{two}>" if S["dct"] else f"k_encode_chunk<{two}, false, false>"
+    if phase == "aggregate":
+        units, bits = (8, 4) if S["P"] <= 8 else (16, 4) if S["P"] <= 15 else (24, 5)
+        return f"k_decode_aggregate<{dct}, {units}, {bits}, false, true, false, 0>"
+    return {"outer": f"k_decode_chunk<{S['P']}, true>", "read": "k_calib_encode", "calib": "k_calib_aggregate",
+            "fill": "k_calib_aggregate", "copy": "k_calib_copy", "linfill": "k_calib_fill<0>", "miner": MINER[0][0]}[phase]
+
+
+# the miner step's launches: kernel, what it does, bytes per chunk, waves a SIMD
+MINER = (("k_ef_step<false>", "the whole step in one launch (no quantiser between its halves)", 3 * 16384 + 176, 2),
+         ("k_encode_chunk<false, true, true>", "update + encode", 3 * 16384 + 176, 3),
+         ("k_decode_chunk<1, true>", "subtract decoded", 2 * 16384 + 176, 3))
 # the measurement build with half of the forward transform on the matrix cores (`TPLR_BUILD_MATRIX_VARIANT=1` makes
 # __graft_entry__.build() write it beside the product library): the set `matrix` profiles its encode launch
 MATRIX_LIB = os.path.join(ROOT, "templar_amd", "libtplr_hip_matrix_variant.so")
@@ -159,6 +177,8 @@ def _stats_table(tag, also=None):
 
 def _trace(tag, kern):
     rows = [r for r in csv.DictReader(open(_csv(tag, "kt", "*kernel_trace.csv"))) if kern in r["Kernel_Name"]]
+    if not rows and "FillFunctor" not in kern:
+        sys.exit(f"no launch of {kern} in the trace of {tag}")
     rows.sort(key=lambda r: int(r["Start_Timestamp"]))
     dur = [(int(r["End_Timestamp"]) - int(r["Start_Timestamp"])) / 1e3 for r in rows]
     return rows, dur
@@ -292,17 +312,15 @@ k_decode_aggregate_cfg3_llama1b_15peers.md (`--profile fill`), beside the launch
 
     for tag, S in SETS.items():
         n, k, Pn, a = S["chunks"], S["k"], S["P"], S["args"]
-        two = "true" if k > 32 else "false"
-        dct = "true" if S["dct"] else "false"
         # ---------------- encode
         if _have(f"{tag}_encode"):
-            kern = f"k_encode_topk_pack<{two}, {dct}, false>"
+            kern = kernel_of(S, "encode")
             tr, dur = _trace(f"{tag}_encode", kern)
             t50 = dur[-50:]
             avg = sum(t50) / len(t50)
             alg_r, alg_w = n * 16384, n * 11 * k // 2
             alg = alg_r + alg_w
-            text = f"""# {_short(tr[-1]['Kernel_Name'])}: {S['what']}, one persistent launch
+            text = f"""# {_short(tr[-1]['Kernel_Name'])}: {S['what']}, one launch ({'resident waves on ranges of the chunk list' if S['dct'] else 'a chunk per short-lived wave'})
 
 ## Kernel trace
 
@@ -343,7 +361,7 @@ Total HBM traffic per launch {fb + wb:,.0f} B = {(fb + wb) / alg:.3f} x the algo
 
 {_cmd(tag, 'encode', 'SQ', a)}
 
-{_sq(f'{tag}_encode', kern, n, 3, 'The kernel issues no matrix-core instruction: the 64-point transform is generated vector code.')}
+{_sq(f'{tag}_encode', kern, n, 3 if S['dct'] else 4, 'The kernel issues no matrix-core instruction: the 64-point transform is generated vector code.')}
 """
             if _have(f"{tag}_read"):
                 _, rd = _trace(f"{tag}_read", "k_calib_encode")
@@ -352,8 +370,8 @@ Total HBM traffic per launch {fb + wb:,.0f} B = {(fb + wb) / alg:.3f} x the algo
                 text += f"""
 ## The memory side alone
 
-`k_calib_encode` (`tplr_calib_encode`) runs the same grid over the same chunk ranges and issues the same 64 streaming row
-loads per chunk, and nothing else.
+`k_calib_encode` (`tplr_calib_encode`) issues the 64 streaming row loads of every chunk, and nothing else, from resident waves on
+ranges of the chunk list.
 
 {_cmd(tag, 'read', 'kt', a)}
 
@@ -366,9 +384,7 @@ The encode launch takes {avg / ravg:.2f} x its memory-only form.
             write(f"k_encode_topk_pack_{S['name']}.md", text)
         # ---------------- aggregate
         if _have(f"{tag}_aggregate"):
-            units = 8 if Pn <= 8 else 16 if Pn <= 15 else 24
-            bits = 4 if Pn <= 15 else 5
-            kern = f"k_decode_aggregate<{dct}, {units}, {bits}, false, true, false, 0>"
+            kern = kernel_of(S, "aggregate")
             tr, dur = _trace(f"{tag}_aggregate", kern)
             t50 = dur[-50:]
             avg = sum(t50) / len(t50)
@@ -381,7 +397,7 @@ The encode launch takes {avg / ravg:.2f} x its memory-only form.
 {_cmd(tag, 'aggregate', 'kt', a)}
 
 ({note}; a step of this phase is the whole aggregate pass: the clip factors from the row figures noted on arrival, the
-fused launch, the norm vectors.)  `p_kernel_stats.csv`, rows of this library's kernels (the {Pn} `k_encode_topk_pack`
+fused launch, the norm vectors.)  `p_kernel_stats.csv`, rows of this library's kernels (the {Pn} encode
 launches build the peers' payloads):
 
 {_stats_table(f'{tag}_aggregate')}
@@ -449,7 +465,7 @@ kernel runs at **{cavg / avg * 100:.1f} %** of its own memory-only form ({avg / 
             write(f"k_decode_aggregate_{S['name']}_{Pn}peers.md", text)
         # ---------------- outer step
         if _have(f"{tag}_outer"):
-            kern = "k_decode_aggregate<true, 16, 4, true, true, false, 0>"
+            kern = kernel_of(S, "outer")
             tr, dur = _trace(f"{tag}_outer", kern)
             t50 = dur[-50:]
             avg = sum(t50) / len(t50)
@@ -478,21 +494,34 @@ HBM traffic by the counters ({nf} dispatches; FETCH_SIZE {f:.1f}, WRITE_SIZE {w:
 {_cmd(tag, 'outer', 'FETCH_SIZE', a)}
 {_cmd(tag, 'outer', 'WRITE_SIZE', a)}
 """
+            if _have(f"{tag}_outer", "SQ"):
+                text += f"""
+{_cmd(tag, 'outer', 'SQ', a)}
+
+{_sq(f'{tag}_outer', kern, n, 3, 'No matrix-core instruction is issued.')}
+"""
             write(f"k_outer_step_{S['name']}_{Pn}peers.md", text)
 
     # ---- miner step
     if _have("cfg3_miner"):
         rows = []
-        for kern, label, b in (("k_ef_step<false>", "the whole step in one launch (no quantiser between its halves)", 294144 * (3 * 16384 + 176)),
-                               ("k_encode_topk_pack<false, true, true>", "update + encode", 294144 * (3 * 16384 + 176)),
-                               ("k_decode_aggregate<true, 8, 4, true, true, false, 0>", "subtract decoded", 294144 * (2 * 16384 + 176))):
-            _, dur = _trace("cfg3_miner", kern)
-            if not dur:
-                continue
+        more = ""
+        n = SETS["cfg3"]["chunks"]
+        for kern, label, per_chunk, waves in MINER:
+            b = n * per_chunk
+            tr, dur = _trace("cfg3_miner", kern)
             t = dur[-50:]
             us = sum(t) / len(t)
             rows.append(f"| `{kern}` | {label} | {len(dur)} | {us:.1f} | {min(t):.1f} | {b:,} | {b / us / 1e3:.0f} | {b / us / 1e3 / 80:.1f} % |")
-        write("error_feedback_step_cfg3_llama1b.md", f"""# Miner-side error-feedback step on the 1B gradient set (294 144 chunks, k=32): one persistent launch, or two where a quantiser sits between its halves
+            more += f"\n## `{kern}`\n\nLaunch geometry: {_geometry(tr[-1])}.\n"
+            c = counted("cfg3_miner", kern)
+            if c:
+                f, nf, fb, w, nw, wb = c
+                more += (f"\nHBM traffic by the counters ({nf} dispatches; FETCH_SIZE {f:.1f}, WRITE_SIZE {w:.1f}, scaled as in "
+                         f"k_calib_copy_1GiB.md):\n{fb:,.0f} B read + {wb:,.0f} B written = {(fb + wb) / b:.3f} x the algorithmic bytes.\n")
+            if _have("cfg3_miner", "SQ"):
+                more += "\n" + _sq("cfg3_miner", kern, n, waves, "No matrix-core instruction is issued.") + "\n"
+        write("error_feedback_step_cfg3_llama1b.md", f"""# Miner-side error-feedback step on the 1B gradient set (294 144 chunks, k=32): one launch, or two where a quantiser sits between its halves
 
 {_cmd('cfg3', 'miner', 'kt', [])}
 
@@ -505,7 +534,13 @@ From `p_kernel_trace.csv` (the last 50 launches of each kernel):
 | kernel | step | launches in the trace | avg us | min us | algorithmic bytes | GB/s | of 8 TB/s |
 |---|---|---|---|---|---|---|---|
 {chr(10).join(rows)}
-""")
+
+Counters:
+
+{_cmd('cfg3', 'miner', 'FETCH_SIZE', [])}
+{_cmd('cfg3', 'miner', 'WRITE_SIZE', [])}
+{_cmd('cfg3', 'miner', 'SQ', [])}
+{more}""")
     if _have("bench_default"):
         write("bench_default_cfg3_llama1b.md", f"""# bench.py (default arguments), 1B gradient set: all kernels of this library
 
@@ -520,7 +555,7 @@ k_decode_aggregate_cfg3_llama1b_15peers.md):
 """)
     # ---------------- the measurement build with half of the forward transform on the matrix cores
     if _have("matrix_encode") and _have("matrix_encode", "MFMA") and _have("cfg3_encode", "MFMA") and _have("cfg3_encode"):
-        kern = "k_encode_topk_pack<false, true, false>"
+        kern = kernel_of(SETS["cfg3"], "encode")
         n = SETS["cfg3"]["chunks"]
         alg = n * 16384 + n * 11 * 32 // 2
         tr, dur = _trace("matrix_encode", kern)

@@ -4,8 +4,11 @@ Untransformed gradients often hold more candidates than the select has slots for
 that then runs over a chunk's 64 registers a lane makes up to thirty passes: with some of them spilled it took 1.1 to 1.6 times
 as long."""
 import struct
+import subprocess
 
 import pytest
+
+import bench_profiles
 
 from templar_amd import _lib
 
@@ -52,3 +55,11 @@ def test_selects_keep_their_chunk_in_registers(kernel, count):
     assert len(found) >= count, sorted(found)
     for name, k in found.items():
         assert k[".private_segment_fixed_size"] == 0 and k[".vgpr_spill_count"] == 0, (name, k)
+
+
+def test_profiled_kernels_are_in_the_library():
+    names = subprocess.run(["c++filt"], input="\n".join(_kernels()), capture_output=True, text=True, check=True).stdout.splitlines()
+    asked = [bench_profiles.kernel_of(S, phase) for S in bench_profiles.SETS.values() for phase in S["phases"]]
+    asked += [m[0] for m in bench_profiles.MINER]
+    for kernel in set(asked):
+        assert any(f"tplr::{kernel}" in n for n in names), kernel
