@@ -3412,7 +3412,8 @@ int tplr_row_sumsq(const float* const* h_val, int n_peers, int k, int64_t n_rows
     const int rows_per_trip = vec ? 256 / w : 64 / w;
     const int64_t trips = (n_rows + rows_per_trip - 1) / rows_per_trip;
     // a wave takes eight trips per round, and workgroups that come and go overlap one round's reduction with the others' loads:
-    // 15 peers of 294 144 rows of 32 in one resident round (2048 workgroups) 111 us, in up to eight 96 (5.9 TB/s), without a cap 98
+    // 15 peers of 294 144 rows of 32 in one resident round (2048 workgroups) 111 us, in up to eight 96 (5.9 TB/s), without a cap 98; of
+    // 64 213 : 191, of 30 337 : 206, 65 536 rows of 32 21.8 : 18.8, of 64 49.5 : 42.4; one peer's 294 144 of 64 16.9 : 17.7, of 128 52.2 : 54.6
     int64_t blocks = (trips + 31) / 32;
     const int64_t cap = (16384 + n_peers - 1) / n_peers;
     blocks = blocks < 1 ? 1 : blocks > cap ? cap : blocks;
