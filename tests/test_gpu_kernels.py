@@ -583,7 +583,7 @@ def test_calibration_copy(dev):
 
 # ---------------------------------------------------------------- persistent loops and batches
 def test_persistent_encode_many_chunks_per_wave(dev):
-    # 4608 chunks: more than one resident set of waves, so every wave walks several chunks
+    # 4608 chunks: more than one resident set of waves
     x = t3((4608, 4096), 2024, row_scale=True).to(dev)
     idx_f, val_f, xshape, _ = tc.encode_compress(x, 32)
     tr = tc.ChunkingTransformer(_Stub([x]), 64)
